@@ -153,6 +153,35 @@ def test_mfma_weight_gradients(width):
         np.testing.assert_allclose(host(db), rdb, rtol=0, atol=1e-5 * np.abs(rdb).max())
 
 
+@pytest.mark.parametrize("width", [32, 64])
+@pytest.mark.parametrize("shape", [(1, 1, 1), (1, 4, 64), (1, 9, 65), (3, 8, 63), (2, 17, 130), (15, 45, 150)])
+def test_weight_gradient_strips_and_stretches(shape, width):
+    """The weight-gradient kernels walk 64-column strips in passes of 4 or 8
+    rows, cut into at most 256 stretches: images smaller than a pass, a
+    column past a strip, rows past a pass, and (the last shape) more passes
+    than stretches for every kind, so that stretches start and end inside
+    strips.  Tolerance: FP32 accumulation over P pixels in chains of at most
+    P / 32 + 256 additions errs by about 6e-8 sqrt(P / 32 + 256) of a partial
+    sum that itself is of the size of the largest entry, below 1e-5 here."""
+    rng = np.random.default_rng(13)
+    n, h, w = shape
+    s = C.c_void_p(0)
+    f, W = (W64 if width == 64 else 0), width
+    for kind, kx, my, mrows in [(5 | f, 8, W, W), (6 | f, W, W, W), (7 | f, W, 8, 16)]:
+        x = rand_bf16(rng, (n, h, w, kx))
+        dy = rand_bf16(rng, (n, h, w, my))
+        dw = torch.full((9 * mrows * kx,), 7.0, dtype=torch.float32, device="cuda")
+        db = torch.zeros(my, dtype=torch.float32, device="cuda")
+        nws = lib().tsu_nn_wgrad_workspace(kind)
+        ws = torch.full((nws,), float("nan"), dtype=torch.float32, device="cuda")
+        ok(lib().tsu_nn_wgrad(kind, P(dev_bf16(x)), P(dev_bf16(dy)), P(dw), P(db), mrows, n, h, w, P(ws), nws, s))
+        rdw, rdb = O.conv_weight_grad(x, dy)
+        got = host(dw).reshape(9, mrows, kx)
+        np.testing.assert_allclose(got[:, :my, :], rdw, rtol=0, atol=1e-5 * np.abs(rdw).max())
+        assert np.all(got[:, my:, :] == 7.0)
+        np.testing.assert_allclose(host(db), rdb, rtol=0, atol=1e-5 * np.abs(rdb).max())
+
+
 def test_wide_conv_workgroups_loop_over_tiles():
     """The 64-channel kernels keep one workgroup per CU and loop over 8 x 64
     pixel tiles (prefetching the next one): an image set with more than

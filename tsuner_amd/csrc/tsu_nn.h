@@ -20,7 +20,8 @@ enum NnKind {
     NN_W64 = 16,        // flag: hidden width 64 (8 -> 64 -> ... -> 64 -> 4)
 };
 
-// Waves of the weight-gradient contraction (partial sums per wave).
+// Most workgroups of a weight-gradient contraction, each of which leaves one
+// set of partial sums (fewer when there are fewer passes).
 constexpr int kWgradWaves = 256;
 
 // Fine cells deeper than this count as wet when a 4x4 block is restricted

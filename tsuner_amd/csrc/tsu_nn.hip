@@ -384,128 +384,514 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
 }
 
-// Weight gradient of out = conv(x, w): dW[t][m][k] = sum_p dy[p][m] x[p + off(t)][k],
-// contracted over pixels on the MFMA K axis (32 pixels per MFMA: four runs of
-// 8 consecutive columns of one row).  Grid: (WAVES/4, 9 taps); wave w of tap t
-// takes rows w, w + WAVES, ... and writes its partial sums to
-// part[t][w][MY][KX]; the centre tap also writes column sums of dy (the bias
-// gradient) to bpart[w][MY].  The reduction kernel adds the partials in a
-// fixed order, so the result is deterministic.
-template <int KX, int MY>
-__global__ __launch_bounds__(256) void wgrad_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ dy,
-                                                    float* __restrict__ part, float* __restrict__ bpart, int N, int H,
-                                                    int W, int waves)
-{
-    constexpr int MT = (MY + 15) / 16, NT = (KX + 15) / 16;
-    const int lane = threadIdx.x & 63;
-    const int w = blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int t = blockIdx.y;
-    if (w >= waves) return;
-    const int g = lane >> 4, li = lane & 15;
-    const int ty = tap_dy(t), tx = tap_dx(t);
-    f32x4 acc[MT][NT];
-#pragma unroll
-    for (int a = 0; a < MT; a++)
-#pragma unroll
-        for (int b = 0; b < NT; b++) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float bsum[MT];
-#pragma unroll
-    for (int a = 0; a < MT; a++) bsum[a] = 0.f;
+// ---- weight gradients --------------------------------------------------------
+//
+// dW[t][m][k] = sum_p dy[p][m] x[p + off(t)][k], contracted over pixels on the
+// MFMA K axis (32 pixels of one row per MFMA).  Both operands lie in memory
+// with the channel fastest while an MFMA operand wants eight pixels of one
+// channel per lane, so the rows are staged in LDS and read with the
+// transposing ds_read_b64_tr_b16: a group of 16 lanes reads four pixels x 16
+// channels and each lane gets the four pixels of its channel.  (Gathering
+// the operands with 2-byte global loads, one tap per workgroup, took 220 us
+// for 64 -> 64 channels over 8 images of 256^2 and 109 us for 32 -> 32: nine
+// passes over both tensors at two bytes a load.)
+//
+// A workgroup walks down a strip of 64 columns, R rows per pass: the rows of
+// the shifted operand stay in an LDS ring, so that every row is loaded once
+// per strip (plus two at the top of a stretch), and the next rows are loaded
+// into registers while the MFMAs run on the current ones.  The passes of all
+// strips of all images, in order, are cut into one contiguous stretch per
+// workgroup; one workgroup per CU fits (its rings take most of the LDS) and
+// kWgradWaves = 256 of them cover the chip.
+//
+// Measured, 8 images of 256^2, before and now (gradient + reduction):
+//   64 -> 64  220 + 112 us -> 57 + 11 us (680 TFLOP/s; both tensors once are
+//             134 MB, 22 us at the copy kernel's 6.1 TB/s, the MFMAs 15 us at
+//             peak, the transposing reads 17 us of LDS time)
+//   32 -> 32  109 + 110 us -> 24 + 5 us (67 MB, 11 us)
+//   8 -> 64, 64 -> 4   145 and 118 + 112 us -> 21 + 5 us (76 MB, 12 us)
+//   8 -> 32, 32 -> 4    84 and 82 + 110 us -> 13 + 4 us (42 MB, 7 us)
+//
+// Pixels: columns are pitched so that a row is a multiple of 8 pixels, and
+// the 32-byte slots of a pixel (16 channels, what one transposing read takes)
+// are XOR-ed with bits of its column: the 8 consecutive columns that half a
+// wave reads then lie in different banks.  The eight pixels of lane group g
+// in a 32-pixel step are 4g .. 4g+3 and 16+4g .. 16+4g+3, for both operands.
 
-    const long long rows = (long long)N * H;
-    for (long long row = w; row < rows; row += waves) {
-        const int r = (int)(row % H);
-        const int rr = r + ty;
-        const bool rv = rr >= 0 && rr < H;
-        for (int c0 = 0; c0 < W; c0 += 32) {
-            const int cb = c0 + 8 * g;          // this lane's 8 pixels: columns cb .. cb + 7
-            bf16x8 A[MT], B[NT];
+constexpr int kWgradCols = 64;             // columns of a strip
+constexpr int kWgradPitch = 72;            // LDS columns of the shifted operand's rows (66 used)
+
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+typedef __attribute__((address_space(3))) uint4 lds_u4;
+
+// eight pixels of one channel: the transposing reads at byte addresses a and b
+__device__ __forceinline__ bf16x8 read_tr8(uint32_t a, uint32_t b)
+{
+    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uintptr_t)a);
+    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uintptr_t)b);
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
+// XOR of a pixel's 32-byte slots at column c: 64 channels have 4 slots and 2
+// pixels per 256 bytes (all banks once), 32 channels 2 slots and 4 pixels.
+template <int CH>
+__device__ __forceinline__ int slot_xor(int c)
+{
+    return CH == 64 ? (c >> 1) & 3 : CH == 32 ? (c >> 2) & 1 : 0;
+}
+
+// The passes of one workgroup: strip pass i of column (n, seg) starts at row
+// R * (i % passes).
+struct WgradWalk {
+    long long first, last;      // passes [first, last)
+    int segs, passes;           // strips per image, passes per strip
+    int H, W;
+    __device__ WgradWalk(int N, int H_, int W_, int R) : H(H_), W(W_)
+    {
+        segs = (W + kWgradCols - 1) / kWgradCols;
+        passes = (H + R - 1) / R;
+        const long long total = (long long)N * segs * passes;
+        first = total * blockIdx.x / gridDim.x;
+        last = total * (blockIdx.x + 1) / gridDim.x;
+    }
+    __device__ void at(long long i, int R, int& n, int& c0, int& r0) const
+    {
+        r0 = (int)(i % passes) * R;
+        i /= passes;
+        c0 = (int)(i % segs) * kWgradCols;
+        n = (int)(i / segs);
+    }
+};
+
+// Middle layers (x and dy of CH = 32 or 64 channels).  Each of 8 waves holds
+// the nine taps of 32 x 32 channels (CH = 64: four such jobs, two waves of a
+// job taking half of a pass's pixels each; CH = 32: one job, eight waves),
+// and the waves of a job add their sums through LDS at the end.  Partial sums
+// go to part[t][workgroup][m][k], the bias gradient (one MFMA per dy tile
+// against ones, in the jobs of the first 32 input channels) to
+// bpart[workgroup][m].
+template <int CH>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void wgrad_mid_kernel(
+    const uint16_t* __restrict__ x, const uint16_t* __restrict__ dy, float* __restrict__ part,
+    float* __restrict__ bpart, int N, int H, int W)
+{
+    constexpr int R = 4;                           // rows per pass
+    constexpr int KO = CH / 8, PIX = CH * 2;
+    constexpr int XR = 2 * R + 2, DR = 2 * R;      // ring rows: R + 2 in use and R coming, R and R
+    constexpr int XROW = kWgradPitch * PIX, DROW = kWgradCols * PIX;
+    constexpr int JOBS = (CH / 32) * (CH / 32), GROUPS = 8 / JOBS;
+    constexpr int STEPS = 2 * R / GROUPS;          // 32-pixel steps of a wave per pass
+    constexpr int XPT = (R * 66 * KO + 511) / 512, DPT = R * 64 * KO / 512;
+    constexpr int XN = XR * XROW / 16, DN = DR * DROW / 16;
+    constexpr int TILES = 38;                      // accumulator tiles of a wave, bias included
+    constexpr int RED = 4 * TILES * 64;            // those of half of the waves
+    constexpr int LDS = XN + DN > RED ? XN + DN : RED;
+    __shared__ uint4 lds[LDS];
+    const uint32_t xbase = (uint32_t)(uintptr_t)(lds_u4*)lds, dbase = xbase + XN * 16;
+    const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int g = lane >> 4, li = lane & 15;
+    const int job = wv % JOBS, group = wv / JOBS;
+    const int m0 = 2 * (job / (CH / 32)), k0 = 2 * (job % (CH / 32));   // first 16-channel tiles
+    const WgradWalk walk(N, H, W, R);
+
+    f32x4 acc[TILES];                              // [tap][k tile][m tile], then the bias of the m tiles
 #pragma unroll
-            for (int a = 0; a < MT; a++) {
-                const int m = a * 16 + li;
-                uint16_t v[8];
+    for (int v = 0; v < TILES; v++) acc[v] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const uint32_t one2 = 0x3F803F80u;
+    const bf16x8 ones = as_bf16x8(make_uint4(one2, one2, one2, one2));
+
+    // lane addresses within a row: pixel 4g + (li >> 2), 8-byte chunk li & 3
+    const int px = 4 * g + (li >> 2), chunk = (li & 3) * 8;
+    uint32_t xa[3][2], da[2];
 #pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    const int c = cb + j;
-                    v[j] = (m < MY && c < W) ? dy[((size_t)row * W + c) * MY + m] : (uint16_t)0;
-                }
-                uint4 u;
-                u.x = v[0] | ((uint32_t)v[1] << 16);
-                u.y = v[2] | ((uint32_t)v[3] << 16);
-                u.z = v[4] | ((uint32_t)v[5] << 16);
-                u.w = v[6] | ((uint32_t)v[7] << 16);
-                A[a] = as_bf16x8(u);
-                if (t == 4) {
+    for (int d = 0; d < 3; d++)
 #pragma unroll
-                    for (int j = 0; j < 8; j++) bsum[a] += from_bf16(v[j]);
-                }
+        for (int b = 0; b < 2; b++)
+            xa[d][b] = xbase + (px + d) * PIX + (((k0 + b) ^ slot_xor<CH>(px + d)) * 32) + chunk;
+#pragma unroll
+    for (int a = 0; a < 2; a++) da[a] = dbase + px * PIX + (((m0 + a) ^ slot_xor<CH>(px)) * 32) + chunk;
+
+    uint4 sx[XPT], sd[DPT];
+    // x rows r0 + 1 .. r0 + R (columns c0 - 1 .. c0 + 64) and dy rows
+    // r0 .. r0 + R - 1 of image n into registers, zeros outside the image
+    auto fetch = [&](int n, int c0, int r0) {
+#pragma unroll
+        for (int j = 0; j < XPT; j++) {
+            const int idx = tid + 512 * j;
+            const int q = idx % KO, c = (idx / KO) % 66, i = idx / (KO * 66);
+            const int gr = r0 + 1 + i, gc = c0 - 1 + c;
+            sx[j] = make_uint4(0, 0, 0, 0);
+            if (i < R && gr < H && gc >= 0 && gc < W)
+                sx[j] = *(const uint4*)(x + (((size_t)n * H + gr) * W + gc) * CH + 8 * q);
+        }
+#pragma unroll
+        for (int j = 0; j < DPT; j++) {
+            const int idx = tid + 512 * j;
+            const int q = idx % KO, c = (idx / KO) % 64, i = idx / (KO * 64);
+            const int gr = r0 + i, gc = c0 + c;
+            sd[j] = make_uint4(0, 0, 0, 0);
+            if (gr < H && gc < W) sd[j] = *(const uint4*)(dy + (((size_t)n * H + gr) * W + gc) * CH + 8 * q);
+        }
+    };
+    // the fetched rows into ring rows xs + 2, ... and ds, ...
+    auto put = [&](int xs, int ds) {
+#pragma unroll
+        for (int j = 0; j < XPT; j++) {
+            const int idx = tid + 512 * j;
+            const int q = idx % KO, c = (idx / KO) % 66, i = idx / (KO * 66);
+            int s = xs + 2 + i;
+            s = s >= XR ? s - XR : s;
+            if (i < R)
+                lds[(s * XROW + c * PIX) / 16 + (((q >> 1) ^ slot_xor<CH>(c)) * 2 + (q & 1))] = sx[j];
+        }
+#pragma unroll
+        for (int j = 0; j < DPT; j++) {
+            const int idx = tid + 512 * j;
+            const int q = idx % KO, c = (idx / KO) % 64, i = idx / (KO * 64);
+            lds[XN + ((ds + i) * DROW + c * PIX) / 16 + (((q >> 1) ^ slot_xor<CH>(c)) * 2 + (q & 1))] = sd[j];
+        }
+    };
+
+    // at the top of a stretch or strip: x rows r0 - 1 and r0 into ring rows 0, 1
+    auto top = [&](int n, int c0, int r0) {
+        for (int idx = tid; idx < 2 * 66 * KO; idx += 512) {
+            const int q = idx % KO, c = (idx / KO) % 66, i = idx / (KO * 66);
+            const int gr = r0 - 1 + i, gc = c0 - 1 + c;
+            uint4 v = make_uint4(0, 0, 0, 0);
+            if (gr >= 0 && gr < H && gc >= 0 && gc < W)
+                v = *(const uint4*)(x + (((size_t)n * H + gr) * W + gc) * CH + 8 * q);
+            lds[(i * XROW + c * PIX) / 16 + (((q >> 1) ^ slot_xor<CH>(c)) * 2 + (q & 1))] = v;
+        }
+    };
+
+    // ring row of x row r0 - 1 and of dy row r0
+    int xs = 0, ds = 0;
+    int n, c0, r0;
+    walk.at(walk.first, R, n, c0, r0);
+    fetch(n, c0, r0);
+    top(n, c0, r0);
+    put(xs, ds);
+    __syncthreads();
+    for (long long i = walk.first; i < walk.last; i++) {
+        const bool more = i + 1 < walk.last;               // uniform over the workgroup
+        bool down = false;                                  // the next pass continues this strip
+        if (more) {
+            walk.at(i + 1, R, n, c0, r0);
+            down = r0 != 0;
+            fetch(n, c0, r0);
+        }
+#pragma unroll 1
+        for (int s = 0; s < STEPS; s++) {
+            const int st = group * STEPS + s;               // step of the pass: row st / 2, half row st % 2
+            const uint32_t half = (uint32_t)(st & 1) * 32 * PIX;
+            const uint32_t dof = (uint32_t)((ds + (st >> 1)) * DROW) + half;
+            bf16x8 A[2];
+#pragma unroll
+            for (int a = 0; a < 2; a++) A[a] = read_tr8(da[a] + dof, da[a] + dof + 16 * PIX);
+            if (k0 == 0) {
+#pragma unroll
+                for (int a = 0; a < 2; a++)
+                    acc[36 + a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[a], ones, acc[36 + a], 0, 0, 0);
             }
 #pragma unroll
-            for (int b = 0; b < NT; b++) {
-                const int k = b * 16 + li;
-                uint16_t v[8];
+            for (int ty = 0; ty < 3; ty++) {
+                int xrow = xs + (st >> 1) + ty;
+                xrow = xrow >= XR ? xrow - XR : xrow;
+                const uint32_t xo = (uint32_t)(xrow * XROW) + half;
 #pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    const int c = cb + j, cs = c + tx;
-                    v[j] = (k < KX && c < W && rv && cs >= 0 && cs < W)
-                               ? x[((size_t)(row + ty) * W + cs) * KX + k] : (uint16_t)0;
-                }
-                uint4 u;
-                u.x = v[0] | ((uint32_t)v[1] << 16);
-                u.y = v[2] | ((uint32_t)v[3] << 16);
-                u.z = v[4] | ((uint32_t)v[5] << 16);
-                u.w = v[6] | ((uint32_t)v[7] << 16);
-                B[b] = as_bf16x8(u);
+                for (int d = 0; d < 3; d++)
+#pragma unroll
+                    for (int b = 0; b < 2; b++) {
+                        const bf16x8 B = read_tr8(xa[d][b] + xo, xa[d][b] + xo + 16 * PIX);
+#pragma unroll
+                        for (int a = 0; a < 2; a++) {
+                            f32x4& c = acc[((ty * 3 + d) * 2 + b) * 2 + a];
+                            c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[a], B, c, 0, 0, 0);
+                        }
+                    }
             }
+        }
+        if (!more) break;
+        if (down) {
+            // the coming rows have ring rows of their own
+            xs = xs + R >= XR ? xs + R - XR : xs + R;
+            ds = R - ds;
+        } else {
+            __syncthreads();                                // every wave is done with the rings
+            xs = ds = 0;
+            top(n, c0, r0);
+        }
+        put(xs, ds);
+        __syncthreads();
+    }
+
+    // the sums of a job's waves: halves added pairwise through LDS, in a fixed order
+    f32x4* red = (f32x4*)lds;
 #pragma unroll
-            for (int a = 0; a < MT; a++)
+    for (int o = 4; o >= JOBS; o >>= 1) {
+        __syncthreads();
+        if (wv >= o && wv < 2 * o) {
 #pragma unroll
-                for (int b = 0; b < NT; b++)
-                    acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[a], B[b], acc[a][b], 0, 0, 0);
+            for (int v = 0; v < TILES; v++) red[(v * 4 + wv - o) * 64 + lane] = acc[v];
+        }
+        __syncthreads();
+        if (wv < o) {
+#pragma unroll
+            for (int v = 0; v < TILES; v++) acc[v] += red[(v * 4 + wv) * 64 + lane];
         }
     }
-    // D[m][k]: lane holds m = a*16 + 4*g + i, k = b*16 + li
-    float* dst = part + ((size_t)t * waves + w) * MY * KX;
+    if (wv >= JOBS) return;
+    // D[m][k]: lane holds m = tile * 16 + 4 * g + e, k = tile * 16 + li
 #pragma unroll
-    for (int a = 0; a < MT; a++)
+    for (int t = 0; t < 9; t++) {
+        float* dst = part + ((size_t)t * gridDim.x + blockIdx.x) * CH * CH;
 #pragma unroll
-        for (int b = 0; b < NT; b++)
+        for (int b = 0; b < 2; b++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int m = a * 16 + 4 * g + i, k = b * 16 + li;
-                if (m < MY && k < KX) dst[m * KX + k] = acc[a][b][i];
-            }
-    if (t == 4) {
+            for (int a = 0; a < 2; a++)
 #pragma unroll
-        for (int a = 0; a < MT; a++) {
-            float s = bsum[a];
-            s += __shfl_xor(s, 16);
-            s += __shfl_xor(s, 32);
-            const int m = a * 16 + li;
-            if (g == 0 && m < MY) bpart[(size_t)w * MY + m] = s;
-        }
+                for (int e = 0; e < 4; e++)
+                    dst[((m0 + a) * 16 + 4 * g + e) * CH + (k0 + b) * 16 + li] = acc[(t * 2 + b) * 2 + a][e];
+    }
+    if (k0 == 0 && li == 0) {
+#pragma unroll
+        for (int a = 0; a < 2; a++)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                bpart[(size_t)blockIdx.x * CH + (m0 + a) * 16 + 4 * g + e] = acc[36 + a][e];
     }
 }
 
-// dw[t][m][k] = sum_w part[t][w][m][k] in order w = 0, 1, ...; dw has
-// mrows >= my rows per tap (rows my .. mrows-1 are left untouched).
-__global__ void wgrad_reduce_kernel(const float* __restrict__ part, const float* __restrict__ bpart,
-                                    float* __restrict__ dw, float* __restrict__ db, int my, int kx, int mrows,
-                                    int waves)
+// Input and output layers: a wide operand p (CH channels) against a narrow
+// one q (8 channels) at nine shifts, G[s][a][b] = sum_p wide[p][a]
+// narrow[p + off(s)][b].  The input layer is wide = dy, narrow = x, s = t;
+// the output layer sums over x's pixels instead of dy's, wide = x, narrow =
+// dy, s = 8 - t (the opposite offset).  Two shifts fill the 16 columns of an
+// MFMA: five tiles, whose tenth half column is ones (the input layer's bias
+// gradient, sum_p dy).  Every wave holds all shifts and channels; a pass is
+// 8 rows, one per wave, and the waves' sums are added through LDS at the
+// end.  Bound by the wide operand's bytes.
+template <int CH, bool OUTL>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void wgrad_edge_kernel(
+    const uint16_t* __restrict__ wide, const uint16_t* __restrict__ narrow, float* __restrict__ part,
+    float* __restrict__ bpart, int N, int H, int W)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    constexpr int R = 8;
+    constexpr int KO = CH / 8, MT = CH / 16, PIX = CH * 2;
+    constexpr int XR = 2 * R + 2, DR = 2 * R;
+    constexpr int XROW = kWgradPitch * 16, DROW = kWgradCols * PIX;
+    constexpr int XPT = (R * 66 + 511) / 512, DPT = R * 64 * KO / 512;
+    constexpr int XN = XR * XROW / 16, DN = DR * DROW / 16;
+    __shared__ uint4 lds[XN + DN];
+    const uint32_t xbase = (uint32_t)(uintptr_t)(lds_u4*)lds, dbase = xbase + XN * 16;
+    const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int g = lane >> 4, li = lane & 15;
+    const WgradWalk walk(N, H, W, R);
+
+    f32x4 acc[5][MT], bacc;
+#pragma unroll
+    for (int j = 0; j < 5; j++)
+#pragma unroll
+        for (int a = 0; a < MT; a++) acc[j][a] = f32x4{0.f, 0.f, 0.f, 0.f};
+    bacc = f32x4{0.f, 0.f, 0.f, 0.f};
+    const uint32_t one2 = 0x3F803F80u;
+    const bf16x8 ones = as_bf16x8(make_uint4(one2, one2, one2, one2));
+
+    // lane addresses: pixel 4g + (li >> 2); chunks 0, 1 of a narrow tile hold
+    // shift 2j's channels, chunks 2, 3 shift 2j + 1's (the tenth: shift 8's)
+    const int px = 4 * g + (li >> 2), ch = li & 3;
+    int xc[5], xr[5];
+    uint32_t da[MT];
+#pragma unroll
+    for (int j = 0; j < 5; j++) {
+        const int s0 = 2 * j, s1 = 2 * j + 1 < 9 ? 2 * j + 1 : 8;
+        xc[j] = (px + (ch < 2 ? s0 % 3 : s1 % 3)) * 16 + (ch & 1) * 8;
+        xr[j] = ch < 2 ? s0 / 3 : s1 / 3;
+    }
+#pragma unroll
+    for (int a = 0; a < MT; a++) da[a] = dbase + px * PIX + ((a ^ slot_xor<CH>(px)) * 32) + ch * 8;
+
+    uint4 sx[XPT], sd[DPT];
+    auto fetch = [&](int n, int c0, int r0) {
+#pragma unroll
+        for (int j = 0; j < XPT; j++) {
+            const int idx = tid + 512 * j;
+            const int c = idx % 66, i = idx / 66;
+            const int gr = r0 + 1 + i, gc = c0 - 1 + c;
+            sx[j] = make_uint4(0, 0, 0, 0);
+            if (i < R && gr < H && gc >= 0 && gc < W)
+                sx[j] = *(const uint4*)(narrow + (((size_t)n * H + gr) * W + gc) * 8);
+        }
+#pragma unroll
+        for (int j = 0; j < DPT; j++) {
+            const int idx = tid + 512 * j;
+            const int q = idx % KO, c = (idx / KO) % 64, i = idx / (KO * 64);
+            const int gr = r0 + i, gc = c0 + c;
+            sd[j] = make_uint4(0, 0, 0, 0);
+            if (gr < H && gc < W) sd[j] = *(const uint4*)(wide + (((size_t)n * H + gr) * W + gc) * CH + 8 * q);
+        }
+    };
+    auto put = [&](int xs, int ds) {
+#pragma unroll
+        for (int j = 0; j < XPT; j++) {
+            const int idx = tid + 512 * j;
+            const int c = idx % 66, i = idx / 66;
+            int s = xs + 2 + i;
+            s = s >= XR ? s - XR : s;
+            if (i < R) lds[s * kWgradPitch + c] = sx[j];
+        }
+#pragma unroll
+        for (int j = 0; j < DPT; j++) {
+            const int idx = tid + 512 * j;
+            const int q = idx % KO, c = (idx / KO) % 64, i = idx / (KO * 64);
+            lds[XN + ((ds + i) * DROW + c * PIX) / 16 + (((q >> 1) ^ slot_xor<CH>(c)) * 2 + (q & 1))] = sd[j];
+        }
+    };
+
+    auto top = [&](int n, int c0, int r0) {
+        if (tid < 2 * 66) {
+            const int c = tid % 66, i = tid / 66;
+            const int gr = r0 - 1 + i, gc = c0 - 1 + c;
+            uint4 v = make_uint4(0, 0, 0, 0);
+            if (gr >= 0 && gr < H && gc >= 0 && gc < W)
+                v = *(const uint4*)(narrow + (((size_t)n * H + gr) * W + gc) * 8);
+            lds[i * kWgradPitch + c] = v;
+        }
+    };
+
+    int xs = 0, ds = 0;
+    int n, c0, r0;
+    walk.at(walk.first, R, n, c0, r0);
+    fetch(n, c0, r0);
+    top(n, c0, r0);
+    put(xs, ds);
+    __syncthreads();
+    for (long long i = walk.first; i < walk.last; i++) {
+        const bool more = i + 1 < walk.last;
+        bool down = false;
+        if (more) {
+            walk.at(i + 1, R, n, c0, r0);
+            down = r0 != 0;
+            fetch(n, c0, r0);
+        }
+        uint32_t xo[5];                                     // narrow row wv + (shift's row), per lane
+#pragma unroll
+        for (int j = 0; j < 5; j++) {
+            int row = xs + wv + xr[j];
+            row = row >= XR ? row - XR : row;
+            xo[j] = xbase + row * XROW + xc[j];
+        }
+        const uint32_t dof = (uint32_t)((ds + wv) * DROW);
+#pragma unroll
+        for (int half = 0; half < 2; half++) {
+            bf16x8 A[MT];
+#pragma unroll
+            for (int a = 0; a < MT; a++) {
+                const uint32_t p = da[a] + dof + half * 32 * PIX;
+                A[a] = read_tr8(p, p + 16 * PIX);
+            }
+#pragma unroll
+            for (int j = 0; j < 5; j++) {
+                const uint32_t p = xo[j] + half * 32 * 16;
+                bf16x8 B = read_tr8(p, p + 16 * 16);
+                if (!OUTL && j == 4) B = li < 8 ? B : ones;
+                if (OUTL && j == 2) bacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, B, bacc, 0, 0, 0);
+#pragma unroll
+                for (int a = 0; a < MT; a++)
+                    acc[j][a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[a], B, acc[j][a], 0, 0, 0);
+            }
+        }
+        if (!more) break;
+        if (down) {
+            xs = xs + R >= XR ? xs + R - XR : xs + R;
+            ds = R - ds;
+        } else {
+            __syncthreads();
+            xs = ds = 0;
+            top(n, c0, r0);
+        }
+        put(xs, ds);
+        __syncthreads();
+    }
+
+    // the eight waves' sums: halves added pairwise through LDS, in a fixed order
+    f32x4* red = (f32x4*)lds;
+    static_assert(4 * (5 * MT + 1) * 64 <= XN + DN, "half of the waves' sums fit the LDS");
+#pragma unroll
+    for (int o = 4; o > 0; o >>= 1) {
+        __syncthreads();
+        if (wv >= o && wv < 2 * o) {
+#pragma unroll
+            for (int j = 0; j < 5; j++)
+#pragma unroll
+                for (int a = 0; a < MT; a++) red[((j * MT + a) * 4 + wv - o) * 64 + lane] = acc[j][a];
+            red[(5 * MT * 4 + wv - o) * 64 + lane] = bacc;
+        }
+        __syncthreads();
+        if (wv < o) {
+#pragma unroll
+            for (int j = 0; j < 5; j++)
+#pragma unroll
+                for (int a = 0; a < MT; a++) acc[j][a] += red[((j * MT + a) * 4 + wv) * 64 + lane];
+            bacc += red[(5 * MT * 4 + wv) * 64 + lane];
+        }
+    }
+    if (wv != 0) return;
+    // D: lane holds wide channel a * 16 + 4 * g + e of shift 2j + (li >> 3),
+    // narrow channel li & 7
+#pragma unroll
+    for (int j = 0; j < 5; j++) {
+        const int s = 2 * j + (li >> 3);
+#pragma unroll
+        for (int a = 0; a < MT; a++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int m = a * 16 + 4 * g + e;
+                if (s < 9) {
+                    const int t = OUTL ? 8 - s : s;
+                    const int i = OUTL ? (li & 7) * CH + m : m * 8 + (li & 7);
+                    part[((size_t)t * gridDim.x + blockIdx.x) * CH * 8 + i] = acc[j][a][e];
+                } else if (!OUTL && li == 8) {
+                    bpart[(size_t)blockIdx.x * CH + m] = acc[j][a][e];
+                }
+            }
+    }
+    // the centre shift's columns of dy against ones: every row is the sum
+    if (OUTL && g == 0 && li < 8) bpart[(size_t)blockIdx.x * 8 + li] = bacc[0];
+}
+
+// dw[t][m][k] = sum_w part[t][w][m][k]; dw has mrows >= my rows per tap
+// (rows my .. mrows-1 are left untouched).  A workgroup of 1024 takes 64
+// elements, 16 threads each over every sixteenth partial, added through LDS
+// in a fixed order (one thread per element over all 256 partials was a chain
+// of 256 loads: 110 us whatever the layer).  Grid row 9: the biases.
+__global__ __launch_bounds__(1024) void wgrad_reduce_kernel(const float* __restrict__ part,
+                                                            const float* __restrict__ bpart, float* __restrict__ dw,
+                                                            float* __restrict__ db, int my, int kx, int mrows,
+                                                            int waves)
+{
+    __shared__ float sh[16][64];
     const int t = blockIdx.y;
-    const int n = my * kx;
+    const int n = t < 9 ? my * kx : my;
+    const int e = threadIdx.x & 63, j = threadIdx.x >> 6;
+    const int i = blockIdx.x * 64 + e;
+    if (blockIdx.x * 64 >= n) return;                       // whole workgroup
+    const float* src = t < 9 ? part + (size_t)t * waves * n : bpart;
+    float s = 0.f;
     if (i < n) {
-        float s = 0.f;
-        for (int w = 0; w < waves; w++) s += part[((size_t)t * waves + w) * n + i];
+#pragma unroll 16
+        for (int w = j; w < waves; w += 16) s += src[(size_t)w * n + i];
+    }
+    sh[j][e] = s;
+    __syncthreads();
+    if (j != 0 || i >= n) return;
+#pragma unroll
+    for (int o = 1; o < 16; o++) s += sh[o][e];
+    if (t < 9)
         dw[((size_t)t * mrows + i / kx) * kx + i % kx] = s;
-    }
-    if (t == 4 && i < my) {
-        float s = 0.f;
-        for (int w = 0; w < waves; w++) s += bpart[(size_t)w * my + i];
+    else
         db[i] = s;
-    }
 }
 
 // Mean-squared-error gradient of the 4-channel FP32 output against the
@@ -923,47 +1309,43 @@ hipError_t nn_launch_conv(int kind, const uint16_t* in, const uint16_t* w, const
 hipError_t nn_launch_wgrad(int kind, const uint16_t* x, const uint16_t* dy, float* part, float* bpart, float* dw,
                            float* db, int mrows, int N, int H, int W, hipStream_t s)
 {
-    const int waves = kWgradWaves;
-    const dim3 grid((unsigned)((waves + 3) / 4), 9), block(256);
-    int my, kx;
+    // one workgroup per stretch of passes, at most kWgradWaves (the partial
+    // sums the workspace holds)
+    const int width = (kind & NN_W64) ? 64 : 32, base = kind & ~NN_W64;
+    const bool mid = base == NN_WGRAD_MID;
+    const int rows = mid ? 4 : 8;                       // rows per pass (R of the kernels)
+    const long long passes = (long long)N * ((W + kWgradCols - 1) / kWgradCols) * ((H + rows - 1) / rows);
+    const int waves = (int)(passes < kWgradWaves ? passes : kWgradWaves);
+    int my = width, kx = width;
     switch (kind) {
     case NN_WGRAD_IN:
-        wgrad_kernel<8, 32><<<grid, block, 0, s>>>(x, dy, part, bpart, N, H, W, waves);
-        my = 32;
+        wgrad_edge_kernel<32, false><<<waves, 512, 0, s>>>(dy, x, part, bpart, N, H, W);
         kx = 8;
         break;
     case NN_WGRAD_MID:
-        wgrad_kernel<32, 32><<<grid, block, 0, s>>>(x, dy, part, bpart, N, H, W, waves);
-        my = 32;
-        kx = 32;
+        wgrad_mid_kernel<32><<<waves, 512, 0, s>>>(x, dy, part, bpart, N, H, W);
         break;
     case NN_WGRAD_OUT:
-        wgrad_kernel<32, 8><<<grid, block, 0, s>>>(x, dy, part, bpart, N, H, W, waves);
+        wgrad_edge_kernel<32, true><<<waves, 512, 0, s>>>(x, dy, part, bpart, N, H, W);
         my = 8;
-        kx = 32;
         break;
     case NN_WGRAD_IN | NN_W64:
-        wgrad_kernel<8, 64><<<grid, block, 0, s>>>(x, dy, part, bpart, N, H, W, waves);
-        my = 64;
+        wgrad_edge_kernel<64, false><<<waves, 512, 0, s>>>(dy, x, part, bpart, N, H, W);
         kx = 8;
         break;
     case NN_WGRAD_MID | NN_W64:
-        wgrad_kernel<64, 64><<<grid, block, 0, s>>>(x, dy, part, bpart, N, H, W, waves);
-        my = 64;
-        kx = 64;
+        wgrad_mid_kernel<64><<<waves, 512, 0, s>>>(x, dy, part, bpart, N, H, W);
         break;
     case NN_WGRAD_OUT | NN_W64:
-        wgrad_kernel<64, 8><<<grid, block, 0, s>>>(x, dy, part, bpart, N, H, W, waves);
+        wgrad_edge_kernel<64, true><<<waves, 512, 0, s>>>(x, dy, part, bpart, N, H, W);
         my = 8;
-        kx = 64;
         break;
     default:
         return hipErrorInvalidValue;
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    const int n = my * kx;
-    wgrad_reduce_kernel<<<dim3((n + 255) / 256, 9), 256, 0, s>>>(part, bpart, dw, db, my, kx, mrows, waves);
+    wgrad_reduce_kernel<<<dim3((my * kx + 63) / 64, 10), 1024, 0, s>>>(part, bpart, dw, db, my, kx, mrows, waves);
     return hipGetLastError();
 }
 

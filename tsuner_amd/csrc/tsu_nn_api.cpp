@@ -34,7 +34,7 @@ bool wgrad_shape(int kind, int* my, int* kx)
 }
 
 // Workspace of tsu_nn_wgrad_noalloc: the largest weight-gradient workspace
-// (hidden width 64, the 64 -> 64 layer: per-wave partials of 9 x 64 x 64
+// (hidden width 64, the 64 -> 64 layer: 256 sets of partials of 9 x 64 x 64
 // weights and 64 biases), 9,453,568 floats = 37.8 MB.  Every device the
 // library's code object is loaded on holds one copy until the process ends.
 constexpr long long kScratchFloats = 9LL * tsu::kWgradWaves * 64 * 64 + (long long)tsu::kWgradWaves * 64;
@@ -131,8 +131,8 @@ TSU_API int tsu_nn_wgrad_noalloc(int kind, const void* x, const void* dy, float*
     float* ws = nullptr;
     int rc = scratch_of_device(dev, &ws);
     if (rc) return rc;
-    // every wave writes all of its partial sums each call: nothing in the
-    // scratch has to start at zero
+    // every workgroup writes all of its partial sums each call: nothing in
+    // the scratch has to start at zero
     float* part = ws;
     float* bpart = ws + 9LL * tsu::kWgradWaves * my * kx;
     hipError_t e = tsu::nn_launch_wgrad(kind, (const uint16_t*)x, (const uint16_t*)dy, part, bpart, dw, db, mrows, n,
