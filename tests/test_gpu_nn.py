@@ -182,6 +182,31 @@ def test_weight_gradient_strips_and_stretches(shape, width):
         np.testing.assert_allclose(host(db), rdb, rtol=0, atol=1e-5 * np.abs(rdb).max())
 
 
+def test_weight_gradients_take_operands_of_any_alignment():
+    """x and dy one element past a 16-byte boundary: the same sums, bit for
+    bit, as from aligned copies."""
+    rng = np.random.default_rng(14)
+    n, h, w = 2, 9, 70
+    s = C.c_void_p(0)
+    for kind, kx, my in [(5, 8, 32), (6 | W64, 64, 64), (7, 32, 8)]:
+        nws = lib().tsu_nn_wgrad_workspace(kind)
+        ws = torch.zeros(nws, dtype=torch.float32, device="cuda")
+        x = dev_bf16(rand_bf16(rng, n * h * w * kx))
+        dy = dev_bf16(rand_bf16(rng, n * h * w * my))
+        got = []
+        for shift in (0, 1):
+            tx, ty = (torch.zeros(t.numel() + shift, dtype=t.dtype, device="cuda") for t in (x, dy))
+            tx[shift:].copy_(x)
+            ty[shift:].copy_(dy)
+            dw = torch.zeros(9 * my * kx, dtype=torch.float32, device="cuda")
+            db = torch.zeros(my, dtype=torch.float32, device="cuda")
+            ok(lib().tsu_nn_wgrad(kind, P(tx[shift:]), P(ty[shift:]), P(dw), P(db), my, n, h, w, P(ws), nws, s))
+            got.append((host(dw), host(db)))
+        assert np.abs(got[0][0]).max() > 0
+        np.testing.assert_array_equal(got[1][0], got[0][0])
+        np.testing.assert_array_equal(got[1][1], got[0][1])
+
+
 def test_wide_conv_workgroups_loop_over_tiles():
     """The 64-channel kernels keep one workgroup per CU and loop over 8 x 64
     pixel tiles (prefetching the next one): an image set with more than

@@ -433,6 +433,16 @@ __device__ __forceinline__ bf16x8 read_tr8(uint32_t a, uint32_t b)
     return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
+// Eight channels of one pixel.  The weight gradients take operands of any
+// element alignment (global loads need none on this hardware; 16-byte aligned
+// rows are the fast case).
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
+__device__ __forceinline__ uint4 load8(const uint16_t* p)
+{
+    const u32x4_any v = *(const u32x4_any*)p;
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+
 // XOR of a pixel's 32-byte slots at column c: 64 channels have 4 slots and 2
 // pixels per 256 bytes (all banks once), 32 channels 2 slots and 4 pixels.
 template <int CH>
@@ -523,7 +533,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             const int gr = r0 + 1 + i, gc = c0 - 1 + c;
             sx[j] = make_uint4(0, 0, 0, 0);
             if (i < R && gr < H && gc >= 0 && gc < W)
-                sx[j] = *(const uint4*)(x + (((size_t)n * H + gr) * W + gc) * CH + 8 * q);
+                sx[j] = load8(x + (((size_t)n * H + gr) * W + gc) * CH + 8 * q);
         }
 #pragma unroll
         for (int j = 0; j < DPT; j++) {
@@ -531,7 +541,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             const int q = idx % KO, c = (idx / KO) % 64, i = idx / (KO * 64);
             const int gr = r0 + i, gc = c0 + c;
             sd[j] = make_uint4(0, 0, 0, 0);
-            if (gr < H && gc < W) sd[j] = *(const uint4*)(dy + (((size_t)n * H + gr) * W + gc) * CH + 8 * q);
+            if (gr < H && gc < W) sd[j] = load8(dy + (((size_t)n * H + gr) * W + gc) * CH + 8 * q);
         }
     };
     // the fetched rows into ring rows xs + 2, ... and ds, ...
@@ -560,7 +570,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             const int gr = r0 - 1 + i, gc = c0 - 1 + c;
             uint4 v = make_uint4(0, 0, 0, 0);
             if (gr >= 0 && gr < H && gc >= 0 && gc < W)
-                v = *(const uint4*)(x + (((size_t)n * H + gr) * W + gc) * CH + 8 * q);
+                v = load8(x + (((size_t)n * H + gr) * W + gc) * CH + 8 * q);
             lds[(i * XROW + c * PIX) / 16 + (((q >> 1) ^ slot_xor<CH>(c)) * 2 + (q & 1))] = v;
         }
     };
@@ -721,7 +731,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             const int gr = r0 + 1 + i, gc = c0 - 1 + c;
             sx[j] = make_uint4(0, 0, 0, 0);
             if (i < R && gr < H && gc >= 0 && gc < W)
-                sx[j] = *(const uint4*)(narrow + (((size_t)n * H + gr) * W + gc) * 8);
+                sx[j] = load8(narrow + (((size_t)n * H + gr) * W + gc) * 8);
         }
 #pragma unroll
         for (int j = 0; j < DPT; j++) {
@@ -729,7 +739,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             const int q = idx % KO, c = (idx / KO) % 64, i = idx / (KO * 64);
             const int gr = r0 + i, gc = c0 + c;
             sd[j] = make_uint4(0, 0, 0, 0);
-            if (gr < H && gc < W) sd[j] = *(const uint4*)(wide + (((size_t)n * H + gr) * W + gc) * CH + 8 * q);
+            if (gr < H && gc < W) sd[j] = load8(wide + (((size_t)n * H + gr) * W + gc) * CH + 8 * q);
         }
     };
     auto put = [&](int xs, int ds) {
@@ -755,7 +765,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             const int gr = r0 - 1 + i, gc = c0 - 1 + c;
             uint4 v = make_uint4(0, 0, 0, 0);
             if (gr >= 0 && gr < H && gc >= 0 && gc < W)
-                v = *(const uint4*)(narrow + (((size_t)n * H + gr) * W + gc) * 8);
+                v = load8(narrow + (((size_t)n * H + gr) * W + gc) * 8);
             lds[i * kWgradPitch + c] = v;
         }
     };
