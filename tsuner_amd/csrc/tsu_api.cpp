@@ -41,7 +41,6 @@ int fail(int code, const std::string& msg)
         if (e_ != hipSuccess) return fail(TSU_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(e_)); \
     } while (0)
 
-constexpr unsigned long long kInfBits = 0x7FF0000000000000ull;
 
 unsigned long long dbits(double v)
 {
@@ -154,6 +153,7 @@ struct tsu_state {
     void* B = nullptr;
     uint8_t* fix = nullptr;
     Ctrl* ctrl = nullptr;
+    tsu::DtSlots* dts = nullptr;
     double* ext = nullptr;
     double* CC = nullptr;
     double* tCC = nullptr;
@@ -238,6 +238,7 @@ void free_state(tsu_state* st)
     (void)hipFree(st->B);
     (void)hipFree(st->fix);
     (void)hipFree(st->ctrl);
+    (void)hipFree(st->dts);
     (void)hipFree(st->ext);
     (void)hipFree(st->CC);
     (void)hipFree(st->tCC);
@@ -254,10 +255,14 @@ tsu::StageArgs stage_args(const tsu_state* st, int k)
     a.Hin = (const char*)st->A + 3 * plane;
     a.fix = st->fix;
     a.ctrl = st->ctrl;
+    a.dts = st->dts;
     a.ext = st->s.extrema ? st->ext : nullptr;
     a.tile_rows = st->tile_rows;
     a.nstrips = st->nstrips;
     a.ntiles = st->ntiles;
+    a.npx = st->P.npx;
+    a.npy = st->P.npy;
+    a.periodic = tsu::periodic_sides(st->P);
     a.P = st->dP;
     a.k = k;
     if (st->s.order == 1) {
@@ -303,13 +308,27 @@ int enqueue_step(tsu_state* st)
             st->ev_used++;
         }
     }
-    HIPCHK(tsu::launch_advance(st->ctrl, st->P, st->stream));
+    if (st->s.order == 1) HIPCHK(tsu::launch_advance(st->ctrl, st->dts, st->P, st->stream));
     return TSU_OK;
 }
 
 int read_ctrl(tsu_state* st, Ctrl* c)
 {
     HIPCHK(hipMemcpyAsync(c, st->ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, st->stream));
+    HIPCHK(hipStreamSynchronize(st->stream));
+    return TSU_OK;
+}
+
+// The control block and every dt slot as before the first step.
+int reset_ctrl(tsu_state* st)
+{
+    Ctrl c{};
+    c.stop_time = INFINITY;
+    c.stop_step = LLONG_MAX;
+    tsu::DtSlots d;
+    tsu::reset_dt_slots(&d);
+    HIPCHK(hipMemcpyAsync(st->ctrl, &c, sizeof(c), hipMemcpyHostToDevice, st->stream));
+    HIPCHK(hipMemcpyAsync(st->dts, &d, sizeof(d), hipMemcpyHostToDevice, st->stream));
     HIPCHK(hipStreamSynchronize(st->stream));
     return TSU_OK;
 }
@@ -387,6 +406,7 @@ TSU_API int tsu_state_create(tsu_state** out, const tsu_sim_params* p, const tsu
     if (e == hipSuccess) e = hipMalloc(&st->B, state_bytes);
     if (e == hipSuccess) e = hipMalloc((void**)&st->fix, (size_t)st->nvol);
     if (e == hipSuccess) e = hipMalloc((void**)&st->ctrl, sizeof(Ctrl));
+    if (e == hipSuccess) e = hipMalloc((void**)&st->dts, sizeof(tsu::DtSlots));
     if (e == hipSuccess) e = hipMalloc((void**)&st->mass_buf, (2 * (size_t)st->mass_nb + 2) * sizeof(double));
     if (e == hipSuccess) e = hipMalloc((void**)&st->dP, sizeof(DevParams));
     if (e == hipSuccess) e = hipMemcpy(st->dP, &st->P, sizeof(DevParams), hipMemcpyHostToDevice);
@@ -396,16 +416,9 @@ TSU_API int tsu_state_create(tsu_state** out, const tsu_sim_params* p, const tsu
         (void)hipGetLastError();
         return fail(TSU_ERR_DEVICE_MEMORY, std::string("device allocation failed: ") + hipGetErrorString(e));
     }
-    Ctrl c{};
-    c.t = 0.0;
-    c.stop_time = INFINITY;
-    c.dt_bits[0] = c.dt_bits[1] = kInfBits;
-    c.step = 0;
-    c.stop_step = LLONG_MAX;
-    e = hipMemcpy(st->ctrl, &c, sizeof(Ctrl), hipMemcpyHostToDevice);
-    if (e != hipSuccess) {
+    if (int rc2 = reset_ctrl(st)) {
         free_state(st);
-        return fail(TSU_ERR_HIP, std::string("ctrl init: ") + hipGetErrorString(e));
+        return rc2;
     }
     *out = st;
     return TSU_OK;
@@ -449,15 +462,8 @@ TSU_API int tsu_state_upload(tsu_state* st, const double* V, const int* fixH)
     }
     HIPCHK(hipMemcpyAsync(st->B, st->A, bytes, hipMemcpyDeviceToDevice, st->stream));
     HIPCHK(hipMemcpyAsync(st->fix, fx.data(), (size_t)nv, hipMemcpyHostToDevice, st->stream));
-    Ctrl c{};
-    c.t = 0.0;
-    c.stop_time = INFINITY;
-    c.dt_bits[0] = c.dt_bits[1] = kInfBits;
-    c.step = 0;
-    c.stop_step = LLONG_MAX;
-    HIPCHK(hipMemcpyAsync(st->ctrl, &c, sizeof(Ctrl), hipMemcpyHostToDevice, st->stream));
     if (st->ext) HIPCHK(tsu::launch_fill(st->ext, 3 * nv, -1e30, st->stream));
-    HIPCHK(hipStreamSynchronize(st->stream));
+    if (int rc = reset_ctrl(st)) return rc;                 // waits for the stream
     st->uploaded = true;
     return TSU_OK;
 }
@@ -538,10 +544,11 @@ TSU_API int tsu_init_dt(tsu_state* st)
     Ctrl c;
     rc = read_ctrl(st, &c);
     if (rc) return rc;
-    c.dt_bits[0] = c.dt_bits[1] = kInfBits;
-    HIPCHK(hipMemcpyAsync(st->ctrl, &c, sizeof(Ctrl), hipMemcpyHostToDevice, st->stream));
+    tsu::DtSlots d;
+    tsu::reset_dt_slots(&d);
+    HIPCHK(hipMemcpyAsync(st->dts, &d, sizeof(d), hipMemcpyHostToDevice, st->stream));
     void* cur = (st->s.order == 1 && (c.step & 1)) ? st->B : st->A;
-    HIPCHK(tsu::launch_init_dt(cur, st->P, st->ctrl, st->precision, st->stream));
+    HIPCHK(tsu::launch_init_dt(cur, st->P, st->dts, c.step, st->precision, st->stream));
     HIPCHK(hipStreamSynchronize(st->stream));
     return TSU_OK;
 }
@@ -596,10 +603,12 @@ TSU_API int tsu_get_time(tsu_state* st, double* t, double* dt, long long* steps)
     if (!st) return fail(TSU_ERR_ARG, "null state");
     DeviceGuard g(st->device);
     Ctrl c;
-    int rc = read_ctrl(st, &c);
+    tsu::DtSlots d;
+    HIPCHK(hipMemcpyAsync(&d, st->dts, sizeof(d), hipMemcpyDeviceToHost, st->stream));
+    int rc = read_ctrl(st, &c);                             // waits for the stream
     if (rc) return rc;
     if (t) *t = c.t;
-    if (dt) *dt = finalize_host(st->P, c.dt_bits[c.step & 1]);
+    if (dt) *dt = finalize_host(st->P, tsu::min_dt_bits(d, c.step));
     if (steps) *steps = c.step;
     return TSU_OK;
 }
@@ -613,8 +622,10 @@ TSU_API int tsu_set_time(tsu_state* st, double t, double dt)
     if (rc) return rc;
     c.t = t;
     if (dt > 0) {
-        c.dt_bits[c.step & 1] = dbits(dt);
-        c.dt_bits[(c.step + 1) & 1] = kInfBits;
+        tsu::DtSlots d;
+        tsu::reset_dt_slots(&d, c.step, dbits(dt));
+        HIPCHK(hipMemcpyAsync(st->dts, &d, sizeof(d), hipMemcpyHostToDevice, st->stream));
+        HIPCHK(hipStreamSynchronize(st->stream));
     }
     HIPCHK(hipMemcpyAsync(st->ctrl, &c, sizeof(Ctrl), hipMemcpyHostToDevice, st->stream));
     HIPCHK(hipStreamSynchronize(st->stream));

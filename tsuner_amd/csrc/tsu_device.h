@@ -75,25 +75,51 @@ struct DevParams {
     double tcc0, dtcc, tcc_end;   // tCC[0], tCC[1]-tCC[0], tCC[timeCC-2]
 };
 
-// Step control block, resident in device memory.  t and step change only in
-// the advance kernel; dt_bits[s & 1] holds the IEEE bits of the minimum cell
-// dt of step s (positive doubles order like their bit patterns).
+// Step control block, resident in device memory.
+//
+// Two-stage scheme: the first stage of a step reads t and step and leaves
+// the running step's time, dt and number in run_*; the last stage reads those
+// and leaves the next step's t and step.  Neither stage reads what it writes,
+// so one wave of each does the writing and a step needs no launch of its own
+// to advance (a one-thread launch cost 5 us and its gap, of 43 us for a step
+// of 100 x 100 cells).  The single-stage scheme has no second launch to
+// alternate with and keeps an advance launch.
 struct Ctrl {
     double t;
     double stop_time;
-    unsigned long long dt_bits[2];
     long long step;
     long long stop_step;   // steps enqueued once step >= stop_step do nothing
     long long clamp;       // 1: the step crossing stop_time ends on it (dt = stop_time - t)
-    long long pad;
+    double run_t, run_dt;
+    long long run_step;
+    long long running;     // 0: the last first stage found nothing to do
+    long long pad[7];      // 128 bytes: members of an ensemble share no cache line
+};
+
+// Smallest cell dt of a step, as the IEEE bits of the minima of kDtSlots
+// groups of waves (positive doubles order like their bit patterns): slots
+// v[s & 1][...][0] belong to step s, and its dt is the least of them.  One
+// address for all waves took their atomics one after the other, 6.5 ns each:
+// 14 us of a last stage of 512 x 512 cells (2304 waves, 41 us), 0.2 ms of one
+// of 8192 x 8192.  A slot has a cache line of its own.
+constexpr int kDtSlots = 16;
+constexpr unsigned long long kInfBits = 0x7FF0000000000000ull;
+struct DtSlots {
+    unsigned long long v[2][kDtSlots][16];
 };
 
 // dt of the step starting at t: the finalized minimum, shortened to land on
-// stop_time when clamping is on.  Stage and advance kernels use the same rule.
-__device__ __forceinline__ double clamp_dt(const Ctrl* C, double t, double dt)
+// stop_time when clamping is on.
+__device__ __forceinline__ double clamp_dt(const Ctrl& C, double t, double dt)
 {
-    if (C->clamp && !(dt < C->stop_time - t)) return C->stop_time - t;
+    if (C.clamp && !(dt < C.stop_time - t)) return C.stop_time - t;
     return dt;
+}
+
+// t after that step; a shortened step ends exactly on stop_time.
+__device__ __forceinline__ double next_time(long long clamp, double stop_time, double t, double dt)
+{
+    return (clamp && !(dt < stop_time - t)) ? stop_time : t + dt;
 }
 
 // ---- primitive operations per compute type --------------------------------
@@ -912,9 +938,8 @@ __device__ __forceinline__ R cell_dt(const DevParams& P, R h, R qx, R qy)
 // nvol > 4096 the reference's partial minima pass through fminf (rounding is
 // monotone, so this is the float-rounded minimum) and the host minimum starts
 // from 1e30.
-__device__ __forceinline__ double finalize_dt(const DevParams& P, unsigned long long bits)
+__device__ __forceinline__ double finalize_dt(const DevParams& P, double m)
 {
-    double m = __longlong_as_double((long long)bits);
     if (P.dt_narrow && P.nvol > 4096) m = (double)(float)m;
     return (m < 1e30) ? m : 1e30;
 }

@@ -24,8 +24,6 @@ using tsu::DevParams;
 
 namespace {
 
-constexpr unsigned long long kInfBits = 0x7FF0000000000000ull;
-
 #define ECHK(expr)                                                                                    \
     do {                                                                                              \
         hipError_t e_ = (expr);                                                                       \
@@ -57,7 +55,9 @@ struct tsu_ensemble {
     double* ext = nullptr;          // hmax, max H, eta_max planes per member with extrema on
     size_t ext_doubles = 0;
     Ctrl* ctrl = nullptr;
+    tsu::DtSlots* dts = nullptr;
     Ctrl* snapC = nullptr;
+    tsu::DtSlots* snapD = nullptr;
     DevParams* dP = nullptr;
     tsu::StageArgs* dargs = nullptr;    // [2][n]: stage 0 and stage 1 arguments (hooks)
     tsu::BatchMember* dmem = nullptr;   // [n]: members as the batched stage kernel sees them
@@ -106,7 +106,9 @@ void destroy(tsu_ensemble* e)
     (void)hipFree(e->fix);
     (void)hipFree(e->ext);
     (void)hipFree(e->ctrl);
+    (void)hipFree(e->dts);
     (void)hipFree(e->snapC);
+    (void)hipFree(e->snapD);
     (void)hipFree(e->dP);
     (void)hipFree(e->dargs);
     (void)hipFree(e->dmem);
@@ -139,6 +141,9 @@ int build_launch_tables(tsu_ensemble* e)
         bm.nstrips = nstrips(e, i);
         bm.ntiles = bm.nstrips * nchunks(e, i);
         bm.order = e->s[i].order;
+        bm.npx = e->P[i].npx;
+        bm.npy = e->P[i].npy;
+        bm.periodic = tsu::periodic_sides(e->P[i]);
         for (int k = 0; k < 2; k++) {
             tsu::StageArgs a{};
             char* Ai = e->A + e->off[i];
@@ -146,10 +151,14 @@ int build_launch_tables(tsu_ensemble* e)
             a.Hin = Ai + 3 * plane;
             a.fix = e->fix + e->foff[i];
             a.ctrl = e->ctrl + i;
+            a.dts = e->dts + i;
             a.ext = e->s[i].extrema ? e->ext + e->xoff[i] : nullptr;
             a.tile_rows = e->rows[i];
             a.nstrips = nstrips(e, i);
             a.ntiles = a.nstrips * nchunks(e, i);
+            a.npx = bm.npx;
+            a.npy = bm.npy;
+            a.periodic = bm.periodic;
             a.P = e->dP + i;
             if (e->s[i].order == 1) {
                 a.in = Ai;
@@ -184,13 +193,13 @@ int build_launch_tables(tsu_ensemble* e)
 int enqueue_step(tsu_ensemble* e)
 {
     const int order = e->s[0].order;
-    const tsu::BatchPools pools{e->A, e->B, e->fix, e->ctrl, e->ext, e->dP};
+    const tsu::BatchPools pools{e->A, e->B, e->fix, e->ctrl, e->dts, e->ext, e->dP};
     bool fast_bed = true;
     for (int i = 0; i < e->n; i++) fast_bed = fast_bed && tsu::fast_bedload(e->P[i]);
     for (int k = 0; k < order; k++)
         ECHK(tsu::launch_stage_batch(pools, e->dmem, e->tiles, e->ntiles, k, k == order - 1, e->sed, e->precision,
                                      e->stream, fast_bed));
-    ECHK(tsu::launch_advance_batch(e->ctrl, e->dP, e->n, e->stream));
+    if (order == 1) ECHK(tsu::launch_advance_batch(e->ctrl, e->dts, e->dP, e->n, e->stream));
     return TSU_OK;
 }
 
@@ -212,6 +221,20 @@ int members_ready(const tsu_ensemble* e)
                 return tsu::set_error(TSU_ERR_ARG, "member " + std::to_string(i) +
                                                        " has an inflow side: tsu_ensemble_set_inflow first");
     }
+    return TSU_OK;
+}
+
+// A member's control block and dt slots as before its first step.
+int reset_ctrl(tsu_ensemble* e, int i)
+{
+    Ctrl c{};
+    c.stop_time = INFINITY;
+    c.stop_step = LLONG_MAX;
+    tsu::DtSlots d;
+    tsu::reset_dt_slots(&d);
+    ECHK(hipMemcpyAsync(e->ctrl + i, &c, sizeof(c), hipMemcpyHostToDevice, e->stream));
+    ECHK(hipMemcpyAsync(e->dts + i, &d, sizeof(d), hipMemcpyHostToDevice, e->stream));
+    ECHK(hipStreamSynchronize(e->stream));
     return TSU_OK;
 }
 
@@ -284,6 +307,7 @@ TSU_API int tsu_ensemble_create(tsu_ensemble** out, int n, const tsu_sim_params*
     if (err == hipSuccess) err = hipMalloc((void**)&e->fix, e->fix_bytes);
     if (err == hipSuccess && e->ext_doubles) err = hipMalloc((void**)&e->ext, e->ext_doubles * sizeof(double));
     if (err == hipSuccess) err = hipMalloc((void**)&e->ctrl, n * sizeof(Ctrl));
+    if (err == hipSuccess) err = hipMalloc((void**)&e->dts, n * sizeof(tsu::DtSlots));
     if (err == hipSuccess) err = hipMalloc((void**)&e->dP, n * sizeof(DevParams));
     if (err == hipSuccess) err = hipMalloc((void**)&e->dargs, 2 * (size_t)n * sizeof(tsu::StageArgs));
     if (err == hipSuccess) err = hipMalloc((void**)&e->dmem, (size_t)n * sizeof(tsu::BatchMember));
@@ -294,17 +318,11 @@ TSU_API int tsu_ensemble_create(tsu_ensemble** out, int n, const tsu_sim_params*
         (void)hipGetLastError();
         return tsu::set_error(TSU_ERR_DEVICE_MEMORY, std::string("ensemble allocation: ") + hipGetErrorString(err));
     }
-    std::vector<Ctrl> c(n);
-    for (int i = 0; i < n; i++) {
-        std::memset(&c[i], 0, sizeof(Ctrl));
-        c[i].stop_time = INFINITY;
-        c[i].stop_step = LLONG_MAX;
-        c[i].dt_bits[0] = c[i].dt_bits[1] = kInfBits;
-    }
-    if (hipMemcpy(e->ctrl, c.data(), n * sizeof(Ctrl), hipMemcpyHostToDevice) != hipSuccess) {
-        destroy(e);
-        return tsu::set_error(TSU_ERR_HIP, "ensemble ctrl init failed");
-    }
+    for (int i = 0; i < n; i++)
+        if (int rc = reset_ctrl(e, i)) {
+            destroy(e);
+            return rc;
+        }
     int rc = build_launch_tables(e);
     if (rc) {
         destroy(e);
@@ -355,13 +373,7 @@ TSU_API int tsu_ensemble_upload(tsu_ensemble* e, int i, const double* V, const i
     ECHK(hipMemcpyAsync(e->B + e->off[i], e->A + e->off[i], bytes, hipMemcpyDeviceToDevice, e->stream));
     ECHK(hipMemcpyAsync(e->fix + e->foff[i], fx.data(), (size_t)nv, hipMemcpyHostToDevice, e->stream));
     if (e->s[i].extrema) ECHK(tsu::launch_fill(e->ext + e->xoff[i], 3 * nv, -1e30, e->stream));
-    Ctrl c;
-    std::memset(&c, 0, sizeof(c));
-    c.stop_time = INFINITY;
-    c.stop_step = LLONG_MAX;
-    c.dt_bits[0] = c.dt_bits[1] = kInfBits;
-    ECHK(hipMemcpyAsync(e->ctrl + i, &c, sizeof(Ctrl), hipMemcpyHostToDevice, e->stream));
-    ECHK(hipStreamSynchronize(e->stream));
+    if ((rc = reset_ctrl(e, i))) return rc;                 // waits for the stream
     e->uploaded[i] = true;
     return TSU_OK;
 }
@@ -433,14 +445,15 @@ TSU_API int tsu_ensemble_init_dt(tsu_ensemble* e)
     if (!e) return tsu::set_error(TSU_ERR_ARG, "null ensemble");
     Guard g(e->device);
     if (int rc = members_ready(e)) return rc;
+    tsu::DtSlots d;
+    tsu::reset_dt_slots(&d);
     for (int i = 0; i < e->n; i++) {
         Ctrl c;
         ECHK(hipMemcpyAsync(&c, e->ctrl + i, sizeof(Ctrl), hipMemcpyDeviceToHost, e->stream));
         ECHK(hipStreamSynchronize(e->stream));
-        c.dt_bits[0] = c.dt_bits[1] = kInfBits;
-        ECHK(hipMemcpyAsync(e->ctrl + i, &c, sizeof(Ctrl), hipMemcpyHostToDevice, e->stream));
+        ECHK(hipMemcpyAsync(e->dts + i, &d, sizeof(d), hipMemcpyHostToDevice, e->stream));
         char* cur = ((e->s[i].order == 1 && (c.step & 1)) ? e->B : e->A) + e->off[i];
-        ECHK(tsu::launch_init_dt(cur, e->P[i], e->ctrl + i, e->precision, e->stream));
+        ECHK(tsu::launch_init_dt(cur, e->P[i], e->dts + i, c.step, e->precision, e->stream));
     }
     ECHK(hipStreamSynchronize(e->stream));
     return TSU_OK;
@@ -502,12 +515,14 @@ TSU_API int tsu_ensemble_get_time(tsu_ensemble* e, int i, double* t, double* dt,
     if (rc) return rc;
     Guard g(e->device);
     Ctrl c;
+    tsu::DtSlots d;
     ECHK(hipMemcpyAsync(&c, e->ctrl + i, sizeof(Ctrl), hipMemcpyDeviceToHost, e->stream));
+    ECHK(hipMemcpyAsync(&d, e->dts + i, sizeof(d), hipMemcpyDeviceToHost, e->stream));
     ECHK(hipStreamSynchronize(e->stream));
     if (t) *t = c.t;
     if (dt) {
         double m;
-        unsigned long long b = c.dt_bits[c.step & 1];
+        unsigned long long b = tsu::min_dt_bits(d, c.step);
         std::memcpy(&m, &b, 8);
         if (e->P[i].dt_narrow && e->P[i].nvol > 4096) m = (double)(float)m;
         *dt = (m < 1e30) ? m : 1e30;
@@ -560,14 +575,17 @@ TSU_API int tsu_ensemble_snapshot(tsu_ensemble* e, int restore)
         if (restore) return tsu::set_error(TSU_ERR_ARG, "no snapshot taken");
         ECHK(hipMalloc((void**)&e->snapA, e->pool_bytes));
         ECHK(hipMalloc((void**)&e->snapC, e->n * sizeof(Ctrl)));
+        ECHK(hipMalloc((void**)&e->snapD, e->n * sizeof(tsu::DtSlots)));
     }
     if (restore) {
         ECHK(hipMemcpyAsync(e->A, e->snapA, e->pool_bytes, hipMemcpyDeviceToDevice, e->stream));
         ECHK(hipMemcpyAsync(e->B, e->snapA, e->pool_bytes, hipMemcpyDeviceToDevice, e->stream));
         ECHK(hipMemcpyAsync(e->ctrl, e->snapC, e->n * sizeof(Ctrl), hipMemcpyDeviceToDevice, e->stream));
+        ECHK(hipMemcpyAsync(e->dts, e->snapD, e->n * sizeof(tsu::DtSlots), hipMemcpyDeviceToDevice, e->stream));
     } else {
         ECHK(hipMemcpyAsync(e->snapA, e->A, e->pool_bytes, hipMemcpyDeviceToDevice, e->stream));
         ECHK(hipMemcpyAsync(e->snapC, e->ctrl, e->n * sizeof(Ctrl), hipMemcpyDeviceToDevice, e->stream));
+        ECHK(hipMemcpyAsync(e->snapD, e->dts, e->n * sizeof(tsu::DtSlots), hipMemcpyDeviceToDevice, e->stream));
     }
     ECHK(hipStreamSynchronize(e->stream));
     return TSU_OK;

@@ -20,14 +20,40 @@ struct StageArgs {
     int pingpong;         // 1: on odd steps in and out swap roles (single-stage scheme)
     const uint8_t* fix;   // 1 = erodible bed, 0 = fixed
     Ctrl* ctrl;
+    DtSlots* dts;
     double* ext;          // hmax, max H, eta_max planes (nvol each) or null
     int k;                // RK stage index
     int last;             // 1 on the last stage of a step (dt epilogue)
     int tile_rows;
     int nstrips;
     int ntiles;
+    int npx, npy;         // the grid and periodic sides (bit 0 x, bit 1 y) of P
+    int periodic;
     const DevParams* P;   // run constants in device memory
 };
+
+inline int periodic_sides(const DevParams& P)
+{
+    return (P.bc[0] == BC_PERIODIC ? 1 : 0) | (P.bc[2] == BC_PERIODIC ? 2 : 0);
+}
+
+// Every slot at +inf; then, if bits is not +inf, slot 0 of step s at bits.
+inline void reset_dt_slots(DtSlots* d, long long s = 0, unsigned long long bits = kInfBits)
+{
+    for (auto& parity : d->v)
+        for (auto& slot : parity)
+            for (auto& w : slot) w = kInfBits;
+    d->v[s & 1][0][0] = bits;
+}
+
+// Bits of the smallest cell dt of step s.
+inline unsigned long long min_dt_bits(const DtSlots& d, long long s)
+{
+    unsigned long long m = kInfBits;
+    for (auto& slot : d.v[s & 1])
+        if (slot[0] < m) m = slot[0];
+    return m;
+}
 
 // precision: 0 = FP64, 1 = FP32 planes and arithmetic (compensated h, H, hc).  fast_bed:
 // the run constants satisfy fast_bedload (tsu_device.h); with sediment the
@@ -45,12 +71,14 @@ struct BatchMember {
     long long foff;       // mask offset (bytes)
     long long xoff;       // extrema offset (doubles), -1: none
     int tile_rows, nstrips, ntiles, order;
+    int npx, npy, periodic;
 };
 struct BatchPools {
     char* A;              // U^n (stage 2 writes it in place)
     char* B;              // stage-1 result
     const uint8_t* fix;
     Ctrl* ctrl;           // one per member
+    DtSlots* dts;         // one per member
     double* ext;
     const DevParams* P;   // one per member
 };
@@ -58,11 +86,15 @@ struct BatchPools {
 // fast_bed: every member's run constants satisfy fast_bedload.
 hipError_t launch_stage_batch(const BatchPools& pools, const BatchMember* mem, const int2* tiles, int ntiles, int k,
                               int last, bool sed, int precision, hipStream_t s, bool fast_bed = false);
-hipError_t launch_advance_batch(Ctrl* ctrl, const DevParams* P, int n, hipStream_t s);
-hipError_t launch_init_dt(const void* V, const DevParams& P, Ctrl* ctrl, int precision, hipStream_t s);
+hipError_t launch_advance_batch(Ctrl* ctrl, DtSlots* dts, const DevParams* P, int n, hipStream_t s);
+// Smallest cell dt of the state V into step `step`'s slots (armed before).
+hipError_t launch_init_dt(const void* V, const DevParams& P, DtSlots* dts, long long step, int precision,
+                          hipStream_t s);
 hipError_t launch_warmup(hipStream_t s);
 hipError_t launch_copy(const void* src, void* dst, long long bytes, hipStream_t s);
-hipError_t launch_advance(Ctrl* ctrl, const DevParams& P, hipStream_t s);
+// After a step of the single-stage scheme (the two-stage scheme's stages
+// advance the control block themselves).
+hipError_t launch_advance(Ctrl* ctrl, DtSlots* dts, const DevParams& P, hipStream_t s);
 hipError_t launch_fill(double* p, long long n, double v, hipStream_t s);
 // Sums of h and of (H + hc) in FP64 into out[0], out[1] (device pointer),
 // using partial (>= 2 * nblocks doubles) as scratch.

@@ -12,9 +12,11 @@
 //     edge flux is evaluated exactly once per stage;
 //   * the last stage of a step also computes the per-cell CFL dt
 //     (Volume_kernel.cu:19-43), reduces it over the wave with shuffles and
-//     folds it into the device-resident step control block with one 64-bit
-//     atomicMin per wave (Reduction_kernel_min.cu:155-196), so dt never
-//     leaves the device.
+//     folds it into one of 16 device-resident minima with a 64-bit atomicMin
+//     per wave (Reduction_kernel_min.cu:155-196), so dt never leaves the
+//     device;
+//   * the two stages of a step keep t and the step number themselves
+//     (GPU/main_TSUNER.cu:185; see Ctrl).
 //
 // Two arithmetic variants share the code: R = double (reference arithmetic,
 // FP64 planes) and R = float (FP32 planes and fluxes; h, H and hc carried as
@@ -32,8 +34,6 @@
 namespace tsu {
 
 namespace {
-
-constexpr unsigned long long kInfBits = 0x7FF0000000000000ull;
 
 __device__ __forceinline__ int map_index(int i, int n, bool periodic)
 {
@@ -339,44 +339,95 @@ template <typename R, typename S, bool SED, bool FB>
 __device__ __forceinline__ void stage_body(const StageArgs& a, const int tile)
 {
     constexpr bool COMP = sizeof(R) == 4;   // FP32 solver: compensated h, H, hc
+    const int lane = threadIdx.x;
+    const int strip = tile % a.nstrips, chunk = tile / a.nstrips;
+    const int npx = a.npx, npy = a.npy;
+    const bool perx = a.periodic & 1, pery = (a.periodic & 2) != 0;
+    const long long nv = (long long)npx * npy;
+    const int x = strip * kStripOut + lane - 2;
+    const int xc = map_index(x, npx, perx);
+    const int y0 = chunk * a.tile_rows;
+    const int y1 = min(y0 + a.tile_rows, npy);
+    auto row_off = [&](int r) -> long long { return (long long)map_index(r, npy, pery) * npx + xc; };
+
+    // The loads of the run constants, the control block, the dt slots and the
+    // first rows depend on kernel arguments only and are issued together,
+    // before any is used: one after the other they cost four memory
+    // latencies, a good part of a launch on a small grid.
+    constexpr int kPWords = sizeof(DevParams) / 8;
+    static_assert(sizeof(DevParams) % 8 == 0 && kPWords <= 64, "one 8-byte word per lane");
+    unsigned long long pword = 0;
+    if (lane < kPWords) pword = reinterpret_cast<const unsigned long long*>(a.P)[lane];
+    Ctrl* C = a.ctrl;
+    const bool first = a.k == 0;
+    unsigned long long d0 = kInfBits, d1 = kInfBits;
+    if (first) {
+        d0 = a.dts->v[0][lane & (kDtSlots - 1)][0];
+        d1 = a.dts->v[1][lane & (kDtSlots - 1)][0];
+    }
+    const S* in = (const S*)a.in;
+    S* out = (S*)a.out;
+    if (a.pingpong) {
+        if (C->step & 1) {
+            in = (const S*)a.out;
+            out = (S*)a.in;
+        }
+    }
+    const S* Hin = SED ? in + 3 * nv : (const S*)a.Hin;
+    const S* v0p = (a.k == 0) ? in : (const S*)a.v0;
+    const uint8_t* fix = a.fix;
+    Cell<R> Rm, R0, R1;
+    load_cell<R, S, SED>(in, Hin, nv, row_off(y0 - 1), Rm);
+    load_cell<R, S, SED>(in, Hin, nv, row_off(y0), R0);
+    load_cell<R, S, SED>(in, Hin, nv, row_off(y0 + 1), R1);
+    const Ctrl c0 = *C;
+
     // Run constants, copied into LDS once per workgroup (one wave).  Read
     // through the global pointer, every use in the row loop was a vector
     // load, since the kernel's own stores might alias the constants; in LDS
     // they cannot, and a use is a short LDS read.  The loop re-reads them
     // per row (see there) rather than holding them in registers.
     __shared__ DevParams Ps;
-    static_assert(sizeof(DevParams) % 8 == 0 && sizeof(DevParams) <= 64 * 8, "one 8-byte word per lane");
-    if (threadIdx.x < sizeof(DevParams) / 8)
-        reinterpret_cast<unsigned long long*>(&Ps)[threadIdx.x] =
-            reinterpret_cast<const unsigned long long*>(a.P)[threadIdx.x];
+    if (lane < kPWords) reinterpret_cast<unsigned long long*>(&Ps)[lane] = pword;
     __syncthreads();
     const DevParams& P = Ps;
-    const int lane = threadIdx.x;
-    const int strip = tile % a.nstrips, chunk = tile / a.nstrips;
 
-    Ctrl* C = a.ctrl;
-    const double ct = C->t;
-    if (!(ct < C->stop_time) || C->step >= C->stop_step) return;
-    const long long step = C->step;
-    const double dtd = clamp_dt(C, ct, finalize_dt(P, C->dt_bits[step & 1]));
-
-    const int npx = P.npx, npy = P.npy;
-    const long long nv = P.nvol;
-    const S* in = (const S*)a.in;
-    S* out = (S*)a.out;
-    if (a.pingpong && (step & 1)) {
-        in = (const S*)a.out;
-        out = (S*)a.in;
+    // The running step: found by its first stage, read from the control
+    // block by its last (see Ctrl).  The first wave keeps the block.
+    double ct, dtd;
+    long long step;
+    if (first) {
+        ct = c0.t;
+        step = c0.step;
+        const bool run = ct < c0.stop_time && step < c0.stop_step;
+        if (!run) {
+            if (tile == 0 && lane == 0) C->running = 0;
+            return;
+        }
+        double m = __longlong_as_double((long long)((step & 1) ? d1 : d0));
+        for (int o = kDtSlots / 2; o > 0; o >>= 1) m = fmin(m, __shfl_xor(m, o, 64));
+        dtd = clamp_dt(c0, ct, finalize_dt(P, m));
+        if (tile == 0 && !a.last) {
+            if (lane == 0) {
+                C->run_t = ct;
+                C->run_dt = dtd;
+                C->run_step = step;
+                C->running = 1;
+            }
+            // armed for the last stage; step - 1, whose slots they were, is over
+            if (lane < kDtSlots) a.dts->v[(step + 1) & 1][lane][0] = kInfBits;
+        }
+    } else {
+        if (!c0.running) return;
+        ct = c0.run_t;
+        dtd = c0.run_dt;
+        step = c0.run_step;
+        if (tile == 0 && lane == 0) {
+            C->t = next_time(c0.clamp, c0.stop_time, ct, dtd);
+            C->step = step + 1;
+        }
     }
-    const S* Hin = SED ? in + 3 * nv : (const S*)a.Hin;
-    const S* v0p = (a.k == 0) ? in : (const S*)a.v0;
-    const uint8_t* fix = a.fix;
 
-    const bool perx = P.bc[0] == BC_PERIODIC, pery = P.bc[2] == BC_PERIODIC;
-    const int x = strip * kStripOut + lane - 2;
-    const int xc = map_index(x, npx, perx);
-    const int y0 = chunk * a.tile_rows;
-    const int y1 = min(y0 + a.tile_rows, npy);
     const bool out_lane = lane >= 2 && lane < 62 && x < npx;
     const int lim = P.limiter;
     const bool second = P.order == 2;
@@ -389,14 +440,9 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int tile)
     const R dtaxG = (R)(invxd * kG), dtayG = (R)(invyd * kG);   // Reconstructor.cu:197,274
     const R dtFR = (R)(dtd * P.FR);                               // Reconstructor.cu:45
 
-    auto row_off = [&](int r) -> long long { return (long long)map_index(r, npy, pery) * npx + xc; };
     auto fix_at = [&](int r) -> int { return need_fix ? (int)fix[row_off(r)] : 0; };
 
     // ---- prologue: faces of row y0 and the edge y0 - 1/2 -----------------
-    Cell<R> Rm, R0, R1;
-    load_cell<R, S, SED>(in, Hin, nv, row_off(y0 - 1), Rm);
-    load_cell<R, S, SED>(in, Hin, nv, row_off(y0), R0);
-    load_cell<R, S, SED>(in, Hin, nv, row_off(y0 + 1), R1);
     derive_cell<R, SED>(Rm);
     derive_cell<R, SED>(R0);
     derive_cell<R, SED>(R1);
@@ -754,7 +800,8 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int tile)
         lymax = wave_max(lymax);
         const double m = (double)dt_of_speeds(P, lxmax, lymax);
         if (lane == 0 && m < __longlong_as_double((long long)kInfBits))
-            atomicMin(&C->dt_bits[(step + 1) & 1], (unsigned long long)__double_as_longlong(m));
+            atomicMin(&a.dts->v[(step + 1) & 1][tile & (kDtSlots - 1)][0],
+                      (unsigned long long)__double_as_longlong(m));
     }
 }
 
@@ -814,19 +861,23 @@ void stage_kernel_batch(BatchPools pools, const BatchMember* __restrict__ mem, c
     a.Hin = Ai + 3 * m.plane;
     a.fix = pools.fix + m.foff;
     a.ctrl = pools.ctrl + e.x;
+    a.dts = pools.dts + e.x;
     a.ext = m.xoff >= 0 ? pools.ext + m.xoff : nullptr;
     a.k = k;
     a.last = last;
     a.tile_rows = m.tile_rows;
     a.nstrips = m.nstrips;
     a.ntiles = m.ntiles;
+    a.npx = m.npx;
+    a.npy = m.npy;
+    a.periodic = m.periodic;
     a.P = pools.P + e.x;
     stage_body<R, S, SED, FB>(a, e.y);
 }
 
-// GPU/main_TSUNER.cu:147-148: dt of the initial state into dt_bits[step & 1].
+// GPU/main_TSUNER.cu:147-148: dt of the initial state into the step's slots.
 template <typename R, typename S>
-__global__ __launch_bounds__(256) void init_dt_kernel(const S* V, DevParams P, Ctrl* C)
+__global__ __launch_bounds__(256) void init_dt_kernel(const S* V, DevParams P, DtSlots* dts, int parity)
 {
     const long long nv = P.nvol;
     double m = __longlong_as_double((long long)kInfBits);
@@ -834,34 +885,33 @@ __global__ __launch_bounds__(256) void init_dt_kernel(const S* V, DevParams P, C
         m = fmin(m, (double)cell_dt(P, (R)V[i], (R)V[nv + i], (R)V[2 * nv + i]));
     m = wave_min(m);
     if ((threadIdx.x & 63) == 0 && m < __longlong_as_double((long long)kInfBits))
-        atomicMin(&C->dt_bits[C->step & 1], (unsigned long long)__double_as_longlong(m));
+        atomicMin(&dts->v[parity][blockIdx.x & (kDtSlots - 1)][0], (unsigned long long)__double_as_longlong(m));
 }
 
-// GPU/main_TSUNER.cu:185: t += dt after the stages; the dt slot of the
-// finished step is re-armed for step + 2.
-__device__ __forceinline__ void advance_one(Ctrl* C, const DevParams& P)
+// GPU/main_TSUNER.cu:185 for the single-stage scheme: t += dt after the
+// stage; the dt slots of the finished step are re-armed for step + 2.  One
+// wave per control block.
+__device__ __forceinline__ void advance_one(Ctrl* C, DtSlots* dts, const DevParams& P)
 {
-    const double t = C->t;
-    const long long s = C->step;
-    if (!(t < C->stop_time) || s >= C->stop_step) return;
-    const double dt = finalize_dt(P, C->dt_bits[s & 1]);
-    // a clamped step (see clamp_dt) ends exactly on stop_time
-    C->t = (C->clamp && !(dt < C->stop_time - t)) ? C->stop_time : t + dt;
-    C->dt_bits[s & 1] = kInfBits;
-    C->step = s + 1;
+    const Ctrl c = *C;
+    if (!(c.t < c.stop_time) || c.step >= c.stop_step) return;
+    const int lane = threadIdx.x & (kDtSlots - 1);
+    double m = __longlong_as_double((long long)dts->v[c.step & 1][lane][0]);
+    for (int o = kDtSlots / 2; o > 0; o >>= 1) m = fmin(m, __shfl_xor(m, o, 64));
+    const double dt = finalize_dt(P, m);
+    if (threadIdx.x < kDtSlots) dts->v[c.step & 1][lane][0] = kInfBits;
+    if (threadIdx.x == 0) {
+        C->t = next_time(c.clamp, c.stop_time, c.t, dt);
+        C->step = c.step + 1;
+    }
 }
 
-__global__ void advance_kernel(Ctrl* C, DevParams P)
-{
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    advance_one(C, P);
-}
+__global__ __launch_bounds__(64) void advance_kernel(Ctrl* C, DtSlots* dts, DevParams P) { advance_one(C, dts, P); }
 
-// One thread per ensemble member.
-__global__ void advance_batch_kernel(Ctrl* C, const DevParams* __restrict__ P, int n)
+// One workgroup (one wave) per ensemble member.
+__global__ __launch_bounds__(64) void advance_batch_kernel(Ctrl* C, DtSlots* dts, const DevParams* __restrict__ P)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) advance_one(C + i, P[i]);
+    advance_one(C + blockIdx.x, dts + blockIdx.x, P[blockIdx.x]);
 }
 
 __global__ void warmup_kernel() {}
@@ -1094,20 +1144,24 @@ hipError_t launch_stage_batch(const BatchPools& pools, const BatchMember* mem, c
     return hipGetLastError();
 }
 
-hipError_t launch_advance_batch(Ctrl* ctrl, const DevParams* P, int n, hipStream_t s)
+hipError_t launch_advance_batch(Ctrl* ctrl, DtSlots* dts, const DevParams* P, int n, hipStream_t s)
 {
-    hipLaunchKernelGGL(advance_batch_kernel, dim3((n + 63) / 64), dim3(64), 0, s, ctrl, P, n);
+    hipLaunchKernelGGL(advance_batch_kernel, dim3(n), dim3(64), 0, s, ctrl, dts, P);
     return hipGetLastError();
 }
 
-hipError_t launch_init_dt(const void* V, const DevParams& P, Ctrl* ctrl, int precision, hipStream_t s)
+hipError_t launch_init_dt(const void* V, const DevParams& P, DtSlots* dts, long long step, int precision,
+                          hipStream_t s)
 {
     long long nb = (P.nvol + 255) / 256;
     int grid = (int)(nb < 4096 ? (nb > 0 ? nb : 1) : 4096);
+    const int parity = (int)(step & 1);
     if (precision == 0)
-        hipLaunchKernelGGL((init_dt_kernel<double, double>), dim3(grid), dim3(256), 0, s, (const double*)V, P, ctrl);
+        hipLaunchKernelGGL((init_dt_kernel<double, double>), dim3(grid), dim3(256), 0, s, (const double*)V, P, dts,
+                           parity);
     else
-        hipLaunchKernelGGL((init_dt_kernel<float, float>), dim3(grid), dim3(256), 0, s, (const float*)V, P, ctrl);
+        hipLaunchKernelGGL((init_dt_kernel<float, float>), dim3(grid), dim3(256), 0, s, (const float*)V, P, dts,
+                           parity);
     return hipGetLastError();
 }
 
@@ -1127,9 +1181,9 @@ hipError_t launch_copy(const void* src, void* dst, long long bytes, hipStream_t 
     return hipGetLastError();
 }
 
-hipError_t launch_advance(Ctrl* ctrl, const DevParams& P, hipStream_t s)
+hipError_t launch_advance(Ctrl* ctrl, DtSlots* dts, const DevParams& P, hipStream_t s)
 {
-    hipLaunchKernelGGL(advance_kernel, dim3(1), dim3(64), 0, s, ctrl, P);
+    hipLaunchKernelGGL(advance_kernel, dim3(1), dim3(64), 0, s, ctrl, dts, P);
     return hipGetLastError();
 }
 
