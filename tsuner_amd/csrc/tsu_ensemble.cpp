@@ -280,7 +280,6 @@ TSU_API int tsu_ensemble_create(tsu_ensemble** out, int n, const tsu_sim_params*
     e->off.resize(n);
     e->foff.resize(n);
     e->xoff.assign(n, 0);
-    e->rows.assign(n, 16);
     e->uploaded.assign(n, false);
     e->cc.assign(n, nullptr);
     e->tcc.assign(n, nullptr);
@@ -301,6 +300,9 @@ TSU_API int tsu_ensemble_create(tsu_ensemble** out, int n, const tsu_sim_params*
     }
     e->mass_nb = tsu::mass_blocks(maxnv);
     Guard g(device);
+    std::vector<std::pair<int, int>> grids;
+    for (int i = 0; i < n; i++) grids.emplace_back(params[i].npx, params[i].npy);
+    e->rows.assign(n, tsu::choose_tile_rows(grids, tsu::stage_waves_per_simd(e->sed, precision), device));
     hipError_t err = hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking);
     if (err == hipSuccess) err = hipMalloc((void**)&e->A, e->pool_bytes);
     if (err == hipSuccess) err = hipMalloc((void**)&e->B, e->pool_bytes);

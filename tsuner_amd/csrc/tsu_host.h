@@ -2,6 +2,8 @@
 #pragma once
 
 #include <string>
+#include <utility>
+#include <vector>
 
 #include "../../include/tsuner.h"
 #include "tsu_device.h"
@@ -14,5 +16,8 @@ void make_dev_params(const tsu_sim_params* p, const tsu_scheme* s, DevParams* P)
 int validate_scheme(const tsu_scheme* s);
 // Records msg as the calling thread's last error and returns code.
 int set_error(int code, const std::string& msg);
+// Tile height for one launch over grids of (npx, npy) cells with a stage
+// kernel of that many waves per SIMD (tsu_api.cpp).
+int choose_tile_rows(const std::vector<std::pair<int, int>>& grids, int waves_per_simd, int device);
 
 }  // namespace tsu

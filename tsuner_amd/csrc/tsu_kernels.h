@@ -59,6 +59,7 @@ inline unsigned long long min_dt_bits(const DtSlots& d, long long s)
 // the run constants satisfy fast_bedload (tsu_device.h); with sediment the
 // launch then takes the kernel that evaluates bedload among the HLL
 // arithmetic.
+int stage_waves_per_simd(bool sed, int precision);   // the launched kernel's occupancy
 hipError_t launch_stage(const StageArgs& a, bool sed, int precision, hipStream_t s, bool fast_bed = false);
 
 // Ensemble member as seen by the batched stage kernel: byte offsets into

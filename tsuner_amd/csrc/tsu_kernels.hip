@@ -1097,6 +1097,12 @@ __global__ void kat_point_kernel(int what, int law, int n, const double* a, cons
 
 }  // namespace
 
+int stage_waves_per_simd(bool sed, int precision)
+{
+    if (precision != 0) return stage_waves<float, true>();
+    return sed ? stage_waves<double, true>() : stage_waves<double, false>();
+}
+
 hipError_t launch_stage(const StageArgs& a, bool sed, int precision, hipStream_t s, bool fast_bed)
 {
     dim3 grid(a.ntiles), block(64);
