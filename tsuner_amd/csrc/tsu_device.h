@@ -145,6 +145,19 @@ __device__ __forceinline__ int sgn(R x)
     return (rabs(x) < (R)kEpsilon) ? 0 : ((x > (R)0) ? 1 : -1);
 }
 
+// The word that holds the sign, and a value with its sign changed or not (no
+// branch).
+__device__ __forceinline__ int sign_word(double x) { return __double2hiint(x); }
+__device__ __forceinline__ int sign_word(float x) { return __float_as_int(x); }
+__device__ __forceinline__ double flip_sign(double x, bool flip)
+{
+    return __hiloint2double(__double2hiint(x) ^ (flip ? (int)0x80000000u : 0), __double2loint(x));
+}
+__device__ __forceinline__ float flip_sign(float x, bool flip)
+{
+    return __int_as_float(__float_as_int(x) ^ (flip ? (int)0x80000000u : 0));
+}
+
 // Reconstructor.cu:19-31.  When a and b do not share a strict sign the
 // numerator a|b| + b|a| is exactly zero (for finite products), so the
 // division is only evaluated for same-sign slopes; there a|b| and b|a| are
@@ -222,10 +235,12 @@ struct Vel {
 // rsqrt estimate, one Newton step on (g, h) = (x y, y / 2) and two residual
 // corrections, the compiler's own sequence for sqrt() with the scale
 // factors at 1 (they act only below 2^-767).  Equal to sqrt(x) for x in
-// [2^-767, DBL_MAX]; sqrt_unscaled0 also returns 0 for x = 0.
-__device__ __forceinline__ double sqrt_unscaled(double x)
+// [2^-767, DBL_MAX]; sqrt_unscaled0 also returns 0 for x = 0: the estimate is
+// taken of at least the smallest denormal, so that it stays finite and every
+// product with x is 0 (a test for 0 became a branch per square root, ten
+// serial chains in the Riemann solver where one block can interleave them).
+__device__ __forceinline__ double sqrt_newton(double x, double y)
 {
-    const double y = __builtin_amdgcn_rsq(x);
     double g = x * y, h = y * 0.5;
     const double r = fma(-h, g, 0.5);
     g = fma(g, r, g);
@@ -235,7 +250,11 @@ __device__ __forceinline__ double sqrt_unscaled(double x)
     d = fma(-g, g, x);
     return fma(d, h, g);
 }
-__device__ __forceinline__ double sqrt_unscaled0(double x) { return x == 0.0 ? x : sqrt_unscaled(x); }
+__device__ __forceinline__ double sqrt_unscaled(double x) { return sqrt_newton(x, __builtin_amdgcn_rsq(x)); }
+__device__ __forceinline__ double sqrt_unscaled0(double x)
+{
+    return sqrt_newton(x, __builtin_amdgcn_rsq(fmax(x, 0x1p-1074)));
+}
 // x > 0 and below the unscaled square root's range
 __device__ __forceinline__ bool sqrt_needs_scaling(double x) { return x > 0.0 && x < 0x1p-767; }
 
@@ -322,7 +341,71 @@ __device__ __forceinline__ Vel<double> velocity64(double h, double qx, double qy
     return u;
 }
 
-__device__ __forceinline__ Vel<double> velocity(double h, double qx, double qy) { return velocity64(h, qx, qy); }
+// Zero whose register is written where this stands: the zeros of a path that
+// skips its arithmetic, which otherwise are set ahead of the branch on every
+// path (about 70 moves per row of a moving wave).
+__device__ __forceinline__ double zero_here(double z = 0.0)
+{
+    asm volatile("" : "+v"(z));
+    return z;
+}
+__device__ __forceinline__ float zero_here(float z)
+{
+    asm volatile("" : "+v"(z));
+    return z;
+}
+
+// The FP64 solver's own velocities: values of velocity64, with wave-wide
+// votes around the divisions and around the cap instead of a branch per
+// quotient, and selects.
+//
+// The speed cap of an uncapped (u.x, u.y): |u| > 10 m/s is scaled to 10 m/s,
+// and u.s set.
+__device__ __forceinline__ void scale_to_cap(Vel<double>& u, bool over)
+{
+    const Den<double> Dm = den(sqrt(over ? u.s : 1.0));
+    const double x = qdiv(u.x, Dm) * kVmax, y = qdiv(u.y, Dm) * kVmax;
+    u.x = over ? x : u.x;
+    u.y = over ? y : u.y;
+    u.s = u.x * u.x + u.y * u.y;
+}
+__device__ __forceinline__ void cap_speed(Vel<double>& u)
+{
+    u.s = u.x * u.x + u.y * u.y;
+    const bool over = u.s > kVmax2Cut;
+    if (wave_any(over)) scale_to_cap(u, over);
+}
+__device__ __forceinline__ void cap_speeds(Vel<double>& u0, Vel<double>& u1)
+{
+    u0.s = u0.x * u0.x + u0.y * u0.y;
+    u1.s = u1.x * u1.x + u1.y * u1.y;
+    const bool over0 = u0.s > kVmax2Cut, over1 = u1.s > kVmax2Cut;
+    if (wave_any(over0 || over1)) {
+        scale_to_cap(u0, over0);
+        scale_to_cap(u1, over1);
+    }
+}
+
+// velocity64 with D = den(h + DBL_EPSILON) at hand.
+__device__ __forceinline__ Vel<double> velocity_over(double h, double qx, double qy, const Den<double>& D)
+{
+    Vel<double> u;
+    const double x = qdiv(qx, D), y = qdiv(qy, D);
+    const bool wet = h >= kEps;
+    u.x = wet ? x : 0.0;
+    u.y = wet ? y : 0.0;
+    cap_speed(u);
+    return u;
+}
+
+__device__ __forceinline__ Vel<double> velocity(double h, double qx, double qy)
+{
+    if (__builtin_amdgcn_ballot_w64(h >= kEps && (qx != 0.0 || qy != 0.0)) == 0) {
+        const double z = zero_here();
+        return {z, z, z};
+    }
+    return velocity_over(h, qx, qy, den(h + kEpsilon));
+}
 
 // FP32 solver: near-dry cells take the reference's FP64 desingularisation,
 // wet cells a single reciprocal.  rh, when given, is rcp(h + DBL_EPSILON)
@@ -352,25 +435,9 @@ __device__ __forceinline__ Vel<float> velocity(float h, float qx, float qy, cons
     return u;
 }
 
-// Velocity and concentration hc / (h + DBL_EPSILON) of one state
-// (SedFlux.cuh:26-49, 103-132); in FP64 the three quotients share one
-// reciprocal of h + DBL_EPSILON.
-// The speed cap of velocity64 on an uncapped (u.x, u.y): |u| > 10 m/s is
-// scaled to 10 m/s, and u.s set.
-__device__ __forceinline__ void cap_speed(Vel<double>& u)
-{
-    double s = u.x * u.x + u.y * u.y;
-    if (s > kVmax2Cut) {
-        const Den<double> Dm = den(sqrt(s));
-        u.x = qdiv(u.x, Dm) * kVmax;
-        u.y = qdiv(u.y, Dm) * kVmax;
-        s = u.x * u.x + u.y * u.y;
-    }
-    u.s = s;
-}
-
-// velocity_conc for the two sides of an edge at once (values identical):
-// one wave-wide test whether any lane of either side divides, then both
+// Velocity and concentration hc / (h + DBL_EPSILON) (SedFlux.cuh:26-49,
+// 103-132) of the two sides of an edge at once; the three quotients of a side
+// share one reciprocal of h + DBL_EPSILON.  One wave-wide test whether any lane of either side divides, then both
 // sides' reciprocals and quotients for every lane in one basic block, the
 // unused ones discarded by selects (h + DBL_EPSILON is a valid shared
 // denominator for any face depth).  Returns true (uniform over the wave)
@@ -382,41 +449,55 @@ __device__ __forceinline__ bool velocity_conc_pair(double h0, double qx0, double
 {
     const bool nu0 = h0 >= kEps && (qx0 != 0.0 || qy0 != 0.0), nc0 = SED && hc0 != 0.0;
     const bool nu1 = h1 >= kEps && (qx1 != 0.0 || qy1 != 0.0), nc1 = SED && hc1 != 0.0;
-    u0.x = u0.y = u0.s = 0.0;
-    u1.x = u1.y = u1.s = 0.0;
-    c0 = c1 = 0.0;
-    if (__builtin_amdgcn_ballot_w64(nu0 || nc0 || nu1 || nc1) == 0) return true;
+    if (__builtin_amdgcn_ballot_w64(nu0 || nc0 || nu1 || nc1) == 0) {
+        const double z = zero_here();
+        u0 = {z, z, z};
+        u1 = {z, z, z};
+        c0 = c1 = z;
+        return true;
+    }
     const Den<double> D0 = den(h0 + kEpsilon), D1 = den(h1 + kEpsilon);
     const double x0 = qdiv(qx0, D0), y0 = qdiv(qy0, D0);
     const double x1 = qdiv(qx1, D1), y1 = qdiv(qy1, D1);
+    c0 = c1 = 0.0;
     if (SED) {
-        const bool slow = wave_any(qtiny(hc0) || qtiny(hc1));
-        const double k0 = qdiv(hc0, D0, slow), k1 = qdiv(hc1, D1, slow);
-        c0 = nc0 ? k0 : 0.0;
-        c1 = nc1 ? k1 : 0.0;
+        // a zero hc gives the quotient 0
+        c0 = qdiv(hc0, D0);
+        c1 = qdiv(hc1, D1);
+        if (wave_any(qtiny(hc0) || qtiny(hc1))) {
+            c0 = hc0 / D0.d;
+            c1 = hc1 / D1.d;
+        }
     }
-    u0.x = (nu0 && qx0 != 0.0) ? x0 : 0.0;
-    u0.y = (nu0 && qy0 != 0.0) ? y0 : 0.0;
-    u1.x = (nu1 && qx1 != 0.0) ? x1 : 0.0;
-    u1.y = (nu1 && qy1 != 0.0) ? y1 : 0.0;
-    cap_speed(u0);
-    cap_speed(u1);
+    // zero momenta give zero quotients
+    u0.x = h0 >= kEps ? x0 : 0.0;
+    u0.y = h0 >= kEps ? y0 : 0.0;
+    u1.x = h1 >= kEps ? x1 : 0.0;
+    u1.y = h1 >= kEps ? y1 : 0.0;
+    cap_speeds(u0, u1);
     return false;
 }
 
+// The same of one state.
 template <bool SED>
 __device__ __forceinline__ void velocity_conc(double h, double qx, double qy, double hc, Vel<double>& u, double& c)
 {
-    c = 0.0;
     const bool need_u = h >= kEps && (qx != 0.0 || qy != 0.0);
     const bool need_c = SED && hc != 0.0;
-    if (need_u || need_c) {
-        const Den<double> D = den(h + kEpsilon);
-        if (need_c) c = qdiv(hc, D, wave_any(qtiny(hc)));
-        u = velocity64(h, qx, qy, &D);
-    } else {
-        u = velocity64(h, qx, qy);
+    if (__builtin_amdgcn_ballot_w64(need_u || need_c) == 0) {
+        const double z = zero_here();
+        u = {z, z, z};
+        c = z;
+        return;
     }
+    const Den<double> D = den(h + kEpsilon);
+    c = 0.0;
+    if (SED) {
+        c = qdiv(hc, D);
+        if (wave_any(qtiny(hc))) c = hc / D.d;
+        c = need_c ? c : 0.0;
+    }
+    u = velocity_over(h, qx, qy, D);
 }
 
 template <bool SED>
@@ -781,9 +862,13 @@ __device__ __forceinline__ void rp_solve(const DevParams& P, bool bed_mobile, co
         R F04 = hc0 * u0.x, F14 = hc1 * u1.x;
         R df3 = F13 - F03, df4 = F14 - F04;
         R DU4 = hc1 - hc0;
-        int s0 = sgn(e.zr - e.zl), s1 = sgn(df3), s2 = sgn(a1);
-        s1 = (s0 != 0) ? s1 * s0 : 0;
-        R v3 = (s2 == s1) ? a1 * df3 : -a1 * df3;
+        // sgn(a1) == sgn(df3) sgn(dz), as both zero or both not and the
+        // three signs' product positive (masks in scalar registers; a NaN
+        // dz counts as negative, as in sgn)
+        const R dz = e.zr - e.zl, eps = (R)kEpsilon;
+        const bool n1 = !(rabs(df3) < eps) & !(rabs(dz) < eps), n2 = !(rabs(a1) < eps);
+        const bool odd = ((sign_word(a1) ^ sign_word(df3)) < 0) ^ !(dz > zero);
+        const R v3 = flip_sign(a1 * df3, (n1 ^ n2) | (n2 & odd));
         R v4 = rmad(a0, DU4, a1 * df4);
         Dm[3] = rmad(half, df3 - v3, F03);
         Dm[4] = rmad(half, df4 - v4, F04);
@@ -848,8 +933,9 @@ __device__ __forceinline__ void riemann_pair(const DevParams& P, const bool (&mo
         quiet = quiet && q;
     }
     if (quiet && __builtin_amdgcn_ballot_w64(rp_has_jump(e[0]) || rp_has_jump(e[1])) == 0) {
+        const R z = zero_here((R)0);
         for (int i = 0; i < 2; i++)
-            for (int f = 0; f < NF; f++) Dm[i][f] = Dp[i][f] = (R)0;
+            for (int f = 0; f < NF; f++) Dm[i][f] = Dp[i][f] = z;
         return;
     }
     RPSpeeds<R> sp[2];

@@ -151,47 +151,63 @@ __device__ __forceinline__ void derive_cell(Cell<R>& v)
     v.us = u.s;
 }
 
+// Differences b - a of neighbouring cells along an axis (Reconstructor.cu:
+// 146-168): depth, hydrostatic surface, velocity, concentration.  A cell's
+// difference to its plus neighbour is that neighbour's difference to its
+// minus one, so each is evaluated once and handed on (x: by a lane shift, y:
+// to the next row).
+template <typename R>
+struct Diff {
+    R h, eta, ux, uy, c;
+};
+
+template <typename R, bool SED>
+__device__ __forceinline__ Diff<R> cell_diff(const Cell<R>& a, const Cell<R>& b)
+{
+    const R zero = (R)0, zm = rmin(a.H, b.H);
+    Diff<R> d;
+    d.h = b.h - a.h;
+    d.eta = rmax(b.h - b.H + zm, zero) - rmax(a.h - a.H + zm, zero);
+    d.ux = b.ux - a.ux;
+    d.uy = b.uy - a.uy;
+    d.c = SED ? b.c - a.c : zero;
+    return d;
+}
+
 // Reconstructor.cu:146-194 along one axis: faces on the minus side (Fm) and
-// plus side (Fp) of the centre cell from its minus (l) and plus (r)
-// neighbours; returns the limited free-surface slope used by the
+// plus side (Fp) of the centre cell from its differences to its minus (l)
+// and plus (r) neighbours; returns the limited free-surface slope used by the
 // non-conservative source (Reconstructor.cu:197,274).
 template <typename R, bool SED>
-__device__ __forceinline__ R recons_axis(int lim, const Cell<R>& ci, R hl, R Hl, R cl, R ulx, R uly, R hr, R Hr, R cr,
-                                         R urx, R ury, R* Fm, R* Fp)
+__device__ __forceinline__ R recons_axis(int lim, const Cell<R>& ci, const Diff<R>& l, const Diff<R>& r, R* Fm, R* Fp)
 {
     const R half = (R)0.5, zero = (R)0;
     const R hi = ci.h, Hi = ci.H;
-    R dl = hi - hl, dr = hr - hi;
-    R dh = limiter(lim, dl, dr);
-    if (half * rabs(dh) > hi) dh = (R)2.0 * hi * (R)sgn(dh);
+    R dh = limiter(lim, l.h, r.h);
+    const bool steep = half * rabs(dh) > hi;   // shallow water on a slope: at the coast only
+    if (wave_any(steep)) dh = steep ? (R)2.0 * hi * (R)sgn(dh) : dh;
     Fm[0] = hi - half * dh;
     Fp[0] = hi + half * dh;
 
-    R zm = rmin(Hl, Hi);
-    const R dle = rmax(hi - Hi + zm, zero) - rmax(hl - Hl + zm, zero);
-    zm = rmin(Hr, Hi);
-    const R dre = rmax(hr - Hr + zm, zero) - rmax(hi - Hi + zm, zero);
-    const R dlu = ci.ux - ulx, dru = urx - ci.ux;
-    const R dlv = ci.uy - uly, drv = ury - ci.uy;
-    const R dlc = SED ? ci.c - cl : zero, drc = SED ? cr - ci.c : zero;
     R deta, dux, duy, dc = zero;
     if (lim == LIM_MINMOD) {
-        deta = lim_minmod(dle, dre);
-        dux = lim_minmod(dlu, dru);
-        duy = lim_minmod(dlv, drv);
-        if (SED) dc = lim_minmod(dlc, drc);
+        deta = lim_minmod(l.eta, r.eta);
+        dux = lim_minmod(l.ux, r.ux);
+        duy = lim_minmod(l.uy, r.uy);
+        if (SED) dc = lim_minmod(l.c, r.c);
     } else {
         // Free-surface, velocity and concentration slopes all vanish in
         // still water: one wave-wide vote skips their quotients when no lane
         // takes one (the limited slopes are then the limiter's zeros).
-        const bool ue = vl_use(dle, dre), uu = vl_use(dlu, dru), uv = vl_use(dlv, drv);
-        const bool uc = SED && vl_use(dlc, drc);
-        deta = dux = duy = zero;
+        const bool ue = vl_use(l.eta, r.eta), uu = vl_use(l.ux, r.ux), uv = vl_use(l.uy, r.uy);
+        const bool uc = SED && vl_use(l.c, r.c);
         if (__builtin_amdgcn_ballot_w64(ue || uu || uv || uc) != 0) {
-            deta = vl_val(dle, dre, ue);
-            dux = vl_val(dlu, dru, uu);
-            duy = vl_val(dlv, drv, uv);
-            if (SED) dc = vl_val(dlc, drc, uc);
+            deta = vl_val(l.eta, r.eta, ue);
+            dux = vl_val(l.ux, r.ux, uu);
+            duy = vl_val(l.uy, r.uy, uv);
+            if (SED) dc = vl_val(l.c, r.c, uc);
+        } else {
+            deta = dux = duy = dc = zero_here(zero);
         }
     }
     R dz = dh - deta;
@@ -339,6 +355,7 @@ template <typename R, typename S, bool SED, bool FB>
 __device__ __forceinline__ void stage_body(const StageArgs& a, const int tile)
 {
     constexpr bool COMP = sizeof(R) == 4;   // FP32 solver: compensated h, H, hc
+    constexpr bool CARRY = SED;   // a row's differences to the next kept for it (else they spill)
     const int lane = threadIdx.x;
     const int strip = tile % a.nstrips, chunk = tile / a.nstrips;
     const int npx = a.npx, npy = a.npy;
@@ -360,10 +377,10 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int tile)
     if (lane < kPWords) pword = reinterpret_cast<const unsigned long long*>(a.P)[lane];
     Ctrl* C = a.ctrl;
     const bool first = a.k == 0;
-    unsigned long long d0 = kInfBits, d1 = kInfBits;
+    unsigned long long slot0 = kInfBits, slot1 = kInfBits;
     if (first) {
-        d0 = a.dts->v[0][lane & (kDtSlots - 1)][0];
-        d1 = a.dts->v[1][lane & (kDtSlots - 1)][0];
+        slot0 = a.dts->v[0][lane & (kDtSlots - 1)][0];
+        slot1 = a.dts->v[1][lane & (kDtSlots - 1)][0];
     }
     const S* in = (const S*)a.in;
     S* out = (S*)a.out;
@@ -404,7 +421,7 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int tile)
             if (tile == 0 && lane == 0) C->running = 0;
             return;
         }
-        double m = __longlong_as_double((long long)((step & 1) ? d1 : d0));
+        double m = __longlong_as_double((long long)((step & 1) ? slot1 : slot0));
         for (int o = kDtSlots / 2; o > 0; o >>= 1) m = fmin(m, __shfl_xor(m, o, 64));
         dtd = clamp_dt(c0, ct, finalize_dt(P, m));
         if (tile == 0 && !a.last) {
@@ -450,8 +467,11 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int tile)
 
     R D0[5], U0[5], FD0[5];
     R detay0 = (R)0;
+    Diff<R> dm1, d0;   // rows y0 - 1 to y0; row r to r + 1, carried down the tile
     if (second) {
-        detay0 = recons_axis<R, SED>(lim, R0, Rm.h, Rm.H, Rm.c, Rm.ux, Rm.uy, R1.h, R1.H, R1.c, R1.ux, R1.uy, D0, U0);
+        dm1 = cell_diff<R, SED>(Rm, R0);
+        d0 = cell_diff<R, SED>(R0, R1);
+        detay0 = recons_axis<R, SED>(lim, R0, dm1, d0, D0, U0);
         filter_faces<R, SED>(D0, U0);
     } else {
         cell_face(R0, D0);
@@ -467,8 +487,7 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int tile)
             Cell<R> Rmm;
             load_cell<R, S, SED>(in, Hin, nv, row_off(y0 - 2), Rmm);
             derive_cell<R, SED>(Rmm);
-            recons_axis<R, SED>(lim, Rm, Rmm.h, Rmm.H, Rmm.c, Rmm.ux, Rmm.uy, R0.h, R0.H, R0.c, R0.ux, R0.uy, Dd,
-                                Um);
+            recons_axis<R, SED>(lim, Rm, cell_diff<R, SED>(Rmm, Rm), dm1, Dd, Um);
             filter_face<R, SED>(Um);
         } else {
             cell_face(Rm, Um);
@@ -522,16 +541,17 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int tile)
         }
 
         // x faces of row r (Reconstructor.cu:120-197)
-        R hl = up1(R0.h), Hl = up1(R0.H), ulx = up1(R0.ux), uly = up1(R0.uy);
-        R hr = dn1(R0.h), Hr = dn1(R0.H), urx = dn1(R0.ux), ury = dn1(R0.uy);
-        R cl = (R)0, cr = (R)0;
-        if (SED) {
-            cl = up1(R0.c);
-            cr = dn1(R0.c);
-        }
         R Lf[5], Rf[5], detax = (R)0;
         if (second) {
-            detax = recons_axis<R, SED>(lim, R0, hl, Hl, cl, ulx, uly, hr, Hr, cr, urx, ury, Lf, Rf);
+            Cell<R> left;
+            left.h = up1(R0.h);
+            left.H = up1(R0.H);
+            left.ux = up1(R0.ux);
+            left.uy = up1(R0.uy);
+            left.c = SED ? up1(R0.c) : (R)0;
+            const Diff<R> l = cell_diff<R, SED>(left, R0);
+            const Diff<R> rt = {dn1(l.h), dn1(l.eta), dn1(l.ux), dn1(l.uy), SED ? dn1(l.c) : (R)0};
+            detax = recons_axis<R, SED>(lim, R0, l, rt, Lf, Rf);
             filter_faces<R, SED>(Lf, Rf);
         } else {
             cell_face(R0, Lf);
@@ -566,8 +586,10 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int tile)
         derive_cell<R, SED>(R2);
         R D1[5], U1[5], detay1 = (R)0;
         if (second) {
-            detay1 = recons_axis<R, SED>(lim, R1, R0.h, R0.H, R0.c, R0.ux, R0.uy, R2.h, R2.H, R2.c, R2.ux, R2.uy, D1,
-                                         U1);
+            if (!CARRY) d0 = cell_diff<R, SED>(R0, R1);
+            const Diff<R> d1 = cell_diff<R, SED>(R1, R2);
+            detay1 = recons_axis<R, SED>(lim, R1, d0, d1, D1, U1);
+            if (CARRY) d0 = d1;
             filter_faces<R, SED>(D1, U1);
         } else {
             cell_face(R1, D1);
@@ -628,9 +650,10 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int tile)
             } else if (__builtin_amdgcn_ballot_w64(v0[0] >= (R)kEps && (v0[1] != (R)0 || v0[2] != (R)0)) != 0) {
                 Dh = den(v0[0] + (R)kEpsilon);
                 have_dh = true;
-                un = velocity64(v0[0], v0[1], v0[2], &Dh);
+                un = velocity_over(v0[0], v0[1], v0[2], Dh);
             } else {
-                un = velocity64(v0[0], v0[1], v0[2]);   // no lane divides
+                const R z = zero_here((R)0);   // no lane divides
+                un = {z, z, z};
             }
             // |u| of U^n (friction, exchange).  In FP64 a wave at rest (|u| =
             // 0 on every lane) has c = 0 and divides both momenta by 1 + 0 =
