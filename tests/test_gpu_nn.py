@@ -154,6 +154,39 @@ def test_mfma_weight_gradients(width):
 
 
 @pytest.mark.parametrize("width", [32, 64])
+@pytest.mark.parametrize("shape", [(1, 1, 1), (1, 4, 64), (1, 9, 65), (3, 8, 63), (2, 26, 129), None])
+def test_conv_strips_and_stretches(shape, width):
+    """The convolutions walk 64-column strips in passes of 4 or 8 rows through
+    an LDS ring: images smaller than a pass, a column past a strip, rows past
+    a pass, several turns of the ring, and (None) more passes than
+    workgroups, so that stretches start and end inside strips.  Tolerances as
+    for the single kinds (one BF16 rounding step; FP32 output 1e-5)."""
+    rng = np.random.default_rng(15)
+    s = C.c_void_p(0)
+    f, W = (W64 if width == 64 else 0), width
+    for kind, k, m in [(0, 8, W), (1, W, W), (2, W, 4), (3, 8, W), (4, W, W)]:
+        n, h, w = shape or ((58 if k == 8 else 15), 45, 150)
+        x = rand_bf16(rng, (n, h, w, k))
+        rows = 16 if kind == 2 else m
+        wt = rand_bf16(rng, (9, rows, k), 0.2)
+        wt[:, m:] = 0
+        b = rng.normal(0, 0.1, size=64).astype(np.float32)
+        act = np.maximum(rand_bf16(rng, (n, h, w, m)), 0)
+        out = torch.full((n * h * w * m,), 9.0, dtype=torch.float32 if kind == 2 else torch.bfloat16, device="cuda")
+        ok(lib().tsu_nn_conv(kind | f, P(dev_bf16(x)), P(dev_bf16(wt)), P(dev_f32(b)), P(dev_bf16(act)), P(out), n, h,
+                             w, s))
+        got = host(out).reshape(n, h, w, m)
+        if kind >= 3:      # the kernel's weights are the per-tap transposes: out[p] = sum_t wt[t] in[p - off(t)]
+            ref = O.conv_input_grad(x, np.transpose(wt, (0, 2, 1))) * (act > 0)
+        else:
+            ref = O.conv(x, wt[:, :m], b[:m])
+        if kind == 2:
+            np.testing.assert_allclose(got, ref, rtol=0, atol=1e-5 * np.abs(ref).max())
+        else:
+            assert_bf16_close(got, O.bf16((np.maximum(ref, 0) if kind < 2 else ref).astype(np.float32)))
+
+
+@pytest.mark.parametrize("width", [32, 64])
 @pytest.mark.parametrize("shape", [(1, 1, 1), (1, 4, 64), (1, 9, 65), (3, 8, 63), (2, 17, 130), (15, 45, 150)])
 def test_weight_gradient_strips_and_stretches(shape, width):
     """The weight-gradient kernels walk 64-column strips in passes of 4 or 8

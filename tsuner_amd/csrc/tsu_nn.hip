@@ -8,8 +8,8 @@
 // Every convolution is computed transposed, D^T[m][p] = sum_k Wt[m][k] X^T[k][p]
 // with m = output channel and p = pixel, so that both MFMA operands are
 // 16-byte vectors along the channel axis of an NHWC row (weights [tap][m][k],
-// activations [pixel][k]) and each lane's four results are four consecutive
-// output channels of one pixel (one 8-byte store).  The K axis of an MFMA
+// activations [pixel][k]) and each lane's results are consecutive output
+// channels of one pixel.  The K axis of an MFMA
 // (32 values) is four "octets" of 8 channels; octet o of the flattened
 // (tap, channel) axis is tap o / (K/8), channels 8*(o % (K/8)) + 0..7, so an
 // 8-channel layer packs four taps into one MFMA and a 32-channel layer one
@@ -41,181 +41,95 @@ __device__ __forceinline__ bf16x8 as_bf16x8(uint4 v) { return __builtin_bit_cast
 __device__ __forceinline__ int tap_dy(int t) { return t / 3 - 1; }
 __device__ __forceinline__ int tap_dx(int t) { return t % 3 - 1; }
 
+// ---- walking down strips -----------------------------------------------------
+//
+// Every convolution kernel walks down strips of 64 columns, R rows per pass,
+// with its input rows in an LDS ring: a row is loaded once per strip (plus two
+// at the top of a stretch), and the next pass's rows are loaded into registers
+// while the MFMAs run on the current ones.  The passes of all strips of all
+// images, in order, are cut into one contiguous stretch per workgroup.
+constexpr int kStripCols = 64;
+
+// The stretch of one workgroup: `left` passes from image n, column c0, row r0.
+struct StripWalk {
+    long long left;
+    int n, c0, r0;
+    int H, W;
+    __device__ StripWalk(int N, int H_, int W_, int R) : H(H_), W(W_)
+    {
+        const int segs = (W + kStripCols - 1) / kStripCols, passes = (H + R - 1) / R;
+        const long long total = (long long)N * segs * passes;
+        long long i = total * blockIdx.x / gridDim.x;
+        left = total * (blockIdx.x + 1) / gridDim.x - i;
+        r0 = (int)(i % passes) * R;
+        i /= passes;
+        c0 = (int)(i % segs) * kStripCols;
+        n = (int)(i / segs);
+    }
+    // to the next pass; true if it continues the strip
+    __device__ bool next(int R)
+    {
+        r0 += R;
+        if (r0 < H) return true;
+        r0 = 0;
+        c0 += kStripCols;
+        if (c0 >= W) {
+            c0 = 0;
+            n++;
+        }
+        return false;
+    }
+};
+
+// Barrier for LDS only: the workgroup's waves share nothing in global memory,
+// and __syncthreads() would wait for every store of the pass to reach memory
+// (8 -> 64 channels, 32 images: 107 us with it).
+__device__ __forceinline__ void lds_barrier()
+{
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
 // out[p][m] = post( sum_t sum_k in[p + SIGN*off(t)][k] * Wt[t][m][k] )
-//   K: input channels (8 or 32), M: output channels held by the weights
-//   (multiple of 16), MOUT: channels stored per output pixel.
+//   K: input channels (8, 32 or 64), MOUT: channels stored per output pixel,
+//   M = 16 MTW MG: output channels held by the weights.
 //   POST 0: + bias, ReLU, BF16 out.  1: + bias, FP32 out.  2: zero where
 //   act[p][m] == 0 (ReLU derivative), BF16 out.
-// A workgroup of 4 waves covers 4 consecutive rows x 64 columns of one
-// image, one row per wave.  The input rows r0-1 .. r0+4 and columns
-// c0-1 .. c0+64 are staged in LDS once (zeros outside the image: the 'same'
-// padding), so every tap's B operand is one 16-byte LDS read instead of a
-// global load re-fetched by nine taps and three waves.
-constexpr int kConvRows = 4;
-constexpr int kTileRows = kConvRows + 2, kTileCols = 64 + 2;
-
-// LDS slot of octet q of tile pixel p: the 16 lanes of a ds_read_b128 read
-// the same octet of 16 consecutive pixels, which with KO octets per pixel
-// are KO*16 bytes apart and would share banks; XOR-ing q with the pixel's
-// bits above log2(16/KO) spreads them over all 64 banks.
-template <int KO>
-__device__ __forceinline__ int swz(int p, int q)
+//
+// A pass is R = 4 rows of 64 columns (more with 8 input channels, whose passes
+// are short beside a load's latency, taken four rows at a time: 8 -> 64 for 32
+// images 106 us with 4 rows, 70 with 8).  A wave covers
+// 16 columns x RW = 4 / RG rows x 16 MTW output channels and keeps its weights of all nine taps in
+// registers (144 for 64 channels in and 32 out), so that only the input is
+// read from LDS, and each 16-byte read of an input row serves the output rows
+// above, at and below it: one read per four MFMAs of 64 -> 64 and 32 -> 32
+// channels.  The workgroup has 4 waves side by side, times MG groups of
+// output channels, times RG groups of rows.  With two tiles of output
+// channels, row 4g + e of tile a is channel 8g + 4a + e, so that a lane's
+// results are eight consecutive channels of a pixel, one 16-byte store.
+//
+// Bound by the bytes of both tensors for the narrow layers and by how well the
+// MFMAs, the epilogue and the loads of one workgroup overlap for 64 -> 64
+// (matrix pipe 52 % busy).  Before (weights and a 10 x 66 pixel tile in LDS, one
+// read per two MFMAs, the tile's loads and stores between barriers) and now, us:
+//            8->32  32->32  32->4  8->64  64->64  64->4, and the data
+//   32 images  41     89     48    106     200     95    gradients 4<-32 60,
+//   of 256^2   27     49     44     70     163     70    32<-32 103, 4<-64 181,
+//   8 images   14     25     14     28      55     27    64<-64 259 -> 53, 97,
+//              10     17     12     16      47     21    124, 215 (32 images)
+// 32 -> 32 moves 268 MB in 49 us, 5.5 TB/s of the copy kernel's 6.1.  Accumulation
+// order and results are those of one tap after the other.
+//
+// LDS: the ring is three blocks of a pass's rows and copies of its first two
+// rows behind them, so that the R + 2 rows of a pass lie in order wherever it
+// starts and a read's row is an immediate.  A pixel's octets are XOR-ed with bits of its column:
+// the 16 lanes of a read (one octet of 16 consecutive pixels) cover all banks.
+template <int K>
+__device__ __forceinline__ int octet_xor(int c)
 {
-    return q ^ ((p / (16 / KO)) & (KO - 1));
+    return K == 64 ? (c >> 1) & 7 : K == 32 ? (c >> 2) & 3 : 0;
 }
-
-template <int K, int M, int MOUT, int SIGN, int POST>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void conv_kernel(const uint16_t* __restrict__ in, const uint16_t* __restrict__ Wt,
-                                                   const float* __restrict__ bias, const uint16_t* __restrict__ act,
-                                                   void* __restrict__ out, int N, int H, int W)
-{
-    constexpr int KO = K / 8;                  // octets per tap
-    constexpr int STEPS = (9 * KO + 3) / 4;    // MFMAs per (m-tile, n-tile)
-    constexpr int MT = M / 16;
-    constexpr int TILE = kTileRows * kTileCols * KO;
-    constexpr int PER_THREAD = (TILE + 255) / 256;
-    constexpr int AHEAD = 2;                   // weight operands prefetched this many steps ahead
-    __shared__ uint4 tile[TILE];
-    const int segs = (W + 63) / 64, rblocks = (H + kConvRows - 1) / kConvRows;
-    long long blk = blockIdx.x;
-    const int seg = (int)(blk % segs);
-    blk /= segs;
-    const int r0 = (int)(blk % rblocks) * kConvRows;
-    const long long n = blk / rblocks;
-    if (n >= N) return;
-    const int c0 = seg * 64;
-    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int g = lane >> 4, li = lane & 15;
-
-    // weight operands of step s: A[a] = Wt[t][a*16 + li][8q .. 8q+7] for this
-    // lane's octet o = 4s + g (t = o / KO, q = o % KO; zero past the 9 taps)
-    auto load_a = [&](int s, bf16x8* A) {
-        const int o = 4 * s + g;
-        const int t = o / KO, q = o % KO;
-#pragma unroll
-        for (int a = 0; a < MT; a++) {
-            uint4 v = make_uint4(0, 0, 0, 0);
-            if (t < 9) v = *(const uint4*)(Wt + ((size_t)(t * M + a * 16 + li) * K + 8 * q));
-            A[a] = as_bf16x8(v);
-        }
-    };
-    // the first steps' weights are in flight while the input tile is staged
-    bf16x8 Abuf[AHEAD + 1][MT];
-#pragma unroll
-    for (int s = 0; s < AHEAD && s < STEPS; s++) load_a(s, Abuf[s]);
-
-    // input tile, in batches of up to 7 loads per thread, each batch's loads
-    // issued before its LDS stores
-    constexpr int BATCH = PER_THREAD < 7 ? PER_THREAD : 7;
-#pragma unroll
-    for (int j0 = 0; j0 < PER_THREAD; j0 += BATCH) {
-        uint4 stage[BATCH];
-#pragma unroll
-        for (int j = 0; j < BATCH; j++) {
-            const int idx = threadIdx.x + 256 * (j0 + j);
-            const int q = idx % KO, rest = idx / KO;
-            const int gc = c0 - 1 + rest % kTileCols, gr = r0 - 1 + rest / kTileCols;
-            stage[j] = make_uint4(0, 0, 0, 0);
-            if (j0 + j < PER_THREAD && idx < TILE && gr >= 0 && gr < H && gc >= 0 && gc < W)
-                stage[j] = *(const uint4*)(in + (((size_t)n * H + gr) * W + gc) * K + 8 * q);
-        }
-#pragma unroll
-        for (int j = 0; j < BATCH; j++) {
-            const int idx = threadIdx.x + 256 * (j0 + j);
-            const int q = idx % KO, rest = idx / KO;
-            if (j0 + j < PER_THREAD && idx < TILE) tile[rest * KO + swz<KO>(rest, q)] = stage[j];
-        }
-    }
-    __syncthreads();
-    const int r = r0 + wv;
-    if (r >= H) return;                        // no barrier follows
-    const long long row = n * H + r;
-
-    f32x4 acc[MT][4];
-#pragma unroll
-    for (int a = 0; a < MT; a++)
-#pragma unroll
-        for (int b = 0; b < 4; b++) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-#pragma unroll
-    for (int s = 0; s < STEPS; s++) {
-        if (s + AHEAD < STEPS) load_a(s + AHEAD, Abuf[(s + AHEAD) % (AHEAD + 1)]);
-        const bf16x8* A = Abuf[s % (AHEAD + 1)];
-        const int o = 4 * s + g;               // this lane's octet
-        const int t = o / KO, q = o % KO;
-        const bool tv = t < 9;
-        const int dy = SIGN * tap_dy(t), dx = SIGN * tap_dx(t);
-        const int lrow = (wv + 1 + dy) * kTileCols + 1 + dx + li;
-#pragma unroll
-        for (int b = 0; b < 4; b++) {
-            uint4 v = make_uint4(0, 0, 0, 0);
-            if (tv) v = tile[(lrow + b * 16) * KO + swz<KO>(lrow + b * 16, q)];
-            const bf16x8 B = as_bf16x8(v);
-#pragma unroll
-            for (int a = 0; a < MT; a++)
-                acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[a], B, acc[a][b], 0, 0, 0);
-        }
-    }
-
-#pragma unroll
-    for (int b = 0; b < 4; b++) {
-        const int c = c0 + b * 16 + li;
-        if (c >= W) continue;
-        const size_t p = (size_t)row * W + c;
-#pragma unroll
-        for (int a = 0; a < MT; a++) {
-            const int m0 = a * 16 + 4 * g;
-            if (m0 >= MOUT) continue;
-            float v[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) v[i] = acc[a][b][i];
-            if (POST == 0 || POST == 1) {
-#pragma unroll
-                for (int i = 0; i < 4; i++) v[i] += bias[m0 + i];
-            }
-            if (POST == 0) {
-#pragma unroll
-                for (int i = 0; i < 4; i++) v[i] = fmaxf(v[i], 0.f);
-            }
-            if (POST == 1) {
-                *(float4*)((float*)out + p * MOUT + m0) = make_float4(v[0], v[1], v[2], v[3]);
-            } else {
-                if (POST == 2) {
-                    const uint2 av = *(const uint2*)(act + p * MOUT + m0);
-                    // ReLU outputs are >= 0: only +0 / -0 bit patterns mean inactive
-                    if ((av.x & 0x7FFFu) == 0) v[0] = 0.f;
-                    if ((av.x & 0x7FFF0000u) == 0) v[1] = 0.f;
-                    if ((av.y & 0x7FFFu) == 0) v[2] = 0.f;
-                    if ((av.y & 0x7FFF0000u) == 0) v[3] = 0.f;
-                }
-                uint2 st;
-                st.x = (uint32_t)to_bf16(v[0]) | ((uint32_t)to_bf16(v[1]) << 16);
-                st.y = (uint32_t)to_bf16(v[2]) | ((uint32_t)to_bf16(v[3]) << 16);
-                *(uint2*)((uint16_t*)out + p * MOUT + m0) = st;
-            }
-        }
-    }
-}
-
-// Convolutions of the wide (64-channel) network: 64 -> 64 (middle layers
-// and their data gradients), 8 -> 64 (input layer) and 64 -> 4 (output
-// layer).  Same arithmetic and operand layout as conv_kernel, arranged so
-// that neither memory latency nor address arithmetic bounds it:
-//   * the layer's weights are staged in LDS once per workgroup, as
-//     [tap][octet][output channel] 16-byte rows, so a step's A operands are
-//     LDS reads (16 lanes read 16 consecutive rows);
-//   * the input tile is planar by octet, [octet][pixel]: the 16 lanes of a
-//     read take 16 consecutive pixels (256 contiguous bytes, no bank
-//     conflicts) and a tap's pixel offset is a constant, so with the steps
-//     unrolled every LDS address is a per-lane base plus an immediate;
-//   * a workgroup of 8 waves covers 8 rows x 64 columns, one row per wave
-//     (two waves per SIMD hide each other's LDS latency);
-//   * workgroups are persistent (one per CU: for 64 -> 64 the weights and
-//     the 10 x 66 pixel input tile fill 155 KB of the 160 KB LDS) and load
-//     the next tile's input into registers while computing the current one.
-constexpr int kWideRows = 8;
-constexpr int kWideTileRows = kWideRows + 2;
-constexpr int kWidePix = kWideTileRows * kTileCols;          // 660 pixels per tile
 
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -226,161 +140,214 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float a, float b)
     return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, bf16x2));
 }
 
-template <int K, int M, int MOUT, int SIGN, int POST>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void conv_wide_kernel(
+// max(x, 0), 0 for a NaN, in one instruction (fmaxf quiets its operand first)
+__device__ __forceinline__ float relu(float x) { return __builtin_amdgcn_fmed3f(x, 0.f, __builtin_inff()); }
+
+// waves per SIMD: what the registers allow (weights + accumulators + input)
+template <int K>
+constexpr int conv_waves() { return K == 8 ? 4 : 2; }
+
+// rows of a pass, and of the ring: three blocks of them, and the copies
+template <int K>
+constexpr int conv_rows() { return K == 8 ? 8 : 4; }
+constexpr int conv_ring(int rows) { return 3 * rows + 2; }
+
+template <int K, int MTW, int MG, int RG, int MOUT, int SIGN, int POST>
+__global__ __launch_bounds__(256 * MG * RG)
+__attribute__((amdgpu_waves_per_eu(conv_waves<K>(), conv_waves<K>()))) void conv_kernel(
     const uint16_t* __restrict__ in, const uint16_t* __restrict__ Wt, const float* __restrict__ bias,
     const uint16_t* __restrict__ act, void* __restrict__ out, int N, int H, int W)
 {
-    constexpr int KO = K / 8, MT = M / 16;
-    constexpr int STEPS = (9 * KO + 3) / 4;
-    constexpr bool TAP_UNIFORM = KO >= 4;                    // a step's 4 octets lie in one tap
-    constexpr int TILE = KO * kWidePix;
-    constexpr int WSLOTS = 9 * KO * M;
-    constexpr int PER_THREAD = (TILE + 511) / 512;
-    constexpr int WPER = (WSLOTS + 511) / 512;
-    constexpr int SLOTS = PER_THREAD > WPER ? PER_THREAD : WPER;
-    __shared__ uint4 wl[WSLOTS];
-    __shared__ uint4 tile[TILE];
-    const int segs = (W + 63) / 64, rblocks = (H + kWideRows - 1) / kWideRows;
-    const long long nblk = (long long)N * rblocks * segs;
-    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    constexpr int T = 256 * MG * RG, R = conv_rows<K>(), RW = 4 / RG, M = 16 * MTW * MG;
+    constexpr int KO = K / 8, KK = K == 8 ? 1 : K / 32;
+    constexpr int XCOL = kStripCols + 2, XROW = XCOL * KO;  // ring row, in uint4
+    constexpr int SLOTS = kStripCols * KO;                  // a row's octets but for the last two columns'
+    constexpr int SWEEP = T / SLOTS;                        // rows per sweep of the workgroup
+    constexpr int LOADS = SWEEP >= R ? 1 : R / SWEEP;
+    constexpr int STEPS = K == 8 ? 3 : 9 * KK;
+    static_assert(T % SLOTS == 0 && 2 * KO * R <= T, "one slot per thread and sweep");
+    __shared__ uint4 ring[conv_ring(R) * XROW];
+    const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int g = lane >> 4, li = lane & 15;
-    if ((long long)blockIdx.x >= nblk) return;              // whole workgroup, before any barrier
+    const int seg = wv & 3, mg = (wv >> 2) % MG, rg = (wv >> 2) / MG;
+    StripWalk walk(N, H, W, R);
 
-    uint4 stage[SLOTS];
-    // weights: global [tap][m][k] -> LDS [tap][octet][m]
+    // weights: step (offset ry, rx; 32 channels kk) of input offset (ry - 1,
+    // rx - 1), tap 3 ry + rx, or its opposite for the data gradients.  With 8
+    // channels a step holds four offsets, one per lane group.
+    bf16x8 A[STEPS][MTW];
 #pragma unroll
-    for (int j = 0; j < WPER; j++) {
-        const int idx = threadIdx.x + 512 * j;              // over (tap, m, octet), octet fastest
-        if (idx < WSLOTS) stage[j] = *(const uint4*)(Wt + (size_t)idx * 8);
-    }
+    for (int s = 0; s < STEPS; s++)
 #pragma unroll
-    for (int j = 0; j < WPER; j++) {
-        const int idx = threadIdx.x + 512 * j;
-        const int q = idx % KO, m = (idx / KO) % M, t = idx / (KO * M);
-        if (idx < WSLOTS) wl[(t * KO + q) * M + m] = stage[j];
-    }
+        for (int a = 0; a < MTW; a++) {
+            const int o = K == 8 ? 4 * s + g : s / KK, k = K == 8 ? 0 : 32 * (s % KK) + 8 * g;
+            const int t = SIGN > 0 ? o : 8 - o;
+            const int m = 16 * MTW * mg + (MTW == 2 ? 8 * (li >> 2) + 4 * a + (li & 3) : li);
+            uint4 v = make_uint4(0, 0, 0, 0);
+            if (o < 9) v = *(const uint4*)(Wt + ((size_t)(t * M + m) * K + k));
+            A[s][a] = as_bf16x8(v);
+        }
+    const int m0 = 16 * MTW * mg + 4 * MTW * g;             // this lane's 4 MTW consecutive output channels
+    f32x4 bias_of[MTW];
+#pragma unroll
+    for (int a = 0; a < MTW; a++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) bias_of[a][e] = POST == 2 ? 0.f : bias[m0 + 4 * a + e];
 
-    auto origin = [&](long long b, long long& n, int& r0, int& c0) {
-        c0 = (int)(b % segs) * 64;
-        b /= segs;
-        r0 = (int)(b % rblocks) * kWideRows;
-        n = b / rblocks;
+    // staging: this thread's octet and column (and row, if a sweep takes
+    // several), and one of the last two columns' for the first threads
+    const int q = tid % KO, col = tid / KO % kStripCols, row = SWEEP > 1 ? tid / SLOTS : 0;
+    const int put_at = row * XROW + col * KO + (q ^ octet_xor<K>(col));
+    const bool has_edge = tid < 2 * KO * R;
+    const int ecol = kStripCols + tid / KO % 2, erow = tid / (2 * KO);
+    const int eput_at = erow * XROW + ecol * KO + (q ^ octet_xor<K>(ecol));
+    uint4 stage[LOADS], estage;
+    auto load = [&](int gr, int gc) {                       // zeros outside the image
+        uint4 v = make_uint4(0, 0, 0, 0);
+        if (gr >= 0 && gr < H && gc >= 0 && gc < W)
+            v = *(const uint4*)((const char*)in + ((size_t)walk.n * H + gr) * W * (2 * K) +
+                                (uint32_t)((gc * K + 8 * q) * 2));
+        return v;
     };
-    auto fetch = [&](long long b) {
-        long long n;
-        int r0, c0;
-        origin(b, n, r0, c0);
+    // the pass's new rows, r0 + 1 .. r0 + R (columns c0 - 1 .. c0 + 64), into registers
+    auto fetch = [&]() {
 #pragma unroll
-        for (int j = 0; j < PER_THREAD; j++) {
-            const int idx = threadIdx.x + 512 * j;          // over (pixel, octet), octet fastest
-            const int q = idx % KO, pix = idx / KO;
-            const int gc = c0 - 1 + pix % kTileCols, gr = r0 - 1 + pix / kTileCols;
-            stage[j] = make_uint4(0, 0, 0, 0);
-            if (idx < TILE && gr >= 0 && gr < H && gc >= 0 && gc < W)
-                stage[j] = *(const uint4*)(in + (((size_t)n * H + gr) * W + gc) * K + 8 * q);
+        for (int j = 0; j < LOADS; j++)
+            if (SWEEP <= R || row < R) stage[j] = load(walk.r0 + 1 + j * SWEEP + row, walk.c0 - 1 + col);
+        if (has_edge) estage = load(walk.r0 + 1 + erow, walk.c0 - 1 + ecol);
+    };
+    // ... and into ring rows R ph + 2 .. R ph + R + 1; the last two of block 2
+    // are also the first two of block 0
+    auto put = [&](int ph) {
+#pragma unroll
+        for (int j = 0; j < LOADS; j++) {
+            const int r = j * SWEEP + row;
+            if (SWEEP <= R || row < R) {
+                ring[(R * ph + 2 + j * SWEEP) * XROW + put_at] = stage[j];
+                if (ph == 2 && r >= R - 2) ring[(j * SWEEP - (R - 2)) * XROW + put_at] = stage[j];
+            }
+        }
+        if (has_edge) {
+            ring[(R * ph + 2) * XROW + eput_at] = estage;
+            if (ph == 2 && erow >= R - 2) ring[-(R - 2) * XROW + eput_at] = estage;
         }
     };
-    auto put = [&]() {
-#pragma unroll
-        for (int j = 0; j < PER_THREAD; j++) {
-            const int idx = threadIdx.x + 512 * j;
-            const int q = idx % KO, pix = idx / KO;
-            if (idx < TILE) tile[q * kWidePix + pix] = stage[j];
+    // at the top of a stretch or strip: rows r0 - 1 and r0 into ring rows 0, 1
+    auto top = [&]() {
+        for (int idx = tid; idx < 2 * XROW; idx += T) {
+            const int o = idx % KO, c = idx / KO % XCOL, i = idx / XROW;
+            const int gr = walk.r0 - 1 + i, gc = walk.c0 - 1 + c;
+            uint4 v = make_uint4(0, 0, 0, 0);
+            if (gr >= 0 && gr < H && gc >= 0 && gc < W)
+                v = *(const uint4*)(in + (((size_t)walk.n * H + gr) * W + gc) * K + 8 * o);
+            ring[i * XROW + c * KO + (o ^ octet_xor<K>(c))] = v;
         }
     };
 
-    long long blk = blockIdx.x;
-    fetch(blk);
-    put();
-    __syncthreads();
-    // per-lane bases: this lane's pixel (row wv + 1, column 1 + li) and octet g
-    const uint4* tbase = tile + g * kWidePix + (wv + 1) * kTileCols + 1 + li;
-    const uint4* wbase = wl + g * M + li;
+    // this lane's reads in the first of the wave's rows: column 16 seg + li +
+    // rx, octet 4 kk + g; with 8 channels, the offset of step rx and lane group g
+    int at[3][KK];
+#pragma unroll
+    for (int rx = 0; rx < 3; rx++)
+#pragma unroll
+        for (int kk = 0; kk < KK; kk++) {
+            const int o = 4 * rx + g < 9 ? 4 * rx + g : 8;
+            const int cl = 16 * seg + li + (K == 8 ? o % 3 : rx);
+            at[rx][kk] = (RW * rg + (K == 8 ? o / 3 : 0)) * XROW + cl * KO + ((K == 8 ? 0 : 4 * kk + g) ^ octet_xor<K>(cl));
+        }
+
+    int ph = 0;                                             // ring row of input row r0 - 1, over R
+    fetch();
+    top();
+    put(0);
+    lds_barrier();
     for (;;) {
-        const long long next = blk + gridDim.x;
-        const bool more = next < nblk;                       // uniform over the workgroup
-        if (more) fetch(next);                               // in flight during the MFMAs
-        long long n;
-        int r0, c0;
-        origin(blk, n, r0, c0);
-        f32x4 acc[MT][4];
-#pragma unroll
-        for (int a = 0; a < MT; a++)
-#pragma unroll
-            for (int b = 0; b < 4; b++) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int s = 0; s < STEPS; s++) {
-            // octet o = 4s + g: tap t = o / KO, octet q = o % KO; with
-            // TAP_UNIFORM, t and q - g are constants of the step
-            bf16x8 A[MT];
-            const int t = TAP_UNIFORM ? (4 * s) / KO : (4 * s + g) / KO;
-            const int q = TAP_UNIFORM ? (4 * s) % KO + g : (4 * s + g) % KO;
-            const bool tv = t < 9;
-            const int d = SIGN * (tap_dy(t) * kTileCols + tap_dx(t));   // tap's pixel offset
-#pragma unroll
-            for (int a = 0; a < MT; a++) {
-                uint4 v = make_uint4(0, 0, 0, 0);
-                if (TAP_UNIFORM)
-                    v = wbase[((4 * s) / KO * KO + (4 * s) % KO) * M + a * 16];
-                else if (tv)
-                    v = wl[(t * KO + q) * M + a * 16 + li];
-                A[a] = as_bf16x8(v);
-            }
-#pragma unroll
-            for (int b = 0; b < 4; b++) {
-                uint4 v = make_uint4(0, 0, 0, 0);
-                if (TAP_UNIFORM)
-                    v = tbase[((4 * s) % KO) * kWidePix + d + b * 16];
-                else if (tv)
-                    v = tile[q * kWidePix + (wv + 1) * kTileCols + 1 + li + d + b * 16];
-                const bf16x8 B = as_bf16x8(v);
-#pragma unroll
-                for (int a = 0; a < MT; a++)
-                    acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[a], B, acc[a][b], 0, 0, 0);
-            }
+        int cr0 = walk.r0 + RW * rg;                        // this pass: the wave's first row, this lane's column
+        const int c = walk.c0 + 16 * seg + li;
+        size_t p0 = ((size_t)walk.n * H + cr0) * W + c;
+        const bool more = --walk.left > 0;                  // uniform over the workgroup
+        bool down = false;                                  // the next pass continues this strip
+        if (more) {
+            down = walk.next(R);
+            fetch();
         }
+        const uint4* rows = ring + R * ph * XROW;
+#pragma unroll 1
+        for (int part = 0; part < R / 4; part++) {
+            f32x4 acc[RW][MTW];
 #pragma unroll
-        for (int b = 0; b < 4; b++) {
-            const int r = r0 + wv, c = c0 + b * 16 + li;
-            if (r >= H || c >= W) continue;
-            const size_t p = ((size_t)n * H + r) * W + c;
+            for (int r = 0; r < RW; r++)
 #pragma unroll
-            for (int a = 0; a < MT; a++) {
-                const int m0 = a * 16 + 4 * g;
-                if (m0 >= MOUT) continue;
-                float v[4];
+                for (int a = 0; a < MTW; a++) acc[r][a] = f32x4{0.f, 0.f, 0.f, 0.f};
+            // by input row: an output row then takes its taps in their order
+            // (and with 8 channels, a row's steps, whose offsets the lanes hold)
 #pragma unroll
-                for (int i = 0; i < 4; i++) v[i] = acc[a][b][i];
-                if (POST == 0 || POST == 1) {
+            for (int j = 0; j < (K == 8 ? RW : RW + 2); j++)
 #pragma unroll
-                    for (int i = 0; i < 4; i++) v[i] += bias[m0 + i];
-                }
-                if (POST == 0) {
+                for (int rx = 0; rx < 3; rx++)
 #pragma unroll
-                    for (int i = 0; i < 4; i++) v[i] = fmaxf(v[i], 0.f);
-                }
-                if (POST == 1) {
+                    for (int kk = 0; kk < KK; kk++) {
+                        uint4 v = rows[at[rx][kk] + j * XROW];
+                        if (K == 8 && rx == 2 && g > 0) v = make_uint4(0, 0, 0, 0);   // past the ninth offset
+                        const bf16x8 B = as_bf16x8(v);
+#pragma unroll
+                        for (int ry = 0; ry < (K == 8 ? 1 : 3); ry++) {
+                            const int r = j - ry;
+                            if (r < 0 || r >= RW) continue;
+#pragma unroll
+                            for (int a = 0; a < MTW; a++)
+                                acc[r][a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                                    A[K == 8 ? rx : (3 * ry + rx) * KK + kk][a], B, acc[r][a], 0, 0, 0);
+                        }
+                    }
+#pragma unroll
+            for (int r = 0; r < RW; r++) {
+                if (cr0 + r >= H || c >= W || m0 >= MOUT) continue;
+                const size_t p = p0 + (size_t)r * W;
+                float v[4 * MTW];
+#pragma unroll
+                for (int a = 0; a < MTW; a++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const float o = POST == 2 ? acc[r][a][e] : acc[r][a][e] + bias_of[a][e];
+                        v[4 * a + e] = POST == 0 ? relu(o) : o;
+                    }
+                if constexpr (POST == 1) {
+                    static_assert(MTW == 1, "one tile of output channels");
                     *(float4*)((float*)out + p * MOUT + m0) = make_float4(v[0], v[1], v[2], v[3]);
                 } else {
+                    static_assert(MTW == 2, "16-byte stores");
                     if (POST == 2) {
-                        const uint2 av = *(const uint2*)(act + p * MOUT + m0);
+                        // (loading it ahead of the MFMAs costs registers: 21
+                        // spilled with 64 channels, 50 -> 76 us for 8 images)
+                        const uint4 av = *(const uint4*)(act + p * MOUT + m0);
+                        const uint32_t aw[4] = {av.x, av.y, av.z, av.w};
                         // ReLU outputs are >= 0: only +0 / -0 bit patterns mean inactive
-                        if ((av.x & 0x7FFFu) == 0) v[0] = 0.f;
-                        if ((av.x & 0x7FFF0000u) == 0) v[1] = 0.f;
-                        if ((av.y & 0x7FFFu) == 0) v[2] = 0.f;
-                        if ((av.y & 0x7FFF0000u) == 0) v[3] = 0.f;
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            if ((aw[e] & 0x7FFFu) == 0) v[2 * e] = 0.f;
+                            if ((aw[e] & 0x7FFF0000u) == 0) v[2 * e + 1] = 0.f;
+                        }
                     }
-                    *(uint2*)((uint16_t*)out + p * MOUT + m0) = make_uint2(pack_bf16x2(v[0], v[1]),
-                                                                           pack_bf16x2(v[2], v[3]));
+                    *(uint4*)((uint16_t*)out + p * MOUT + m0) =
+                        make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]),
+                                   pack_bf16x2(v[6], v[7]));
                 }
             }
+            rows += 4 * XROW;
+            cr0 += 4;
+            p0 += 4 * (size_t)W;
         }
-        __syncthreads();                                     // every wave is done reading the tile
         if (!more) break;
-        put();
-        __syncthreads();
-        blk = next;
+        if (down) {
+            ph = ph == 2 ? 0 : ph + 1;                      // the coming rows have ring rows of their own
+        } else {
+            lds_barrier();                                // every wave is done with the ring
+            ph = 0;
+            top();
+        }
+        put(ph);
+        lds_barrier();
     }
 }
 
@@ -418,7 +385,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // wave reads then lie in different banks.  The eight pixels of lane group g
 // in a 32-pixel step are 4g .. 4g+3 and 16+4g .. 16+4g+3, for both operands.
 
-constexpr int kWgradCols = 64;             // columns of a strip
 constexpr int kWgradPitch = 72;            // LDS columns of the shifted operand's rows (66 used)
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
@@ -451,29 +417,6 @@ __device__ __forceinline__ int slot_xor(int c)
     return CH == 64 ? (c >> 1) & 3 : CH == 32 ? (c >> 2) & 1 : 0;
 }
 
-// The passes of one workgroup: strip pass i of column (n, seg) starts at row
-// R * (i % passes).
-struct WgradWalk {
-    long long first, last;      // passes [first, last)
-    int segs, passes;           // strips per image, passes per strip
-    int H, W;
-    __device__ WgradWalk(int N, int H_, int W_, int R) : H(H_), W(W_)
-    {
-        segs = (W + kWgradCols - 1) / kWgradCols;
-        passes = (H + R - 1) / R;
-        const long long total = (long long)N * segs * passes;
-        first = total * blockIdx.x / gridDim.x;
-        last = total * (blockIdx.x + 1) / gridDim.x;
-    }
-    __device__ void at(long long i, int R, int& n, int& c0, int& r0) const
-    {
-        r0 = (int)(i % passes) * R;
-        i /= passes;
-        c0 = (int)(i % segs) * kWgradCols;
-        n = (int)(i / segs);
-    }
-};
-
 // Middle layers (x and dy of CH = 32 or 64 channels).  Each of 8 waves holds
 // the nine taps of 32 x 32 channels (CH = 64: four such jobs, two waves of a
 // job taking half of a pass's pixels each; CH = 32: one job, eight waves),
@@ -489,7 +432,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     constexpr int R = 4;                           // rows per pass
     constexpr int KO = CH / 8, PIX = CH * 2;
     constexpr int XR = 2 * R + 2, DR = 2 * R;      // ring rows: R + 2 in use and R coming, R and R
-    constexpr int XROW = kWgradPitch * PIX, DROW = kWgradCols * PIX;
+    constexpr int XROW = kWgradPitch * PIX, DROW = kStripCols * PIX;
     constexpr int JOBS = (CH / 32) * (CH / 32), GROUPS = 8 / JOBS;
     constexpr int STEPS = 2 * R / GROUPS;          // 32-pixel steps of a wave per pass
     constexpr int XPT = (R * 66 * KO + 511) / 512, DPT = R * 64 * KO / 512;
@@ -503,7 +446,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int g = lane >> 4, li = lane & 15;
     const int job = wv % JOBS, group = wv / JOBS;
     const int m0 = 2 * (job / (CH / 32)), k0 = 2 * (job % (CH / 32));   // first 16-channel tiles
-    const WgradWalk walk(N, H, W, R);
+    StripWalk walk(N, H, W, R);
 
     f32x4 acc[TILES];                              // [tap][k tile][m tile], then the bias of the m tiles
 #pragma unroll
@@ -577,19 +520,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
     // ring row of x row r0 - 1 and of dy row r0
     int xs = 0, ds = 0;
-    int n, c0, r0;
-    walk.at(walk.first, R, n, c0, r0);
-    fetch(n, c0, r0);
-    top(n, c0, r0);
+    fetch(walk.n, walk.c0, walk.r0);
+    top(walk.n, walk.c0, walk.r0);
     put(xs, ds);
     __syncthreads();
-    for (long long i = walk.first; i < walk.last; i++) {
-        const bool more = i + 1 < walk.last;               // uniform over the workgroup
+    for (;;) {
+        const bool more = --walk.left > 0;                  // uniform over the workgroup
         bool down = false;                                  // the next pass continues this strip
         if (more) {
-            walk.at(i + 1, R, n, c0, r0);
-            down = r0 != 0;
-            fetch(n, c0, r0);
+            down = walk.next(R);
+            fetch(walk.n, walk.c0, walk.r0);
         }
 #pragma unroll 1
         for (int s = 0; s < STEPS; s++) {
@@ -630,7 +570,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         } else {
             __syncthreads();                                // every wave is done with the rings
             xs = ds = 0;
-            top(n, c0, r0);
+            top(walk.n, walk.c0, walk.r0);
         }
         put(xs, ds);
         __syncthreads();
@@ -690,14 +630,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     constexpr int R = 8;
     constexpr int KO = CH / 8, MT = CH / 16, PIX = CH * 2;
     constexpr int XR = 2 * R + 2, DR = 2 * R;
-    constexpr int XROW = kWgradPitch * 16, DROW = kWgradCols * PIX;
+    constexpr int XROW = kWgradPitch * 16, DROW = kStripCols * PIX;
     constexpr int XPT = (R * 66 + 511) / 512, DPT = R * 64 * KO / 512;
     constexpr int XN = XR * XROW / 16, DN = DR * DROW / 16;
     __shared__ uint4 lds[XN + DN];
     const uint32_t xbase = (uint32_t)(uintptr_t)(lds_u4*)lds, dbase = xbase + XN * 16;
     const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int g = lane >> 4, li = lane & 15;
-    const WgradWalk walk(N, H, W, R);
+    StripWalk walk(N, H, W, R);
 
     f32x4 acc[5][MT], bacc;
 #pragma unroll
@@ -771,19 +711,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     };
 
     int xs = 0, ds = 0;
-    int n, c0, r0;
-    walk.at(walk.first, R, n, c0, r0);
-    fetch(n, c0, r0);
-    top(n, c0, r0);
+    fetch(walk.n, walk.c0, walk.r0);
+    top(walk.n, walk.c0, walk.r0);
     put(xs, ds);
     __syncthreads();
-    for (long long i = walk.first; i < walk.last; i++) {
-        const bool more = i + 1 < walk.last;
+    for (;;) {
+        const bool more = --walk.left > 0;
         bool down = false;
         if (more) {
-            walk.at(i + 1, R, n, c0, r0);
-            down = r0 != 0;
-            fetch(n, c0, r0);
+            down = walk.next(R);
+            fetch(walk.n, walk.c0, walk.r0);
         }
         uint32_t xo[5];                                     // narrow row wv + (shift's row), per lane
 #pragma unroll
@@ -819,7 +756,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         } else {
             __syncthreads();
             xs = ds = 0;
-            top(n, c0, r0);
+            top(walk.n, walk.c0, walk.r0);
         }
         put(xs, ds);
         __syncthreads();
@@ -1257,62 +1194,54 @@ hipError_t nn_launch_target(const StageArgs* fine, const StageArgs* coarse, int 
 }
 
 namespace {
-// conv_wide_kernel's persistent grid: one workgroup per CU (its LDS holds one),
-// at most one per tile.
-dim3 wide_grid(int N, int H, int W)
+// One workgroup per stretch of passes, as many as the chip holds at once.
+template <int K, int MTW, int MG, int RG, int MOUT, int SIGN, int POST>
+hipError_t launch_conv(const uint16_t* in, const uint16_t* w, const float* bias, const uint16_t* act, void* out, int N,
+                       int H, int W, hipStream_t s)
 {
-    static int cus = 0;
-    if (cus == 0) {
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
-            cus = 256;
-    }
-    const long long tiles = (long long)N * ((H + kWideRows - 1) / kWideRows) * ((W + 63) / 64);
-    return dim3((unsigned)(tiles < cus ? tiles : cus));
+    constexpr int R = conv_rows<K>(), lds = conv_ring(R) * (kStripCols + 2) * K * 2;
+    // by LDS (160 KB) and by waves per SIMD
+    constexpr int by_lds = 163840 / lds, by_waves = conv_waves<K>() / (MG * RG);
+    constexpr int per_cu = by_lds < by_waves ? by_lds : (by_waves > 0 ? by_waves : 1);
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
+        cus = 256;
+    const long long passes = (long long)N * ((W + kStripCols - 1) / kStripCols) * ((H + R - 1) / R);
+    const long long most = (long long)cus * per_cu;
+    conv_kernel<K, MTW, MG, RG, MOUT, SIGN, POST><<<(unsigned)(passes < most ? passes : most), 256 * MG * RG, 0, s>>>(
+        in, w, bias, act, out, N, H, W);
+    return hipGetLastError();
 }
 }  // namespace
 
 hipError_t nn_launch_conv(int kind, const uint16_t* in, const uint16_t* w, const float* bias, const uint16_t* act,
                           void* out, int N, int H, int W, hipStream_t s)
 {
-    const long long blocks = (long long)N * ((H + kConvRows - 1) / kConvRows) * ((W + 63) / 64);
-    const dim3 grid((unsigned)blocks), block(256);
     switch (kind) {
     case NN_FWD_IN:      // 8 -> 32, ReLU
-        conv_kernel<8, 32, 32, 1, 0><<<grid, block, 0, s>>>(in, w, bias, act, out, N, H, W);
-        break;
+        return launch_conv<8, 2, 1, 1, 32, 1, 0>(in, w, bias, act, out, N, H, W, s);
     case NN_FWD_MID:     // 32 -> 32, ReLU
-        conv_kernel<32, 32, 32, 1, 0><<<grid, block, 0, s>>>(in, w, bias, act, out, N, H, W);
-        break;
+        return launch_conv<32, 2, 1, 1, 32, 1, 0>(in, w, bias, act, out, N, H, W, s);
     case NN_FWD_OUT:     // 32 -> 4 (weights padded to 16 rows), FP32 out
-        conv_kernel<32, 16, 4, 1, 1><<<grid, block, 0, s>>>(in, w, bias, act, out, N, H, W);
-        break;
+        return launch_conv<32, 1, 1, 1, 4, 1, 1>(in, w, bias, act, out, N, H, W, s);
     case NN_DGRAD_OUT:   // dy 8 channels (4 used) -> dx 32, ReLU mask
-        conv_kernel<8, 32, 32, -1, 2><<<grid, block, 0, s>>>(in, w, bias, act, out, N, H, W);
-        break;
+        return launch_conv<8, 2, 1, 1, 32, -1, 2>(in, w, bias, act, out, N, H, W, s);
     case NN_DGRAD_MID:   // dy 32 -> dx 32, ReLU mask
-        conv_kernel<32, 32, 32, -1, 2><<<grid, block, 0, s>>>(in, w, bias, act, out, N, H, W);
-        break;
+        return launch_conv<32, 2, 1, 1, 32, -1, 2>(in, w, bias, act, out, N, H, W, s);
     case NN_FWD_IN | NN_W64:
-        conv_wide_kernel<8, 64, 64, 1, 0><<<wide_grid(N, H, W), 512, 0, s>>>(in, w, bias, act, out, N, H, W);
-        break;
+        return launch_conv<8, 2, 2, 1, 64, 1, 0>(in, w, bias, act, out, N, H, W, s);
     case NN_FWD_MID | NN_W64:
-        conv_wide_kernel<64, 64, 64, 1, 0><<<wide_grid(N, H, W), 512, 0, s>>>(in, w, bias, act, out, N, H, W);
-        break;
+        return launch_conv<64, 2, 2, 1, 64, 1, 0>(in, w, bias, act, out, N, H, W, s);
     case NN_FWD_OUT | NN_W64:
-        conv_wide_kernel<64, 16, 4, 1, 1><<<wide_grid(N, H, W), 512, 0, s>>>(in, w, bias, act, out, N, H, W);
-        break;
+        return launch_conv<64, 1, 1, 2, 4, 1, 1>(in, w, bias, act, out, N, H, W, s);
     case NN_DGRAD_OUT | NN_W64:
-        conv_wide_kernel<8, 64, 64, -1, 2><<<wide_grid(N, H, W), 512, 0, s>>>(in, w, bias, act, out, N, H, W);
-        break;
+        return launch_conv<8, 2, 2, 1, 64, -1, 2>(in, w, bias, act, out, N, H, W, s);
     case NN_DGRAD_MID | NN_W64:
-        conv_wide_kernel<64, 64, 64, -1, 2><<<wide_grid(N, H, W), 512, 0, s>>>(in, w, bias, act, out, N, H, W);
-        break;
+        return launch_conv<64, 2, 2, 1, 64, -1, 2>(in, w, bias, act, out, N, H, W, s);
     default:
         return hipErrorInvalidValue;
     }
-    return hipGetLastError();
 }
 
 hipError_t nn_launch_wgrad(int kind, const uint16_t* x, const uint16_t* dy, float* part, float* bpart, float* dw,
@@ -1323,7 +1252,7 @@ hipError_t nn_launch_wgrad(int kind, const uint16_t* x, const uint16_t* dy, floa
     const int width = (kind & NN_W64) ? 64 : 32, base = kind & ~NN_W64;
     const bool mid = base == NN_WGRAD_MID;
     const int rows = mid ? 4 : 8;                       // rows per pass (R of the kernels)
-    const long long passes = (long long)N * ((W + kWgradCols - 1) / kWgradCols) * ((H + rows - 1) / rows);
+    const long long passes = (long long)N * ((W + kStripCols - 1) / kStripCols) * ((H + rows - 1) / rows);
     const int waves = (int)(passes < kWgradWaves ? passes : kWgradWaves);
     int my = width, kx = width;
     switch (kind) {
