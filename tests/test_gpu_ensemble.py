@@ -139,3 +139,25 @@ def test_inflow_member_without_series_is_refused():
     with pytest.raises(_lib.TsuError) as e:
         Ensemble([sc], precision="fp32")
     assert "tsu_ensemble_set_inflow" in str(e.value)
+
+
+@pytest.mark.parametrize("n", [1, 2, 3])
+@pytest.mark.parametrize("order", [1, 2])
+@pytest.mark.parametrize("chunk", [0, 4])
+def test_halves_on_two_streams_equal_single_solver(n, order, chunk):
+    """One member (one half), two, and three of unequal sizes; calls that
+    enqueue whole chunks, a remainder and a single step, with work on the
+    ensemble's stream (a mass sum) between them."""
+    scs = [S.gaussian_source(n=k, dx=40.0, seed=k, order=order) for k in (48, 130, 61)][:n]
+    ens = Ensemble(scs, precision="fp32", graph_chunk=chunk)
+    masses = []
+    for k in (9, 1, 4, 0):
+        ens.step(k, sync=False)
+        masses.append([ens.mass(i) for i in range(n)])
+    for i, sc in enumerate(scs):
+        g = Solver.from_scenario(sc, precision="fp32")
+        for k, m in zip((9, 1, 4, 0), masses):
+            g.step(k)
+            assert g.mass() == m[i]
+        assert np.array_equal(ens.state(i), g.state()), "member %d" % i
+        assert ens.time(i) == g.time()

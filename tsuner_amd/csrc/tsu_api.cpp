@@ -154,7 +154,7 @@ int set_error(int code, const std::string& msg) { return fail(code, msg); }
 // r + 0.87 rows per tile, until a run's own latency shows: the hypotenuse of
 // the work and half of the time alone.
 //
-// An ensemble brings its own parallelism and is judged alone, a single grid
+// Half an ensemble (what steps on one stream) is judged alone, a single grid
 // by the product of both.  The constants are fits to sweeps of the height
 // over 36 grids of 100^2 .. 4096^2 cells in both precisions, with and without
 // sediment, alone and beside two others.  Against powers of two from 32 down

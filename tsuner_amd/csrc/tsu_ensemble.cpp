@@ -1,14 +1,16 @@
 // tsu_ensemble.cpp -- many independent scenarios on grids of uneven size,
-// advanced together: one stage launch covers every tile of every member
-// (stage_kernel_batch), each member keeps its own buffers, run constants and
-// step-control block (so its own dt and time), and whole-ensemble steps are
-// replayed from a captured HIP graph.  The reference runs one scenario per
+// advanced together: one stage launch covers every tile of half the members
+// (stage_kernel_batch), the other half's beside it on a second stream, each
+// member keeps its own buffers, run constants and step-control block (so its
+// own dt and time), and each half's steps are replayed from a captured HIP
+// graph.  The reference runs one scenario per
 // process (GPU/main_TSUNER.cu:21-222); this is the batched form of that loop.
 #define TSU_BUILDING_LIBRARY 1
 #include "../../include/tsuner.h"
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <climits>
 #include <cmath>
 #include <cstring>
@@ -61,14 +63,17 @@ struct tsu_ensemble {
     DevParams* dP = nullptr;
     tsu::StageArgs* dargs = nullptr;    // [2][n]: stage 0 and stage 1 arguments (hooks)
     tsu::BatchMember* dmem = nullptr;   // [n]: members as the batched stage kernel sees them
-    int2* tiles = nullptr;
-    int ntiles = 0;
+    int2* tiles = nullptr;          // the first half's tiles, then the second's
+    int ntiles[2] = {0, 0};
+    std::vector<int> half;          // 0 or 1 per member (see split_members)
     double* mass_buf = nullptr;
     int mass_nb = 0;
     hipStream_t stream = nullptr;
+    hipStream_t stream2 = nullptr;  // the second half's steps; joined to stream when a call returns
+    hipEvent_t forked = nullptr, joined = nullptr;
     int graph_chunk = 0;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t gexec = nullptr;
+    hipGraph_t graph[2] = {nullptr, nullptr};
+    hipGraphExec_t gexec[2] = {nullptr, nullptr};
 };
 
 namespace {
@@ -88,10 +93,12 @@ struct Guard {
 
 void drop_graph(tsu_ensemble* e)
 {
-    if (e->gexec) (void)hipGraphExecDestroy(e->gexec);
-    if (e->graph) (void)hipGraphDestroy(e->graph);
-    e->gexec = nullptr;
-    e->graph = nullptr;
+    for (int h = 0; h < 2; h++) {
+        if (e->gexec[h]) (void)hipGraphExecDestroy(e->gexec[h]);
+        if (e->graph[h]) (void)hipGraphDestroy(e->graph[h]);
+        e->gexec[h] = nullptr;
+        e->graph[h] = nullptr;
+    }
 }
 
 void destroy(tsu_ensemble* e)
@@ -99,6 +106,7 @@ void destroy(tsu_ensemble* e)
     if (!e) return;
     Guard g(e->device);
     drop_graph(e);
+    if (e->stream2) (void)hipStreamSynchronize(e->stream2);
     if (e->stream) (void)hipStreamSynchronize(e->stream);
     (void)hipFree(e->A);
     (void)hipFree(e->B);
@@ -116,12 +124,37 @@ void destroy(tsu_ensemble* e)
     (void)hipFree(e->mass_buf);
     for (double* p : e->cc) (void)hipFree(p);
     for (double* p : e->tcc) (void)hipFree(p);
+    if (e->forked) (void)hipEventDestroy(e->forked);
+    if (e->joined) (void)hipEventDestroy(e->joined);
+    if (e->stream2) (void)hipStreamDestroy(e->stream2);
     if (e->stream) (void)hipStreamDestroy(e->stream);
     delete e;
 }
 
 int nstrips(const tsu_ensemble* e, int i) { return (e->p[i].npx + tsu::kStripOut - 1) / tsu::kStripOut; }
 int nchunks(const tsu_ensemble* e, int i) { return (e->p[i].npy + e->rows[i] - 1) / e->rows[i]; }
+
+// Members in two halves of about equal cell counts, the largest first, each
+// to the smaller half.  The halves step on streams of their own: where one
+// half's stage runs out of tiles, the other's fill the chip.  In one launch
+// per stage the last round of tiles left it half empty, and two stages of a
+// step cannot overlap.  Eight members of 2.2 million cells in FP32: 146 ->
+// 107 us a step; three parts 112, four 144 (they share hardware queues).  A
+// single member is one part.  Members do not read each other, so results are
+// the same.
+void split_members(tsu_ensemble* e)
+{
+    std::vector<int> order((size_t)e->n);
+    for (int i = 0; i < e->n; i++) order[(size_t)i] = i;
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return e->P[a].nvol > e->P[b].nvol; });
+    long long cells[2] = {0, 0};
+    e->half.assign((size_t)e->n, 0);
+    for (int i : order) {
+        const int h = cells[1] < cells[0];
+        e->half[(size_t)i] = h;
+        cells[h] += e->P[i].nvol;
+    }
+}
 
 // Per-member stage arguments and the tile table (member, tile) for the
 // current tile heights.
@@ -141,6 +174,7 @@ int build_launch_tables(tsu_ensemble* e)
         bm.nstrips = nstrips(e, i);
         bm.ntiles = bm.nstrips * nchunks(e, i);
         bm.order = e->s[i].order;
+        bm.half = e->half[(size_t)i];
         bm.npx = e->P[i].npx;
         bm.npy = e->P[i].npy;
         bm.periodic = tsu::periodic_sides(e->P[i]);
@@ -176,13 +210,16 @@ int build_launch_tables(tsu_ensemble* e)
             }
             args[(size_t)k * e->n + i] = a;
         }
-        const int nt = args[i].ntiles;
-        for (int t = 0; t < nt; t++) tiles.push_back(make_int2(i, t));
+    }
+    for (int h = 0; h < 2; h++) {
+        const size_t before = tiles.size();
+        for (int i = 0; i < e->n; i++)
+            for (int t = 0; e->half[(size_t)i] == h && t < args[i].ntiles; t++) tiles.push_back(make_int2(i, t));
+        e->ntiles[h] = (int)(tiles.size() - before);
     }
     drop_graph(e);
     (void)hipFree(e->tiles);
     e->tiles = nullptr;
-    e->ntiles = (int)tiles.size();
     ECHK(hipMalloc((void**)&e->tiles, tiles.size() * sizeof(int2)));
     ECHK(hipMemcpy(e->tiles, tiles.data(), tiles.size() * sizeof(int2), hipMemcpyHostToDevice));
     ECHK(hipMemcpy(e->dargs, args.data(), args.size() * sizeof(tsu::StageArgs), hipMemcpyHostToDevice));
@@ -190,17 +227,67 @@ int build_launch_tables(tsu_ensemble* e)
     return TSU_OK;
 }
 
-int enqueue_step(tsu_ensemble* e)
+hipStream_t half_stream(const tsu_ensemble* e, int h) { return h ? e->stream2 : e->stream; }
+
+// One step of a half's members, on the half's stream.
+int enqueue_step(tsu_ensemble* e, int h)
 {
     const int order = e->s[0].order;
     const tsu::BatchPools pools{e->A, e->B, e->fix, e->ctrl, e->dts, e->ext, e->dP};
+    const int2* tiles = e->tiles + (h ? e->ntiles[0] : 0);
     bool fast_bed = true;
     for (int i = 0; i < e->n; i++) fast_bed = fast_bed && tsu::fast_bedload(e->P[i]);
     for (int k = 0; k < order; k++)
-        ECHK(tsu::launch_stage_batch(pools, e->dmem, e->tiles, e->ntiles, k, k == order - 1, e->sed, e->precision,
-                                     e->stream, fast_bed));
-    if (order == 1) ECHK(tsu::launch_advance_batch(e->ctrl, e->dts, e->dP, e->n, e->stream));
+        ECHK(tsu::launch_stage_batch(pools, e->dmem, tiles, e->ntiles[h], k, k == order - 1, e->sed, e->precision,
+                                     half_stream(e, h), fast_bed));
+    if (order == 1) ECHK(tsu::launch_advance_batch(e->ctrl, e->dts, e->dP, e->dmem, e->n, h, half_stream(e, h)));
     return TSU_OK;
+}
+
+// A half's graph of graph_chunk steps.
+int capture_steps(tsu_ensemble* e, int h)
+{
+    ECHK(hipStreamBeginCapture(half_stream(e, h), hipStreamCaptureModeThreadLocal));
+    for (int k = 0; k < e->graph_chunk; k++) {
+        if (int rc = enqueue_step(e, h)) {
+            hipGraph_t gph = nullptr;
+            (void)hipStreamEndCapture(half_stream(e, h), &gph);
+            if (gph) (void)hipGraphDestroy(gph);
+            return rc;
+        }
+    }
+    ECHK(hipStreamEndCapture(half_stream(e, h), &e->graph[h]));
+    ECHK(hipGraphInstantiate(&e->gexec[h], e->graph[h], nullptr, nullptr, 0));
+    return TSU_OK;
+}
+
+// nsteps steps of every member behind the work on e->stream; work enqueued on
+// it afterwards comes after them.  With graphs, whole chunks are replayed.
+int enqueue_steps(tsu_ensemble* e, int nsteps, bool graphs)
+{
+    const int halves = e->ntiles[1] > 0 ? 2 : 1;
+    graphs = graphs && e->graph_chunk > 0 && nsteps >= e->graph_chunk;
+    if (graphs)
+        for (int h = 0; h < halves; h++)
+            if (!e->gexec[h])
+                if (int rc = capture_steps(e, h)) return rc;
+    if (nsteps == 0) return TSU_OK;
+    if (halves == 2) {
+        ECHK(hipEventRecord(e->forked, e->stream));
+        ECHK(hipStreamWaitEvent(e->stream2, e->forked, 0));
+    }
+    int rc = TSU_OK, done = 0;
+    for (; graphs && rc == TSU_OK && nsteps - done >= e->graph_chunk; done += e->graph_chunk)
+        for (int h = 0; h < halves && rc == TSU_OK; h++)
+            if (hipError_t er = hipGraphLaunch(e->gexec[h], half_stream(e, h)))
+                rc = tsu::set_error(TSU_ERR_HIP, std::string("graph launch: ") + hipGetErrorString(er));
+    for (; rc == TSU_OK && done < nsteps; done++)
+        for (int h = 0; h < halves && rc == TSU_OK; h++) rc = enqueue_step(e, h);
+    if (halves == 2) {   // after an error too: what was enqueued is waited for
+        ECHK(hipEventRecord(e->joined, e->stream2));
+        ECHK(hipStreamWaitEvent(e->stream, e->joined, 0));
+    }
+    return rc;
 }
 
 int member_ok(const tsu_ensemble* e, int i)
@@ -300,10 +387,21 @@ TSU_API int tsu_ensemble_create(tsu_ensemble** out, int n, const tsu_sim_params*
     }
     e->mass_nb = tsu::mass_blocks(maxnv);
     Guard g(device);
-    std::vector<std::pair<int, int>> grids;
-    for (int i = 0; i < n; i++) grids.emplace_back(params[i].npx, params[i].npy);
-    e->rows.assign(n, tsu::choose_tile_rows(grids, tsu::stage_waves_per_simd(e->sed, precision), device));
+    split_members(e);
+    e->rows.assign(n, 1);
+    for (int h = 0; h < 2; h++) {
+        std::vector<std::pair<int, int>> grids;
+        for (int i = 0; i < n; i++)
+            if (e->half[(size_t)i] == h) grids.emplace_back(params[i].npx, params[i].npy);
+        if (grids.empty()) continue;
+        const int rows = tsu::choose_tile_rows(grids, tsu::stage_waves_per_simd(e->sed, precision), device);
+        for (int i = 0; i < n; i++)
+            if (e->half[(size_t)i] == h) e->rows[(size_t)i] = rows;
+    }
     hipError_t err = hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking);
+    if (err == hipSuccess && n > 1) err = hipStreamCreateWithFlags(&e->stream2, hipStreamNonBlocking);
+    if (err == hipSuccess && n > 1) err = hipEventCreateWithFlags(&e->forked, hipEventDisableTiming);
+    if (err == hipSuccess && n > 1) err = hipEventCreateWithFlags(&e->joined, hipEventDisableTiming);
     if (err == hipSuccess) err = hipMalloc((void**)&e->A, e->pool_bytes);
     if (err == hipSuccess) err = hipMalloc((void**)&e->B, e->pool_bytes);
     if (err == hipSuccess) err = hipMalloc((void**)&e->fix, e->fix_bytes);
@@ -478,29 +576,7 @@ TSU_API int tsu_ensemble_step(tsu_ensemble* e, int nsteps)
     if (nsteps < 0) return tsu::set_error(TSU_ERR_ARG, "negative step count");
     if (int rc = members_ready(e)) return rc;
     Guard g(e->device);
-    int done = 0, rc;
-    if (e->graph_chunk > 0 && nsteps >= e->graph_chunk) {
-        if (!e->gexec) {
-            ECHK(hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
-            for (int k = 0; k < e->graph_chunk; k++) {
-                if ((rc = enqueue_step(e))) {
-                    hipGraph_t gph = nullptr;
-                    (void)hipStreamEndCapture(e->stream, &gph);
-                    if (gph) (void)hipGraphDestroy(gph);
-                    return rc;
-                }
-            }
-            ECHK(hipStreamEndCapture(e->stream, &e->graph));
-            ECHK(hipGraphInstantiate(&e->gexec, e->graph, nullptr, nullptr, 0));
-        }
-        while (nsteps - done >= e->graph_chunk) {
-            ECHK(hipGraphLaunch(e->gexec, e->stream));
-            done += e->graph_chunk;
-        }
-    }
-    for (; done < nsteps; done++)
-        if ((rc = enqueue_step(e))) return rc;
-    return TSU_OK;
+    return enqueue_steps(e, nsteps, true);
 }
 
 TSU_API int tsu_ensemble_synchronize(tsu_ensemble* e)
@@ -602,7 +678,7 @@ TSU_API int tsu_ensemble_time_steps(tsu_ensemble* e, int nsteps, double* ms)
     ECHK(hipEventCreate(&b));
     int rc = TSU_OK;
     hipError_t er = hipEventRecord(a, e->stream);
-    for (int k = 0; k < nsteps && er == hipSuccess && rc == TSU_OK; k++) rc = enqueue_step(e);
+    if (er == hipSuccess) rc = enqueue_steps(e, nsteps, false);
     if (er == hipSuccess) er = hipEventRecord(b, e->stream);
     if (er == hipSuccess) er = hipEventSynchronize(b);
     float f = 0.0f;

@@ -73,6 +73,7 @@ struct BatchMember {
     long long xoff;       // extrema offset (doubles), -1: none
     int tile_rows, nstrips, ntiles, order;
     int npx, npy, periodic;
+    int half;             // the part of the ensemble that it steps with
 };
 struct BatchPools {
     char* A;              // U^n (stage 2 writes it in place)
@@ -87,7 +88,9 @@ struct BatchPools {
 // fast_bed: every member's run constants satisfy fast_bedload.
 hipError_t launch_stage_batch(const BatchPools& pools, const BatchMember* mem, const int2* tiles, int ntiles, int k,
                               int last, bool sed, int precision, hipStream_t s, bool fast_bed = false);
-hipError_t launch_advance_batch(Ctrl* ctrl, DtSlots* dts, const DevParams* P, int n, hipStream_t s);
+// The members of one half, of n in all.
+hipError_t launch_advance_batch(Ctrl* ctrl, DtSlots* dts, const DevParams* P, const BatchMember* mem, int n, int half,
+                                hipStream_t s);
 // Smallest cell dt of the state V into step `step`'s slots (armed before).
 hipError_t launch_init_dt(const void* V, const DevParams& P, DtSlots* dts, long long step, int precision,
                           hipStream_t s);

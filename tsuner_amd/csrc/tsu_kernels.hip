@@ -931,9 +931,11 @@ __device__ __forceinline__ void advance_one(Ctrl* C, DtSlots* dts, const DevPara
 
 __global__ __launch_bounds__(64) void advance_kernel(Ctrl* C, DtSlots* dts, DevParams P) { advance_one(C, dts, P); }
 
-// One workgroup (one wave) per ensemble member.
-__global__ __launch_bounds__(64) void advance_batch_kernel(Ctrl* C, DtSlots* dts, const DevParams* __restrict__ P)
+// One workgroup (one wave) per ensemble member; those of one half advance.
+__global__ __launch_bounds__(64) void advance_batch_kernel(Ctrl* C, DtSlots* dts, const DevParams* __restrict__ P,
+                                                           const BatchMember* __restrict__ mem, int half)
 {
+    if (mem[blockIdx.x].half != half) return;
     advance_one(C + blockIdx.x, dts + blockIdx.x, P[blockIdx.x]);
 }
 
@@ -1173,9 +1175,10 @@ hipError_t launch_stage_batch(const BatchPools& pools, const BatchMember* mem, c
     return hipGetLastError();
 }
 
-hipError_t launch_advance_batch(Ctrl* ctrl, DtSlots* dts, const DevParams* P, int n, hipStream_t s)
+hipError_t launch_advance_batch(Ctrl* ctrl, DtSlots* dts, const DevParams* P, const BatchMember* mem, int n, int half,
+                                hipStream_t s)
 {
-    hipLaunchKernelGGL(advance_batch_kernel, dim3(n), dim3(64), 0, s, ctrl, dts, P);
+    hipLaunchKernelGGL(advance_batch_kernel, dim3(n), dim3(64), 0, s, ctrl, dts, P, mem, half);
     return hipGetLastError();
 }
 
