@@ -355,6 +355,36 @@ def test_tile_height_independent(rows):
     run_pair(sc, 12, tile_rows=rows)
 
 
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("order", [1, 2])
+@pytest.mark.parametrize("nx,ny,bc", [
+    (1, 1, [S.BC_WALL] * 4), (1, 7, [S.BC_PERIODIC] * 4), (59, 2, [S.BC_FREE] * 4), (60, 3, [S.BC_INFLOW] * 4),
+    (61, 33, [S.BC_PERIODIC] * 2 + [S.BC_WALL] * 2), (62, 40, [S.BC_FREE, S.BC_WALL] + [S.BC_PERIODIC] * 2),
+    (121, 31, [S.BC_INFLOW, S.BC_WALL, S.BC_FREE, S.BC_INFLOW]),
+    # the largest grids of one row per workgroup in FP64 and FP32, and one row more
+    (60, 682, [S.BC_WALL] * 4), (60, 683, [S.BC_WALL] * 4), (30, 1024, [S.BC_PERIODIC] * 4),
+    (30, 1025, [S.BC_PERIODIC] * 4)])
+def test_small_grid_equals_one_wave_per_tile(precision, order, nx, ny, bc):
+    """Default tiling (rows shared by three waves on these grids) against one
+    wave per tile, with and without sediment, extrema on."""
+    for sediment in (1, 0):
+        sc = S.sediment_shelf(n=nx, ny=ny, dx=40.0, seed=nx + ny)
+        sc.scheme.update(bc=bc, order=order, extrema=1, bedload=sediment, suspension=sediment)
+        if nx * ny == 1:                  # the generated bed has no relief to scale: NaN
+            sc.V[:] = np.array([5.0, 0.0, 0.0, 5.0, 0.0])[:, None, None]
+        sc.V[1] += sc.V[0] * 0.5
+        if not sediment:
+            sc.V[4] = 0.0
+        a, b = (Solver.from_scenario(sc, precision=precision, tile_rows=r) for r in (0, 4))
+        say("%s order %d %d x %d sediment %d" % (precision, order, nx, ny, sediment))
+        a.step(10)
+        b.step(10)
+        cmp_state(a.state(), b.state(), "%d x %d" % (nx, ny))
+        assert a.time() == b.time()
+        for p, q in zip(a.extrema(), b.extrema()):
+            assert np.array_equal(p, q)
+
+
 def test_graph_replay_matches_eager():
     sc = S.sediment_shelf(n=90, ny=60, dx=40.0, seed=6)
     a = Solver.from_scenario(sc)

@@ -220,6 +220,7 @@ struct tsu_state {
     DevParams* dP = nullptr;   // device copy of P read by the stage kernels
     hipStream_t stream = nullptr;
     int tile_rows = 0, nstrips = 0, nchunks = 0, ntiles = 0;
+    bool split = false;        // stage_split_kernel (tile_rows 1)
     bool rows_given = false;   // tile_rows by the caller, not by default
     int graph_chunk = 0;
     hipGraphExec_t gexec = nullptr;
@@ -253,14 +254,34 @@ struct DeviceGuard {
 // parts of h, H and hc (compensated accumulation).
 size_t planes_of(const tsu_state* st) { return st->precision == TSU_FP64 ? 5 : 8; }
 
-int default_tile_rows(const tsu_state* st)
+// Whether all rows of a grid, each with three waves (stage_split_kernel), run
+// at once with at most two waves per SIMD in FP64 and three in FP32.  Above
+// that its extra work (a row's edge along y is solved by both its rows, with a
+// reconstruction more) costs more than the shorter chain gives, first beside
+// other runs.  us a step, alone and with two others of its size beside it (a
+// third of their time), against one wave per tile: FP64 with sediment 100^2
+// 26.9 -> 16.3 and 12.1 -> 7.4, 160^2 28.5 -> 20.9 and 12.7 -> 10.5, past the
+// line 200^2 28.8 -> 26.8 and 14.0 -> 14.6, 320^2 40 -> 48 and 26.8 -> 30.9;
+// FP32 100^2 21.1 -> 14.1 and 9.0 -> 6.6, 240 x 256 23.3 -> 18.0 and 10.2 ->
+// 10.4, past it 320^2 24.1 -> 27.2 and 12.4 -> 15.8.
+bool split_rows(const tsu_state* st)
 {
-    return tsu::choose_tile_rows({{st->p.npx, st->p.npy}}, tsu::stage_waves_per_simd(st->sed, st->precision),
-                                 st->device);
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, st->device) != hipSuccess || cus < 1)
+        cus = 256;
+    const long long strips = (st->p.npx + tsu::kStripOut - 1) / tsu::kStripOut;
+    return tsu::kSplitWaves * strips * st->p.npy <= 4LL * cus * (st->precision == TSU_FP64 ? 2 : 3);
 }
 
+// rows 0: the default for the grid, precision and scheme.
 void set_tiling(tsu_state* st, int rows)
 {
+    st->split = rows == 0 && split_rows(st);
+    if (st->split)
+        rows = 1;
+    else if (rows == 0)
+        rows = tsu::choose_tile_rows({{st->p.npx, st->p.npy}}, tsu::stage_waves_per_simd(st->sed, st->precision),
+                                     st->device);
     st->tile_rows = rows;
     st->nstrips = (st->p.npx + tsu::kStripOut - 1) / tsu::kStripOut;
     st->nchunks = (st->p.npy + rows - 1) / rows;
@@ -308,6 +329,7 @@ tsu::StageArgs stage_args(const tsu_state* st, int k)
     a.tile_rows = st->tile_rows;
     a.nstrips = st->nstrips;
     a.ntiles = st->ntiles;
+    a.split = st->split;
     a.npx = st->P.npx;
     a.npy = st->P.npy;
     a.periodic = tsu::periodic_sides(st->P);
@@ -445,7 +467,7 @@ TSU_API int tsu_state_create(tsu_state** out, const tsu_sim_params* p, const tsu
     st->nvol = (long long)p->npx * p->npy;
     tsu::make_dev_params(&st->p, &st->s, &st->P);
     st->sed = s->bedload || s->suspension;
-    set_tiling(st, default_tile_rows(st));
+    set_tiling(st, 0);
 
     DeviceGuard g(device);
     const size_t state_bytes = planes_of(st) * (size_t)st->nvol * st->esize;
@@ -493,7 +515,7 @@ TSU_API int tsu_state_upload(tsu_state* st, const double* V, const int* fixH)
     st->sed = st->s.bedload || st->s.suspension || !hc_zero;
     DeviceGuard g(st->device);
     drop_graph(st);
-    if (!st->rows_given) set_tiling(st, default_tile_rows(st));
+    if (!st->rows_given) set_tiling(st, 0);
     const size_t bytes = planes_of(st) * (size_t)nv * st->esize;
     if (st->precision == TSU_FP64) {
         HIPCHK(hipMemcpyAsync(st->A, V, bytes, hipMemcpyHostToDevice, st->stream));
@@ -737,7 +759,7 @@ TSU_API int tsu_set_tile_rows(tsu_state* st, int rows)
     if (rows < 0 || rows > 4096) return fail(TSU_ERR_ARG, "tile rows out of range");
     drop_graph(st);
     st->rows_given = rows != 0;
-    set_tiling(st, rows == 0 ? default_tile_rows(st) : rows);
+    set_tiling(st, rows);
     return TSU_OK;
 }
 

@@ -27,6 +27,7 @@ struct StageArgs {
     int tile_rows;
     int nstrips;
     int ntiles;
+    int split;            // 1: the kernel of small grids (tile_rows 1)
     int npx, npy;         // the grid and periodic sides (bit 0 x, bit 1 y) of P
     int periodic;
     const DevParams* P;   // run constants in device memory
@@ -59,6 +60,7 @@ inline unsigned long long min_dt_bits(const DtSlots& d, long long s)
 // the run constants satisfy fast_bedload (tsu_device.h); with sediment the
 // launch then takes the kernel that evaluates bedload among the HLL
 // arithmetic.
+constexpr int kSplitWaves = 3;   // of a workgroup of stage_split_kernel: one row of a strip
 int stage_waves_per_simd(bool sed, int precision);   // the launched kernel's occupancy
 hipError_t launch_stage(const StageArgs& a, bool sed, int precision, hipStream_t s, bool fast_bed = false);
 

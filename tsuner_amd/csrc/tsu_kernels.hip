@@ -16,7 +16,9 @@
 //     per wave (Reduction_kernel_min.cu:155-196), so dt never leaves the
 //     device;
 //   * the two stages of a step keep t and the step number themselves
-//     (GPU/main_TSUNER.cu:185; see Ctrl).
+//     (GPU/main_TSUNER.cu:185; see Ctrl);
+//   * on small grids a row of a tile is shared by three waves instead
+//     (stage_split_kernel).
 //
 // Two arithmetic variants share the code: R = double (reference arithmetic,
 // FP64 planes) and R = float (FP32 planes and fluxes; h, H and hc carried as
@@ -161,13 +163,20 @@ struct Diff {
     R h, eta, ux, uy, c;
 };
 
+template <typename R>
+__device__ __forceinline__ R eta_diff(const Cell<R>& a, const Cell<R>& b)
+{
+    const R zero = (R)0, zm = rmin(a.H, b.H);
+    return rmax(b.h - b.H + zm, zero) - rmax(a.h - a.H + zm, zero);
+}
+
 template <typename R, bool SED>
 __device__ __forceinline__ Diff<R> cell_diff(const Cell<R>& a, const Cell<R>& b)
 {
-    const R zero = (R)0, zm = rmin(a.H, b.H);
+    const R zero = (R)0;
     Diff<R> d;
     d.h = b.h - a.h;
-    d.eta = rmax(b.h - b.H + zm, zero) - rmax(a.h - a.H + zm, zero);
+    d.eta = eta_diff(a, b);
     d.ux = b.ux - a.ux;
     d.uy = b.uy - a.uy;
     d.c = SED ? b.c - a.c : zero;
@@ -350,21 +359,291 @@ __device__ __forceinline__ void edge_flux_pair(const DevParams& P, int ka, bool 
     }
 }
 
+// The running step: found by its first stage, read from the control block by
+// its last (see Ctrl).  False when there is none.  The keeper (one wave of
+// the launch) keeps the block.  slot0, slot1: this lane's dt slots (first
+// stage only).
+__device__ __forceinline__ bool open_step(const StageArgs& a, const DevParams& P, const Ctrl& c0,
+                                          unsigned long long slot0, unsigned long long slot1, bool keeper, int lane,
+                                          double& ct, double& dtd, long long& step)
+{
+    Ctrl* C = a.ctrl;
+    if (a.k == 0) {
+        ct = c0.t;
+        step = c0.step;
+        const bool run = ct < c0.stop_time && step < c0.stop_step;
+        if (!run) {
+            if (keeper && lane == 0) C->running = 0;
+            return false;
+        }
+        double m = __longlong_as_double((long long)((step & 1) ? slot1 : slot0));
+        for (int o = kDtSlots / 2; o > 0; o >>= 1) m = fmin(m, __shfl_xor(m, o, 64));
+        dtd = clamp_dt(c0, ct, finalize_dt(P, m));
+        if (keeper && !a.last) {
+            if (lane == 0) {
+                C->run_t = ct;
+                C->run_dt = dtd;
+                C->run_step = step;
+                C->running = 1;
+            }
+            // armed for the last stage; step - 1, whose slots they were, is over
+            if (lane < kDtSlots) a.dts->v[(step + 1) & 1][lane][0] = kInfBits;
+        }
+    } else {
+        if (!c0.running) return false;
+        ct = c0.run_t;
+        dtd = c0.run_dt;
+        step = c0.run_step;
+        if (keeper && lane == 0) {
+            C->t = next_time(c0.clamp, c0.stop_time, ct, dtd);
+            C->step = step + 1;
+        }
+    }
+    return true;
+}
+
+// Per-step constants, in the reference's evaluation order.
+template <typename R>
+struct StepConsts {
+    double dtd;
+    R dt, invx, invy, dtaxG, dtayG, dtFR;
+};
+
+template <typename R>
+__device__ __forceinline__ StepConsts<R> step_consts(const DevParams& P, double dtd)
+{
+    const double invxd = dtd * P.inv_dx, invyd = dtd * P.inv_dy;   // main_TSUNER.cu:182
+    StepConsts<R> K;
+    K.dtd = dtd;
+    K.dt = (R)dtd;
+    K.invx = (R)invxd;
+    K.invy = (R)invyd;
+    K.dtaxG = (R)(invxd * kG);   // Reconstructor.cu:197,274
+    K.dtayG = (R)(invyd * kG);
+    K.dtFR = (R)(dtd * P.FR);    // Reconstructor.cu:45
+    return K;
+}
+
+// The momenta k1, k2 of a cell after the free-surface source (Reconstructor.cu:
+// 197,274) and friction from U^n = v0 (Reconstructor.cu:45-53); returns the bed
+// exchange rate.
+template <typename R, bool SED>
+__device__ __forceinline__ R source_terms(const DevParams& P, const StepConsts<R>& K, int k, bool second,
+                                          const Cell<R>& R0, R detax, R detay, const R* v0, R& k1, R& k2)
+{
+    constexpr bool COMP = sizeof(R) == 4;
+    k1 = R0.qx;
+    k2 = R0.qy;
+    if (second) {
+        k1 -= K.dtaxG * R0.h * detax;
+        k2 -= K.dtayG * R0.h * detay;
+    }
+    Vel<R> un;
+    // the quadratic law divides by h^n + DBL_EPSILON, the velocity's
+    // denominator: one shared reciprocal, computed where a quotient
+    // needs it (have_dh is uniform over the wave)
+    Den<R> Dh = {(R)1, (R)1};
+    bool have_dh = false;
+    if constexpr (COMP) {
+        Dh = den(v0[0] + (R)kEpsilon);
+        have_dh = true;
+    }
+    if (k == 0) {   // U^n is this stage's input: its velocity is known
+        un.x = R0.ux;
+        un.y = R0.uy;
+        un.s = R0.us;
+    } else if constexpr (COMP) {
+        un = velocity(v0[0], v0[1], v0[2], &Dh.y);
+    } else if (__builtin_amdgcn_ballot_w64(v0[0] >= (R)kEps && (v0[1] != (R)0 || v0[2] != (R)0)) != 0) {
+        Dh = den(v0[0] + (R)kEpsilon);
+        have_dh = true;
+        un = velocity_over(v0[0], v0[1], v0[2], Dh);
+    } else {
+        const R z = zero_here((R)0);   // no lane divides
+        un = {z, z, z};
+    }
+    // |u| of U^n (friction, exchange).  In FP64 a wave at rest (|u| =
+    // 0 on every lane) has c = 0 and divides both momenta by 1 + 0 =
+    // 1, which leaves them unchanged: it skips the friction step (the
+    // FP32 solver, where the step is a few instructions, measured
+    // slower with the vote).
+    R modu = (R)0;
+    const bool still = !COMP && __builtin_amdgcn_ballot_w64(un.s != (R)0) == 0;
+    if (!still) {
+        modu = sqrt_voted(un.s);
+        if (!have_dh) Dh = den(v0[0] + (R)kEpsilon);
+        R cf;
+        if (P.friction_law == FRIC_MANNING) {
+            R hp = v0[0] + (R)kEpsilon;
+            R dtGnn = (R)(K.dtd * kG * P.manning_n * P.manning_n);
+            if constexpr (COMP)
+                cf = dtGnn * modu / (hp * cbrtf(hp));
+            else
+                cf = dtGnn * modu / (hp * cbrt(hp));
+        } else {
+            cf = qdiv(K.dtFR * modu, Dh);
+        }
+        // both momenta divided by 1 + c
+        const Den<R> Dc = den((R)1 + cf);
+        k1 = qdiv(k1, Dc);
+        k2 = qdiv(k2, Dc);
+    }
+    R phi = (R)0;
+    if (SED && P.suspension) phi = erosion_rate(P, v0[0], modu, v0[4], still);
+    return phi;
+}
+
+// The next dt from the largest wave speeds of a wave's cells.
+template <typename R>
+__device__ __forceinline__ void fold_dt(const StageArgs& a, const DevParams& P, int tile, int lane, long long step,
+                                        R lxmax, R lymax)
+{
+    lxmax = wave_max(lxmax);
+    lymax = wave_max(lymax);
+    const double m = (double)dt_of_speeds(P, lxmax, lymax);
+    if (lane == 0 && m < __longlong_as_double((long long)kInfBits))
+        atomicMin(&a.dts->v[(step + 1) & 1][tile & (kDtSlots - 1)][0], (unsigned long long)__double_as_longlong(m));
+}
+
+// A row of a strip of a small grid in a workgroup of three waves: one for each
+// of the row's edges along y, one for its edges along x and the update.
+//
+// On a grid that leaves most of the chip idle a stage lasts as long as one
+// wave: in stage_body its loads, then the lower edge, then the edges along x
+// and the upper edge, each a chain of dependent FP64 quotients and square
+// roots.  Here the three are side by side, and one copy of the edge solve
+// serves all waves.  A neighbour's edge is solved once more instead of being
+// handed on.  100 x 100 cells in motion, FP64 with sediment: 13.4 -> 8.1 us a
+// stage.  What is left is the launch, the loads, and one chain each of face
+// reconstruction, edge and update.  The sums are stage_body's, in its order.
+
+//
+// The part between the loads and the update: M, A, B, Q are the rows y - 2 ..
+// y + 1 in wave 0 and y - 1 .. y + 2 in the others (Q not in wave 2).  True in
+// wave 2, with the fluctuations of the edges along x (Dm, Dp) and of the
+// edges along y that enter row y (FD, FU), and the source terms (own: lanes
+// that store a cell; v0: their U^n).
+template <typename R, bool SED, bool FB>
+__device__ __forceinline__ bool split_edges(const StageArgs& a, const DevParams& P, const StepConsts<R>& K, int wave,
+                                            int lane, int x, int xc, int y, double ct, Cell<R>& M, Cell<R>& A,
+                                            Cell<R>& B, Cell<R>& Q, int fa, int fb, bool own, const R* v0, R* Dm,
+                                            R* Dp, R* FD, R* FU, R& k1, R& k2, R& phi)
+{
+    __shared__ R flux[2][5][64];   // what enters row y through its lower and upper edges
+    const int npx = a.npx, npy = a.npy;
+    const bool perx = a.periodic & 1, pery = (a.periodic & 2) != 0;
+    const int lim = P.limiter;
+    const bool second = P.order == 2;
+    const bool along_x = wave == 2;
+
+    // both sides of the wave's edges
+    R El[5], Er[5], detax = (R)0, detay = (R)0;
+    int kind, fixed;
+    bool right_ghost = false;
+    derive_cell<R, SED>(A);
+    if (along_x) {
+        R Lf[5], Rf[5];
+        if (second) {
+            Cell<R> left;
+            left.h = up1(A.h);
+            left.H = up1(A.H);
+            left.ux = up1(A.ux);
+            left.uy = up1(A.uy);
+            left.c = SED ? up1(A.c) : (R)0;
+            const Diff<R> l = cell_diff<R, SED>(left, A);
+            const Diff<R> rt = {dn1(l.h), dn1(l.eta), dn1(l.ux), dn1(l.uy), SED ? dn1(l.c) : (R)0};
+            detax = recons_axis<R, SED>(lim, A, l, rt, Lf, Rf);
+            filter_faces<R, SED>(Lf, Rf);
+            detay = limiter(lim, eta_diff(M, A), eta_diff(A, B));
+        } else {
+            cell_face(A, Lf);
+            cell_face(A, Rf);
+        }
+        R Rl[5];
+        for (int f = 0; f < 5; f++) Rl[f] = up1(Rf[f]);
+        const int fxl = up1i(fa);
+        kind = N_PX;
+        if (x == 0 && !perx) {
+            for (int f = 0; f < 5; f++) El[f] = Lf[f];
+            ghost_state(P, 0, Lf, Er, 2LL * npx + npy + y, 1, ct);
+            kind = N_MX;
+            fixed = fa;
+        } else if (x == npx && !perx) {
+            for (int f = 0; f < 5; f++) El[f] = Rl[f];
+            ghost_state(P, 1, Rl, Er, (long long)npx + y, 1, ct);
+            fixed = fxl;
+        } else {
+            for (int f = 0; f < 5; f++) {
+                El[f] = Rl[f];
+                Er[f] = Lf[f];
+            }
+            fixed = (perx && (x == 0 || x == npx)) ? fxl : fxl * fa;
+        }
+    } else {
+        derive_cell<R, SED>(B);
+        if (second) {
+            R other[5];
+            derive_cell<R, SED>(M);
+            derive_cell<R, SED>(Q);
+            const Diff<R> d = cell_diff<R, SED>(A, B);
+            recons_axis<R, SED>(lim, A, cell_diff<R, SED>(M, A), d, other, El);
+            recons_axis<R, SED>(lim, B, d, cell_diff<R, SED>(B, Q), Er, other);
+            filter_faces<R, SED>(El, Er);
+        } else {
+            cell_face(A, El);
+            cell_face(B, Er);
+        }
+        kind = N_PY;
+        const bool end = wave == 0 ? y == 0 : y + 1 == npy;
+        fixed = end ? fa : fa * fb;   // periodic wrap edge: VolumeSolver.cu:386
+        if (end && !pery) {
+            if (wave == 0) {
+                for (int f = 0; f < 5; f++) El[f] = Er[f];
+                ghost_state(P, 2, El, Er, (long long)xc, 2, ct);
+                kind = N_MY;
+                fixed = fb;
+                right_ghost = true;
+            } else {
+                ghost_state(P, 3, El, Er, (long long)npx + npy + xc, 2, ct);
+            }
+        }
+    }
+
+    edge_flux<R, SED, FB>(P, kind, fixed != 0, El, Er, Dm, Dp);
+
+    constexpr int nf = SED ? 5 : 3;
+    if (along_x) {
+        if (own) phi = source_terms<R, SED>(P, K, a.k, second, A, detax, detay, v0, k1, k2);
+    } else {
+        const bool minus = wave == 1 || right_ghost;
+        for (int f = 0; f < nf; f++) flux[wave][f][lane] = minus ? Dm[f] : Dp[f];
+    }
+    __syncthreads();
+    if (!along_x) return false;
+    for (int f = 0; f < 5; f++) {
+        FD[f] = f < nf ? flux[0][f][lane] : (R)0;
+        FU[f] = f < nf ? flux[1][f][lane] : (R)0;
+    }
+    return true;
+}
+
 // FB: the run constants satisfy fast_bedload (kernels with sediment only).
-template <typename R, typename S, bool SED, bool FB>
+// SPLIT: one row per workgroup of three waves (split_edges).
+template <typename R, typename S, bool SED, bool FB, bool SPLIT = false>
 __device__ __forceinline__ void stage_body(const StageArgs& a, const int tile)
 {
     constexpr bool COMP = sizeof(R) == 4;   // FP32 solver: compensated h, H, hc
     constexpr bool CARRY = SED;   // a row's differences to the next kept for it (else they spill)
-    const int lane = threadIdx.x;
+    const int lane = SPLIT ? (int)threadIdx.x & 63 : (int)threadIdx.x;
+    const int wave = SPLIT ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) : 0;
     const int strip = tile % a.nstrips, chunk = tile / a.nstrips;
     const int npx = a.npx, npy = a.npy;
     const bool perx = a.periodic & 1, pery = (a.periodic & 2) != 0;
     const long long nv = (long long)npx * npy;
     const int x = strip * kStripOut + lane - 2;
     const int xc = map_index(x, npx, perx);
-    const int y0 = chunk * a.tile_rows;
-    const int y1 = min(y0 + a.tile_rows, npy);
+    const int y0 = SPLIT ? chunk : chunk * a.tile_rows;
+    const int y1 = SPLIT ? y0 + 1 : min(y0 + a.tile_rows, npy);
     auto row_off = [&](int r) -> long long { return (long long)map_index(r, npy, pery) * npx + xc; };
 
     // The loads of the run constants, the control block, the dt slots and the
@@ -394,107 +673,75 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int tile)
     const S* v0p = (a.k == 0) ? in : (const S*)a.v0;
     const uint8_t* fix = a.fix;
     Cell<R> Rm, R0, R1;
-    load_cell<R, S, SED>(in, Hin, nv, row_off(y0 - 1), Rm);
-    load_cell<R, S, SED>(in, Hin, nv, row_off(y0), R0);
-    load_cell<R, S, SED>(in, Hin, nv, row_off(y0 + 1), R1);
+    const int rc = SPLIT && wave == 0 ? y0 - 1 : y0;   // row of R0
+    load_cell<R, S, SED>(in, Hin, nv, row_off(rc - 1), Rm);
+    load_cell<R, S, SED>(in, Hin, nv, row_off(rc), R0);
+    load_cell<R, S, SED>(in, Hin, nv, row_off(rc + 1), R1);
+    Cell<R> R2;
+    if (SPLIT && wave != 2) load_cell<R, S, SED>(in, Hin, nv, row_off(rc + 2), R2);
     const Ctrl c0 = *C;
 
-    // Run constants, copied into LDS once per workgroup (one wave).  Read
+    // Run constants, copied into LDS once per workgroup.  Read
     // through the global pointer, every use in the row loop was a vector
     // load, since the kernel's own stores might alias the constants; in LDS
     // they cannot, and a use is a short LDS read.  The loop re-reads them
     // per row (see there) rather than holding them in registers.
     __shared__ DevParams Ps;
-    if (lane < kPWords) reinterpret_cast<unsigned long long*>(&Ps)[lane] = pword;
+    if (lane < kPWords && wave == 0) reinterpret_cast<unsigned long long*>(&Ps)[lane] = pword;
     __syncthreads();
     const DevParams& P = Ps;
 
-    // The running step: found by its first stage, read from the control
-    // block by its last (see Ctrl).  The first wave keeps the block.
     double ct, dtd;
     long long step;
-    if (first) {
-        ct = c0.t;
-        step = c0.step;
-        const bool run = ct < c0.stop_time && step < c0.stop_step;
-        if (!run) {
-            if (tile == 0 && lane == 0) C->running = 0;
-            return;
-        }
-        double m = __longlong_as_double((long long)((step & 1) ? slot1 : slot0));
-        for (int o = kDtSlots / 2; o > 0; o >>= 1) m = fmin(m, __shfl_xor(m, o, 64));
-        dtd = clamp_dt(c0, ct, finalize_dt(P, m));
-        if (tile == 0 && !a.last) {
-            if (lane == 0) {
-                C->run_t = ct;
-                C->run_dt = dtd;
-                C->run_step = step;
-                C->running = 1;
-            }
-            // armed for the last stage; step - 1, whose slots they were, is over
-            if (lane < kDtSlots) a.dts->v[(step + 1) & 1][lane][0] = kInfBits;
-        }
-    } else {
-        if (!c0.running) return;
-        ct = c0.run_t;
-        dtd = c0.run_dt;
-        step = c0.run_step;
-        if (tile == 0 && lane == 0) {
-            C->t = next_time(c0.clamp, c0.stop_time, ct, dtd);
-            C->step = step + 1;
-        }
-    }
+    if (!open_step(a, P, c0, slot0, slot1, tile == 0 && wave == 0, lane, ct, dtd, step)) return;
 
-    const bool out_lane = lane >= 2 && lane < 62 && x < npx;
+    const bool out_lane = lane >= 2 && lane < 62 && x < npx && (!SPLIT || wave == 2);
     const int lim = P.limiter;
     const bool second = P.order == 2;
     const bool need_fix = SED && P.bedload;
 
-    // Per-step constants, in the reference's evaluation order.
-    const double invxd = dtd * P.inv_dx, invyd = dtd * P.inv_dy;  // main_TSUNER.cu:182
-    const R dt = (R)dtd;
-    const R invx = (R)invxd, invy = (R)invyd;
-    const R dtaxG = (R)(invxd * kG), dtayG = (R)(invyd * kG);   // Reconstructor.cu:197,274
-    const R dtFR = (R)(dtd * P.FR);                               // Reconstructor.cu:45
+    const StepConsts<R> K = step_consts<R>(P, dtd);
+    const R dt = K.dt, invx = K.invx, invy = K.invy;
 
     auto fix_at = [&](int r) -> int { return need_fix ? (int)fix[row_off(r)] : 0; };
 
-    // ---- prologue: faces of row y0 and the edge y0 - 1/2 -----------------
-    derive_cell<R, SED>(Rm);
-    derive_cell<R, SED>(R0);
-    derive_cell<R, SED>(R1);
-    int fx0 = fix_at(y0), fx1;
-
+    int fx0 = fix_at(rc), fx1;
     R D0[5], U0[5], FD0[5];
     R detay0 = (R)0;
     Diff<R> dm1, d0;   // rows y0 - 1 to y0; row r to r + 1, carried down the tile
-    if (second) {
-        dm1 = cell_diff<R, SED>(Rm, R0);
-        d0 = cell_diff<R, SED>(R0, R1);
-        detay0 = recons_axis<R, SED>(lim, R0, dm1, d0, D0, U0);
-        filter_faces<R, SED>(D0, U0);
-    } else {
-        cell_face(R0, D0);
-        cell_face(R0, U0);
-    }
-    if (y0 == 0 && !pery) {
-        R G5[5], dp[5];
-        ghost_state(P, 2, D0, G5, (long long)xc, 2, ct);
-        edge_flux<R, SED, FB>(P, N_MY, fx0 != 0, D0, G5, FD0, dp);
-    } else {
-        R Um[5], Dd[5], dm[5];
+    // ---- prologue: faces of row y0 and the edge y0 - 1/2 -----------------
+    if constexpr (!SPLIT) {
+        derive_cell<R, SED>(Rm);
+        derive_cell<R, SED>(R0);
+        derive_cell<R, SED>(R1);
         if (second) {
-            Cell<R> Rmm;
-            load_cell<R, S, SED>(in, Hin, nv, row_off(y0 - 2), Rmm);
-            derive_cell<R, SED>(Rmm);
-            recons_axis<R, SED>(lim, Rm, cell_diff<R, SED>(Rmm, Rm), dm1, Dd, Um);
-            filter_face<R, SED>(Um);
+            dm1 = cell_diff<R, SED>(Rm, R0);
+            d0 = cell_diff<R, SED>(R0, R1);
+            detay0 = recons_axis<R, SED>(lim, R0, dm1, d0, D0, U0);
+            filter_faces<R, SED>(D0, U0);
         } else {
-            cell_face(Rm, Um);
+            cell_face(R0, D0);
+            cell_face(R0, U0);
         }
-        int fxm = fix_at(y0 - 1);
-        int fixed = (y0 == 0) ? fxm : fxm * fx0;   // periodic wrap edge: VolumeSolver.cu:386
-        edge_flux<R, SED, FB>(P, N_PY, fixed != 0, Um, D0, dm, FD0);
+        if (y0 == 0 && !pery) {
+            R G5[5], dp[5];
+            ghost_state(P, 2, D0, G5, (long long)xc, 2, ct);
+            edge_flux<R, SED, FB>(P, N_MY, fx0 != 0, D0, G5, FD0, dp);
+        } else {
+            R Um[5], Dd[5], dm[5];
+            if (second) {
+                Cell<R> Rmm;
+                load_cell<R, S, SED>(in, Hin, nv, row_off(y0 - 2), Rmm);
+                derive_cell<R, SED>(Rmm);
+                recons_axis<R, SED>(lim, Rm, cell_diff<R, SED>(Rmm, Rm), dm1, Dd, Um);
+                filter_face<R, SED>(Um);
+            } else {
+                cell_face(Rm, Um);
+            }
+            int fxm = fix_at(y0 - 1);
+            int fixed = (y0 == 0) ? fxm : fxm * fx0;   // periodic wrap edge: VolumeSolver.cu:386
+            edge_flux<R, SED, FB>(P, N_PY, fixed != 0, Um, D0, dm, FD0);
+        }
     }
 
     // largest wave speeds of the tile's updated cells (last stage: the next dt)
@@ -507,12 +754,11 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int tile)
         // of hoisting all of them into registers ahead of the loop
         typedef const __attribute__((address_space(3))) DevParams* LdsParams;
         LdsParams Pl = (LdsParams)&Ps;
-        asm volatile("" : "+s"(Pl));
+        if constexpr (!SPLIT) asm volatile("" : "+s"(Pl));
         const DevParams& P = *(const DevParams*)Pl;
         // next row (r + 2): issued first, consumed after the x work below
-        Cell<R> R2;
-        load_cell<R, S, SED>(in, Hin, nv, row_off(r + 2), R2);
-        fx1 = fix_at(r + 1);
+        if constexpr (!SPLIT) load_cell<R, S, SED>(in, Hin, nv, row_off(r + 2), R2);
+        fx1 = fix_at(SPLIT ? rc + 1 : r + 1);
         R v0[5];
         R lo_in[3] = {(R)0, (R)0, (R)0}, lo_v0[3] = {(R)0, (R)0, (R)0};
         const long long pos = (long long)r * npx + xc;
@@ -540,84 +786,11 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int tile)
             }
         }
 
-        // x faces of row r (Reconstructor.cu:120-197)
-        R Lf[5], Rf[5], detax = (R)0;
-        if (second) {
-            Cell<R> left;
-            left.h = up1(R0.h);
-            left.H = up1(R0.H);
-            left.ux = up1(R0.ux);
-            left.uy = up1(R0.uy);
-            left.c = SED ? up1(R0.c) : (R)0;
-            const Diff<R> l = cell_diff<R, SED>(left, R0);
-            const Diff<R> rt = {dn1(l.h), dn1(l.eta), dn1(l.ux), dn1(l.uy), SED ? dn1(l.c) : (R)0};
-            detax = recons_axis<R, SED>(lim, R0, l, rt, Lf, Rf);
-            filter_faces<R, SED>(Lf, Rf);
-        } else {
-            cell_face(R0, Lf);
-            cell_face(R0, Rf);
-        }
-
-        // x edge at x - 1/2 (VolumeSolver.cu:227-317)
-        R Rl[5];
-        for (int f = 0; f < 5; f++) Rl[f] = up1(Rf[f]);
-        int fxl = need_fix ? up1i(fx0) : 0;
-        R El[5], Er[5];
-        int kind = N_PX;
-        int fixed;
-        if (x == 0 && !perx) {
-            for (int f = 0; f < 5; f++) El[f] = Lf[f];
-            ghost_state(P, 0, Lf, Er, 2LL * npx + npy + r, 1, ct);
-            kind = N_MX;
-            fixed = fx0;
-        } else if (x == npx && !perx) {
-            for (int f = 0; f < 5; f++) El[f] = Rl[f];
-            ghost_state(P, 1, Rl, Er, (long long)npx + r, 1, ct);
-            fixed = fxl;
-        } else {
-            for (int f = 0; f < 5; f++) {
-                El[f] = Rl[f];
-                Er[f] = Lf[f];
-            }
-            fixed = (perx && (x == 0 || x == npx)) ? fxl : fxl * fx0;
-        }
-
-        // y faces of row r + 1 and the edge r + 1/2
-        derive_cell<R, SED>(R2);
-        R D1[5], U1[5], detay1 = (R)0;
-        if (second) {
-            if (!CARRY) d0 = cell_diff<R, SED>(R0, R1);
-            const Diff<R> d1 = cell_diff<R, SED>(R1, R2);
-            detay1 = recons_axis<R, SED>(lim, R1, d0, d1, D1, U1);
-            if (CARRY) d0 = d1;
-            filter_faces<R, SED>(D1, U1);
-        } else {
-            cell_face(R1, D1);
-            cell_face(R1, U1);
-        }
-        // upper side of the edge r + 1/2: row r + 1's lower faces, or the
-        // ghost state above the domain's last row
-        R Yr[5];
-        if (r + 1 == npy && !pery)
-            ghost_state(P, 3, U0, Yr, (long long)npx + npy + xc, 2, ct);
-        else
-            for (int f = 0; f < 5; f++) Yr[f] = D1[f];
-        const int fy = (r + 1 == npy) ? fx0 : fx0 * fx1;
-
-        // the x edge x - 1/2 and the y edge r + 1/2, solved side by side
+        R detax = (R)0, detay1 = (R)0, U1[5];
         R Dmx[5], Dpx[5], FU0[5], FD1[5];   // FD1: not used after the domain's last row
-        edge_flux_pair<R, SED, FB>(P, kind, fixed != 0, El, Er, Dmx, Dpx, N_PY, fy != 0, U0, Yr, FU0, FD1);
-        R FL[5], FR[5];
-        const bool left_wall = (x == 0 && !perx);
-        for (int f = 0; f < 5; f++) {
-            FL[f] = left_wall ? Dmx[f] : Dpx[f];
-            FR[f] = dn1(Dmx[f]);
-        }
-
-        // cell update of row r (Reconstructor.cu:197,274,353-354;
-        // Volume_kernel.cu:191-195,244-282)
-        if (out_lane) {
-            if (a.k == 0) {
+        R k1 = (R)0, k2 = (R)0, phi = (R)0;
+        if constexpr (SPLIT) {
+            if (out_lane && a.k == 0) {
                 v0[0] = R0.h;
                 v0[1] = R0.qx;
                 v0[2] = R0.qy;
@@ -626,64 +799,97 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int tile)
                 if (COMP)
                     for (int j = 0; j < 3; j++) lo_v0[j] = lo_in[j];
             }
-            R k1 = R0.qx, k2 = R0.qy;
+            if (!split_edges<R, SED, FB>(a, P, K, wave, lane, x, xc, r, ct, Rm, R0, R1, R2, fx0, fx1, out_lane, v0, Dmx,
+                                         Dpx, FD0, FU0, k1, k2, phi))
+                return;
+        } else {
+            // x faces of row r (Reconstructor.cu:120-197)
+            R Lf[5], Rf[5];
             if (second) {
-                k1 -= dtaxG * R0.h * detax;
-                k2 -= dtayG * R0.h * detay0;
-            }
-            Vel<R> un;
-            // the quadratic law divides by h^n + DBL_EPSILON, the velocity's
-            // denominator: one shared reciprocal, computed where a quotient
-            // needs it (have_dh is uniform over the wave)
-            Den<R> Dh = {(R)1, (R)1};
-            bool have_dh = false;
-            if constexpr (COMP) {
-                Dh = den(v0[0] + (R)kEpsilon);
-                have_dh = true;
-            }
-            if (a.k == 0) {   // U^n is this stage's input: its velocity is known
-                un.x = R0.ux;
-                un.y = R0.uy;
-                un.s = R0.us;
-            } else if constexpr (COMP) {
-                un = velocity(v0[0], v0[1], v0[2], &Dh.y);
-            } else if (__builtin_amdgcn_ballot_w64(v0[0] >= (R)kEps && (v0[1] != (R)0 || v0[2] != (R)0)) != 0) {
-                Dh = den(v0[0] + (R)kEpsilon);
-                have_dh = true;
-                un = velocity_over(v0[0], v0[1], v0[2], Dh);
+                Cell<R> left;
+                left.h = up1(R0.h);
+                left.H = up1(R0.H);
+                left.ux = up1(R0.ux);
+                left.uy = up1(R0.uy);
+                left.c = SED ? up1(R0.c) : (R)0;
+                const Diff<R> l = cell_diff<R, SED>(left, R0);
+                const Diff<R> rt = {dn1(l.h), dn1(l.eta), dn1(l.ux), dn1(l.uy), SED ? dn1(l.c) : (R)0};
+                detax = recons_axis<R, SED>(lim, R0, l, rt, Lf, Rf);
+                filter_faces<R, SED>(Lf, Rf);
             } else {
-                const R z = zero_here((R)0);   // no lane divides
-                un = {z, z, z};
+                cell_face(R0, Lf);
+                cell_face(R0, Rf);
             }
-            // |u| of U^n (friction, exchange).  In FP64 a wave at rest (|u| =
-            // 0 on every lane) has c = 0 and divides both momenta by 1 + 0 =
-            // 1, which leaves them unchanged: it skips the friction step (the
-            // FP32 solver, where the step is a few instructions, measured
-            // slower with the vote).
-            R modu = (R)0;
-            const bool still = !COMP && __builtin_amdgcn_ballot_w64(un.s != (R)0) == 0;
-            if (!still) {
-                modu = sqrt_voted(un.s);
-                if (!have_dh) Dh = den(v0[0] + (R)kEpsilon);
-                R cf;
-                if (P.friction_law == FRIC_MANNING) {
-                    R hp = v0[0] + (R)kEpsilon;
-                    R dtGnn = (R)(dtd * kG * P.manning_n * P.manning_n);
-                    if constexpr (COMP)
-                        cf = dtGnn * modu / (hp * cbrtf(hp));
-                    else
-                        cf = dtGnn * modu / (hp * cbrt(hp));
-                } else {
-                    cf = qdiv(dtFR * modu, Dh);
-                }
-                // Reconstructor.cu:52-53: both momenta divided by 1 + c
-                const Den<R> Dc = den((R)1 + cf);
-                k1 = qdiv(k1, Dc);
-                k2 = qdiv(k2, Dc);
-            }
-            R phi = (R)0;
-            if (SED && P.suspension) phi = erosion_rate(P, v0[0], modu, v0[4], still);
 
+            // x edge at x - 1/2 (VolumeSolver.cu:227-317)
+            R Rl[5];
+            for (int f = 0; f < 5; f++) Rl[f] = up1(Rf[f]);
+            int fxl = need_fix ? up1i(fx0) : 0;
+            R El[5], Er[5];
+            int kind = N_PX;
+            int fixed;
+            if (x == 0 && !perx) {
+                for (int f = 0; f < 5; f++) El[f] = Lf[f];
+                ghost_state(P, 0, Lf, Er, 2LL * npx + npy + r, 1, ct);
+                kind = N_MX;
+                fixed = fx0;
+            } else if (x == npx && !perx) {
+                for (int f = 0; f < 5; f++) El[f] = Rl[f];
+                ghost_state(P, 1, Rl, Er, (long long)npx + r, 1, ct);
+                fixed = fxl;
+            } else {
+                for (int f = 0; f < 5; f++) {
+                    El[f] = Rl[f];
+                    Er[f] = Lf[f];
+                }
+                fixed = (perx && (x == 0 || x == npx)) ? fxl : fxl * fx0;
+            }
+
+            // y faces of row r + 1 and the edge r + 1/2
+            derive_cell<R, SED>(R2);
+            R D1[5];
+            if (second) {
+                if (!CARRY) d0 = cell_diff<R, SED>(R0, R1);
+                const Diff<R> d1 = cell_diff<R, SED>(R1, R2);
+                detay1 = recons_axis<R, SED>(lim, R1, d0, d1, D1, U1);
+                if (CARRY) d0 = d1;
+                filter_faces<R, SED>(D1, U1);
+            } else {
+                cell_face(R1, D1);
+                cell_face(R1, U1);
+            }
+            // upper side of the edge r + 1/2: row r + 1's lower faces, or the
+            // ghost state above the domain's last row
+            R Yr[5];
+            if (r + 1 == npy && !pery)
+                ghost_state(P, 3, U0, Yr, (long long)npx + npy + xc, 2, ct);
+            else
+                for (int f = 0; f < 5; f++) Yr[f] = D1[f];
+            const int fy = (r + 1 == npy) ? fx0 : fx0 * fx1;
+
+            // the x edge x - 1/2 and the y edge r + 1/2, solved side by side
+            edge_flux_pair<R, SED, FB>(P, kind, fixed != 0, El, Er, Dmx, Dpx, N_PY, fy != 0, U0, Yr, FU0, FD1);
+        }
+        R FL[5], FR[5];
+        const bool left_wall = (x == 0 && !perx);
+        for (int f = 0; f < 5; f++) {
+            FL[f] = left_wall ? Dmx[f] : Dpx[f];
+            FR[f] = dn1(Dmx[f]);
+        }
+
+        if (out_lane) {
+            if constexpr (!SPLIT) {
+                if (a.k == 0) {
+                    v0[0] = R0.h;
+                    v0[1] = R0.qx;
+                    v0[2] = R0.qy;
+                    v0[3] = R0.H;
+                    v0[4] = R0.hc;
+                    if (COMP)
+                        for (int j = 0; j < 3; j++) lo_v0[j] = lo_in[j];
+                }
+                phi = source_terms<R, SED>(P, K, a.k, second, R0, detax, detay0, v0, k1, k2);
+            }
             R W[5];
             W[1] = k1 - (invx * (FL[1] + FR[1]) + invy * (FD0[1] + FU0[1]));
             W[2] = k2 - (invx * (FL[2] + FR[2]) + invy * (FD0[2] + FU0[2]));
@@ -808,24 +1014,19 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int tile)
         }
 
         // slide the window
-        R0 = R1;
-        R1 = R2;
-        for (int f = 0; f < 5; f++) {
-            U0[f] = U1[f];
-            FD0[f] = FD1[f];
+        if constexpr (!SPLIT) {
+            R0 = R1;
+            R1 = R2;
+            for (int f = 0; f < 5; f++) {
+                U0[f] = U1[f];
+                FD0[f] = FD1[f];
+            }
+            detay0 = detay1;
+            fx0 = fx1;
         }
-        detay0 = detay1;
-        fx0 = fx1;
     }
 
-    if (a.last) {
-        lxmax = wave_max(lxmax);
-        lymax = wave_max(lymax);
-        const double m = (double)dt_of_speeds(P, lxmax, lymax);
-        if (lane == 0 && m < __longlong_as_double((long long)kInfBits))
-            atomicMin(&a.dts->v[(step + 1) & 1][tile & (kDtSlots - 1)][0],
-                      (unsigned long long)__double_as_longlong(m));
-    }
+    if (a.last) fold_dt(a, P, tile, lane, step, lxmax, lymax);
 }
 
 // Waves per SIMD the register allocation targets.  Measured on the 8192^2
@@ -848,11 +1049,25 @@ constexpr int stage_waves()
     return sizeof(R) == 4 ? TSU_WAVES_FP32 : (SED ? TSU_WAVES_FP64 : TSU_WAVES_FP64_NOSED);
 }
 
+// 130 VGPRs in FP64 with sediment, 92 to 112 otherwise: nothing spills.
+template <typename R, bool SED>
+constexpr int split_waves()
+{
+    return sizeof(R) == 8 && SED ? 3 : 4;
+}
+
 template <typename R, typename S, bool SED, bool FB = false>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(stage_waves<R, SED>(), stage_waves<R, SED>())))
 void stage_kernel(StageArgs a)
 {
     stage_body<R, S, SED, FB>(a, xcd_tile(blockIdx.x, gridDim.x));
+}
+
+template <typename R, typename S, bool SED, bool FB = false>
+__global__ __launch_bounds__(64 * kSplitWaves) __attribute__((amdgpu_waves_per_eu(split_waves<R, SED>(), split_waves<R, SED>())))
+void stage_split_kernel(StageArgs a)
+{
+    stage_body<R, S, SED, FB, true>(a, xcd_tile(blockIdx.x, gridDim.x));
 }
 
 // Ensemble: one launch covers every tile of every scenario.  tiles[b] =
@@ -1128,23 +1343,33 @@ int stage_waves_per_simd(bool sed, int precision)
     return sed ? stage_waves<double, true>() : stage_waves<double, false>();
 }
 
+namespace {
+template <typename R, bool SED, bool FB>
+void launch_stage_of(const StageArgs& a, hipStream_t s)
+{
+    if (a.split)
+        hipLaunchKernelGGL((stage_split_kernel<R, R, SED, FB>), dim3(a.ntiles), dim3(64 * kSplitWaves), 0, s, a);
+    else
+        hipLaunchKernelGGL((stage_kernel<R, R, SED, FB>), dim3(a.ntiles), dim3(64), 0, s, a);
+}
+}  // namespace
+
 hipError_t launch_stage(const StageArgs& a, bool sed, int precision, hipStream_t s, bool fast_bed)
 {
-    dim3 grid(a.ntiles), block(64);
     if (precision == 0) {
         if (sed && fast_bed)
-            hipLaunchKernelGGL((stage_kernel<double, double, true, true>), grid, block, 0, s, a);
+            launch_stage_of<double, true, true>(a, s);
         else if (sed)
-            hipLaunchKernelGGL((stage_kernel<double, double, true>), grid, block, 0, s, a);
+            launch_stage_of<double, true, false>(a, s);
         else
-            hipLaunchKernelGGL((stage_kernel<double, double, false>), grid, block, 0, s, a);
+            launch_stage_of<double, false, false>(a, s);
     } else {
         if (sed && fast_bed)
-            hipLaunchKernelGGL((stage_kernel<float, float, true, true>), grid, block, 0, s, a);
+            launch_stage_of<float, true, true>(a, s);
         else if (sed)
-            hipLaunchKernelGGL((stage_kernel<float, float, true>), grid, block, 0, s, a);
+            launch_stage_of<float, true, false>(a, s);
         else
-            hipLaunchKernelGGL((stage_kernel<float, float, false>), grid, block, 0, s, a);
+            launch_stage_of<float, false, false>(a, s);
     }
     return hipGetLastError();
 }
