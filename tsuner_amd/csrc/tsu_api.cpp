@@ -142,12 +142,14 @@ int set_error(int code, const std::string& msg) { return fail(code, msg); }
 //
 // Alone on the GPU: a tile of r rows costs its wave r + 0.6 rows (the
 // prologue's faces and edge, partly under the launch's start); k waves that
-// share a SIMD take k (1 + 0.4 (w - k) / (w - 1)) rows' time per row, w the
-// kernel's waves per SIMD (a wave alone leaves issue slots idle: 6.6 us
-// against 4.3 us per row in FP64).  Tiles that fit the chip at once last as
-// long as the SIMD with most waves; more run in rounds, the last one partly
-// filled, and with more rounds the tiles' uneven costs (still, dry) blur them
-// into a steady rate.  The 0.4 is the wait for the slowest wave.
+// share a SIMD take from 1.4 (FP64) or 1.7 (FP32) rows' time per row for one
+// to w for w, the kernel's waves per SIMD (a wave alone leaves issue slots
+// idle: 256^2 in FP32 takes 23.8 us a step with up to two one-row waves per
+// SIMD, 29.5 with one of two rows).
+// Tiles that fit the chip at once last as long as the SIMD with most waves;
+// more run in rounds, the last one partly filled, and with more rounds the
+// tiles' uneven costs (still, dry) blur them into a steady rate.  The 0.4 is
+// the wait for the slowest wave.
 //
 // Beside other runs on the GPU (two to three simulations on streams of their
 // own) idle slots are filled by the others and what counts is the work,
@@ -156,19 +158,20 @@ int set_error(int code, const std::string& msg) { return fail(code, msg); }
 //
 // Half an ensemble (what steps on one stream) is judged alone, a single grid
 // by the product of both.  The constants are fits to sweeps of the height
-// over 36 grids of 100^2 .. 4096^2 cells in both precisions, with and without
-// sediment, alone and beside two others.  Against powers of two from 32 down
-// to 2 (at least 8192 tiles, then at least 2048) the chosen heights take
-// 10 % less time alone (at most 3 % more) and 5 % less beside others, on
-// average; us a step alone: 100^2 FP64 43.5 -> 30.0 (1 row for 2), 700^2 143
-// -> 117 (5 for 4), 4096^2 2399 -> 2336 (24 for 32); ensembles of 2.2 million
-// cells in FP32 214 -> 158 (5 for a fixed 16).
-int choose_tile_rows(const std::vector<std::pair<int, int>>& grids, int waves, int device)
+// over 40 grids of 256^2 .. 2048^2 cells in both precisions, with and without
+// sediment, alone and beside two others: over these the chosen heights are
+// 0.4 % from the best alone and 4 % beside others, on average.  Against
+// powers of two from 32 down to 2 (at least 8192 tiles, then at least 2048),
+// us a step alone: 700^2 FP64 143 -> 117 (5 rows for 4), 4096^2 2399 -> 2336
+// (24 for 32); ensembles of 2.2 million cells in FP32 214 -> 158 (5 for a
+// fixed 16).
+int choose_tile_rows(const std::vector<std::pair<int, int>>& grids, bool sed, int precision, int device)
 {
     int cus = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus < 1) cus = 256;
-    const double simds = 4.0 * cus, slots = simds * waves;
-    auto together = [&](double k) { return waves > 1 ? k * (1.0 + 0.4 * (waves - k) / (waves - 1)) : k; };
+    const int waves = stage_waves_per_simd(sed, precision);
+    const double simds = 4.0 * cus, slots = simds * waves, lone = precision == TSU_FP64 ? 1.4 : 1.7;
+    auto together = [&](double k) { return waves > 1 ? lone + (waves - lone) * (k - 1.0) / (waves - 1.0) : k; };
     int best = 1;
     double best_cost = INFINITY;
     for (int r = 1; r <= 32; r++) {
@@ -280,8 +283,7 @@ void set_tiling(tsu_state* st, int rows)
     if (st->split)
         rows = 1;
     else if (rows == 0)
-        rows = tsu::choose_tile_rows({{st->p.npx, st->p.npy}}, tsu::stage_waves_per_simd(st->sed, st->precision),
-                                     st->device);
+        rows = tsu::choose_tile_rows({{st->p.npx, st->p.npy}}, st->sed, st->precision, st->device);
     st->tile_rows = rows;
     st->nstrips = (st->p.npx + tsu::kStripOut - 1) / tsu::kStripOut;
     st->nchunks = (st->p.npy + rows - 1) / rows;

@@ -394,7 +394,7 @@ TSU_API int tsu_ensemble_create(tsu_ensemble** out, int n, const tsu_sim_params*
         for (int i = 0; i < n; i++)
             if (e->half[(size_t)i] == h) grids.emplace_back(params[i].npx, params[i].npy);
         if (grids.empty()) continue;
-        const int rows = tsu::choose_tile_rows(grids, tsu::stage_waves_per_simd(e->sed, precision), device);
+        const int rows = tsu::choose_tile_rows(grids, e->sed, precision, device);
         for (int i = 0; i < n; i++)
             if (e->half[(size_t)i] == h) e->rows[(size_t)i] = rows;
     }

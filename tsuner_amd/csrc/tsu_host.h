@@ -16,8 +16,8 @@ void make_dev_params(const tsu_sim_params* p, const tsu_scheme* s, DevParams* P)
 int validate_scheme(const tsu_scheme* s);
 // Records msg as the calling thread's last error and returns code.
 int set_error(int code, const std::string& msg);
-// Tile height for one launch over grids of (npx, npy) cells with a stage
-// kernel of that many waves per SIMD (tsu_api.cpp).
-int choose_tile_rows(const std::vector<std::pair<int, int>>& grids, int waves_per_simd, int device);
+// Tile height for one launch of the stage kernel over grids of (npx, npy)
+// cells (tsu_api.cpp).
+int choose_tile_rows(const std::vector<std::pair<int, int>>& grids, bool sed, int precision, int device);
 
 }  // namespace tsu
