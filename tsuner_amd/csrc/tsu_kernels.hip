@@ -762,6 +762,14 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int tile)
         R v0[5];
         R lo_in[3] = {(R)0, (R)0, (R)0}, lo_v0[3] = {(R)0, (R)0, (R)0};
         const long long pos = (long long)r * npx + xc;
+        // small grids: the running maxima, which otherwise are two more
+        // memory latencies at the end (loads after stores): 18.5 -> 18.0 us a
+        // step of 100 x 100 cells
+        double peak[3];
+        if constexpr (SPLIT) {
+            if (out_lane && a.last && a.ext)
+                for (int j = 0; j < 3; j++) peak[j] = a.ext[j * nv + pos];
+        }
         if (out_lane) {
             if (a.k != 0) {
                 v0[0] = (R)v0p[pos];
@@ -1005,10 +1013,10 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int tile)
                     double* bmax = a.ext + nv;
                     double* emax = a.ext + 2 * nv;
                     if (hd > P.epsilon_h) {
-                        hmax[pos] = fmax(hmax[pos], hd);
-                        emax[pos] = fmax(emax[pos], hd - Hs);
+                        hmax[pos] = fmax(SPLIT ? peak[0] : hmax[pos], hd);
+                        emax[pos] = fmax(SPLIT ? peak[2] : emax[pos], hd - Hs);
                     }
-                    bmax[pos] = fmax(bmax[pos], Hs);
+                    bmax[pos] = fmax(SPLIT ? peak[1] : bmax[pos], Hs);
                 }
             }
         }
