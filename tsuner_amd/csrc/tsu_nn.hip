@@ -111,13 +111,13 @@ __device__ __forceinline__ void lds_barrier()
 //
 // Bound by the bytes of both tensors for the narrow layers and by how well the
 // MFMAs, the epilogue and the loads of one workgroup overlap for 64 -> 64
-// (matrix pipe 52 % busy).  Before (weights and a 10 x 66 pixel tile in LDS, one
+// (matrix pipe 51 % busy; without its loads and stores 120 us).  Before (weights and a 10 x 66 pixel tile in LDS, one
 // read per two MFMAs, the tile's loads and stores between barriers) and now, us:
 //            8->32  32->32  32->4  8->64  64->64  64->4, and the data
 //   32 images  41     89     48    106     200     95    gradients 4<-32 60,
-//   of 256^2   27     49     44     70     163     70    32<-32 103, 4<-64 181,
-//   8 images   14     25     14     28      55     27    64<-64 259 -> 53, 97,
-//              10     17     12     16      47     21    124, 215 (32 images)
+//   of 256^2   27     49     40     71     150     68    32<-32 103, 4<-64 181,
+//   8 images   14     25     14     28      55     27    64<-64 259 -> 53, 80,
+//              10     17     11     15      42     20    126, 181 (32 images)
 // 32 -> 32 moves 268 MB in 49 us, 5.5 TB/s of the copy kernel's 6.1.  Accumulation
 // order and results are those of one tap after the other.
 //
@@ -165,6 +165,8 @@ __attribute__((amdgpu_waves_per_eu(conv_waves<K>(), conv_waves<K>()))) void conv
     constexpr int SWEEP = T / SLOTS;                        // rows per sweep of the workgroup
     constexpr int LOADS = SWEEP >= R ? 1 : R / SWEEP;
     constexpr int STEPS = K == 8 ? 3 : 9 * KK;
+    constexpr int READS = (K == 8 ? RW : RW + 2) * 3 * KK, AHEAD = K == 64 ? 2 : 0;
+    constexpr bool EARLY = K == 64 || (K == 32 && POST == 2);   // see put
     static_assert(T % SLOTS == 0 && 2 * KO * R <= T, "one slot per thread and sweep");
     __shared__ uint4 ring[conv_ring(R) * XROW];
     const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -202,19 +204,19 @@ __attribute__((amdgpu_waves_per_eu(conv_waves<K>(), conv_waves<K>()))) void conv
     const int ecol = kStripCols + tid / KO % 2, erow = tid / (2 * KO);
     const int eput_at = erow * XROW + ecol * KO + (q ^ octet_xor<K>(ecol));
     uint4 stage[LOADS], estage;
-    auto load = [&](int gr, int gc) {                       // zeros outside the image
+    auto load = [&](int gr, int gc, int rows) {             // zeros outside the image's first rows
         uint4 v = make_uint4(0, 0, 0, 0);
-        if (gr >= 0 && gr < H && gc >= 0 && gc < W)
+        if (gr >= 0 && gr < rows && gc >= 0 && gc < W)
             v = *(const uint4*)((const char*)in + ((size_t)walk.n * H + gr) * W * (2 * K) +
                                 (uint32_t)((gc * K + 8 * q) * 2));
         return v;
     };
     // the pass's new rows, r0 + 1 .. r0 + R (columns c0 - 1 .. c0 + 64), into registers
-    auto fetch = [&]() {
+    auto fetch = [&](int rows) {
 #pragma unroll
         for (int j = 0; j < LOADS; j++)
-            if (SWEEP <= R || row < R) stage[j] = load(walk.r0 + 1 + j * SWEEP + row, walk.c0 - 1 + col);
-        if (has_edge) estage = load(walk.r0 + 1 + erow, walk.c0 - 1 + ecol);
+            if (SWEEP <= R || row < R) stage[j] = load(walk.r0 + 1 + j * SWEEP + row, walk.c0 - 1 + col, rows);
+        if (has_edge) estage = load(walk.r0 + 1 + erow, walk.c0 - 1 + ecol, rows);
     };
     // ... and into ring rows R ph + 2 .. R ph + R + 1; the last two of block 2
     // are also the first two of block 0
@@ -232,15 +234,16 @@ __attribute__((amdgpu_waves_per_eu(conv_waves<K>(), conv_waves<K>()))) void conv
             if (ph == 2 && erow >= R - 2) ring[-(R - 2) * XROW + eput_at] = estage;
         }
     };
-    // at the top of a stretch or strip: rows r0 - 1 and r0 into ring rows 0, 1
-    auto top = [&]() {
+    // at the top of a stretch or strip: rows r0 - 1 and r0 into ring rows R ph
+    // and R ph + 1
+    auto top = [&](int ph) {
         for (int idx = tid; idx < 2 * XROW; idx += T) {
             const int o = idx % KO, c = idx / KO % XCOL, i = idx / XROW;
             const int gr = walk.r0 - 1 + i, gc = walk.c0 - 1 + c;
             uint4 v = make_uint4(0, 0, 0, 0);
             if (gr >= 0 && gr < H && gc >= 0 && gc < W)
                 v = *(const uint4*)(in + (((size_t)walk.n * H + gr) * W + gc) * K + 8 * o);
-            ring[i * XROW + c * KO + (o ^ octet_xor<K>(c))] = v;
+            ring[(R * ph + i) * XROW + c * KO + (o ^ octet_xor<K>(c))] = v;
         }
     };
 
@@ -257,20 +260,20 @@ __attribute__((amdgpu_waves_per_eu(conv_waves<K>(), conv_waves<K>()))) void conv
         }
 
     int ph = 0;                                             // ring row of input row r0 - 1, over R
-    fetch();
-    top();
+    fetch(H);
+    top(0);
     put(0);
     lds_barrier();
     for (;;) {
         int cr0 = walk.r0 + RW * rg;                        // this pass: the wave's first row, this lane's column
         const int c = walk.c0 + 16 * seg + li;
+        const int pass_n = walk.n;
         size_t p0 = ((size_t)walk.n * H + cr0) * W + c;
         const bool more = --walk.left > 0;                  // uniform over the workgroup
         bool down = false;                                  // the next pass continues this strip
-        if (more) {
-            down = walk.next(R);
-            fetch();
-        }
+        if (more) down = walk.next(R);
+        if (EARLY || more) fetch(more ? H : 0);
+        const int next_ph = ph == 2 ? 0 : ph + 1;           // the coming rows have ring rows of their own
         const uint4* rows = ring + R * ph * XROW;
 #pragma unroll 1
         for (int part = 0; part < R / 4; part++) {
@@ -280,26 +283,51 @@ __attribute__((amdgpu_waves_per_eu(conv_waves<K>(), conv_waves<K>()))) void conv
 #pragma unroll
                 for (int a = 0; a < MTW; a++) acc[r][a] = f32x4{0.f, 0.f, 0.f, 0.f};
             // by input row: an output row then takes its taps in their order
-            // (and with 8 channels, a row's steps, whose offsets the lanes hold)
+            // (and with 8 channels, a row's steps, whose offsets the lanes
+            // hold).  With 64 channels AHEAD reads are kept in flight: the
+            // compiler, short of registers, issued each and waited for it by
+            // itself.
+            auto read = [&](int i) {
+                const int j = i / (3 * KK), rx = i / KK % 3, kk = i % KK;
+                uint4 v = rows[at[rx][kk] + j * XROW];
+                if (K == 8 && rx == 2 && g > 0) v = make_uint4(0, 0, 0, 0);   // past the ninth offset
+                return v;
+            };
+            uint4 ahead[AHEAD + 1];
 #pragma unroll
-            for (int j = 0; j < (K == 8 ? RW : RW + 2); j++)
+            for (int i = 0; i < AHEAD; i++) ahead[i] = read(i);
 #pragma unroll
-                for (int rx = 0; rx < 3; rx++)
+            for (int i = 0; i < READS; i++) {
+                if (i + AHEAD < READS) ahead[(i + AHEAD) % (AHEAD + 1)] = read(i + AHEAD);
+                if (AHEAD > 0) __builtin_amdgcn_sched_barrier(0);
+                const int j = i / (3 * KK), rx = i / KK % 3, kk = i % KK;
+                const bf16x8 B = as_bf16x8(ahead[i % (AHEAD + 1)]);
 #pragma unroll
-                    for (int kk = 0; kk < KK; kk++) {
-                        uint4 v = rows[at[rx][kk] + j * XROW];
-                        if (K == 8 && rx == 2 && g > 0) v = make_uint4(0, 0, 0, 0);   // past the ninth offset
-                        const bf16x8 B = as_bf16x8(v);
+                for (int ry = 0; ry < (K == 8 ? 1 : 3); ry++) {
+                    const int r = j - ry;
+                    if (r < 0 || r >= RW) continue;
 #pragma unroll
-                        for (int ry = 0; ry < (K == 8 ? 1 : 3); ry++) {
-                            const int r = j - ry;
-                            if (r < 0 || r >= RW) continue;
+                    for (int a = 0; a < MTW; a++)
+                        acc[r][a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            A[K == 8 ? rx : (3 * ry + rx) * KK + kk][a], B, acc[r][a], 0, 0, 0);
+                }
+            }
+            // the activations of all rows at once (a row's load behind the
+            // stores of the rows before it waits for them as well)
+            uint4 mask[RW];
+            if constexpr (POST == 2 && K != 8) {
 #pragma unroll
-                            for (int a = 0; a < MTW; a++)
-                                acc[r][a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                                    A[K == 8 ? rx : (3 * ry + rx) * KK + kk][a], B, acc[r][a], 0, 0, 0);
-                        }
-                    }
+                for (int r = 0; r < RW; r++)
+                    mask[r] = *(const uint4*)(act + (((size_t)pass_n * H + min(cr0 + r, H - 1)) * W + min(c, W - 1)) * MOUT +
+                                              m0);
+            }
+            // EARLY: the coming rows go into the ring ahead of the results'
+            // stores, in every pass.  A wait for these loads behind stores
+            // that lanes may skip is a wait for the stores too: 64 -> 64, 32
+            // images, 162 -> 150 us with the reads ahead.  Short passes have
+            // the loads come later than the stores go: 8 -> 32, 8 images,
+            // 9.2 us so and 10.0 early, 32 -> 32 16.9 and 17.7.
+            if (EARLY) put(next_ph);
 #pragma unroll
             for (int r = 0; r < RW; r++) {
                 if (cr0 + r >= H || c >= W || m0 >= MOUT) continue;
@@ -318,10 +346,8 @@ __attribute__((amdgpu_waves_per_eu(conv_waves<K>(), conv_waves<K>()))) void conv
                 } else {
                     static_assert(MTW == 2, "16-byte stores");
                     if (POST == 2) {
-                        // (loading it ahead of the MFMAs costs registers: 21
-                        // spilled with 64 channels, 50 -> 76 us for 8 images)
-                        const uint4 av = *(const uint4*)(act + p * MOUT + m0);
-                        const uint32_t aw[4] = {av.x, av.y, av.z, av.w};
+                        if (K == 8) mask[r] = *(const uint4*)(act + p * MOUT + m0);
+                        const uint32_t aw[4] = {mask[r].x, mask[r].y, mask[r].z, mask[r].w};
                         // ReLU outputs are >= 0: only +0 / -0 bit patterns mean inactive
 #pragma unroll
                         for (int e = 0; e < 4; e++) {
@@ -339,14 +365,12 @@ __attribute__((amdgpu_waves_per_eu(conv_waves<K>(), conv_waves<K>()))) void conv
             p0 += 4 * (size_t)W;
         }
         if (!more) break;
-        if (down) {
-            ph = ph == 2 ? 0 : ph + 1;                      // the coming rows have ring rows of their own
-        } else {
-            lds_barrier();                                // every wave is done with the ring
-            ph = 0;
-            top();
+        if (!EARLY) put(next_ph);
+        ph = next_ph;
+        if (!down) {
+            lds_barrier();                                // every wave is done with the rows above
+            top(ph);
         }
-        put(ph);
         lds_barrier();
     }
 }
