@@ -396,10 +396,10 @@ __attribute__((amdgpu_waves_per_eu(conv_waves<K>(), conv_waves<K>()))) void conv
 // kWgradWaves = 256 of them cover the chip.
 //
 // Measured, 8 images of 256^2, before and now (gradient + reduction):
-//   64 -> 64  220 + 112 us -> 57 + 11 us (680 TFLOP/s; both tensors once are
+//   64 -> 64  220 + 112 us -> 50 + 7 us (770 TFLOP/s; both tensors once are
 //             134 MB, 22 us at the copy kernel's 6.1 TB/s, the MFMAs 15 us at
 //             peak, the transposing reads 17 us of LDS time)
-//   32 -> 32  109 + 110 us -> 24 + 5 us (67 MB, 11 us)
+//   32 -> 32  109 + 110 us -> 21 + 4 us (67 MB, 11 us)
 //   8 -> 64, 64 -> 4   145 and 118 + 112 us -> 21 + 5 us (76 MB, 12 us)
 //   8 -> 32, 32 -> 4    84 and 82 + 110 us -> 13 + 4 us (42 MB, 7 us)
 //
@@ -461,6 +461,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     constexpr int STEPS = 2 * R / GROUPS;          // 32-pixel steps of a wave per pass
     constexpr int XPT = (R * 66 * KO + 511) / 512, DPT = R * 64 * KO / 512;
     constexpr int XN = XR * XROW / 16, DN = DR * DROW / 16;
+    constexpr int AHEAD = 1;                       // operands read ahead of their MFMAs
     constexpr int TILES = 38;                      // accumulator tiles of a wave, bias included
     constexpr int RED = 4 * TILES * 64;            // those of half of the waves
     constexpr int LDS = XN + DN > RED ? XN + DN : RED;
@@ -563,27 +564,37 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             bf16x8 A[2];
 #pragma unroll
             for (int a = 0; a < 2; a++) A[a] = read_tr8(da[a] + dof, da[a] + dof + 16 * PIX);
+            uint32_t xo[3];
+#pragma unroll
+            for (int ty = 0; ty < 3; ty++) {
+                int xrow = xs + (st >> 1) + ty;
+                xrow = xrow >= XR ? xrow - XR : xrow;
+                xo[ty] = (uint32_t)(xrow * XROW) + half;
+            }
+            // input operands (ty, d, b), each read while its predecessor's two
+            // MFMAs run: the compiler, short of registers, waited for each read
+            // (64 -> 64 60.5 us with its reduction, one ahead 56.7, two 57.3,
+            // three, which spill, 59.2)
+            auto read = [&](int i) {
+                const uint32_t at = xa[i / 2 % 3][i % 2] + xo[i / 6];
+                return read_tr8(at, at + 16 * PIX);
+            };
+            bf16x8 B[AHEAD + 1];
+#pragma unroll
+            for (int i = 0; i < AHEAD; i++) B[i] = read(i);
             if (k0 == 0) {
 #pragma unroll
                 for (int a = 0; a < 2; a++)
                     acc[36 + a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[a], ones, acc[36 + a], 0, 0, 0);
             }
 #pragma unroll
-            for (int ty = 0; ty < 3; ty++) {
-                int xrow = xs + (st >> 1) + ty;
-                xrow = xrow >= XR ? xrow - XR : xrow;
-                const uint32_t xo = (uint32_t)(xrow * XROW) + half;
+            for (int i = 0; i < 18; i++) {
+                if (i + AHEAD < 18) B[(i + AHEAD) % (AHEAD + 1)] = read(i + AHEAD);
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int d = 0; d < 3; d++)
-#pragma unroll
-                    for (int b = 0; b < 2; b++) {
-                        const bf16x8 B = read_tr8(xa[d][b] + xo, xa[d][b] + xo + 16 * PIX);
-#pragma unroll
-                        for (int a = 0; a < 2; a++) {
-                            f32x4& c = acc[((ty * 3 + d) * 2 + b) * 2 + a];
-                            c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[a], B, c, 0, 0, 0);
-                        }
-                    }
+                for (int a = 0; a < 2; a++)
+                    acc[2 * i + a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[a], B[i % (AHEAD + 1)], acc[2 * i + a], 0,
+                                                                             0, 0);
             }
         }
         if (!more) break;
