@@ -290,6 +290,14 @@ TSU_API int tsu_nn_adam(float *p, const float *g, float *m, float *v, long long 
 /* FP32 [9][m][k] -> BF16 same layout (wb) and, if wt != NULL, the per-tap
  * transpose wt[9][k][mt] of rows m < mt. */
 TSU_API int tsu_nn_pack(const float *w, void *wb, void *wt, int m, int k, int mt, void *stream);
+/* tsu_nn_adam on the parameters of a whole network (8 -> width, mids times
+ * width -> width, width -> 4 held as 16 rows, each layer's [9][m][k] weights
+ * followed by its bias; width 32 or 64) and tsu_nn_pack of every layer, in one
+ * launch.  wb: the layers' BF16 weights one after the other; wt: the
+ * transposes of layers 1, 2, ... one after the other, [9][width][width] each
+ * and [9][width][8] of the last. */
+TSU_API int tsu_nn_adam_pack(float *p, const float *g, float *m, float *v, float lr_t, float beta1, float beta2,
+                             float eps, int width, int mids, void *wb, void *wt, void *stream);
 /* Network inputs of every member of a two-stage ensemble whose members share
  * one grid: x[member][y][x][8] BF16 = (h, qx, qy, z = -H, dz/dx, dz/dy, eta if
  * h > wet_h else 0, wet flag) times scale_in[0..7]. */

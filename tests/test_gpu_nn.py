@@ -294,6 +294,35 @@ def test_mse_and_adam_kernels():
                                atol=1e-7)
 
 
+@pytest.mark.parametrize("width,mids", [(32, 0), (32, 2), (64, 1), (64, 4)])
+def test_adam_pack_equals_step_and_packs(width, mids):
+    """One launch for the step and all layers' BF16 copies against the step
+    and one packing per layer: the same values."""
+    import math
+    import torch
+    from tsuner_amd import nn
+    arch = nn.Arch(width, mids)
+    rng = np.random.default_rng(width + mids)
+    g, m, v = (rng.normal(size=arch.nparam).astype(np.float32) for _ in range(3))
+    nets = [nn.Net(nn.init_params(3, arch), max_batch=1, h=8, w=8, arch=arch) for _ in range(2)]
+    for net in nets:
+        net.g.copy_(dev_f32(g))
+        net.m.copy_(dev_f32(1e-3 * m))
+        net.v.copy_(dev_f32(1e-6 * v * v))
+    a, b = nets
+    a.adam(1e-2)
+    lr_t = 1e-2 * math.sqrt(1.0 - 0.999) / (1.0 - 0.9)
+    ok(lib().tsu_nn_adam(P(b.p), P(b.g), P(b.m), P(b.v), arch.nparam, C.c_float(lr_t), C.c_float(0.9), C.c_float(0.999),
+                         C.c_float(1e-8), C.c_void_p(0)))
+    b.pack()
+    for x, y in zip([a.p, a.m, a.v] + a.wb + a.wt[1:], [b.p, b.m, b.v] + b.wb + b.wt[1:]):
+        assert torch.equal(x, y)
+    assert not torch.equal(a.p, dev_f32(nn.init_params(3, arch)))
+    s = C.c_void_p(0)
+    assert lib().tsu_nn_adam_pack(P(a.p), P(a.g), P(a.m), P(a.v), C.c_float(0), C.c_float(0), C.c_float(0), C.c_float(1),
+                                  48, 1, P(a.p), P(a.p), s) != 0
+
+
 @pytest.mark.parametrize("width,mids", [(32, 2), (64, 1), (32, 4)])
 def test_network_gradients_match_oracle(width, mids):
     """Full forward + backward on the GPU against the oracle's loss_and_grads

@@ -131,6 +131,8 @@ _PROTOS = {
                              C.c_void_p]),
     "tsu_nn_adam": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_longlong, C.c_float, C.c_float,
                               C.c_float, C.c_float, C.c_void_p]),
+    "tsu_nn_adam_pack": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_float, C.c_float, C.c_float,
+                                   C.c_float, C.c_int, C.c_int, C.c_void_p, C.c_void_p, C.c_void_p]),
     "tsu_nn_pack": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_void_p]),
     "tsu_ensemble_nn_features": (C.c_int, [C.c_void_p, C.POINTER(C.c_float), C.c_float, C.c_void_p]),
     "tsu_ensemble_nn_apply": (C.c_int, [C.c_void_p, C.POINTER(C.c_float), C.c_float, C.c_void_p, C.c_longlong,

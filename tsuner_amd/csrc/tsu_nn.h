@@ -47,6 +47,8 @@ hipError_t nn_launch_mse(const float* out, const float* tgt, uint16_t* dy, doubl
                          long long npix, float scale, hipStream_t s);
 hipError_t nn_launch_adam(float* p, const float* g, float* m, float* v, long long n, float lr_t, float b1, float b2,
                           float eps, hipStream_t s);
+hipError_t nn_launch_adam_pack(float* p, const float* g, float* m, float* v, float lr_t, float b1, float b2, float eps,
+                               int width, int mids, uint16_t* wb, uint16_t* wt, hipStream_t s);
 hipError_t nn_launch_pack(const float* w, uint16_t* wb, uint16_t* wt, int m, int k, int mt, hipStream_t s);
 
 // Ensemble-side kernels.  args: the members' last-stage arguments (their

@@ -905,21 +905,63 @@ __global__ __launch_bounds__(256) void mse_kernel(const float* __restrict__ out,
 }
 
 // Adam (Kingma & Ba 2015) with bias correction folded into the step size.
+__device__ __forceinline__ float adam_one(float* __restrict__ p, const float* __restrict__ gr, float* __restrict__ m,
+                                          float* __restrict__ v, long long i, float lr_t, float b1, float b2, float eps)
+{
+    const float gi = gr[i];
+    const float mi = b1 * m[i] + (1.f - b1) * gi;
+    const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
+    m[i] = mi;
+    v[i] = vi;
+    return p[i] -= lr_t * mi / (sqrtf(vi) + eps);
+}
+
 __global__ void adam_kernel(float* __restrict__ p, const float* __restrict__ gr, float* __restrict__ m,
                             float* __restrict__ v, long long n, float lr_t, float b1, float b2, float eps)
 {
     for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
-        const float gi = gr[i];
-        const float mi = b1 * m[i] + (1.f - b1) * gi;
-        const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-        m[i] = mi;
-        v[i] = vi;
-        p[i] -= lr_t * mi / (sqrtf(vi) + eps);
+        adam_one(p, gr, m, v, i, lr_t, b1, b2, eps);
     }
 }
 
-// FP32 master weights [9][m][k] -> BF16 forward weights (same layout) and,
-// if wt != null, BF16 per-tap transposes wt[9][k][mt] keeping m < mt.
+// The step of a whole network's parameters (layer l's weights [9][m][k], then
+// its bias) with every layer's BF16 copies, one parameter per thread: a launch
+// for each layer's copies is all latency.  8 images of 256^2: a training step
+// of the 32-wide network 206 -> 200 us; the 64-wide one takes the same 692.
+//
+// A wave takes 8 rows x 8 input channels of a tap, so that the transposed
+// copies are written 16 bytes at a time (with a row of 64 channels per wave,
+// 2-byte stores to 64 lines each, 697 us).
+template <int W>
+__global__ __launch_bounds__(256) void adam_pack_kernel(float* __restrict__ p, const float* __restrict__ gr,
+                                                        float* __restrict__ m, float* __restrict__ v, float lr_t,
+                                                        float b1, float b2, float eps, int mids,
+                                                        uint16_t* __restrict__ wb, uint16_t* __restrict__ wt)
+{
+    constexpr int FIRST = 9 * W * 8, MID = 9 * W * W, LAST = 9 * 16 * W;   // weights of a layer
+    const long long i = blockIdx.x * 256LL + threadIdx.x;
+    const long long weights = FIRST + mids * (long long)MID + LAST;
+    if (i >= weights) {                                                    // a bias
+        const long long b = i - weights;
+        const long long l = min(b / W, mids + 1LL);
+        if (b < (mids + 1LL) * W + 16)
+            adam_one(p, gr, m, v, (l <= mids ? FIRST + l * (long long)MID : weights) + b, lr_t, b1, b2, eps);
+        return;
+    }
+    const int l = i < FIRST ? 0 : 1 + (int)min((i - FIRST) / MID, (long long)mids);
+    const bool last = l == mids + 1;
+    const long long base = l == 0 ? 0 : FIRST + (l - 1) * (long long)MID;  // of the layer in wb
+    const int rows = last ? 16 : W, ks = l == 0 ? 8 : W;
+    const int at = (int)(i - base), tile = at / 64, lane = at % 64;
+    const int t = at / (rows * ks), in_tap = tile - t * (rows * ks / 64);
+    const int row = in_tap / (ks / 8) * 8 + lane % 8, k = in_tap % (ks / 8) * 8 + lane / 8;
+    const int w = (t * rows + row) * ks + k;
+    const uint16_t b = to_bf16(adam_one(p, gr, m, v, base + l * (long long)W + w, lr_t, b1, b2, eps));
+    wb[base + w] = b;
+    const int mt = last ? 8 : W;
+    if (l > 0 && row < mt) wt[base - FIRST + (t * W + k) * mt + row] = b;
+}
+
 __global__ void pack_kernel(const float* __restrict__ w, uint16_t* __restrict__ wb, uint16_t* __restrict__ wt, int m,
                             int k, int mt)
 {
@@ -1334,6 +1376,18 @@ hipError_t nn_launch_adam(float* p, const float* g, float* m, float* v, long lon
 {
     adam_kernel<<<(unsigned)((n + 255) / 256 < 1024 ? (n + 255) / 256 : 1024), 256, 0, s>>>(p, g, m, v, n, lr_t, b1,
                                                                                            b2, eps);
+    return hipGetLastError();
+}
+
+hipError_t nn_launch_adam_pack(float* p, const float* g, float* m, float* v, float lr_t, float b1, float b2, float eps,
+                               int width, int mids, uint16_t* wb, uint16_t* wt, hipStream_t s)
+{
+    const long long n = 9LL * width * 8 + width + mids * (9LL * width * width + width) + 9LL * 16 * width + 16;
+    const unsigned blocks = (unsigned)((n + 255) / 256);
+    if (width == 32)
+        adam_pack_kernel<32><<<blocks, 256, 0, s>>>(p, g, m, v, lr_t, b1, b2, eps, mids, wb, wt);
+    else
+        adam_pack_kernel<64><<<blocks, 256, 0, s>>>(p, g, m, v, lr_t, b1, b2, eps, mids, wb, wt);
     return hipGetLastError();
 }
 

@@ -159,6 +159,16 @@ TSU_API int tsu_nn_adam(float* p, const float* g, float* m, float* v, long long 
     return e == hipSuccess ? TSU_OK : hip_fail("tsu_nn_adam", e);
 }
 
+TSU_API int tsu_nn_adam_pack(float* p, const float* g, float* m, float* v, float lr_t, float beta1, float beta2,
+                             float eps, int width, int mids, void* wb, void* wt, void* stream)
+{
+    if (!p || !g || !m || !v || !wb || !wt || (width != 32 && width != 64) || mids < 0)
+        return tsu::set_error(TSU_ERR_ARG, "tsu_nn_adam_pack: bad argument");
+    hipError_t e = tsu::nn_launch_adam_pack(p, g, m, v, lr_t, beta1, beta2, eps, width, mids, (uint16_t*)wb,
+                                            (uint16_t*)wt, (hipStream_t)stream);
+    return e == hipSuccess ? TSU_OK : hip_fail("tsu_nn_adam_pack", e);
+}
+
 TSU_API int tsu_nn_pack(const float* w, void* wb, void* wt, int m, int k, int mt, void* stream)
 {
     if (!w || !wb || m < 1 || k < 1 || (wt && (mt < 1 || mt > m)))

@@ -113,9 +113,11 @@ class Net:
         self.t = 0
         bf = dict(dtype=torch.bfloat16, device=self.dev)
         W, L = arch.width, arch.nlayers
-        self.wb = [torch.zeros(9 * m * k, **bf) for m, k in arch.layers]
-        # per-tap transposes used by the data gradients of layers 1 .. L-1
-        self.wt = [None] + [torch.zeros(9 * W * W, **bf) for _ in range(arch.mids)] + [torch.zeros(9 * W * 8, **bf)]
+        # BF16 weights of the layers, and per-tap transposes used by the data
+        # gradients of layers 1 .. L-1: parts of one buffer each
+        wb, wt = [9 * m * k for m, k in arch.layers], [9 * W * W] * arch.mids + [9 * W * 8]
+        self._wb, self._wt = torch.zeros(sum(wb), **bf), torch.zeros(sum(wt), **bf)
+        self.wb, self.wt = list(self._wb.split(wb)), [None] + list(self._wt.split(wt))
         npix = max_batch * h * w
         self.acts = [torch.zeros(npix * W, **bf) for _ in range(L - 1)]
         self.out = torch.zeros(npix * COUT, **f32)
@@ -194,9 +196,9 @@ class Net:
     def adam(self, lr: float, b1: float = 0.9, b2: float = 0.999, eps: float = 1e-8):
         self.t += 1
         lr_t = lr * math.sqrt(1.0 - b2 ** self.t) / (1.0 - b1 ** self.t)
-        check(lib().tsu_nn_adam(_ptr(self.p), _ptr(self.g), _ptr(self.m), _ptr(self.v), self.arch.nparam, C.c_float(lr_t),
-                                C.c_float(b1), C.c_float(b2), C.c_float(eps), _stream()), "adam")
-        self.pack()
+        check(lib().tsu_nn_adam_pack(_ptr(self.p), _ptr(self.g), _ptr(self.m), _ptr(self.v), C.c_float(lr_t),
+                                     C.c_float(b1), C.c_float(b2), C.c_float(eps), self.arch.width, self.arch.mids,
+                                     _ptr(self._wb), _ptr(self._wt), _stream()), "adam")
 
     def train_step(self, x, target, n: int, lr: float) -> None:
         self.forward(x, n)
