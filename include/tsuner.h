@@ -214,6 +214,8 @@ TSU_API int tsu_ensemble_create(tsu_ensemble **out, int n, const tsu_sim_params 
 TSU_API int tsu_ensemble_destroy(tsu_ensemble *e);
 TSU_API int tsu_ensemble_upload(tsu_ensemble *e, int member, const double *V, const int *fixH);
 TSU_API int tsu_ensemble_download(tsu_ensemble *e, int member, double *V);
+/* One plane of it: 0 h, 1 qx, 2 qy, 3 H, 4 hc. */
+TSU_API int tsu_ensemble_download_plane(tsu_ensemble *e, int member, int plane, double *out);
 TSU_API int tsu_ensemble_init_dt(tsu_ensemble *e);
 /* Boundary series of one member, in the layout of tsu_state_set_inflow
  * (VolumeSolver.cu:172-202 read per member at that member's time). */

@@ -161,3 +161,23 @@ def test_halves_on_two_streams_equal_single_solver(n, order, chunk):
             assert g.mass() == m[i]
         assert np.array_equal(ens.state(i), g.state()), "member %d" % i
         assert ens.time(i) == g.time()
+
+
+@pytest.mark.parametrize("nx,ny", [(1, 1), (63, 5), (1100, 801)])
+def test_fp32_states_keep_hi_and_lo_parts(nx, ny):
+    """FP64 planes -> float pairs (q: floats) -> FP64 planes; the last grid's
+    five planes take more than one transfer of 4 Mi values."""
+    rng = np.random.default_rng(nx)
+    V = rng.normal(size=(5, ny, nx)) * 10.0 ** rng.integers(-42, 6, size=(5, ny, nx))
+    V.reshape(5, -1)[:, 0] = [0.0, -0.0, 1e-45, 3e38, 1e-300]
+    want = V.astype(np.float32).astype(np.float64)
+    for f in (0, 3, 4):
+        want[f] += (V[f] - want[f]).astype(np.float32).astype(np.float64)
+    sc = S.Scenario("random", S.base_params(nx, ny, 10.0, 10.0), S.default_scheme(), V, np.ones((ny, nx), np.int32))
+    s = Solver.from_scenario(sc, precision="fp32", init_dt=False)
+    assert np.array_equal(s.state(), want)
+    ens = Ensemble([sc, sc], precision="fp32")
+    for i in range(2):
+        assert np.array_equal(ens.state(i), want)
+        for f in range(5):
+            assert np.array_equal(ens.plane(i, f), want[f])

@@ -295,7 +295,7 @@ class RunResult:
 def _bed_change(ens, i, H0: np.ndarray, factor: int) -> np.ndarray:
     """H_end - H0 of member i, averaged over factor x factor blocks (the
     restriction's bed is the block mean)."""
-    d = ens.state(i)[3] - H0
+    d = ens.plane(i, 3) - H0
     if factor == 1:
         return d
     n = d.shape[0] // factor

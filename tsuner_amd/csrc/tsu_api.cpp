@@ -138,6 +138,63 @@ int validate_scheme(const tsu_scheme* s) { return check_scheme(s); }
 
 int set_error(int code, const std::string& msg) { return fail(code, msg); }
 
+namespace {
+int reserve(Staging* g, long long count)
+{
+    const long long want = std::min(count, 4LL << 20);
+    if (g->cap >= want) return TSU_OK;
+    free_staging(g);
+    if (hipMalloc((void**)&g->buf, (size_t)want * sizeof(double)) != hipSuccess) {
+        (void)hipGetLastError();
+        g->buf = nullptr;
+        return fail(TSU_ERR_DEVICE_MEMORY, "transfer buffer allocation failed");
+    }
+    g->cap = want;
+    return TSU_OK;
+}
+}  // namespace
+
+void free_staging(Staging* g)
+{
+    (void)hipFree(g->buf);
+    *g = Staging{};
+}
+
+int upload_planes(Staging* g, const double* host, void* state, int precision, long long nv, hipStream_t s)
+{
+    const long long count = 5 * nv;
+    if (precision == TSU_FP64) {
+        HIPCHK(hipMemcpyAsync(state, host, (size_t)count * sizeof(double), hipMemcpyHostToDevice, s));
+    } else {
+        if (int rc = reserve(g, count)) return rc;
+        for (long long o = 0; o < count; o += g->cap) {
+            const long long n = std::min(g->cap, count - o);
+            HIPCHK(hipMemcpyAsync(g->buf, host + o, (size_t)n * sizeof(double), hipMemcpyHostToDevice, s));
+            HIPCHK(launch_narrow(g->buf, (float*)state, nv, o, n, s));
+        }
+    }
+    HIPCHK(hipStreamSynchronize(s));
+    return TSU_OK;
+}
+
+int download_planes(Staging* g, const void* state, double* host, int precision, long long nv, long long first,
+                    long long count, hipStream_t s)
+{
+    if (precision == TSU_FP64) {
+        HIPCHK(hipMemcpyAsync(host, (const double*)state + first, (size_t)count * sizeof(double),
+                              hipMemcpyDeviceToHost, s));
+    } else {
+        if (int rc = reserve(g, count)) return rc;
+        for (long long o = 0; o < count; o += g->cap) {
+            const long long n = std::min(g->cap, count - o);
+            HIPCHK(launch_widen((const float*)state, g->buf, nv, first + o, n, s));
+            HIPCHK(hipMemcpyAsync(host + o, g->buf, (size_t)n * sizeof(double), hipMemcpyDeviceToHost, s));
+        }
+    }
+    HIPCHK(hipStreamSynchronize(s));
+    return TSU_OK;
+}
+
 // The tile height with the least estimated cost of a stage.
 //
 // Alone on the GPU: a tile of r rows costs its wave r + 0.6 rows (the
@@ -214,6 +271,7 @@ struct tsu_state {
     uint8_t* fix = nullptr;
     Ctrl* ctrl = nullptr;
     tsu::DtSlots* dts = nullptr;
+    tsu::Staging staging;
     double* ext = nullptr;
     double* CC = nullptr;
     double* tCC = nullptr;
@@ -310,6 +368,7 @@ void free_state(tsu_state* st)
     (void)hipFree(st->fix);
     (void)hipFree(st->ctrl);
     (void)hipFree(st->dts);
+    tsu::free_staging(&st->staging);
     (void)hipFree(st->ext);
     (void)hipFree(st->CC);
     (void)hipFree(st->tCC);
@@ -519,21 +578,7 @@ TSU_API int tsu_state_upload(tsu_state* st, const double* V, const int* fixH)
     drop_graph(st);
     if (!st->rows_given) set_tiling(st, 0);
     const size_t bytes = planes_of(st) * (size_t)nv * st->esize;
-    if (st->precision == TSU_FP64) {
-        HIPCHK(hipMemcpyAsync(st->A, V, bytes, hipMemcpyHostToDevice, st->stream));
-    } else {
-        // hi planes 0-4, then the lo parts of h, H, hc (planes 5-7)
-        std::vector<float> f((size_t)8 * nv);
-        for (size_t i = 0; i < (size_t)5 * nv; i++) f[i] = (float)V[i];
-        const int src[3] = {0, 3, 4};
-        for (int j = 0; j < 3; j++)
-            for (size_t i = 0; i < (size_t)nv; i++) {
-                const size_t k = (size_t)src[j] * nv + i;
-                f[(size_t)(5 + j) * nv + i] = (float)(V[k] - (double)f[k]);
-            }
-        HIPCHK(hipMemcpyAsync(st->A, f.data(), bytes, hipMemcpyHostToDevice, st->stream));
-        HIPCHK(hipStreamSynchronize(st->stream));
-    }
+    if (int rc = tsu::upload_planes(&st->staging, V, st->A, st->precision, nv, st->stream)) return rc;
     HIPCHK(hipMemcpyAsync(st->B, st->A, bytes, hipMemcpyDeviceToDevice, st->stream));
     HIPCHK(hipMemcpyAsync(st->fix, fx.data(), (size_t)nv, hipMemcpyHostToDevice, st->stream));
     if (st->ext) HIPCHK(tsu::launch_fill(st->ext, 3 * nv, -1e30, st->stream));
@@ -549,21 +594,7 @@ TSU_API int tsu_state_download(tsu_state* st, double* V)
     void* cur;
     int rc = current_buffer(st, &cur);
     if (rc) return rc;
-    const long long nv = st->nvol;
-    const size_t bytes = planes_of(st) * (size_t)nv * st->esize;
-    if (st->precision == TSU_FP64) {
-        HIPCHK(hipMemcpyAsync(V, cur, bytes, hipMemcpyDeviceToHost, st->stream));
-        HIPCHK(hipStreamSynchronize(st->stream));
-    } else {
-        std::vector<float> f((size_t)8 * nv);
-        HIPCHK(hipMemcpyAsync(f.data(), cur, bytes, hipMemcpyDeviceToHost, st->stream));
-        HIPCHK(hipStreamSynchronize(st->stream));
-        for (size_t i = 0; i < (size_t)5 * nv; i++) V[i] = (double)f[i];
-        const int dst[3] = {0, 3, 4};
-        for (int j = 0; j < 3; j++)
-            for (size_t i = 0; i < (size_t)nv; i++) V[(size_t)dst[j] * nv + i] += (double)f[(size_t)(5 + j) * nv + i];
-    }
-    return TSU_OK;
+    return tsu::download_planes(&st->staging, cur, V, st->precision, st->nvol, 0, 5 * st->nvol, st->stream);
 }
 
 TSU_API int tsu_state_set_inflow(tsu_state* st, const double* CC, const double* tCC, unsigned long timeCC)

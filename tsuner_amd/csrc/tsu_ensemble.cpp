@@ -58,6 +58,7 @@ struct tsu_ensemble {
     size_t ext_doubles = 0;
     Ctrl* ctrl = nullptr;
     tsu::DtSlots* dts = nullptr;
+    tsu::Staging staging;
     Ctrl* snapC = nullptr;
     tsu::DtSlots* snapD = nullptr;
     DevParams* dP = nullptr;
@@ -115,6 +116,7 @@ void destroy(tsu_ensemble* e)
     (void)hipFree(e->ext);
     (void)hipFree(e->ctrl);
     (void)hipFree(e->dts);
+    tsu::free_staging(&e->staging);
     (void)hipFree(e->snapC);
     (void)hipFree(e->snapD);
     (void)hipFree(e->dP);
@@ -455,21 +457,7 @@ TSU_API int tsu_ensemble_upload(tsu_ensemble* e, int i, const double* V, const i
     Guard g(e->device);
     drop_graph(e);
     const size_t bytes = e->planes * (size_t)nv * e->esize;
-    if (e->precision == TSU_FP64) {
-        ECHK(hipMemcpyAsync(e->A + e->off[i], V, bytes, hipMemcpyHostToDevice, e->stream));
-        ECHK(hipStreamSynchronize(e->stream));
-    } else {
-        std::vector<float> f((size_t)8 * nv);
-        for (size_t k = 0; k < (size_t)5 * nv; k++) f[k] = (float)V[k];
-        const int src[3] = {0, 3, 4};
-        for (int j = 0; j < 3; j++)
-            for (size_t k = 0; k < (size_t)nv; k++) {
-                const size_t q = (size_t)src[j] * nv + k;
-                f[(size_t)(5 + j) * nv + k] = (float)(V[q] - (double)f[q]);
-            }
-        ECHK(hipMemcpyAsync(e->A + e->off[i], f.data(), bytes, hipMemcpyHostToDevice, e->stream));
-        ECHK(hipStreamSynchronize(e->stream));
-    }
+    if ((rc = tsu::upload_planes(&e->staging, V, e->A + e->off[i], e->precision, nv, e->stream))) return rc;
     ECHK(hipMemcpyAsync(e->B + e->off[i], e->A + e->off[i], bytes, hipMemcpyDeviceToDevice, e->stream));
     ECHK(hipMemcpyAsync(e->fix + e->foff[i], fx.data(), (size_t)nv, hipMemcpyHostToDevice, e->stream));
     if (e->s[i].extrema) ECHK(tsu::launch_fill(e->ext + e->xoff[i], 3 * nv, -1e30, e->stream));
@@ -487,20 +475,19 @@ TSU_API int tsu_ensemble_download(tsu_ensemble* e, int i, double* V)
     char* cur;
     if ((rc = current_buffer(e, i, &cur))) return rc;
     const long long nv = e->P[i].nvol;
-    const size_t bytes = e->planes * (size_t)nv * e->esize;
-    if (e->precision == TSU_FP64) {
-        ECHK(hipMemcpyAsync(V, cur, bytes, hipMemcpyDeviceToHost, e->stream));
-        ECHK(hipStreamSynchronize(e->stream));
-    } else {
-        std::vector<float> f((size_t)8 * nv);
-        ECHK(hipMemcpyAsync(f.data(), cur, bytes, hipMemcpyDeviceToHost, e->stream));
-        ECHK(hipStreamSynchronize(e->stream));
-        for (size_t k = 0; k < (size_t)5 * nv; k++) V[k] = (double)f[k];
-        const int dst[3] = {0, 3, 4};
-        for (int j = 0; j < 3; j++)
-            for (size_t k = 0; k < (size_t)nv; k++) V[(size_t)dst[j] * nv + k] += (double)f[(size_t)(5 + j) * nv + k];
-    }
-    return TSU_OK;
+    return tsu::download_planes(&e->staging, cur, V, e->precision, nv, 0, 5 * nv, e->stream);
+}
+
+TSU_API int tsu_ensemble_download_plane(tsu_ensemble* e, int i, int plane, double* out)
+{
+    int rc = member_ok(e, i);
+    if (rc) return rc;
+    if (!out || plane < 0 || plane > 4) return tsu::set_error(TSU_ERR_ARG, "bad argument");
+    Guard g(e->device);
+    char* cur;
+    if ((rc = current_buffer(e, i, &cur))) return rc;
+    const long long nv = e->P[i].nvol;
+    return tsu::download_planes(&e->staging, cur, out, e->precision, nv, plane * nv, nv, e->stream);
 }
 
 TSU_API int tsu_ensemble_set_inflow(tsu_ensemble* e, int i, const double* CC, const double* tCC, unsigned long timeCC)

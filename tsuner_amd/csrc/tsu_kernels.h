@@ -101,6 +101,13 @@ hipError_t launch_copy(const void* src, void* dst, long long bytes, hipStream_t 
 // After a step of the single-stage scheme (the two-stage scheme's stages
 // advance the control block themselves).
 hipError_t launch_advance(Ctrl* ctrl, DtSlots* dts, const DevParams& P, hipStream_t s);
+// The FP32 solver's state planes (hi 0-4, lo parts of h, H, hc 5-7; nv cells
+// each) from and to the caller's five FP64 planes: values [first, first +
+// count) of the five planes in a row, which are in `wide` (device).
+hipError_t launch_narrow(const double* wide, float* state, long long nv, long long first, long long count,
+                         hipStream_t s);
+hipError_t launch_widen(const float* state, double* wide, long long nv, long long first, long long count,
+                        hipStream_t s);
 hipError_t launch_fill(double* p, long long n, double v, hipStream_t s);
 // Sums of h and of (H + hc) in FP64 into out[0], out[1] (device pointer),
 // using partial (>= 2 * nblocks doubles) as scratch.

@@ -77,6 +77,12 @@ class Ensemble:
         check(lib().tsu_ensemble_download(self._h, int(i), ptr(out)), "tsu_ensemble_download")
         return out
 
+    def plane(self, i: int, f: int) -> np.ndarray:
+        """state(i)[f] alone: 0 h, 1 qx, 2 qy, 3 H, 4 hc."""
+        out = np.empty(self.shapes[i], dtype=np.float64)
+        check(lib().tsu_ensemble_download_plane(self._h, int(i), int(f), ptr(out)), "tsu_ensemble_download_plane")
+        return out
+
     def time(self, i: int):
         t, dt, n = C.c_double(), C.c_double(), C.c_longlong()
         check(lib().tsu_ensemble_get_time(self._h, int(i), C.byref(t), C.byref(dt), C.byref(n)),
