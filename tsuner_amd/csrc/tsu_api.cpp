@@ -141,13 +141,14 @@ int set_error(int code, const std::string& msg) { return fail(code, msg); }
 namespace {
 int reserve(Staging* g, long long count)
 {
-    const long long want = std::min(count, 4LL << 20);
+    long long want = std::min(count, 4LL << 20);
     if (g->cap >= want) return TSU_OK;
     free_staging(g);
-    if (hipMalloc((void**)&g->buf, (size_t)want * sizeof(double)) != hipSuccess) {
+    // a smaller buffer, and more transfers, where memory is short
+    for (; hipMalloc((void**)&g->buf, (size_t)want * sizeof(double)) != hipSuccess; want /= 4) {
         (void)hipGetLastError();
         g->buf = nullptr;
-        return fail(TSU_ERR_DEVICE_MEMORY, "transfer buffer allocation failed");
+        if (want < 1024) return fail(TSU_ERR_DEVICE_MEMORY, "transfer buffer allocation failed");
     }
     g->cap = want;
     return TSU_OK;
