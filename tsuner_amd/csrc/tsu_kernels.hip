@@ -516,9 +516,9 @@ __device__ __forceinline__ void fold_dt(const StageArgs& a, const DevParams& P, 
 // roots.  Here the three are side by side, and one copy of the edge solve
 // serves all waves.  A neighbour's edge is solved once more instead of being
 // handed on.  100 x 100 cells in motion, FP64 with sediment: 13.4 -> 8.1 us a
-// stage.  What is left is the launch, the loads, and one chain each of face
-// reconstruction, edge and update.  The sums are stage_body's, in its order.
-
+// stage (8.9 with running maxima).  What is left is the launch, the loads, and
+// one chain each of face reconstruction, edge and update.  The sums are
+// stage_body's, in its order.
 //
 // The part between the loads and the update: M, A, B, Q are the rows y - 2 ..
 // y + 1 in wave 0 and y - 1 .. y + 2 in the others (Q not in wave 2).  True in

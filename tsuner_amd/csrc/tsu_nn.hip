@@ -111,8 +111,9 @@ __device__ __forceinline__ void lds_barrier()
 //
 // Bound by the bytes of both tensors for the narrow layers and by how well the
 // MFMAs, the epilogue and the loads of one workgroup overlap for 64 -> 64
-// (matrix pipe 51 % busy; without its loads and stores 120 us).  Before (weights and a 10 x 66 pixel tile in LDS, one
-// read per two MFMAs, the tile's loads and stores between barriers) and now, us:
+// (matrix pipe 51 % busy; without its loads and stores 120 us).  Before
+// (weights and a 10 x 66 pixel tile in LDS, one read per two MFMAs, the tile's
+// loads and stores between barriers) and now, us:
 //            8->32  32->32  32->4  8->64  64->64  64->4, and the data
 //   32 images  41     89     48    106     200     95    gradients 4<-32 60,
 //   of 256^2   27     49     40     71     150     68    32<-32 103, 4<-64 181,
@@ -318,8 +319,8 @@ __attribute__((amdgpu_waves_per_eu(conv_waves<K>(), conv_waves<K>()))) void conv
             if constexpr (POST == 2 && K != 8) {
 #pragma unroll
                 for (int r = 0; r < RW; r++)
-                    mask[r] = *(const uint4*)(act + (((size_t)pass_n * H + min(cr0 + r, H - 1)) * W + min(c, W - 1)) * MOUT +
-                                              m0);
+                    mask[r] = *(const uint4*)(act + m0 +
+                                              (((size_t)pass_n * H + min(cr0 + r, H - 1)) * W + min(c, W - 1)) * MOUT);
             }
             // EARLY: the coming rows go into the ring ahead of the results'
             // stores, in every pass.  A wait for these loads behind stores
