@@ -8,6 +8,10 @@
  * V[f*nvol + j*npx + i] with f = 0 h, 1 qx, 2 qy, 3 H (depth below datum,
  * bed z = -H), 4 hc (reference layout, GPU/main_TSUNER.cu:104-111).
  *
+ * Threads: calls on different handles are independent.  Calls on one handle
+ * take their turns, except tsu_synchronize and tsu_ensemble_synchronize, which
+ * keep no other call waiting; a handle is destroyed after its last call.
+ *
  * Reference interfaces replaced (paths relative to the TSUNER source tree):
  *   TSUNER()            TSUNER.h:39, GPU/main_TSUNER.cu:21-222
  *   checkCUDAsupport()  TSUNER.h:41, GPU/CheckCUDASupport.cu:49-73

@@ -258,6 +258,7 @@ int choose_tile_rows(const std::vector<std::pair<int, int>>& grids, bool sed, in
 }  // namespace tsu
 
 struct tsu_state {
+    std::recursive_mutex calls;
     int device = 0;
     int precision = TSU_FP64;
     bool sed = true;
@@ -574,8 +575,8 @@ TSU_API int tsu_state_upload(tsu_state* st, const double* V, const int* fixH)
     }
     bool hc_zero = true;
     for (long long i = 0; i < nv && hc_zero; i++) hc_zero = V[4 * nv + i] == 0.0;
+    tsu::HandleGuard g(st->calls, st->device);
     st->sed = st->s.bedload || st->s.suspension || !hc_zero;
-    DeviceGuard g(st->device);
     drop_graph(st);
     if (!st->rows_given) set_tiling(st, 0);
     const size_t bytes = planes_of(st) * (size_t)nv * st->esize;
@@ -591,7 +592,7 @@ TSU_API int tsu_state_upload(tsu_state* st, const double* V, const int* fixH)
 TSU_API int tsu_state_download(tsu_state* st, double* V)
 {
     if (!st || !V) return fail(TSU_ERR_ARG, "null argument");
-    DeviceGuard g(st->device);
+    tsu::HandleGuard g(st->calls, st->device);
     void* cur;
     int rc = current_buffer(st, &cur);
     if (rc) return rc;
@@ -608,7 +609,7 @@ TSU_API int tsu_state_set_inflow(tsu_state* st, const double* CC, const double* 
     for (unsigned long k = 0; k < timeCC; k++)
         if (!std::isfinite(tCC[k]) || (k > 0 && !(tCC[k] > tCC[k - 1])))
             return fail(TSU_ERR_ARG, "inflow times must be finite and strictly increasing");
-    DeviceGuard g(st->device);
+    tsu::HandleGuard g(st->calls, st->device);
     // steps already enqueued may still read the old series and run constants
     HIPCHK(hipStreamSynchronize(st->stream));
     drop_graph(st);
@@ -646,7 +647,7 @@ TSU_API int tsu_init_dt(tsu_state* st)
 {
     int rc = check_ready(st);
     if (rc) return rc;
-    DeviceGuard g(st->device);
+    tsu::HandleGuard g(st->calls, st->device);
     Ctrl c;
     rc = read_ctrl(st, &c);
     if (rc) return rc;
@@ -664,7 +665,7 @@ TSU_API int tsu_step(tsu_state* st, int nsteps)
     int rc = check_ready(st);
     if (rc) return rc;
     if (nsteps < 0) return fail(TSU_ERR_ARG, "negative step count");
-    DeviceGuard g(st->device);
+    tsu::HandleGuard g(st->calls, st->device);
     int done = 0;
     if (st->graph_chunk > 0 && nsteps >= st->graph_chunk) {
         if (!st->gexec) {
@@ -699,7 +700,7 @@ TSU_API int tsu_step(tsu_state* st, int nsteps)
 TSU_API int tsu_synchronize(tsu_state* st)
 {
     if (!st) return fail(TSU_ERR_ARG, "null state");
-    DeviceGuard g(st->device);
+    DeviceGuard g(st->device);   // no call is kept waiting
     HIPCHK(hipStreamSynchronize(st->stream));
     return TSU_OK;
 }
@@ -707,7 +708,7 @@ TSU_API int tsu_synchronize(tsu_state* st)
 TSU_API int tsu_get_time(tsu_state* st, double* t, double* dt, long long* steps)
 {
     if (!st) return fail(TSU_ERR_ARG, "null state");
-    DeviceGuard g(st->device);
+    tsu::HandleGuard g(st->calls, st->device);
     Ctrl c;
     tsu::DtSlots d;
     HIPCHK(hipMemcpyAsync(&d, st->dts, sizeof(d), hipMemcpyDeviceToHost, st->stream));
@@ -722,7 +723,7 @@ TSU_API int tsu_get_time(tsu_state* st, double* t, double* dt, long long* steps)
 TSU_API int tsu_set_time(tsu_state* st, double t, double dt)
 {
     if (!st) return fail(TSU_ERR_ARG, "null state");
-    DeviceGuard g(st->device);
+    tsu::HandleGuard g(st->calls, st->device);
     Ctrl c;
     int rc = read_ctrl(st, &c);
     if (rc) return rc;
@@ -741,7 +742,7 @@ TSU_API int tsu_set_time(tsu_state* st, double t, double dt)
 TSU_API int tsu_set_stop_time(tsu_state* st, double stop_time)
 {
     if (!st) return fail(TSU_ERR_ARG, "null state");
-    DeviceGuard g(st->device);
+    tsu::HandleGuard g(st->calls, st->device);
     static_assert(offsetof(Ctrl, stop_time) == 8, "ctrl layout");
     HIPCHK(hipMemcpyAsync((char*)st->ctrl + offsetof(Ctrl, stop_time), &stop_time, sizeof(double),
                           hipMemcpyHostToDevice, st->stream));
@@ -752,7 +753,7 @@ TSU_API int tsu_set_stop_time(tsu_state* st, double stop_time)
 TSU_API int tsu_set_clamp(tsu_state* st, int on)
 {
     if (!st) return fail(TSU_ERR_ARG, "null state");
-    DeviceGuard g(st->device);
+    tsu::HandleGuard g(st->calls, st->device);
     const long long v = on ? 1 : 0;
     HIPCHK(hipMemcpyAsync((char*)st->ctrl + offsetof(Ctrl, clamp), &v, sizeof(long long), hipMemcpyHostToDevice,
                           st->stream));
@@ -763,7 +764,7 @@ TSU_API int tsu_set_clamp(tsu_state* st, int on)
 TSU_API int tsu_mass(tsu_state* st, double out[2])
 {
     if (!st || !out) return fail(TSU_ERR_ARG, "null argument");
-    DeviceGuard g(st->device);
+    tsu::HandleGuard g(st->calls, st->device);
     void* cur;
     int rc = current_buffer(st, &cur);
     if (rc) return rc;
@@ -778,7 +779,7 @@ TSU_API int tsu_get_extrema(tsu_state* st, double* hmax, double* bmax, double* e
 {
     if (!st) return fail(TSU_ERR_ARG, "null state");
     if (!st->ext) return fail(TSU_ERR_ARG, "extrema are not enabled in the scheme");
-    DeviceGuard g(st->device);
+    tsu::HandleGuard g(st->calls, st->device);
     const size_t b = (size_t)st->nvol * sizeof(double);
     if (hmax) HIPCHK(hipMemcpyAsync(hmax, st->ext, b, hipMemcpyDeviceToHost, st->stream));
     if (bmax) HIPCHK(hipMemcpyAsync(bmax, st->ext + st->nvol, b, hipMemcpyDeviceToHost, st->stream));
@@ -791,6 +792,7 @@ TSU_API int tsu_set_tile_rows(tsu_state* st, int rows)
 {
     if (!st) return fail(TSU_ERR_ARG, "null state");
     if (rows < 0 || rows > 4096) return fail(TSU_ERR_ARG, "tile rows out of range");
+    tsu::HandleGuard g(st->calls, st->device);
     drop_graph(st);
     st->rows_given = rows != 0;
     set_tiling(st, rows);
@@ -804,6 +806,7 @@ TSU_API int tsu_set_graph_chunk(tsu_state* st, int chunk)
     if (!st) return fail(TSU_ERR_ARG, "null state");
     if (chunk < 0) return fail(TSU_ERR_ARG, "negative graph chunk");
     if (st->s.order == 1 && (chunk & 1)) return fail(TSU_ERR_ARG, "single-stage graphs need an even chunk");
+    tsu::HandleGuard g(st->calls, st->device);
     drop_graph(st);
     st->graph_chunk = chunk;
     return TSU_OK;
@@ -812,6 +815,7 @@ TSU_API int tsu_set_graph_chunk(tsu_state* st, int chunk)
 TSU_API int tsu_set_timing(tsu_state* st, int on)
 {
     if (!st) return fail(TSU_ERR_ARG, "null state");
+    tsu::HandleGuard g(st->calls, st->device);
     st->timing = on != 0;
     return TSU_OK;
 }
@@ -819,7 +823,7 @@ TSU_API int tsu_set_timing(tsu_state* st, int on)
 TSU_API int tsu_get_timing(tsu_state* st, double stage_ms[2], long long launches[2], int reset)
 {
     if (!st) return fail(TSU_ERR_ARG, "null state");
-    DeviceGuard g(st->device);
+    tsu::HandleGuard g(st->calls, st->device);
     HIPCHK(hipStreamSynchronize(st->stream));
     for (size_t i = 0; i < st->ev_used; i++) {
         float ms = 0.0f;

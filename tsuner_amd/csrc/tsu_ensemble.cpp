@@ -38,6 +38,7 @@ size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 }  // namespace
 
 struct tsu_ensemble {
+    std::recursive_mutex calls;
     int device = 0, precision = TSU_FP64, n = 0;
     bool sed = false;
     std::vector<tsu_sim_params> p;
@@ -454,7 +455,7 @@ TSU_API int tsu_ensemble_upload(tsu_ensemble* e, int i, const double* V, const i
     bool hc_zero = true;
     for (long long k = 0; k < nv && hc_zero; k++) hc_zero = V[4 * nv + k] == 0.0;
     if (!hc_zero && !e->sed) return tsu::set_error(TSU_ERR_UNSUPPORTED, "nonzero hc needs a sediment scheme");
-    Guard g(e->device);
+    tsu::HandleGuard g(e->calls, e->device);
     drop_graph(e);
     const size_t bytes = e->planes * (size_t)nv * e->esize;
     if ((rc = tsu::upload_planes(&e->staging, V, e->A + e->off[i], e->precision, nv, e->stream))) return rc;
@@ -471,7 +472,7 @@ TSU_API int tsu_ensemble_download(tsu_ensemble* e, int i, double* V)
     int rc = member_ok(e, i);
     if (rc) return rc;
     if (!V) return tsu::set_error(TSU_ERR_ARG, "null argument");
-    Guard g(e->device);
+    tsu::HandleGuard g(e->calls, e->device);
     char* cur;
     if ((rc = current_buffer(e, i, &cur))) return rc;
     const long long nv = e->P[i].nvol;
@@ -483,7 +484,7 @@ TSU_API int tsu_ensemble_download_plane(tsu_ensemble* e, int i, int plane, doubl
     int rc = member_ok(e, i);
     if (rc) return rc;
     if (!out || plane < 0 || plane > 4) return tsu::set_error(TSU_ERR_ARG, "bad argument");
-    Guard g(e->device);
+    tsu::HandleGuard g(e->calls, e->device);
     char* cur;
     if ((rc = current_buffer(e, i, &cur))) return rc;
     const long long nv = e->P[i].nvol;
@@ -499,7 +500,7 @@ TSU_API int tsu_ensemble_set_inflow(tsu_ensemble* e, int i, const double* CC, co
     for (unsigned long k = 0; k < timeCC; k++)
         if (!std::isfinite(tCC[k]) || (k > 0 && !(tCC[k] > tCC[k - 1])))
             return tsu::set_error(TSU_ERR_ARG, "inflow times must be finite and strictly increasing");
-    Guard g(e->device);
+    tsu::HandleGuard g(e->calls, e->device);
     // steps already enqueued may still read the member's old series
     ECHK(hipStreamSynchronize(e->stream));
     drop_graph(e);
@@ -530,7 +531,7 @@ TSU_API int tsu_ensemble_set_inflow(tsu_ensemble* e, int i, const double* CC, co
 TSU_API int tsu_ensemble_init_dt(tsu_ensemble* e)
 {
     if (!e) return tsu::set_error(TSU_ERR_ARG, "null ensemble");
-    Guard g(e->device);
+    tsu::HandleGuard g(e->calls, e->device);
     if (int rc = members_ready(e)) return rc;
     tsu::DtSlots d;
     tsu::reset_dt_slots(&d);
@@ -549,7 +550,7 @@ TSU_API int tsu_ensemble_init_dt(tsu_ensemble* e)
 TSU_API int tsu_ensemble_set_stop_step(tsu_ensemble* e, long long stop_step)
 {
     if (!e) return tsu::set_error(TSU_ERR_ARG, "null ensemble");
-    Guard g(e->device);
+    tsu::HandleGuard g(e->calls, e->device);
     for (int i = 0; i < e->n; i++)
         ECHK(hipMemcpyAsync((char*)(e->ctrl + i) + offsetof(Ctrl, stop_step), &stop_step, sizeof(long long),
                             hipMemcpyHostToDevice, e->stream));
@@ -562,14 +563,14 @@ TSU_API int tsu_ensemble_step(tsu_ensemble* e, int nsteps)
     if (!e) return tsu::set_error(TSU_ERR_ARG, "null ensemble");
     if (nsteps < 0) return tsu::set_error(TSU_ERR_ARG, "negative step count");
     if (int rc = members_ready(e)) return rc;
-    Guard g(e->device);
+    tsu::HandleGuard g(e->calls, e->device);
     return enqueue_steps(e, nsteps, true);
 }
 
 TSU_API int tsu_ensemble_synchronize(tsu_ensemble* e)
 {
     if (!e) return tsu::set_error(TSU_ERR_ARG, "null ensemble");
-    Guard g(e->device);
+    Guard g(e->device);   // no call is kept waiting
     ECHK(hipStreamSynchronize(e->stream));
     return TSU_OK;
 }
@@ -578,7 +579,7 @@ TSU_API int tsu_ensemble_get_time(tsu_ensemble* e, int i, double* t, double* dt,
 {
     int rc = member_ok(e, i);
     if (rc) return rc;
-    Guard g(e->device);
+    tsu::HandleGuard g(e->calls, e->device);
     Ctrl c;
     tsu::DtSlots d;
     ECHK(hipMemcpyAsync(&c, e->ctrl + i, sizeof(Ctrl), hipMemcpyDeviceToHost, e->stream));
@@ -601,7 +602,7 @@ TSU_API int tsu_ensemble_mass(tsu_ensemble* e, int i, double out[2])
     int rc = member_ok(e, i);
     if (rc) return rc;
     if (!out) return tsu::set_error(TSU_ERR_ARG, "null argument");
-    Guard g(e->device);
+    tsu::HandleGuard g(e->calls, e->device);
     char* cur;
     if ((rc = current_buffer(e, i, &cur))) return rc;
     double* res = e->mass_buf + 2 * e->mass_nb;
@@ -616,8 +617,8 @@ TSU_API int tsu_ensemble_set_tile_rows(tsu_ensemble* e, const int* rows)
     if (!e || !rows) return tsu::set_error(TSU_ERR_ARG, "null argument");
     for (int i = 0; i < e->n; i++)
         if (rows[i] < 1 || rows[i] > 4096) return tsu::set_error(TSU_ERR_ARG, "tile rows out of range");
+    tsu::HandleGuard g(e->calls, e->device);
     e->rows.assign(rows, rows + e->n);
-    Guard g(e->device);
     return build_launch_tables(e);
 }
 
@@ -625,7 +626,7 @@ TSU_API int tsu_ensemble_set_graph_chunk(tsu_ensemble* e, int chunk)
 {
     if (!e || chunk < 0) return tsu::set_error(TSU_ERR_ARG, "bad argument");
     if (e->s[0].order == 1 && (chunk & 1)) return tsu::set_error(TSU_ERR_ARG, "single-stage graphs need an even chunk");
-    Guard g(e->device);
+    tsu::HandleGuard g(e->calls, e->device);
     drop_graph(e);
     e->graph_chunk = chunk;
     return TSU_OK;
@@ -635,7 +636,7 @@ TSU_API int tsu_ensemble_snapshot(tsu_ensemble* e, int restore)
 {
     if (!e) return tsu::set_error(TSU_ERR_ARG, "null ensemble");
     if (e->s[0].order != 2) return tsu::set_error(TSU_ERR_UNSUPPORTED, "snapshots need the two-stage scheme");
-    Guard g(e->device);
+    tsu::HandleGuard g(e->calls, e->device);
     if (!e->snapA) {
         if (restore) return tsu::set_error(TSU_ERR_ARG, "no snapshot taken");
         ECHK(hipMalloc((void**)&e->snapA, e->pool_bytes));
@@ -659,7 +660,7 @@ TSU_API int tsu_ensemble_snapshot(tsu_ensemble* e, int restore)
 TSU_API int tsu_ensemble_time_steps(tsu_ensemble* e, int nsteps, double* ms)
 {
     if (!e || !ms || nsteps < 1) return tsu::set_error(TSU_ERR_ARG, "bad argument");
-    Guard g(e->device);
+    tsu::HandleGuard g(e->calls, e->device);
     hipEvent_t a = nullptr, b = nullptr;
     ECHK(hipEventCreate(&a));
     ECHK(hipEventCreate(&b));
@@ -681,7 +682,7 @@ TSU_API int tsu_ensemble_time_steps(tsu_ensemble* e, int nsteps, double* ms)
 TSU_API int tsu_ensemble_set_stop_time(tsu_ensemble* e, const double* stop_time, int clamp)
 {
     if (!e || !stop_time) return tsu::set_error(TSU_ERR_ARG, "null argument");
-    Guard g(e->device);
+    tsu::HandleGuard g(e->calls, e->device);
     const long long cl = clamp ? 1 : 0;
     for (int i = 0; i < e->n; i++) {
         ECHK(hipMemcpyAsync((char*)(e->ctrl + i) + offsetof(Ctrl, stop_time), stop_time + i, sizeof(double),
@@ -698,7 +699,7 @@ TSU_API int tsu_ensemble_get_extrema(tsu_ensemble* e, int i, double* hmax, doubl
     int rc = member_ok(e, i);
     if (rc) return rc;
     if (!e->s[i].extrema) return tsu::set_error(TSU_ERR_ARG, "extrema are not enabled for this member");
-    Guard g(e->device);
+    tsu::HandleGuard g(e->calls, e->device);
     const size_t nv = (size_t)e->P[i].nvol, b = nv * sizeof(double);
     const double* x = e->ext + e->xoff[i];
     if (hmax) ECHK(hipMemcpyAsync(hmax, x, b, hipMemcpyDeviceToHost, e->stream));
@@ -713,7 +714,7 @@ TSU_API void* tsu_ensemble_stream(tsu_ensemble* e) { return e ? (void*)e->stream
 TSU_API int tsu_ensemble_get_times(tsu_ensemble* e, double* t, long long* steps)
 {
     if (!e || (!t && !steps)) return tsu::set_error(TSU_ERR_ARG, "bad argument");
-    Guard g(e->device);
+    tsu::HandleGuard g(e->calls, e->device);
     std::vector<Ctrl> c((size_t)e->n);
     ECHK(hipMemcpyAsync(c.data(), e->ctrl, e->n * sizeof(Ctrl), hipMemcpyDeviceToHost, e->stream));
     ECHK(hipStreamSynchronize(e->stream));
@@ -775,7 +776,7 @@ TSU_API int tsu_ensemble_nn_features(tsu_ensemble* e, const float scale_in[8], f
     int rc = nn_uniform(e, "tsu_ensemble_nn_features");
     if (rc) return rc;
     if (!scale_in || !x) return tsu::set_error(TSU_ERR_ARG, "null argument");
-    Guard g(e->device);
+    tsu::HandleGuard g(e->calls, e->device);
     ECHK(tsu::nn_launch_features(e->dargs + e->n, e->n, e->p[0].npx, e->p[0].npy, e->precision,
                                  make_scales(scale_in, nullptr, wet_h), (uint16_t*)x, e->stream));
     return TSU_OK;
@@ -787,7 +788,7 @@ TSU_API int tsu_ensemble_nn_apply(tsu_ensemble* e, const float scale_out[4], flo
     int rc = nn_uniform(e, "tsu_ensemble_nn_apply");
     if (rc) return rc;
     if (!scale_out || !out) return tsu::set_error(TSU_ERR_ARG, "null argument");
-    Guard g(e->device);
+    tsu::HandleGuard g(e->calls, e->device);
     tsu::NnScales sc = make_scales(nullptr, scale_out, wet_h);
     sc.shore_h = shore_h;
     ECHK(tsu::nn_launch_apply(e->dargs + e->n, e->n, e->p[0].npx, e->p[0].npy, e->precision, sc, out, expect_step,
@@ -799,7 +800,7 @@ TSU_API int tsu_ensemble_restrict(tsu_ensemble* fine, tsu_ensemble* coarse)
 {
     int rc = nn_pair(fine, coarse, "tsu_ensemble_restrict");
     if (rc) return rc;
-    Guard g(coarse->device);
+    tsu::HandleGuard gf(fine->calls, fine->device), g(coarse->calls, coarse->device);
     ECHK(hipStreamSynchronize(fine->stream));
     ECHK(tsu::nn_launch_restrict(fine->dargs + fine->n, coarse->dargs + coarse->n, coarse->n, coarse->p[0].npx,
                                  coarse->p[0].npy, coarse->precision, coarse->stream));
@@ -817,7 +818,7 @@ TSU_API int tsu_ensemble_nn_target(tsu_ensemble* fine, tsu_ensemble* coarse, con
     int rc = nn_pair(fine, coarse, "tsu_ensemble_nn_target");
     if (rc) return rc;
     if (!scale_out || !target) return tsu::set_error(TSU_ERR_ARG, "null argument");
-    Guard g(coarse->device);
+    tsu::HandleGuard gf(fine->calls, fine->device), g(coarse->calls, coarse->device);
     ECHK(hipStreamSynchronize(fine->stream));
     ECHK(tsu::nn_launch_target(fine->dargs + fine->n, coarse->dargs + coarse->n, coarse->n, coarse->p[0].npx,
                                coarse->p[0].npy, coarse->precision, make_scales(nullptr, scale_out, 0.f), target,

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <mutex>
 #include <string>
 #include <utility>
 #include <vector>
@@ -18,6 +19,27 @@ void make_dev_params(const tsu_sim_params* p, const tsu_scheme* s, DevParams* P)
 int validate_scheme(const tsu_scheme* s);
 // Records msg as the calling thread's last error and returns code.
 int set_error(int code, const std::string& msg);
+// Held by every call on a handle but the waits for its stream: a call's
+// launches and copies follow one another on the handle's streams with nothing
+// of another thread's call between them.  A transfer reuses one buffer piece by
+// piece, and the halves of an ensemble step beside its stream until they are
+// joined.  Calls nest (recursive).
+class HandleGuard {
+public:
+    HandleGuard(std::recursive_mutex& m, int device) : lock_(m)
+    {
+        if (hipGetDevice(&prev_) != hipSuccess) prev_ = -1;
+        (void)hipSetDevice(device);
+    }
+    ~HandleGuard()
+    {
+        if (prev_ >= 0) (void)hipSetDevice(prev_);
+    }
+
+private:
+    std::lock_guard<std::recursive_mutex> lock_;
+    int prev_ = -1;
+};
 // FP64 values on their way to or from a handle's FP32 planes (device memory,
 // at most 32 MB, allocated by the first transfer and kept with the handle).
 struct Staging {
