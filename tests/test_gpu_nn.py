@@ -264,6 +264,25 @@ def test_wide_conv_workgroups_loop_over_tiles():
     assert_bf16_close(host(out).reshape(n, h, w, 64), O.bf16(ref.astype(np.float32)))
 
 
+@pytest.mark.parametrize("width", [32, 64])
+def test_output_layer_takes_four_biases(width):
+    """The output layer's bias is four values (its weights are 16 rows); what
+    lies behind them in memory is not the layer's and changes nothing.
+    Tolerance as for the single kinds (FP32 output 1e-5)."""
+    rng = np.random.default_rng(21)
+    n, h, w = 2, 6, 70
+    x = rand_bf16(rng, (n, h, w, width))
+    wt = rand_bf16(rng, (9, 16, width), 0.2)
+    wt[:, 4:] = 0
+    b = rng.normal(0, 0.1, size=4).astype(np.float32)
+    room = dev_f32(np.concatenate([b, np.full(12, np.nan, np.float32)]))
+    out = torch.zeros(n * h * w * 4, dtype=torch.float32, device="cuda")
+    ok(lib().tsu_nn_conv(2 | (W64 if width == 64 else 0), P(dev_bf16(x)), P(dev_bf16(wt)), P(room[:4]), None, P(out), n,
+                         h, w, C.c_void_p(0)))
+    ref = O.conv(x, wt[:, :4], b)
+    np.testing.assert_allclose(host(out).reshape(ref.shape), ref, rtol=0, atol=1e-5 * np.abs(ref).max())
+
+
 def test_mse_and_adam_kernels():
     rng = np.random.default_rng(4)
     npix = 1000

@@ -191,11 +191,14 @@ __attribute__((amdgpu_waves_per_eu(conv_waves<K>(), conv_waves<K>()))) void conv
             A[s][a] = as_bf16x8(v);
         }
     const int m0 = 16 * MTW * mg + 4 * MTW * g;             // this lane's 4 MTW consecutive output channels
+    // of which MOUT = 4 has those of the first lane group only: the caller's
+    // bias ends there
+    static_assert(MOUT % (4 * MTW) == 0, "a lane's channels are all stored or none");
     f32x4 bias_of[MTW];
 #pragma unroll
     for (int a = 0; a < MTW; a++)
 #pragma unroll
-        for (int e = 0; e < 4; e++) bias_of[a][e] = POST == 2 ? 0.f : bias[m0 + 4 * a + e];
+        for (int e = 0; e < 4; e++) bias_of[a][e] = POST == 2 || m0 >= MOUT ? 0.f : bias[m0 + 4 * a + e];
 
     // staging: this thread's octet and column (and row, if a sweep takes
     // several), and one of the last two columns' for the first threads
