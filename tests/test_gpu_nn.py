@@ -215,6 +215,44 @@ def test_weight_gradient_strips_and_stretches(shape, width):
         np.testing.assert_allclose(host(db), rdb, rtol=0, atol=1e-5 * np.abs(rdb).max())
 
 
+@pytest.mark.parametrize("width", [32, 64])
+@pytest.mark.parametrize("shape", [(1, 1, 1), (2, 5, 9), (1, 9, 65), (1, 8, 64), (2, 11, 130)])
+def test_weight_gradients_of_values_that_are_not_finite(shape, width):
+    """dW[t] = sum_p dy[p] x[p + t] with zeros for x around the image and p
+    over the image alone, for an infinity or a NaN of x, of dy and of both on
+    the image's border and inside: the same entries are infinite, of the same
+    sign, and NaN as in the oracle's sum, and the others are right (tolerance
+    as above)."""
+    rng = np.random.default_rng(22)
+    n, h, w = shape
+    s = C.c_void_p(0)
+    f, W = (W64 if width == 64 else 0), width
+    spots = sorted({(r, c) for r in (0, h // 2, h - 1) for c in (0, w // 2, w - 1)})
+    for kind, kx, my in [(5 | f, 8, W), (6 | f, W, W), (7 | f, W, 8)]:
+        nws = lib().tsu_nn_wgrad_workspace(kind)
+        ws = torch.empty(nws, dtype=torch.float32, device="cuda")
+        for at in spots:
+            for which in (1, 2, 3):
+                x = rand_bf16(rng, (n, h, w, kx))
+                dy = rand_bf16(rng, (n, h, w, my))
+                if which & 1:
+                    x[n - 1, at[0], at[1], 3] = [np.inf, -np.inf, np.nan][rng.integers(3)]
+                if which & 2:
+                    r, c = (at if rng.integers(2) else spots[rng.integers(len(spots))])
+                    dy[n - 1, r, c, 1] = [np.inf, -np.inf, np.nan][rng.integers(3)]
+                dw = torch.zeros(9 * my * kx, dtype=torch.float32, device="cuda")
+                db = torch.zeros(my, dtype=torch.float32, device="cuda")
+                ok(lib().tsu_nn_wgrad(kind, P(dev_bf16(x)), P(dev_bf16(dy)), P(dw), P(db), my, n, h, w, P(ws), nws, s))
+                with np.errstate(invalid="ignore"):
+                    rdw, rdb = O.conv_weight_grad(x, dy)
+                for got, ref in ((host(dw).reshape(9, my, kx), rdw), (host(db), rdb)):
+                    fin = np.isfinite(ref)
+                    np.testing.assert_array_equal(got[~fin], ref[~fin].astype(np.float32))
+                    if fin.any():
+                        np.testing.assert_allclose(got[fin], ref[fin], rtol=0, atol=1e-5 * np.abs(ref[fin]).max())
+        _KEEP.clear()
+
+
 def test_weight_gradients_take_operands_of_any_alignment():
     """x and dy one element past a 16-byte boundary: the same sums, bit for
     bit, as from aligned copies."""

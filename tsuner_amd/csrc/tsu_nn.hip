@@ -412,6 +412,12 @@ __attribute__((amdgpu_waves_per_eu(conv_waves<K>(), conv_waves<K>()))) void conv
 // are XOR-ed with bits of its column: the 8 consecutive columns that half a
 // wave reads then lie in different banks.  The eight pixels of lane group g
 // in a 32-pixel step are 4g .. 4g+3 and 16+4g .. 16+4g+3, for both operands.
+//
+// The sum takes the pixels p of the image and zeros for x around it, also for
+// values that are not finite (0 times an infinity is a NaN): a step's pixels
+// past the image must meet zeros in both operands.  RAGGED: the image's width
+// is no multiple of the strips' 64 columns (64 -> 64, 8 images of 250^2, 50.2
+// -> 51.3 us with it, which widths without a remainder are spared).
 
 constexpr int kWgradPitch = 72;            // LDS columns of the shifted operand's rows (66 used)
 
@@ -452,7 +458,7 @@ __device__ __forceinline__ int slot_xor(int c)
 // go to part[t][workgroup][m][k], the bias gradient (one MFMA per dy tile
 // against ones, in the jobs of the first 32 input channels) to
 // bpart[workgroup][m].
-template <int CH>
+template <int CH, bool RAGGED>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void wgrad_mid_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ dy, float* __restrict__ part,
     float* __restrict__ bpart, int N, int H, int W)
@@ -554,6 +560,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     put(xs, ds);
     __syncthreads();
     for (;;) {
+        const int rows = H - walk.r0, cols = W - walk.c0;   // of the image, from this pass on
         const bool more = --walk.left > 0;                  // uniform over the workgroup
         bool down = false;                                  // the next pass continues this strip
         if (more) {
@@ -563,7 +570,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll 1
         for (int s = 0; s < STEPS; s++) {
             const int st = group * STEPS + s;               // step of the pass: row st / 2, half row st % 2
+            if ((st >> 1) >= rows) break;                   // past the image (see above)
             const uint32_t half = (uint32_t)(st & 1) * 32 * PIX;
+            // the left neighbours of the first column past the image: from the
+            // column itself, which holds zeros
+            const int past = cols - (st & 1) * 32;
+            uint32_t left[2][2];
+#pragma unroll
+            for (int b = 0; b < 2; b++) {
+                left[b][0] = RAGGED && px == past ? xa[1][b] : xa[0][b];
+                left[b][1] = RAGGED && px + 16 == past ? xa[1][b] : xa[0][b];
+            }
             const uint32_t dof = (uint32_t)((ds + (st >> 1)) * DROW) + half;
             bf16x8 A[2];
 #pragma unroll
@@ -580,8 +597,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             // (64 -> 64 60.5 us with its reduction, one ahead 56.7, two 57.3,
             // three, which spill, 59.2)
             auto read = [&](int i) {
-                const uint32_t at = xa[i / 2 % 3][i % 2] + xo[i / 6];
-                return read_tr8(at, at + 16 * PIX);
+                const int d = i / 2 % 3, b = i % 2;
+                const uint32_t at = (d == 0 ? left[b][0] : xa[d][b]) + xo[i / 6];
+                return read_tr8(at, (d == 0 ? left[b][1] + xo[i / 6] : at) + 16 * PIX);
             };
             bf16x8 B[AHEAD + 1];
 #pragma unroll
@@ -652,6 +670,37 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
 }
 
+__device__ __forceinline__ bool wave_any(bool b) { return __builtin_expect(__builtin_amdgcn_ballot_w64(b) != 0, 0); }
+
+__device__ __forceinline__ bool not_finite16(uint32_t bits) { return (bits & 0x7F80u) == 0x7F80u; }
+
+// any of eight values an infinity or a NaN: the largest magnitude bits
+__device__ __forceinline__ bool not_finite(bf16x8 v)
+{
+    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+    const uint4 u = __builtin_bit_cast(uint4, v);
+    const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+    u16x2 most = {0, 0};
+#pragma unroll
+    for (int i = 0; i < 4; i++) most = __builtin_elementwise_max(most, __builtin_bit_cast(u16x2, w[i] & 0x7FFF7FFFu));
+    return (most.x >= 0x7F80) | (most.y >= 0x7F80);
+}
+
+// A lane's eight pixels of the 32 from column c0 on (4g .. 4g + 3 and 16 + 4g
+// ..), with a one of its sign for each value that is not finite and lies on the
+// image's border (row: the whole row does).
+__device__ __forceinline__ bf16x8 border_ones(bf16x8 v, bool row, int g, int c0, int W)
+{
+    typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
+    u16x8 u = __builtin_bit_cast(u16x8, v);
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const int c = c0 + 4 * g + (i & 3) + 4 * (i & 4);
+        if ((row || c == 0 || c == W - 1) && not_finite16(u[i])) u[i] = (u[i] & 0x8000) | 0x3F80;
+    }
+    return __builtin_bit_cast(bf16x8, u);
+}
+
 // Input and output layers: a wide operand p (CH channels) against a narrow
 // one q (8 channels) at nine shifts, G[s][a][b] = sum_p wide[p][a]
 // narrow[p + off(s)][b].  The input layer is wide = dy, narrow = x, s = t;
@@ -661,7 +710,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // gradient, sum_p dy).  Every wave holds all shifts and channels; a pass is
 // 8 rows, one per wave, and the waves' sums are added through LDS at the
 // end.  Bound by the wide operand's bytes.
-template <int CH, bool OUTL>
+//
+// The output layer's pixels of x at the image's border meet dy's zeros outside
+// in products that are none of the sum's, and dy's border pixels x's zeros in
+// products of the sum that it does not form.  Both are 0 unless a value there is
+// not finite.  Then (a vote per half row and row of the border) such values of x
+// are ones to the MFMAs, which keeps the products with infinities of dy, and
+// the products that the sum has are added one by one, for such values of dy
+// with x's zeros too: NaNs.  The votes cost 64 -> 4 0.8 us of 20.5 with its
+// reduction (8 images of 256^2).
+template <int CH, bool OUTL, bool RAGGED>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void wgrad_edge_kernel(
     const uint16_t* __restrict__ wide, const uint16_t* __restrict__ narrow, float* __restrict__ part,
     float* __restrict__ bpart, int N, int H, int W)
@@ -755,6 +813,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     put(xs, ds);
     __syncthreads();
     for (;;) {
+        const int r = walk.r0 + wv, c0 = walk.c0;           // the wave's row, the strip's first column
         const bool more = --walk.left > 0;
         bool down = false;
         if (more) {
@@ -769,23 +828,86 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             xo[j] = xbase + row * XROW + xc[j];
         }
         const uint32_t dof = (uint32_t)((ds + wv) * DROW);
+        // output layer, a row or strip at the image's border: a value of x or
+        // dy that is not finite
+        int own = xs + wv + 1;
+        own = own >= XR ? own - XR : own;
+        const uint4* mine = lds + own * kWgradPitch + 1;    // dy's pixels beside the wave's
+        const bool at_border = r < H && (r == 0 || r == H - 1 || c0 == 0 || W - c0 <= kStripCols);
+        bool bad = false;
+        if (r < H) {                                        // (a row past the image has nothing to add)
+            bf16x8 A[2][MT];
 #pragma unroll
-        for (int half = 0; half < 2; half++) {
-            bf16x8 A[MT];
+            for (int half = 0; half < 2; half++)
 #pragma unroll
-            for (int a = 0; a < MT; a++) {
-                const uint32_t p = da[a] + dof + half * 32 * PIX;
-                A[a] = read_tr8(p, p + 16 * PIX);
+                for (int a = 0; a < MT; a++) {
+                    const uint32_t p = da[a] + dof + half * 32 * PIX;
+                    A[half][a] = read_tr8(p, p + 16 * PIX);
+                }
+            if (OUTL && at_border) {
+                bad = not_finite(as_bf16x8(mine[lane]));
+#pragma unroll
+                for (int half = 0; half < 2; half++)
+#pragma unroll
+                    for (int a = 0; a < MT; a++) bad |= not_finite(A[half][a]);
+                bad = wave_any(bad);
+                if (bad) {
+#pragma unroll
+                    for (int half = 0; half < 2; half++)
+#pragma unroll
+                        for (int a = 0; a < MT; a++)
+                            A[half][a] = border_ones(A[half][a], r == 0 || r == H - 1, g, c0 + 32 * half, W);
+                }
             }
 #pragma unroll
-            for (int j = 0; j < 5; j++) {
-                const uint32_t p = xo[j] + half * 32 * 16;
-                bf16x8 B = read_tr8(p, p + 16 * 16);
-                if (!OUTL && j == 4) B = li < 8 ? B : ones;
-                if (OUTL && j == 2) bacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, B, bacc, 0, 0, 0);
+            for (int half = 0; half < 2; half++) {
+                // input layer: the left neighbours of the first column past
+                // the image from the column itself, which holds zeros (shifts
+                // 0, 3 and 6: chunks 0, 1 of tiles 0 and 3, 2, 3 of tile 1)
+                const int past = W - c0 - 32 * half;
+                const uint32_t lo = RAGGED && px == past ? 16 : 0, hi = RAGGED && px + 16 == past ? 16 : 0;
 #pragma unroll
-                for (int a = 0; a < MT; a++)
-                    acc[j][a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[a], B, acc[j][a], 0, 0, 0);
+                for (int j = 0; j < 5; j++) {
+                    const bool to_left = !OUTL && RAGGED && (j == 1 ? ch >= 2 : (j == 0 || j == 3) && ch < 2);
+                    const uint32_t p = xo[j] + half * 32 * 16;
+                    bf16x8 B = read_tr8(p + (to_left ? lo : 0), p + (to_left ? hi : 0) + 16 * 16);
+                    if (!OUTL && j == 4) B = li < 8 ? B : ones;
+                    if (OUTL && j == 2) bacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, B, bacc, 0, 0, 0);
+#pragma unroll
+                    for (int a = 0; a < MT; a++)
+                        acc[j][a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[half][a], B, acc[j][a], 0, 0, 0);
+                }
+            }
+        }
+        if (OUTL && bad) {
+#pragma unroll 1
+            for (int i = 0; i < kStripCols && c0 + i < W; i++) {
+                int ln = lane;                               // (no register is held for this by the passes)
+                asm volatile("" : "+v"(ln));
+                const int g = ln >> 4, li = ln & 15;
+                const int c = c0 + i;
+                const bool edge = r == 0 || r == H - 1 || c == 0 || c == W - 1;
+                const bool bad_dy = not_finite16(((const uint16_t*)(mine + i))[li & 7]);
+#pragma unroll
+                for (int j = 0; j < 5; j++) {
+                    const int s = 2 * j + (li >> 3), dr = s / 3 - 1, dc = s % 3 - 1;   // this column's shift
+                    const bool in = r + dr >= 0 && r + dr < H && c + dc >= 0 && c + dc < W;
+                    int row = xs + wv + 1 + dr;
+                    row = row >= XR ? row - XR : row;
+                    const uint16_t v = ((const uint16_t*)(lds + row * kWgradPitch + 1 + i + dc))[li & 7];
+                    const bool out = r - dr < 0 || r - dr >= H || c - dc < 0 || c - dc >= W;
+                    const float none = bad_dy && out ? __builtin_nanf("") : 0.f;
+#pragma unroll
+                    for (int a = 0; a < MT; a++) {
+                        const uint16_t* at = (const uint16_t*)lds + (XN * 16 + (ds + wv) * DROW + i * PIX) / 2 +
+                                             (a ^ slot_xor<CH>(i)) * 16 + 4 * g;
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            const bool add = edge && in && not_finite16(at[e]);
+                            acc[j][a][e] += none + (add ? from_bf16(at[e]) * from_bf16(v) : 0.f);
+                        }
+                    }
+                }
             }
         }
         if (!more) break;
@@ -1335,27 +1457,32 @@ hipError_t nn_launch_wgrad(int kind, const uint16_t* x, const uint16_t* dy, floa
     const long long passes = (long long)N * ((W + kStripCols - 1) / kStripCols) * ((H + rows - 1) / rows);
     const int waves = (int)(passes < kWgradWaves ? passes : kWgradWaves);
     int my = width, kx = width;
+    // a: the kernel's first operand; ragged: for widths with a remainder
+    typedef void (*Kernel)(const uint16_t*, const uint16_t*, float*, float*, int, int, int);
+    auto launch = [&](Kernel whole, Kernel ragged, const uint16_t* a, const uint16_t* b) {
+        (W % kStripCols ? ragged : whole)<<<waves, 512, 0, s>>>(a, b, part, bpart, N, H, W);
+    };
     switch (kind) {
     case NN_WGRAD_IN:
-        wgrad_edge_kernel<32, false><<<waves, 512, 0, s>>>(dy, x, part, bpart, N, H, W);
+        launch(wgrad_edge_kernel<32, false, false>, wgrad_edge_kernel<32, false, true>, dy, x);
         kx = 8;
         break;
     case NN_WGRAD_MID:
-        wgrad_mid_kernel<32><<<waves, 512, 0, s>>>(x, dy, part, bpart, N, H, W);
+        launch(wgrad_mid_kernel<32, false>, wgrad_mid_kernel<32, true>, x, dy);
         break;
     case NN_WGRAD_OUT:
-        wgrad_edge_kernel<32, true><<<waves, 512, 0, s>>>(x, dy, part, bpart, N, H, W);
+        launch(wgrad_edge_kernel<32, true, false>, wgrad_edge_kernel<32, true, false>, x, dy);
         my = 8;
         break;
     case NN_WGRAD_IN | NN_W64:
-        wgrad_edge_kernel<64, false><<<waves, 512, 0, s>>>(dy, x, part, bpart, N, H, W);
+        launch(wgrad_edge_kernel<64, false, false>, wgrad_edge_kernel<64, false, true>, dy, x);
         kx = 8;
         break;
     case NN_WGRAD_MID | NN_W64:
-        wgrad_mid_kernel<64><<<waves, 512, 0, s>>>(x, dy, part, bpart, N, H, W);
+        launch(wgrad_mid_kernel<64, false>, wgrad_mid_kernel<64, true>, x, dy);
         break;
     case NN_WGRAD_OUT | NN_W64:
-        wgrad_edge_kernel<64, true><<<waves, 512, 0, s>>>(x, dy, part, bpart, N, H, W);
+        launch(wgrad_edge_kernel<64, true, false>, wgrad_edge_kernel<64, true, false>, x, dy);
         my = 8;
         break;
     default:
