@@ -632,3 +632,35 @@ def test_unscaled_square_root_on_the_device():
     np.testing.assert_array_equal(ref, np.sqrt(a))            # the device's sqrt() is the IEEE one
     bad = np.flatnonzero(got != np.sqrt(a))
     assert bad.size == 0, "differs at %d inputs, e.g. %r" % (bad.size, a[bad[:3]])
+
+
+def test_square_root_of_negative_numbers_is_nan():
+    rng = np.random.default_rng(24)
+    sc = S.sediment_shelf(n=8, dx=10.0, inflow=False)
+    a = -np.concatenate([10.0 ** rng.uniform(-300, 300, 4000), [1.0, 2.0 ** -1022, np.inf], np.full(61, 1e-3)])
+    got, ref = kat_point(sc.params, sc.scheme, 7, a)[:2]
+    assert np.isnan(ref).all() and np.isnan(got).all()
+    assert np.isnan(kat_point(sc.params, sc.scheme, 3, a[:64] * 1e-3, 0 * a[:64], 0 * a[:64])[0]).all()
+    zero = np.array([0.0, -0.0, np.nan])
+    np.testing.assert_array_equal(kat_point(sc.params, sc.scheme, 7, zero)[0], zero)
+
+
+@pytest.mark.parametrize("nx,ny", [(64, 3), (100, 100), (300, 310)])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_negative_depths_leave_the_initial_dt_to_the_other_cells(precision, nx, ny):
+    """A cell of negative depth has no wave speed, so no time step: the initial
+    dt is that of the state with those cells dry, for a whole wave of such
+    cells and for single ones among others."""
+    rng = np.random.default_rng(nx)
+    sc = S.sediment_shelf(n=nx, ny=ny, dx=20.0, seed=nx, inflow=False)
+    sc.V[0] = np.maximum(sc.V[0], 1.0)
+    sc.V[0, ny // 2] = 30.0
+    sc.V[1] = sc.V[0] * rng.uniform(-2, 2, (ny, nx))
+    dry = rng.random((ny, nx)) < 0.05
+    dry[0] = True
+    sc.V[0][dry] = -10.0 ** rng.uniform(-17, 1, dry.sum())
+    sc.V[1][dry] = 0.0
+    dt = Solver.from_scenario(sc, precision=precision).dt
+    sc.V[0][dry] = 0.0
+    assert dt == Solver.from_scenario(sc, precision=precision).dt
+    assert 0.0 < dt < 10.0

@@ -235,10 +235,12 @@ struct Vel {
 // rsqrt estimate, one Newton step on (g, h) = (x y, y / 2) and two residual
 // corrections, the compiler's own sequence for sqrt() with the scale
 // factors at 1 (they act only below 2^-767).  Equal to sqrt(x) for x in
-// [2^-767, DBL_MAX]; sqrt_unscaled0 also returns 0 for x = 0: the estimate is
-// taken of at least the smallest denormal, so that it stays finite and every
-// product with x is 0 (a test for 0 became a branch per square root, ten
-// serial chains in the Riemann solver where one block can interleave them).
+// [2^-767, DBL_MAX]; sqrt_unscaled0 also returns x for x = +-0, and a NaN for
+// x < 0 as sqrt does (the depth of an uploaded state may be negative): the
+// estimate is taken of x plus the smallest denormal, which is x unless x is
+// denormal, so that it stays finite and every product with a zero x is 0 (a
+// test for 0 became a branch per square root, ten serial chains in the Riemann
+// solver where one block can interleave them).
 __device__ __forceinline__ double sqrt_newton(double x, double y)
 {
     double g = x * y, h = y * 0.5;
@@ -253,7 +255,7 @@ __device__ __forceinline__ double sqrt_newton(double x, double y)
 __device__ __forceinline__ double sqrt_unscaled(double x) { return sqrt_newton(x, __builtin_amdgcn_rsq(x)); }
 __device__ __forceinline__ double sqrt_unscaled0(double x)
 {
-    return sqrt_newton(x, __builtin_amdgcn_rsq(fmax(x, 0x1p-1074)));
+    return sqrt_newton(x, __builtin_amdgcn_rsq(x + 0x1p-1074));
 }
 // x > 0 and below the unscaled square root's range
 __device__ __forceinline__ bool sqrt_needs_scaling(double x) { return x > 0.0 && x < 0x1p-767; }
