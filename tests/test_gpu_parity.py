@@ -664,3 +664,38 @@ def test_negative_depths_leave_the_initial_dt_to_the_other_cells(precision, nx, 
     sc.V[0][dry] = 0.0
     assert dt == Solver.from_scenario(sc, precision=precision).dt
     assert 0.0 < dt < 10.0
+
+
+def test_velocity_of_no_momentum_is_zero_at_any_depth():
+    """At an infinite depth, at -DBL_EPSILON and below, in waves whose other
+    lanes move."""
+    sc = S.sediment_shelf(n=8, dx=10.0, inflow=False)
+    h = np.tile(np.array([np.inf, 3.0, -2.0 ** -52, 0.5, -1.0, 1e300, 7.0, 0.0]), 16)
+    qx = np.where(np.tile(np.arange(8) % 2 == 1, 16), 2.0, 0.0)
+    qx[5::8] = 0.0
+    ux, uy, m, _ = kat_point(sc.params, sc.scheme, 1, h, qx, 0 * qx)
+    want = np.where(qx == 0.0, 0.0, np.where(h > 0, 2.0 / (np.abs(h) + 2.0 ** -52), 0.0))
+    np.testing.assert_array_equal(ux, want)
+    np.testing.assert_array_equal(uy, 0 * want)
+    np.testing.assert_array_equal(m, want)
+
+
+@pytest.mark.parametrize("order", [1, 2])
+@pytest.mark.parametrize("nx,ny", [(64, 5), (100, 100), (300, 310)])
+def test_concentration_of_no_load_is_zero_at_minus_epsilon(order, nx, ny):
+    """Land cells uploaded with a depth of -DBL_EPSILON (eta + H rounded) among
+    water that holds a load: the first step from rest is that of dry cells.
+    Tolerance: 2^-52 of depth moves a neighbour's surface by at most an ulp of
+    the bed (7e-15 m), far below 1e-11 of any field's scale."""
+    sc = S.sediment_shelf(n=nx, ny=ny, dx=20.0, seed=nx, inflow=False, order=order)
+    land = sc.V[0] == 0.0
+    assert land.any()
+    sc.V[4] = 1e-3 * sc.V[0]
+    got = []
+    for depth in (-2.0 ** -52, 0.0):
+        sc.V[0][land] = depth
+        s = Solver.from_scenario(sc)
+        s.step(1)
+        got.append(s.state())
+    for a, b in zip(*got):
+        np.testing.assert_allclose(a, b, rtol=0, atol=1e-11 * np.abs(b).max())

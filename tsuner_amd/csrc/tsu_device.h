@@ -402,11 +402,12 @@ __device__ __forceinline__ Vel<double> velocity_over(double h, double qx, double
 
 __device__ __forceinline__ Vel<double> velocity(double h, double qx, double qy)
 {
-    if (__builtin_amdgcn_ballot_w64(h >= kEps && (qx != 0.0 || qy != 0.0)) == 0) {
+    const bool need = h >= kEps && (qx != 0.0 || qy != 0.0);
+    if (__builtin_amdgcn_ballot_w64(need) == 0) {
         const double z = zero_here();
         return {z, z, z};
     }
-    return velocity_over(h, qx, qy, den(h + kEpsilon));
+    return velocity_over(h, qx, qy, den(need ? h + kEpsilon : 1.0));
 }
 
 // FP32 solver: near-dry cells take the reference's FP64 desingularisation,
@@ -439,11 +440,14 @@ __device__ __forceinline__ Vel<float> velocity(float h, float qx, float qy, cons
 
 // Velocity and concentration hc / (h + DBL_EPSILON) (SedFlux.cuh:26-49,
 // 103-132) of the two sides of an edge at once; the three quotients of a side
-// share one reciprocal of h + DBL_EPSILON.  One wave-wide test whether any lane of either side divides, then both
-// sides' reciprocals and quotients for every lane in one basic block, the
-// unused ones discarded by selects (h + DBL_EPSILON is a valid shared
-// denominator for any face depth).  Returns true (uniform over the wave)
-// when no lane divides: every velocity and concentration is then 0.
+// share one reciprocal of h + DBL_EPSILON.  One wave-wide test whether any lane
+// of either side divides, then both sides' reciprocals and quotients for every
+// lane in one basic block, the unused ones discarded by selects.  Where all
+// numerators are zero so are the quotients, whatever the depth: the divisor is
+// then 1, since h + DBL_EPSILON may be 0 or infinite in a cell that the caller
+// uploaded (2048^2 with sediment in motion 1238 us -> 1245; selects of the
+// quotients 1264).  Returns true (uniform over the wave) when no lane divides:
+// every velocity and concentration is then 0.
 template <bool SED>
 __device__ __forceinline__ bool velocity_conc_pair(double h0, double qx0, double qy0, double hc0, double h1,
                                                    double qx1, double qy1, double hc1, Vel<double>& u0, double& c0,
@@ -458,7 +462,8 @@ __device__ __forceinline__ bool velocity_conc_pair(double h0, double qx0, double
         c0 = c1 = z;
         return true;
     }
-    const Den<double> D0 = den(h0 + kEpsilon), D1 = den(h1 + kEpsilon);
+    const Den<double> D0 = den(nu0 || nc0 ? h0 + kEpsilon : 1.0);
+    const Den<double> D1 = den(nu1 || nc1 ? h1 + kEpsilon : 1.0);
     const double x0 = qdiv(qx0, D0), y0 = qdiv(qy0, D0);
     const double x1 = qdiv(qx1, D1), y1 = qdiv(qy1, D1);
     c0 = c1 = 0.0;
@@ -492,7 +497,7 @@ __device__ __forceinline__ void velocity_conc(double h, double qx, double qy, do
         c = z;
         return;
     }
-    const Den<double> D = den(h + kEpsilon);
+    const Den<double> D = den(need_u || need_c ? h + kEpsilon : 1.0);
     c = 0.0;
     if (SED) {
         c = qdiv(hc, D);
