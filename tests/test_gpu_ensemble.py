@@ -181,3 +181,23 @@ def test_fp32_states_keep_hi_and_lo_parts(nx, ny):
         assert np.array_equal(ens.state(i), want)
         for f in range(5):
             assert np.array_equal(ens.plane(i, f), want[f])
+
+
+@pytest.mark.parametrize("nx,ny", [(128, 128), (127, 130)])
+def test_fp32_states_converted_on_the_host_and_on_the_device(nx, ny):
+    """The largest states whose FP64 values the host splits and joins, and
+    larger ones, whose the device does: the same floats, q without low parts."""
+    rng = np.random.default_rng(nx)
+    V = rng.normal(size=(5, ny, nx)) * 10.0 ** rng.integers(-42, 6, size=(5, ny, nx))
+    V.reshape(5, -1)[:, 0] = [0.0, -0.0, 1e-45, 3e38, 1e-300]
+    want = V.astype(np.float32).astype(np.float64)
+    for f in (0, 3, 4):
+        want[f] += (V[f] - want[f]).astype(np.float32).astype(np.float64)
+    sc = S.Scenario("random", S.base_params(nx, ny, 10.0, 10.0), S.default_scheme(), V, np.ones((ny, nx), np.int32))
+    other = S.gaussian_source(n=64, dx=20.0, seed=1)
+    assert np.array_equal(Solver.from_scenario(sc, precision="fp32", init_dt=False).state(), want)
+    ens = Ensemble([other, sc], precision="fp32")
+    assert np.array_equal(ens.state(1), want)
+    for f in range(5):
+        assert np.array_equal(ens.plane(1, f), want[f])
+        assert np.array_equal(ens.plane(0, f), ens.state(0)[f])

@@ -139,20 +139,27 @@ int validate_scheme(const tsu_scheme* s) { return check_scheme(s); }
 int set_error(int code, const std::string& msg) { return fail(code, msg); }
 
 namespace {
-int reserve(Staging* g, long long count)
+// A buffer for transfers of count values.  False where the host converts: few
+// values, whose launch and wait would cost more than they save (a download of
+// 100^2 cells 33 us on the host and 41 on the device, of 256^2 217 and 166),
+// and a device without room.
+bool reserve(Staging* g, long long nv, long long count)
 {
-    long long want = std::min(count, 4LL << 20);
-    if (g->cap >= want) return TSU_OK;
+    if (nv <= 16384) return false;
+    const long long want = std::min(count, 4LL << 20);
+    if (g->cap >= want) return true;
     free_staging(g);
-    // a smaller buffer, and more transfers, where memory is short
-    for (; hipMalloc((void**)&g->buf, (size_t)want * sizeof(double)) != hipSuccess; want /= 4) {
+    if (hipMalloc((void**)&g->buf, (size_t)want * sizeof(double)) != hipSuccess) {
         (void)hipGetLastError();
         g->buf = nullptr;
-        if (want < 1024) return fail(TSU_ERR_DEVICE_MEMORY, "transfer buffer allocation failed");
+        return false;
     }
     g->cap = want;
-    return TSU_OK;
+    return true;
 }
+
+// plane of the low parts of plane f, or -1
+constexpr int kLoPlane[5] = {5, -1, -1, 6, 7};
 }  // namespace
 
 void free_staging(Staging* g)
@@ -166,31 +173,56 @@ int upload_planes(Staging* g, const double* host, void* state, int precision, lo
     const long long count = 5 * nv;
     if (precision == TSU_FP64) {
         HIPCHK(hipMemcpyAsync(state, host, (size_t)count * sizeof(double), hipMemcpyHostToDevice, s));
-    } else {
-        if (int rc = reserve(g, count)) return rc;
+    } else if (reserve(g, nv, count)) {
         for (long long o = 0; o < count; o += g->cap) {
             const long long n = std::min(g->cap, count - o);
             HIPCHK(hipMemcpyAsync(g->buf, host + o, (size_t)n * sizeof(double), hipMemcpyHostToDevice, s));
             HIPCHK(launch_narrow(g->buf, (float*)state, nv, o, n, s));
         }
+    } else {
+        std::vector<float> v((size_t)(8 * nv));
+        for (int f = 0; f < 5; f++) {
+            const double* from = host + f * nv;
+            float* hi = v.data() + f * nv;
+            for (long long i = 0; i < nv; i++) hi[i] = (float)from[i];
+            if (kLoPlane[f] < 0) continue;
+            float* lo = v.data() + kLoPlane[f] * nv;
+            for (long long i = 0; i < nv; i++) lo[i] = (float)(from[i] - (double)hi[i]);
+        }
+        HIPCHK(hipMemcpyAsync(state, v.data(), v.size() * sizeof(float), hipMemcpyHostToDevice, s));
+        HIPCHK(hipStreamSynchronize(s));                    // v ends here
+        return TSU_OK;
     }
     HIPCHK(hipStreamSynchronize(s));
     return TSU_OK;
 }
 
-int download_planes(Staging* g, const void* state, double* host, int precision, long long nv, long long first,
-                    long long count, hipStream_t s)
+int download_planes(Staging* g, const void* state, double* host, int precision, long long nv, int first, int planes,
+                    hipStream_t s)
 {
+    const long long count = planes * nv, at = first * nv;
     if (precision == TSU_FP64) {
-        HIPCHK(hipMemcpyAsync(host, (const double*)state + first, (size_t)count * sizeof(double),
-                              hipMemcpyDeviceToHost, s));
-    } else {
-        if (int rc = reserve(g, count)) return rc;
+        HIPCHK(hipMemcpyAsync(host, (const double*)state + at, (size_t)count * sizeof(double), hipMemcpyDeviceToHost,
+                              s));
+    } else if (reserve(g, nv, count)) {
         for (long long o = 0; o < count; o += g->cap) {
             const long long n = std::min(g->cap, count - o);
-            HIPCHK(launch_widen((const float*)state, g->buf, nv, first + o, n, s));
+            HIPCHK(launch_widen((const float*)state, g->buf, nv, at + o, n, s));
             HIPCHK(hipMemcpyAsync(host + o, g->buf, (size_t)n * sizeof(double), hipMemcpyDeviceToHost, s));
         }
+    } else {
+        // from the first plane to the last low part, in one copy
+        const int last = planes == 5 ? 7 : std::max(first, kLoPlane[first]);
+        std::vector<float> v((size_t)((last - first + 1) * nv));
+        HIPCHK(hipMemcpyAsync(v.data(), (const float*)state + at, v.size() * sizeof(float), hipMemcpyDeviceToHost, s));
+        HIPCHK(hipStreamSynchronize(s));
+        for (int f = 0; f < planes; f++) {
+            const float* hi = v.data() + f * nv;
+            const float* lo = kLoPlane[first + f] < 0 ? nullptr : v.data() + (kLoPlane[first + f] - first) * nv;
+            double* to = host + f * nv;
+            for (long long i = 0; i < nv; i++) to[i] = lo ? (double)hi[i] + (double)lo[i] : (double)hi[i];
+        }
+        return TSU_OK;
     }
     HIPCHK(hipStreamSynchronize(s));
     return TSU_OK;
@@ -596,7 +628,7 @@ TSU_API int tsu_state_download(tsu_state* st, double* V)
     void* cur;
     int rc = current_buffer(st, &cur);
     if (rc) return rc;
-    return tsu::download_planes(&st->staging, cur, V, st->precision, st->nvol, 0, 5 * st->nvol, st->stream);
+    return tsu::download_planes(&st->staging, cur, V, st->precision, st->nvol, 0, 5, st->stream);
 }
 
 TSU_API int tsu_state_set_inflow(tsu_state* st, const double* CC, const double* tCC, unsigned long timeCC)

@@ -476,7 +476,7 @@ TSU_API int tsu_ensemble_download(tsu_ensemble* e, int i, double* V)
     char* cur;
     if ((rc = current_buffer(e, i, &cur))) return rc;
     const long long nv = e->P[i].nvol;
-    return tsu::download_planes(&e->staging, cur, V, e->precision, nv, 0, 5 * nv, e->stream);
+    return tsu::download_planes(&e->staging, cur, V, e->precision, nv, 0, 5, e->stream);
 }
 
 TSU_API int tsu_ensemble_download_plane(tsu_ensemble* e, int i, int plane, double* out)
@@ -488,7 +488,7 @@ TSU_API int tsu_ensemble_download_plane(tsu_ensemble* e, int i, int plane, doubl
     char* cur;
     if ((rc = current_buffer(e, i, &cur))) return rc;
     const long long nv = e->P[i].nvol;
-    return tsu::download_planes(&e->staging, cur, out, e->precision, nv, plane * nv, nv, e->stream);
+    return tsu::download_planes(&e->staging, cur, out, e->precision, nv, plane, 1, e->stream);
 }
 
 TSU_API int tsu_ensemble_set_inflow(tsu_ensemble* e, int i, const double* CC, const double* tCC, unsigned long timeCC)

@@ -41,18 +41,19 @@ private:
     int prev_ = -1;
 };
 // FP64 values on their way to or from a handle's FP32 planes (device memory,
-// at most 32 MB, allocated by the first transfer and kept with the handle).
+// at most 32 MB, allocated by the first transfer that is converted there and
+// kept with the handle).
 struct Staging {
     double* buf = nullptr;
     long long cap = 0;   // doubles
 };
 void free_staging(Staging* g);
-// Values [first, first + count) of the five state planes (nv cells each, one
-// after the other) between the host and a device state of the precision,
-// ordered on the stream and complete on return.
+// The five state planes of nv cells each, or of a download all five or one of
+// them, between the host and a device state of the precision, ordered on the
+// stream and complete on return.
 int upload_planes(Staging* g, const double* host, void* state, int precision, long long nv, hipStream_t s);
-int download_planes(Staging* g, const void* state, double* host, int precision, long long nv, long long first,
-                    long long count, hipStream_t s);
+int download_planes(Staging* g, const void* state, double* host, int precision, long long nv, int first, int planes,
+                    hipStream_t s);
 // Tile height for one launch of the stage kernel over grids of (npx, npy)
 // cells (tsu_api.cpp).
 int choose_tile_rows(const std::vector<std::pair<int, int>>& grids, bool sed, int precision, int device);
