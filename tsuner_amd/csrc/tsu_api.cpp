@@ -43,13 +43,6 @@ int fail(int code, const std::string& msg)
     } while (0)
 
 
-unsigned long long dbits(double v)
-{
-    unsigned long long b;
-    std::memcpy(&b, &v, 8);
-    return b;
-}
-
 double bitsd(unsigned long long b)
 {
     double v;
@@ -191,9 +184,7 @@ int upload_planes(Staging* g, const double* host, void* state, int precision, lo
         }
         HIPCHK(hipMemcpyAsync(state, v.data(), v.size() * sizeof(float), hipMemcpyHostToDevice, s));
         HIPCHK(hipStreamSynchronize(s));                    // v ends here
-        return TSU_OK;
     }
-    HIPCHK(hipStreamSynchronize(s));
     return TSU_OK;
 }
 
@@ -305,6 +296,7 @@ struct tsu_state {
     uint8_t* fix = nullptr;
     Ctrl* ctrl = nullptr;
     tsu::DtSlots* dts = nullptr;
+    tsu::StepReport* report = nullptr;
     tsu::Staging staging;
     double* ext = nullptr;
     double* CC = nullptr;
@@ -402,6 +394,7 @@ void free_state(tsu_state* st)
     (void)hipFree(st->fix);
     (void)hipFree(st->ctrl);
     (void)hipFree(st->dts);
+    (void)hipFree(st->report);
     tsu::free_staging(&st->staging);
     (void)hipFree(st->ext);
     (void)hipFree(st->CC);
@@ -484,20 +477,6 @@ int read_ctrl(tsu_state* st, Ctrl* c)
     return TSU_OK;
 }
 
-// The control block and every dt slot as before the first step.
-int reset_ctrl(tsu_state* st)
-{
-    Ctrl c{};
-    c.stop_time = INFINITY;
-    c.stop_step = LLONG_MAX;
-    tsu::DtSlots d;
-    tsu::reset_dt_slots(&d);
-    HIPCHK(hipMemcpyAsync(st->ctrl, &c, sizeof(c), hipMemcpyHostToDevice, st->stream));
-    HIPCHK(hipMemcpyAsync(st->dts, &d, sizeof(d), hipMemcpyHostToDevice, st->stream));
-    HIPCHK(hipStreamSynchronize(st->stream));
-    return TSU_OK;
-}
-
 // Buffer holding U^n (the single-stage scheme alternates by step parity).
 int current_buffer(tsu_state* st, void** buf)
 {
@@ -573,18 +552,16 @@ TSU_API int tsu_state_create(tsu_state** out, const tsu_sim_params* p, const tsu
     if (e == hipSuccess) e = hipMalloc((void**)&st->fix, (size_t)st->nvol);
     if (e == hipSuccess) e = hipMalloc((void**)&st->ctrl, sizeof(Ctrl));
     if (e == hipSuccess) e = hipMalloc((void**)&st->dts, sizeof(tsu::DtSlots));
+    if (e == hipSuccess) e = hipMalloc((void**)&st->report, sizeof(tsu::StepReport));
     if (e == hipSuccess) e = hipMalloc((void**)&st->mass_buf, (2 * (size_t)st->mass_nb + 2) * sizeof(double));
     if (e == hipSuccess) e = hipMalloc((void**)&st->dP, sizeof(DevParams));
     if (e == hipSuccess) e = hipMemcpy(st->dP, &st->P, sizeof(DevParams), hipMemcpyHostToDevice);
     if (e == hipSuccess && s->extrema) e = hipMalloc((void**)&st->ext, 3 * (size_t)st->nvol * sizeof(double));
+    if (e == hipSuccess) e = tsu::launch_reset_steps(st->ctrl, st->dts, 1, st->stream);
     if (e != hipSuccess) {
         free_state(st);
         (void)hipGetLastError();
         return fail(TSU_ERR_DEVICE_MEMORY, std::string("device allocation failed: ") + hipGetErrorString(e));
-    }
-    if (int rc2 = reset_ctrl(st)) {
-        free_state(st);
-        return rc2;
     }
     *out = st;
     return TSU_OK;
@@ -616,7 +593,8 @@ TSU_API int tsu_state_upload(tsu_state* st, const double* V, const int* fixH)
     HIPCHK(hipMemcpyAsync(st->B, st->A, bytes, hipMemcpyDeviceToDevice, st->stream));
     HIPCHK(hipMemcpyAsync(st->fix, fx.data(), (size_t)nv, hipMemcpyHostToDevice, st->stream));
     if (st->ext) HIPCHK(tsu::launch_fill(st->ext, 3 * nv, -1e30, st->stream));
-    if (int rc = reset_ctrl(st)) return rc;                 // waits for the stream
+    HIPCHK(tsu::launch_reset_steps(st->ctrl, st->dts, 1, st->stream));
+    HIPCHK(hipStreamSynchronize(st->stream));
     st->uploaded = true;
     return TSU_OK;
 }
@@ -683,9 +661,7 @@ TSU_API int tsu_init_dt(tsu_state* st)
     Ctrl c;
     rc = read_ctrl(st, &c);
     if (rc) return rc;
-    tsu::DtSlots d;
-    tsu::reset_dt_slots(&d);
-    HIPCHK(hipMemcpyAsync(st->dts, &d, sizeof(d), hipMemcpyHostToDevice, st->stream));
+    HIPCHK(tsu::launch_arm_dt(st->dts, st->stream));
     void* cur = (st->s.order == 1 && (c.step & 1)) ? st->B : st->A;
     HIPCHK(tsu::launch_init_dt(cur, st->P, st->dts, c.step, st->precision, st->stream));
     HIPCHK(hipStreamSynchronize(st->stream));
@@ -741,14 +717,13 @@ TSU_API int tsu_get_time(tsu_state* st, double* t, double* dt, long long* steps)
 {
     if (!st) return fail(TSU_ERR_ARG, "null state");
     tsu::HandleGuard g(st->calls, st->device);
-    Ctrl c;
-    tsu::DtSlots d;
-    HIPCHK(hipMemcpyAsync(&d, st->dts, sizeof(d), hipMemcpyDeviceToHost, st->stream));
-    int rc = read_ctrl(st, &c);                             // waits for the stream
-    if (rc) return rc;
-    if (t) *t = c.t;
-    if (dt) *dt = finalize_host(st->P, tsu::min_dt_bits(d, c.step));
-    if (steps) *steps = c.step;
+    tsu::StepReport r;
+    HIPCHK(tsu::launch_report(st->ctrl, st->dts, st->report, st->stream));
+    HIPCHK(hipMemcpyAsync(&r, st->report, sizeof(r), hipMemcpyDeviceToHost, st->stream));
+    HIPCHK(hipStreamSynchronize(st->stream));
+    if (t) *t = r.t;
+    if (dt) *dt = finalize_host(st->P, r.dt_bits);
+    if (steps) *steps = r.step;
     return TSU_OK;
 }
 
@@ -756,17 +731,7 @@ TSU_API int tsu_set_time(tsu_state* st, double t, double dt)
 {
     if (!st) return fail(TSU_ERR_ARG, "null state");
     tsu::HandleGuard g(st->calls, st->device);
-    Ctrl c;
-    int rc = read_ctrl(st, &c);
-    if (rc) return rc;
-    c.t = t;
-    if (dt > 0) {
-        tsu::DtSlots d;
-        tsu::reset_dt_slots(&d, c.step, dbits(dt));
-        HIPCHK(hipMemcpyAsync(st->dts, &d, sizeof(d), hipMemcpyHostToDevice, st->stream));
-        HIPCHK(hipStreamSynchronize(st->stream));
-    }
-    HIPCHK(hipMemcpyAsync(st->ctrl, &c, sizeof(Ctrl), hipMemcpyHostToDevice, st->stream));
+    HIPCHK(tsu::launch_set_time(st->ctrl, st->dts, t, dt, st->stream));
     HIPCHK(hipStreamSynchronize(st->stream));
     return TSU_OK;
 }

@@ -59,6 +59,7 @@ struct tsu_ensemble {
     size_t ext_doubles = 0;
     Ctrl* ctrl = nullptr;
     tsu::DtSlots* dts = nullptr;
+    tsu::StepReport* report = nullptr;
     tsu::Staging staging;
     Ctrl* snapC = nullptr;
     tsu::DtSlots* snapD = nullptr;
@@ -117,6 +118,7 @@ void destroy(tsu_ensemble* e)
     (void)hipFree(e->ext);
     (void)hipFree(e->ctrl);
     (void)hipFree(e->dts);
+    (void)hipFree(e->report);
     tsu::free_staging(&e->staging);
     (void)hipFree(e->snapC);
     (void)hipFree(e->snapD);
@@ -314,20 +316,6 @@ int members_ready(const tsu_ensemble* e)
     return TSU_OK;
 }
 
-// A member's control block and dt slots as before its first step.
-int reset_ctrl(tsu_ensemble* e, int i)
-{
-    Ctrl c{};
-    c.stop_time = INFINITY;
-    c.stop_step = LLONG_MAX;
-    tsu::DtSlots d;
-    tsu::reset_dt_slots(&d);
-    ECHK(hipMemcpyAsync(e->ctrl + i, &c, sizeof(c), hipMemcpyHostToDevice, e->stream));
-    ECHK(hipMemcpyAsync(e->dts + i, &d, sizeof(d), hipMemcpyHostToDevice, e->stream));
-    ECHK(hipStreamSynchronize(e->stream));
-    return TSU_OK;
-}
-
 int current_buffer(tsu_ensemble* e, int i, char** buf)
 {
     if (e->s[i].order == 2) {
@@ -411,21 +399,18 @@ TSU_API int tsu_ensemble_create(tsu_ensemble** out, int n, const tsu_sim_params*
     if (err == hipSuccess && e->ext_doubles) err = hipMalloc((void**)&e->ext, e->ext_doubles * sizeof(double));
     if (err == hipSuccess) err = hipMalloc((void**)&e->ctrl, n * sizeof(Ctrl));
     if (err == hipSuccess) err = hipMalloc((void**)&e->dts, n * sizeof(tsu::DtSlots));
+    if (err == hipSuccess) err = hipMalloc((void**)&e->report, sizeof(tsu::StepReport));
     if (err == hipSuccess) err = hipMalloc((void**)&e->dP, n * sizeof(DevParams));
     if (err == hipSuccess) err = hipMalloc((void**)&e->dargs, 2 * (size_t)n * sizeof(tsu::StageArgs));
     if (err == hipSuccess) err = hipMalloc((void**)&e->dmem, (size_t)n * sizeof(tsu::BatchMember));
     if (err == hipSuccess) err = hipMalloc((void**)&e->mass_buf, (2 * (size_t)e->mass_nb + 2) * sizeof(double));
     if (err == hipSuccess) err = hipMemcpy(e->dP, e->P.data(), n * sizeof(DevParams), hipMemcpyHostToDevice);
+    if (err == hipSuccess) err = tsu::launch_reset_steps(e->ctrl, e->dts, n, e->stream);
     if (err != hipSuccess) {
         destroy(e);
         (void)hipGetLastError();
         return tsu::set_error(TSU_ERR_DEVICE_MEMORY, std::string("ensemble allocation: ") + hipGetErrorString(err));
     }
-    for (int i = 0; i < n; i++)
-        if (int rc = reset_ctrl(e, i)) {
-            destroy(e);
-            return rc;
-        }
     int rc = build_launch_tables(e);
     if (rc) {
         destroy(e);
@@ -462,7 +447,8 @@ TSU_API int tsu_ensemble_upload(tsu_ensemble* e, int i, const double* V, const i
     ECHK(hipMemcpyAsync(e->B + e->off[i], e->A + e->off[i], bytes, hipMemcpyDeviceToDevice, e->stream));
     ECHK(hipMemcpyAsync(e->fix + e->foff[i], fx.data(), (size_t)nv, hipMemcpyHostToDevice, e->stream));
     if (e->s[i].extrema) ECHK(tsu::launch_fill(e->ext + e->xoff[i], 3 * nv, -1e30, e->stream));
-    if ((rc = reset_ctrl(e, i))) return rc;                 // waits for the stream
+    ECHK(tsu::launch_reset_steps(e->ctrl + i, e->dts + i, 1, e->stream));
+    ECHK(hipStreamSynchronize(e->stream));
     e->uploaded[i] = true;
     return TSU_OK;
 }
@@ -533,13 +519,11 @@ TSU_API int tsu_ensemble_init_dt(tsu_ensemble* e)
     if (!e) return tsu::set_error(TSU_ERR_ARG, "null ensemble");
     tsu::HandleGuard g(e->calls, e->device);
     if (int rc = members_ready(e)) return rc;
-    tsu::DtSlots d;
-    tsu::reset_dt_slots(&d);
     for (int i = 0; i < e->n; i++) {
         Ctrl c;
         ECHK(hipMemcpyAsync(&c, e->ctrl + i, sizeof(Ctrl), hipMemcpyDeviceToHost, e->stream));
         ECHK(hipStreamSynchronize(e->stream));
-        ECHK(hipMemcpyAsync(e->dts + i, &d, sizeof(d), hipMemcpyHostToDevice, e->stream));
+        ECHK(tsu::launch_arm_dt(e->dts + i, e->stream));
         char* cur = ((e->s[i].order == 1 && (c.step & 1)) ? e->B : e->A) + e->off[i];
         ECHK(tsu::launch_init_dt(cur, e->P[i], e->dts + i, c.step, e->precision, e->stream));
     }
@@ -580,20 +564,18 @@ TSU_API int tsu_ensemble_get_time(tsu_ensemble* e, int i, double* t, double* dt,
     int rc = member_ok(e, i);
     if (rc) return rc;
     tsu::HandleGuard g(e->calls, e->device);
-    Ctrl c;
-    tsu::DtSlots d;
-    ECHK(hipMemcpyAsync(&c, e->ctrl + i, sizeof(Ctrl), hipMemcpyDeviceToHost, e->stream));
-    ECHK(hipMemcpyAsync(&d, e->dts + i, sizeof(d), hipMemcpyDeviceToHost, e->stream));
+    tsu::StepReport r;
+    ECHK(tsu::launch_report(e->ctrl + i, e->dts + i, e->report, e->stream));
+    ECHK(hipMemcpyAsync(&r, e->report, sizeof(r), hipMemcpyDeviceToHost, e->stream));
     ECHK(hipStreamSynchronize(e->stream));
-    if (t) *t = c.t;
+    if (t) *t = r.t;
     if (dt) {
         double m;
-        unsigned long long b = tsu::min_dt_bits(d, c.step);
-        std::memcpy(&m, &b, 8);
+        std::memcpy(&m, &r.dt_bits, 8);
         if (e->P[i].dt_narrow && e->P[i].nvol > 4096) m = (double)(float)m;
         *dt = (m < 1e30) ? m : 1e30;
     }
-    if (steps) *steps = c.step;
+    if (steps) *steps = r.step;
     return TSU_OK;
 }
 

@@ -50,7 +50,7 @@ struct Staging {
 void free_staging(Staging* g);
 // The five state planes of nv cells each, or of a download all five or one of
 // them, between the host and a device state of the precision, ordered on the
-// stream and complete on return.
+// stream; a download is complete on return, an upload once the stream is.
 int upload_planes(Staging* g, const double* host, void* state, int precision, long long nv, hipStream_t s);
 int download_planes(Staging* g, const void* state, double* host, int precision, long long nv, int first, int planes,
                     hipStream_t s);

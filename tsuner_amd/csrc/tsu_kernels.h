@@ -38,23 +38,12 @@ inline int periodic_sides(const DevParams& P)
     return (P.bc[0] == BC_PERIODIC ? 1 : 0) | (P.bc[2] == BC_PERIODIC ? 2 : 0);
 }
 
-// Every slot at +inf; then, if bits is not +inf, slot 0 of step s at bits.
-inline void reset_dt_slots(DtSlots* d, long long s = 0, unsigned long long bits = kInfBits)
-{
-    for (auto& parity : d->v)
-        for (auto& slot : parity)
-            for (auto& w : slot) w = kInfBits;
-    d->v[s & 1][0][0] = bits;
-}
-
-// Bits of the smallest cell dt of step s.
-inline unsigned long long min_dt_bits(const DtSlots& d, long long s)
-{
-    unsigned long long m = kInfBits;
-    for (auto& slot : d.v[s & 1])
-        if (slot[0] < m) m = slot[0];
-    return m;
-}
+// A step's time, dt (the bits of the smallest cell dt) and number.
+struct StepReport {
+    double t;
+    unsigned long long dt_bits;
+    long long step;
+};
 
 // precision: 0 = FP64, 1 = FP32 planes and arithmetic (compensated h, H, hc).  fast_bed:
 // the run constants satisfy fast_bedload (tsu_device.h); with sediment the
@@ -96,6 +85,13 @@ hipError_t launch_advance_batch(Ctrl* ctrl, DtSlots* dts, const DevParams* P, co
 // Smallest cell dt of the state V into step `step`'s slots (armed before).
 hipError_t launch_init_dt(const void* V, const DevParams& P, DtSlots* dts, long long step, int precision,
                           hipStream_t s);
+// Control blocks and dt slots, n of each, as before the first step.
+hipError_t launch_reset_steps(Ctrl* ctrl, DtSlots* dts, int n, hipStream_t s);
+// Every dt slot at +inf.
+hipError_t launch_arm_dt(DtSlots* dts, hipStream_t s);
+// The time, and if dt > 0 the dt, of the running step.
+hipError_t launch_set_time(Ctrl* ctrl, DtSlots* dts, double t, double dt, hipStream_t s);
+hipError_t launch_report(const Ctrl* ctrl, const DtSlots* dts, StepReport* out, hipStream_t s);
 hipError_t launch_warmup(hipStream_t s);
 hipError_t launch_copy(const void* src, void* dst, long long bytes, hipStream_t s);
 // After a step of the single-stage scheme (the two-stage scheme's stages

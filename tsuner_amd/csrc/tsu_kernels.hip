@@ -1164,6 +1164,49 @@ __global__ __launch_bounds__(64) void advance_batch_kernel(Ctrl* C, DtSlots* dts
     advance_one(C + blockIdx.x, dts + blockIdx.x, P[blockIdx.x]);
 }
 
+// What the host sets and reads of a control block and its dt slots, in one
+// launch each.  Copies, one for each of the two, took a read of the time from 23
+// to 31 us, setting it from 12 to 44, a new state of 32^2 cells from 115 to 146.
+__device__ __forceinline__ void arm_dt(DtSlots* dts)
+{
+    for (int i = threadIdx.x; i < 2 * kDtSlots; i += 64) dts->v[i / kDtSlots][i % kDtSlots][0] = kInfBits;
+}
+
+__global__ __launch_bounds__(64) void reset_steps_kernel(Ctrl* C, DtSlots* dts)
+{
+    arm_dt(dts + blockIdx.x);
+    if (threadIdx.x == 0) {
+        Ctrl c = {};
+        c.stop_time = __longlong_as_double((long long)kInfBits);
+        c.stop_step = 0x7FFFFFFFFFFFFFFFll;
+        C[blockIdx.x] = c;
+    }
+}
+
+__global__ __launch_bounds__(64) void arm_dt_kernel(DtSlots* dts) { arm_dt(dts); }
+
+__global__ __launch_bounds__(64) void set_time_kernel(Ctrl* C, DtSlots* dts, double t, double dt)
+{
+    if (dt > 0.0) {
+        arm_dt(dts);
+        __syncthreads();                                    // slot 0 is armed before it is set
+    }
+    if (threadIdx.x != 0) return;
+    C->t = t;
+    if (dt > 0.0) dts->v[C->step & 1][0][0] = (unsigned long long)__double_as_longlong(dt);
+}
+
+__global__ __launch_bounds__(64) void report_kernel(const Ctrl* C, const DtSlots* dts, StepReport* out)
+{
+    const long long step = C->step;
+    unsigned long long m = dts->v[step & 1][threadIdx.x & (kDtSlots - 1)][0];
+    for (int o = kDtSlots / 2; o > 0; o >>= 1) {
+        const unsigned long long v = __shfl_xor(m, o, 64);
+        m = v < m ? v : m;
+    }
+    if (threadIdx.x == 0) *out = {C->t, m, step};
+}
+
 __global__ void warmup_kernel() {}
 
 // Plain streaming copy (16 B per lane per access), the reference point for
@@ -1459,6 +1502,30 @@ hipError_t launch_init_dt(const void* V, const DevParams& P, DtSlots* dts, long 
     else
         hipLaunchKernelGGL((init_dt_kernel<float, float>), dim3(grid), dim3(256), 0, s, (const float*)V, P, dts,
                            parity);
+    return hipGetLastError();
+}
+
+hipError_t launch_reset_steps(Ctrl* ctrl, DtSlots* dts, int n, hipStream_t s)
+{
+    hipLaunchKernelGGL(reset_steps_kernel, dim3(n), dim3(64), 0, s, ctrl, dts);
+    return hipGetLastError();
+}
+
+hipError_t launch_arm_dt(DtSlots* dts, hipStream_t s)
+{
+    hipLaunchKernelGGL(arm_dt_kernel, dim3(1), dim3(64), 0, s, dts);
+    return hipGetLastError();
+}
+
+hipError_t launch_set_time(Ctrl* ctrl, DtSlots* dts, double t, double dt, hipStream_t s)
+{
+    hipLaunchKernelGGL(set_time_kernel, dim3(1), dim3(64), 0, s, ctrl, dts, t, dt);
+    return hipGetLastError();
+}
+
+hipError_t launch_report(const Ctrl* ctrl, const DtSlots* dts, StepReport* out, hipStream_t s)
+{
+    hipLaunchKernelGGL(report_kernel, dim3(1), dim3(64), 0, s, ctrl, dts, out);
     return hipGetLastError();
 }
 
