@@ -201,3 +201,21 @@ def test_fp32_states_converted_on_the_host_and_on_the_device(nx, ny):
     for f in range(5):
         assert np.array_equal(ens.plane(1, f), want[f])
         assert np.array_equal(ens.plane(0, f), ens.state(0)[f])
+
+
+@pytest.mark.parametrize("order", [1, 2])
+@pytest.mark.parametrize("chunk", [0, 2])
+def test_short_and_long_calls_alternate(order, chunk):
+    """Calls of one launch for both halves and calls that fork them (here from
+    21 single-stage and 11 two-stage steps on), eager and in graphs of either,
+    against the single solver."""
+    scs = [S.gaussian_source(n=k, dx=40.0, seed=k, order=order) for k in (300, 181, 240)]
+    ens = Ensemble(scs, precision="fp32", graph_chunk=chunk)
+    calls = (1, 2, 24, 3, 25, 2, 10)
+    for k in calls:
+        ens.step(k, sync=False)
+    for i, sc in enumerate(scs):
+        g = Solver.from_scenario(sc, precision="fp32")
+        g.step(sum(calls))
+        assert np.array_equal(ens.state(i), g.state()), "member %d" % i
+        assert ens.time(i) == g.time()

@@ -1,9 +1,9 @@
 // tsu_ensemble.cpp -- many independent scenarios on grids of uneven size,
 // advanced together: one stage launch covers every tile of half the members
-// (stage_kernel_batch), the other half's beside it on a second stream, each
-// member keeps its own buffers, run constants and step-control block (so its
-// own dt and time), and each half's steps are replayed from a captured HIP
-// graph.  The reference runs one scenario per
+// (stage_kernel_batch), the other half's beside it on a second stream (short
+// calls: one launch for both), each member keeps its own buffers, run constants
+// and step-control block (so its own dt and time), and each half's steps are
+// replayed from a captured HIP graph.  The reference runs one scenario per
 // process (GPU/main_TSUNER.cu:21-222); this is the batched form of that loop.
 #define TSU_BUILDING_LIBRARY 1
 #include "../../include/tsuner.h"
@@ -75,8 +75,8 @@ struct tsu_ensemble {
     hipStream_t stream2 = nullptr;  // the second half's steps; joined to stream when a call returns
     hipEvent_t forked = nullptr, joined = nullptr;
     int graph_chunk = 0;
-    hipGraph_t graph[2] = {nullptr, nullptr};
-    hipGraphExec_t gexec[2] = {nullptr, nullptr};
+    hipGraph_t graph[3] = {nullptr, nullptr, nullptr};      // of each half, and of both (see kBoth)
+    hipGraphExec_t gexec[3] = {nullptr, nullptr, nullptr};
 };
 
 namespace {
@@ -94,9 +94,11 @@ struct Guard {
     }
 };
 
+constexpr int kBoth = 2;   // for a half: the members of both, on the ensemble's stream
+
 void drop_graph(tsu_ensemble* e)
 {
-    for (int h = 0; h < 2; h++) {
+    for (int h = 0; h <= kBoth; h++) {
         if (e->gexec[h]) (void)hipGraphExecDestroy(e->gexec[h]);
         if (e->graph[h]) (void)hipGraphDestroy(e->graph[h]);
         e->gexec[h] = nullptr;
@@ -232,18 +234,19 @@ int build_launch_tables(tsu_ensemble* e)
     return TSU_OK;
 }
 
-hipStream_t half_stream(const tsu_ensemble* e, int h) { return h ? e->stream2 : e->stream; }
+hipStream_t half_stream(const tsu_ensemble* e, int h) { return h == 1 ? e->stream2 : e->stream; }
 
 // One step of a half's members, on the half's stream.
 int enqueue_step(tsu_ensemble* e, int h)
 {
     const int order = e->s[0].order;
     const tsu::BatchPools pools{e->A, e->B, e->fix, e->ctrl, e->dts, e->ext, e->dP};
-    const int2* tiles = e->tiles + (h ? e->ntiles[0] : 0);
+    const int2* tiles = e->tiles + (h == 1 ? e->ntiles[0] : 0);
+    const int ntiles = h == kBoth ? e->ntiles[0] + e->ntiles[1] : e->ntiles[h];
     bool fast_bed = true;
     for (int i = 0; i < e->n; i++) fast_bed = fast_bed && tsu::fast_bedload(e->P[i]);
     for (int k = 0; k < order; k++)
-        ECHK(tsu::launch_stage_batch(pools, e->dmem, tiles, e->ntiles[h], k, k == order - 1, e->sed, e->precision,
+        ECHK(tsu::launch_stage_batch(pools, e->dmem, tiles, ntiles, k, k == order - 1, e->sed, e->precision,
                                      half_stream(e, h), fast_bed));
     if (order == 1) ECHK(tsu::launch_advance_batch(e->ctrl, e->dts, e->dP, e->dmem, e->n, h, half_stream(e, h)));
     return TSU_OK;
@@ -266,29 +269,47 @@ int capture_steps(tsu_ensemble* e, int h)
     return TSU_OK;
 }
 
+// Whether a call of nsteps steps is worth a fork and join of the halves, which
+// take 20 to 45 us of it: by what the halves save, a part of the steps' time,
+// which goes with cells and stages, twice in FP64 and by half with sediment.
+// FP32 with sediment, two-stage, us a step of calls of one step, together and by
+// halves: 3 x 300^2 cells 38 and 49, 2 x 700^2 82 and 85, 2 x 1500^2 275 and
+// 263; FP64 2 x 700^2 192 and 178.  Steps from which a call is faster by halves:
+// 3 x 300^2 FP32 5 and FP64 6, 32 x 64^2 FP32 7, single-stage 2 x 700^2 FP32 4
+// and FP64 2.  A single-stage step alone is one launch: 32 x 256^2 FP32 63 and
+// 80.
+bool worth_halves(const tsu_ensemble* e, int nsteps)
+{
+    const double stages = (double)nsteps * e->s[0].order;
+    if (e->ntiles[1] == 0 || stages < 2) return false;
+    double cells = 0.0;
+    for (const DevParams& P : e->P) cells += (double)P.nvol;
+    return stages * cells * (e->precision == TSU_FP64 ? 2.0 : 1.0) * (e->sed ? 1.5 : 1.0) >= 5.5e6;
+}
+
 // nsteps steps of every member behind the work on e->stream; work enqueued on
 // it afterwards comes after them.  With graphs, whole chunks are replayed.
 int enqueue_steps(tsu_ensemble* e, int nsteps, bool graphs)
 {
-    const int halves = e->ntiles[1] > 0 ? 2 : 1;
+    const bool halves = worth_halves(e, nsteps);
+    const int from = halves ? 0 : kBoth, to = halves ? 1 : kBoth;
     graphs = graphs && e->graph_chunk > 0 && nsteps >= e->graph_chunk;
     if (graphs)
-        for (int h = 0; h < halves; h++)
+        for (int h = from; h <= to; h++)
             if (!e->gexec[h])
                 if (int rc = capture_steps(e, h)) return rc;
-    if (nsteps == 0) return TSU_OK;
-    if (halves == 2) {
+    if (halves) {
         ECHK(hipEventRecord(e->forked, e->stream));
         ECHK(hipStreamWaitEvent(e->stream2, e->forked, 0));
     }
     int rc = TSU_OK, done = 0;
     for (; graphs && rc == TSU_OK && nsteps - done >= e->graph_chunk; done += e->graph_chunk)
-        for (int h = 0; h < halves && rc == TSU_OK; h++)
+        for (int h = from; h <= to && rc == TSU_OK; h++)
             if (hipError_t er = hipGraphLaunch(e->gexec[h], half_stream(e, h)))
                 rc = tsu::set_error(TSU_ERR_HIP, std::string("graph launch: ") + hipGetErrorString(er));
     for (; rc == TSU_OK && done < nsteps; done++)
-        for (int h = 0; h < halves && rc == TSU_OK; h++) rc = enqueue_step(e, h);
-    if (halves == 2) {   // after an error too: what was enqueued is waited for
+        for (int h = from; h <= to && rc == TSU_OK; h++) rc = enqueue_step(e, h);
+    if (halves) {   // after an error too: what was enqueued is waited for
         ECHK(hipEventRecord(e->joined, e->stream2));
         ECHK(hipStreamWaitEvent(e->stream, e->joined, 0));
     }

@@ -79,7 +79,7 @@ struct BatchPools {
 // fast_bed: every member's run constants satisfy fast_bedload.
 hipError_t launch_stage_batch(const BatchPools& pools, const BatchMember* mem, const int2* tiles, int ntiles, int k,
                               int last, bool sed, int precision, hipStream_t s, bool fast_bed = false);
-// The members of one half, of n in all.
+// The members of one half (0, 1) or both (2), of n in all.
 hipError_t launch_advance_batch(Ctrl* ctrl, DtSlots* dts, const DevParams* P, const BatchMember* mem, int n, int half,
                                 hipStream_t s);
 // Smallest cell dt of the state V into step `step`'s slots (armed before).

@@ -1156,11 +1156,12 @@ __device__ __forceinline__ void advance_one(Ctrl* C, DtSlots* dts, const DevPara
 
 __global__ __launch_bounds__(64) void advance_kernel(Ctrl* C, DtSlots* dts, DevParams P) { advance_one(C, dts, P); }
 
-// One workgroup (one wave) per ensemble member; those of one half advance.
+// One workgroup (one wave) per ensemble member; those of one half (0, 1) or of
+// both (2) advance.
 __global__ __launch_bounds__(64) void advance_batch_kernel(Ctrl* C, DtSlots* dts, const DevParams* __restrict__ P,
                                                            const BatchMember* __restrict__ mem, int half)
 {
-    if (mem[blockIdx.x].half != half) return;
+    if (half < 2 && mem[blockIdx.x].half != half) return;
     advance_one(C + blockIdx.x, dts + blockIdx.x, P[blockIdx.x]);
 }
 
