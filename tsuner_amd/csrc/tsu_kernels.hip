@@ -658,18 +658,21 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int tile)
     if (lane < kPWords) pword = reinterpret_cast<const unsigned long long*>(a.P)[lane];
     Ctrl* C = a.ctrl;
     const bool first = a.k == 0;
-    unsigned long long slot0 = kInfBits, slot1 = kInfBits;
-    if (first) {
-        slot0 = a.dts->v[0][lane & (kDtSlots - 1)][0];
-        slot1 = a.dts->v[1][lane & (kDtSlots - 1)][0];
-    }
     const S* in = (const S*)a.in;
     S* out = (S*)a.out;
+    unsigned long long slot0 = kInfBits, slot1 = kInfBits;
     if (a.pingpong) {
-        if (C->step & 1) {
+        // single stage: the step's parity picks the buffers and the step's
+        // slots; the others are being lowered by this launch's atomics
+        const bool odd = C->step & 1;
+        if (odd) {
             in = (const S*)a.out;
             out = (S*)a.in;
         }
+        slot0 = slot1 = a.dts->v[odd][lane & (kDtSlots - 1)][0];
+    } else if (first) {
+        slot0 = a.dts->v[0][lane & (kDtSlots - 1)][0];
+        slot1 = a.dts->v[1][lane & (kDtSlots - 1)][0];
     }
     const S* Hin = SED ? in + 3 * nv : (const S*)a.Hin;
     const S* v0p = (a.k == 0) ? in : (const S*)a.v0;
