@@ -237,15 +237,18 @@ int download_planes(Staging* g, const void* state, double* host, int precision, 
 // r + 0.87 rows per tile, until a run's own latency shows: the hypotenuse of
 // the work and half of the time alone.
 //
-// Half an ensemble (what steps on one stream) is judged alone, a single grid
-// by the product of both.  The constants are fits to sweeps of the height
-// over 40 grids of 256^2 .. 2048^2 cells in both precisions, with and without
-// sediment, alone and beside two others: over these the chosen heights are
-// 0.4 % from the best alone and 4 % beside others, on average.  Against
-// powers of two from 32 down to 2 (at least 8192 tiles, then at least 2048),
-// us a step alone: 700^2 FP64 143 -> 117 (5 rows for 4), 4096^2 2399 -> 2336
-// (24 for 32); ensembles of 2.2 million cells in FP32 214 -> 158 (5 for a
-// fixed 16).
+// The product of both is least for the height chosen: a grid steps alone or
+// beside other runs, half an ensemble beside the other half.  The constants are
+// fits to sweeps of the height over 40 grids of 256^2 .. 2048^2 cells in both
+// precisions, with and without sediment, alone and beside two others: over these
+// the chosen heights are 0.4 % from the best alone and 4 % beside others, on
+// average.  Over ensembles of 0.08 to 8 million cells in two halves, both
+// schemes and precisions, with and without sediment, at rest and in motion, they
+// are 2 % from the best on average and 11 % at most (by the time alone 6 % and
+// 28 %: 8 members of 2.2 million cells in FP32, two-stage, 147 us a step for 122
+// with 6 rows).  Against powers of two from 32 down to 2 (at least 8192 tiles,
+// then at least 2048), us a step alone: 700^2 FP64 143 -> 117 (5 rows for 4),
+// 4096^2 2399 -> 2336 (24 for 32).
 int choose_tile_rows(const std::vector<std::pair<int, int>>& grids, bool sed, int precision, int device)
 {
     int cus = 0;
@@ -269,7 +272,7 @@ int choose_tile_rows(const std::vector<std::pair<int, int>>& grids, bool sed, in
             rounds = hard + (steady - hard) * blur;
         }
         const double alone = (r + 0.6) * (rounds + 0.4);
-        const double cost = grids.size() > 1 ? alone : alone * std::hypot(n / simds * (r + 0.87), 0.5 * alone);
+        const double cost = alone * std::hypot(n / simds * (r + 0.87), 0.5 * alone);
         if (cost < best_cost) {
             best = r;
             best_cost = cost;
