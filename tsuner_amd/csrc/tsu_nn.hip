@@ -116,10 +116,10 @@ __device__ __forceinline__ void lds_barrier()
 // loads and stores between barriers) and now, us:
 //            8->32  32->32  32->4  8->64  64->64  64->4, and the data
 //   32 images  41     89     48    106     200     95    gradients 4<-32 60,
-//   of 256^2   27     49     40     71     150     68    32<-32 103, 4<-64 181,
-//   8 images   14     25     14     28      55     27    64<-64 259 -> 53, 80,
-//              10     17     11     15      42     20    126, 181 (32 images)
-// 32 -> 32 moves 268 MB in 49 us, 5.5 TB/s of the copy kernel's 6.1.  Accumulation
+//   of 256^2   27     50     30     68     140     62    32<-32 103, 4<-64 181,
+//   8 images   14     25     14     28      55     27    64<-64 259 -> 54, 79,
+//               9     16     11     15      36     18    123, 175 (32 images)
+// 32 -> 32 moves 268 MB in 50 us, 5.4 TB/s of the copy kernel's 6.1.  Accumulation
 // order and results are those of one tap after the other.
 //
 // LDS: the ring is three blocks of a pass's rows and copies of its first two
@@ -175,21 +175,6 @@ __attribute__((amdgpu_waves_per_eu(conv_waves<K>(), conv_waves<K>()))) void conv
     const int seg = wv & 3, mg = (wv >> 2) % MG, rg = (wv >> 2) / MG;
     StripWalk walk(N, H, W, R);
 
-    // weights: step (offset ry, rx; 32 channels kk) of input offset (ry - 1,
-    // rx - 1), tap 3 ry + rx, or its opposite for the data gradients.  With 8
-    // channels a step holds four offsets, one per lane group.
-    bf16x8 A[STEPS][MTW];
-#pragma unroll
-    for (int s = 0; s < STEPS; s++)
-#pragma unroll
-        for (int a = 0; a < MTW; a++) {
-            const int o = K == 8 ? 4 * s + g : s / KK, k = K == 8 ? 0 : 32 * (s % KK) + 8 * g;
-            const int t = SIGN > 0 ? o : 8 - o;
-            const int m = 16 * MTW * mg + (MTW == 2 ? 8 * (li >> 2) + 4 * a + (li & 3) : li);
-            uint4 v = make_uint4(0, 0, 0, 0);
-            if (o < 9) v = *(const uint4*)(Wt + ((size_t)(t * M + m) * K + k));
-            A[s][a] = as_bf16x8(v);
-        }
     const int m0 = 16 * MTW * mg + 4 * MTW * g;             // this lane's 4 MTW consecutive output channels
     // of which MOUT = 4 has those of the first lane group only: the caller's
     // bias ends there
@@ -238,17 +223,20 @@ __attribute__((amdgpu_waves_per_eu(conv_waves<K>(), conv_waves<K>()))) void conv
             if (ph == 2 && erow >= R - 2) ring[-(R - 2) * XROW + eput_at] = estage;
         }
     };
-    // at the top of a stretch or strip: rows r0 - 1 and r0 into ring rows R ph
-    // and R ph + 1
-    auto top = [&](int ph) {
-        for (int idx = tid; idx < 2 * XROW; idx += T) {
-            const int o = idx % KO, c = idx / KO % XCOL, i = idx / XROW;
-            const int gr = walk.r0 - 1 + i, gc = walk.c0 - 1 + c;
-            uint4 v = make_uint4(0, 0, 0, 0);
-            if (gr >= 0 && gr < H && gc >= 0 && gc < W)
-                v = *(const uint4*)(in + (((size_t)walk.n * H + gr) * W + gc) * K + 8 * o);
-            ring[(R * ph + i) * XROW + c * KO + (o ^ octet_xor<K>(c))] = v;
-        }
+    // at the top of a stretch or strip: rows r0 - 1 and r0, which go into ring
+    // rows R ph and R ph + 1
+    constexpr int TOP = 2 * XROW;
+    auto load_top = [&](int idx) {
+        const int o = idx % KO, c = idx / KO % XCOL, i = idx / XROW;
+        const int gr = walk.r0 - 1 + i, gc = walk.c0 - 1 + c;
+        uint4 v = make_uint4(0, 0, 0, 0);
+        if (idx < TOP && gr >= 0 && gr < H && gc >= 0 && gc < W)
+            v = *(const uint4*)(in + (((size_t)walk.n * H + gr) * W + gc) * K + 8 * o);
+        return v;
+    };
+    auto put_top = [&](int ph, int idx, uint4 v) {
+        const int o = idx % KO, c = idx / KO % XCOL, i = idx / XROW;
+        if (idx < TOP) ring[(R * ph + i) * XROW + c * KO + (o ^ octet_xor<K>(c))] = v;
     };
 
     // this lane's reads in the first of the wave's rows: column 16 seg + li +
@@ -263,9 +251,53 @@ __attribute__((amdgpu_waves_per_eu(conv_waves<K>(), conv_waves<K>()))) void conv
             at[rx][kk] = (RW * rg + (K == 8 ? o / 3 : 0)) * XROW + cl * KO + ((K == 8 ? 0 : 4 * kk + g) ^ octet_xor<K>(cl));
         }
 
-    int ph = 0;                                             // ring row of input row r0 - 1, over R
+    // weights: step (offset ry, rx; 32 channels kk) of input offset (ry - 1,
+    // rx - 1), tap 3 ry + rx, or its opposite for the data gradients.  With 8
+    // channels a step holds four offsets, one per lane group.
+    //
+    // Many weights (18 reads of a wave and more) go through the ring, which is
+    // free yet: 16 lanes of a wave's own loads take 16 rows of weights, a cache
+    // line each, and the four waves side by side the same ones.  64 -> 64, an
+    // image of 64^2: 13.5 us so, 7.7 here; 2 images of 256^2 19.7 and 14.0, 32
+    // images 144 and 140 (8 -> 64, an image of 64^2: 4.8 and 5.1).
+    constexpr bool BY_RING = STEPS * MTW >= 18;
+    constexpr int WN = 9 * M * KO, WEIGHTS = (WN + T - 1) / T, TOPS = (TOP + T - 1) / T;
+    static_assert(!BY_RING || WN <= conv_ring(R) * XROW, "the ring holds the weights");
     fetch(H);
-    top(0);
+    uint4 tops[TOPS];
+#pragma unroll
+    for (int j = 0; j < TOPS; j++) tops[j] = load_top(tid + T * j);
+    if constexpr (BY_RING) {
+        uint4 w[WEIGHTS];
+#pragma unroll
+        for (int j = 0; j < WEIGHTS; j++) w[j] = ((const uint4*)Wt)[min(tid + T * j, WN - 1)];
+#pragma unroll
+        for (int j = 0; j < WEIGHTS; j++) {
+            const int idx = tid + T * j, row = idx / KO;    // row: of [tap][output channel]
+            if (idx < WN) ring[row * KO + (idx % KO ^ octet_xor<K>(row))] = w[j];
+        }
+        lds_barrier();
+    }
+    bf16x8 A[STEPS][MTW];
+#pragma unroll
+    for (int s = 0; s < STEPS; s++)
+#pragma unroll
+        for (int a = 0; a < MTW; a++) {
+            const int o = K == 8 ? 4 * s + g : s / KK, k = K == 8 ? 0 : 32 * (s % KK) + 8 * g;
+            const int t = SIGN > 0 ? o : 8 - o;
+            const int m = 16 * MTW * mg + (MTW == 2 ? 8 * (li >> 2) + 4 * a + (li & 3) : li);
+            uint4 v = make_uint4(0, 0, 0, 0);
+            if (BY_RING)
+                v = ring[(t * M + m) * KO + (k / 8 ^ octet_xor<K>(m))];
+            else if (o < 9)
+                v = *(const uint4*)(Wt + ((size_t)(t * M + m) * K + k));
+            A[s][a] = as_bf16x8(v);
+        }
+    if (BY_RING) lds_barrier();
+
+    int ph = 0;                                             // ring row of input row r0 - 1, over R
+#pragma unroll
+    for (int j = 0; j < TOPS; j++) put_top(0, tid + T * j, tops[j]);
     put(0);
     lds_barrier();
     for (;;) {
@@ -373,7 +405,7 @@ __attribute__((amdgpu_waves_per_eu(conv_waves<K>(), conv_waves<K>()))) void conv
         ph = next_ph;
         if (!down) {
             lds_barrier();                                // every wave is done with the rows above
-            top(ph);
+            for (int idx = tid; idx < TOP; idx += T) put_top(ph, idx, load_top(idx));
         }
         lds_barrier();
     }
