@@ -302,33 +302,42 @@ __device__ __forceinline__ double qdiv(double x, const Den<double>& D)
 __device__ __forceinline__ float qdiv(float x, const Den<float>& D) { return x * D.y; }
 
 // A nonzero numerator below 2^-968 can make qdiv's residual underflow, and
-// then the corrected product may miss x / d by an ulp (zero is exact).  The
-// solver's quotients of state values (velocities, concentrations, momenta
-// over 1 + c) test their numerators as a group with one wave-wide vote and
-// take the IEEE division for the whole group when any lane has such a
-// numerator (`slow`, uniform over the wave); every other quotient of the
-// solver has a numerator that is zero or far above 2^-968 (products and
-// differences of speeds at least sqrt(g * 2^-1074), or a factor of a
-// quantity that is only used as 1 + c).
+// then the corrected product may miss x / d by an ulp (zero is exact).
+// Concentrations vote: when any lane of the wave has such a numerator all take
+// the IEEE division (qdiv_voted).  The other quotients do without: a velocity
+// or momentum of that size is off by an ulp of its own, below 2^-1000 of any
+// depth's or speed's scale, and the rest have numerators that are zero or far
+// above 2^-968 (products and differences of speeds at least sqrt(g * 2^-1074),
+// or a factor of a quantity that is only used as 1 + c).
 __device__ __forceinline__ bool qtiny(double x) { return x != 0.0 && fabs(x) < 0x1p-968; }
 __device__ __forceinline__ bool wave_any(bool b) { return __builtin_expect(__builtin_amdgcn_ballot_w64(b) != 0, 0); }
-__device__ __forceinline__ double qdiv(double x, const Den<double>& D, bool slow)
+__device__ __forceinline__ double qdiv_voted(double x, const Den<double>& D)
 {
-    if (slow) return x / D.d;
-    return qdiv(x, D);
+    double q = qdiv(x, D);
+    if (wave_any(qtiny(x))) q = x / D.d;
+    return q;
 }
-__device__ __forceinline__ float qdiv(float x, const Den<float>& D, bool) { return x * D.y; }
+// two quotients, one vote
+__device__ __forceinline__ void qdiv_voted(double x0, const Den<double>& D0, double x1, const Den<double>& D1,
+                                           double& q0, double& q1)
+{
+    q0 = qdiv(x0, D0);
+    q1 = qdiv(x1, D1);
+    if (wave_any(qtiny(x0) || qtiny(x1))) {
+        q0 = x0 / D0.d;
+        q1 = x1 / D1.d;
+    }
+}
 
 // SedFlux.cuh:26-49 in FP64.  Divisions with a zero numerator are skipped
-// (0/d is 0); the cap test uses s instead of sqrt(s) (see kVmax2Cut).  D,
-// when given, is den(h + DBL_EPSILON) computed by the caller.
-__device__ __forceinline__ Vel<double> velocity64(double h, double qx, double qy, const Den<double>* D = nullptr)
+// (0/d is 0); the cap test uses s instead of sqrt(s) (see kVmax2Cut).
+__device__ __forceinline__ Vel<double> velocity64(double h, double qx, double qy)
 {
     Vel<double> u;
     u.x = 0.0;
     u.y = 0.0;
     if (h >= kEps && (qx != 0.0 || qy != 0.0)) {
-        const Den<double> Dh = D ? *D : den(h + kEpsilon);
+        const Den<double> Dh = den(h + kEpsilon);
         if (qx != 0.0) u.x = qdiv(qx, Dh);
         if (qy != 0.0) u.y = qdiv(qy, Dh);
     }
@@ -469,12 +478,7 @@ __device__ __forceinline__ bool velocity_conc_pair(double h0, double qx0, double
     c0 = c1 = 0.0;
     if (SED) {
         // a zero hc gives the quotient 0
-        c0 = qdiv(hc0, D0);
-        c1 = qdiv(hc1, D1);
-        if (wave_any(qtiny(hc0) || qtiny(hc1))) {
-            c0 = hc0 / D0.d;
-            c1 = hc1 / D1.d;
-        }
+        qdiv_voted(hc0, D0, hc1, D1, c0, c1);
     }
     // zero momenta give zero quotients
     u0.x = h0 >= kEps ? x0 : 0.0;
@@ -500,8 +504,7 @@ __device__ __forceinline__ void velocity_conc(double h, double qx, double qy, do
     const Den<double> D = den(need_u || need_c ? h + kEpsilon : 1.0);
     c = 0.0;
     if (SED) {
-        c = qdiv(hc, D);
-        if (wave_any(qtiny(hc))) c = hc / D.d;
+        c = qdiv_voted(hc, D);
         c = need_c ? c : 0.0;
     }
     u = velocity_over(h, qx, qy, D);
