@@ -255,12 +255,13 @@ __attribute__((amdgpu_waves_per_eu(conv_waves<K>(), conv_waves<K>()))) void conv
     // rx - 1), tap 3 ry + rx, or its opposite for the data gradients.  With 8
     // channels a step holds four offsets, one per lane group.
     //
-    // Many weights (18 reads of a wave and more) go through the ring, which is
-    // free yet: 16 lanes of a wave's own loads take 16 rows of weights, a cache
-    // line each, and the four waves side by side the same ones.  64 -> 64, an
-    // image of 64^2: 13.5 us so, 7.7 here; 2 images of 256^2 19.7 and 14.0, 32
-    // images 144 and 140 (8 -> 64, an image of 64^2: 4.8 and 5.1).
-    constexpr bool BY_RING = STEPS * MTW >= 18;
+    // The weights of 64 input channels go through the ring, which is free yet: 16
+    // lanes of a wave's own loads take 16 rows of weights, a cache line each, and
+    // the four waves side by side the same ones.  64 -> 64, an image of 64^2: 13.5
+    // us so, 7.7 here; 2 images of 256^2 19.7 and 14.0, 32 images 144 and 140.
+    // With fewer channels the loads wait less than two more barriers take (32 ->
+    // 32, an image of 64^2 4.3 and 4.7 us; training, 8 images, 193.5 and 196.6).
+    constexpr bool BY_RING = K == 64;
     constexpr int WN = 9 * M * KO, WEIGHTS = (WN + T - 1) / T, TOPS = (TOP + T - 1) / T;
     static_assert(!BY_RING || WN <= conv_ring(R) * XROW, "the ring holds the weights");
     fetch(H);
