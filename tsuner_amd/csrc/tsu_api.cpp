@@ -353,7 +353,10 @@ size_t planes_of(const tsu_state* st) { return st->precision == TSU_FP64 ? 5 : 8
 // 26.9 -> 16.3 and 12.1 -> 7.4, 160^2 28.5 -> 20.9 and 12.7 -> 10.5, past the
 // line 200^2 28.8 -> 26.8 and 14.0 -> 14.6, 320^2 40 -> 48 and 26.8 -> 30.9;
 // FP32 100^2 21.1 -> 14.1 and 9.0 -> 6.6, 240 x 256 23.3 -> 18.0 and 10.2 ->
-// 10.4, past it 320^2 24.1 -> 27.2 and 12.4 -> 15.8.
+// 10.4, past it 320^2 24.1 -> 27.2 and 12.4 -> 15.8.  Without sediment, and
+// single-stage, the kernels hold more waves but there is as little left to gain at
+// the line: FP64 100^2 18.9 -> 12.8 and 10.8 -> 8.0, 180 x 200 19.8 -> 18.9 and
+// 11.4 -> 10.6, single-stage 13.6 -> 13.4 and 8.2 -> 8.1.
 bool split_rows(const tsu_state* st)
 {
     int cus = 0;
