@@ -38,9 +38,9 @@ HBM_PEAK_GBS = 8000.0
 # TRAFFIC_PROFILE.  None at other sizes.  The stage kernels' work depends on
 # the state (waves at rest skip quotients and Riemann solves), their HBM
 # traffic does not.
-TRAFFIC_8192 = {"fp64": 7.203e9, "fp32": 5.810e9}
+TRAFFIC_8192 = {"fp64": 7.198e9, "fp32": 5.818e9}
 TRAFFIC_PROFILE = "profiles/stage_kernel_8192_counters.md"
-PROFILE_BUILD = "593c74d"
+PROFILE_BUILD = "2b098d2"
 METRIC = "cell-updates/s at 8192² FP64 vs FP32; ensemble sims/hr coarse+NN vs fine"
 
 
@@ -227,8 +227,8 @@ ENSEMBLE_SIDES = (256, 384, 512, 768, 1024)
 def run_ensemble(members, steps, seed=2024, chunk=50):
     """Fine-grid ensemble: `members` Gaussian-source scenarios with sides drawn
     uniformly from ENSEMBLE_SIDES (dx = 10 m), FP32 state, tile heights
-    autotuned per grid-size class, every member advanced `steps` steps by one
-    batched stage launch per RK stage replayed from HIP graphs.  sims/hr =
+    autotuned per grid-size class, every member advanced `steps` steps by batched
+    stage launches (halves of the members side by side) replayed from HIP graphs.  sims/hr =
     members * 3600 / wall seconds of the whole ensemble run."""
     from tsuner_amd import autotune
     from tsuner_amd import scenarios as S

@@ -204,9 +204,11 @@ TSU_API void *tsu_stream(tsu_state *st);
 TSU_API void *tsu_device_state(tsu_state *st);
 
 /* ---- ensembles ------------------------------------------------------------
- * n independent scenarios (grids of any size) advanced together: one launch
- * per RK stage covers every member, each member keeps its own dt and time,
- * and whole-ensemble steps replay from a captured HIP graph.  The reference
+ * n independent scenarios (grids of any size) advanced together: a launch per
+ * RK stage covers half the members, the halves step on two streams (short
+ * calls: one launch for all), each member keeps its own dt and time, and
+ * whole-ensemble steps replay from captured HIP graphs.  Work enqueued on the
+ * ensemble's stream after a call follows both halves.  The reference
  * runs one scenario per TSUNER() call (GPU/main_TSUNER.cu:21-222); members
  * here follow the same arithmetic.  params and scheme are arrays of n; all
  * members share the RK order.  A member with an inflow side takes its own

@@ -75,7 +75,8 @@ struct BatchPools {
     double* ext;
     const DevParams* P;   // one per member
 };
-// Ensemble: one launch over all tiles of all members (tiles[i] = member, tile).
+// Ensemble: one launch over the tiles of half the members or of all (tiles[i] =
+// member, tile).
 // fast_bed: every member's run constants satisfy fast_bedload.
 hipError_t launch_stage_batch(const BatchPools& pools, const BatchMember* mem, const int2* tiles, int ntiles, int k,
                               int last, bool sed, int precision, hipStream_t s, bool fast_bed = false);

@@ -1043,10 +1043,10 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int tile)
 }
 
 // Waves per SIMD the register allocation targets.  Measured on the 8192^2
-// bench: FP32 at 3 waves (168 VGPRs, a few spilled) runs 24% faster than at
-// 2; 4 waves spill 39 VGPRs and lose.  FP64 with sediment needs 245-255
-// VGPRs; at 3 waves it spills 79 or more and runs at half speed, so it stays
-// at 2.  FP64 without sediment fits 168 VGPRs, i.e. 3 waves, unspilled.
+// bench: FP32 at 3 waves (166 VGPRs now) runs 24% faster than at 2; 4 waves
+// spill 39 VGPRs and lose.  FP64 with sediment takes 231-235 VGPRs; at 3 waves
+// it spilled 79 or more and ran at half speed, so it stays at 2.  FP64 without
+// sediment takes 157 VGPRs, i.e. 3 waves.
 #ifndef TSU_WAVES_FP64
 #define TSU_WAVES_FP64 2
 #endif
@@ -1062,7 +1062,7 @@ constexpr int stage_waves()
     return sizeof(R) == 4 ? TSU_WAVES_FP32 : (SED ? TSU_WAVES_FP64 : TSU_WAVES_FP64_NOSED);
 }
 
-// 130 VGPRs in FP64 with sediment, 92 to 112 otherwise: nothing spills.
+// 138 VGPRs in FP64 with sediment, 116 to 128 otherwise: nothing spills.
 template <typename R, bool SED>
 constexpr int split_waves()
 {
@@ -1083,9 +1083,9 @@ void stage_split_kernel(StageArgs a)
     stage_body<R, S, SED, FB, true>(a, xcd_tile(blockIdx.x, gridDim.x));
 }
 
-// Ensemble: one launch covers every tile of every scenario.  tiles[b] =
-// (scenario, tile within the scenario); scen[s] holds that scenario's
-// buffers, constants and step-control block.
+// Ensemble: one launch covers every tile of half the scenarios or of all.
+// tiles[b] = (scenario, tile within the scenario); mem[s] holds that scenario's
+// place in the pools, its sizes and its half.
 template <typename R, typename S, bool SED, bool FB = false>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(stage_waves<R, SED>(), stage_waves<R, SED>())))
 void stage_kernel_batch(BatchPools pools, const BatchMember* __restrict__ mem, const int2* __restrict__ tiles, int k,

@@ -433,7 +433,7 @@ __attribute__((amdgpu_waves_per_eu(conv_waves<K>(), conv_waves<K>()))) void conv
 // kWgradWaves = 256 of them cover the chip.
 //
 // Measured, 8 images of 256^2, before and now (gradient + reduction):
-//   64 -> 64  220 + 112 us -> 50 + 7 us (770 TFLOP/s; both tensors once are
+//   64 -> 64  220 + 112 us -> 49 + 7 us (790 TFLOP/s; both tensors once are
 //             134 MB, 22 us at the copy kernel's 6.1 TB/s, the MFMAs 15 us at
 //             peak, the transposing reads 17 us of LDS time)
 //   32 -> 32  109 + 110 us -> 21 + 4 us (67 MB, 11 us)

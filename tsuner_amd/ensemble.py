@@ -1,8 +1,9 @@
 """Ensembles of scenarios on uneven grids, advanced together on one GPU.
 
-``Ensemble`` wraps a ``tsu_ensemble`` handle: one stage launch per RK stage
-covers every tile of every member, each member keeps its own dt and time,
-and steps replay from a captured HIP graph.
+``Ensemble`` wraps a ``tsu_ensemble`` handle: a stage launch covers every tile
+of half the members, and the halves step side by side (short calls: every
+member in one launch); each member keeps its own dt and time, and steps replay
+from captured HIP graphs.
 """
 from __future__ import annotations
 
